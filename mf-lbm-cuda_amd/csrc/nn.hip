@@ -16,6 +16,7 @@
 // Weights are kept as W[n][k] with n padded to 16 and k to 32 (zero padding), fp32 master
 // copy plus a bf16 copy for the MFMA operands.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstdint>
 #include <mutex>
 
@@ -25,127 +26,376 @@
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float bf2f(__bf16 v) { return (float)v; }
+
+// Workgroup barrier for data exchanged through LDS only: unlike __syncthreads() it leaves the
+// loads from memory in flight.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 struct Grid3 {
     int D, H, W;
 };
 
+// 16-byte load through a buffer descriptor: a lane past the descriptor's bytes reads zeros, so
+// the zero padding of a convolution costs no select (num = 0 for a whole plane outside the
+// grid, NOWHERE as the offset of a single lane).  Descriptors address less than 2^31 bytes.
+constexpr uint32_t NOWHERE = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t num) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)num, 0x00027000);
+}
+__device__ __forceinline__ bf16x8 buffer_load16(__amdgpu_buffer_rsrc_t rsrc, uint32_t offset, uint32_t uniform_offset) {
+    return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)offset, (int)uniform_offset, 0));
+}
+
 // Taps: 0..26, x fastest (dx = tap % 3 - 1, dy = tap / 3 % 3 - 1, dz = tap / 9 - 1); a tap
 // outside the grid reads zero (zero padding).
 
-// Forward / data-gradient convolution.  One wave: MT x 16 voxels x NT*16 output channels,
-// the 16-channel tiles blockIdx.y * NT .. + NT - 1 (small grids split the channels over
-// blocks); the MT voxel tiles share each weight load.
-// Epilogue: + bias (if given), then either ReLU, or a multiply by the ReLU mask of `gate`
-// (the data gradient of a layer whose input came through a ReLU), stored as bf16 and/or fp32.
-template <int NT, int MT>
-__global__ __launch_bounds__(256) void k_conv3(const __bf16* __restrict__ X, const __bf16* __restrict__ Wb,
-                                               const float* __restrict__ bias, const __bf16* __restrict__ gate,
-                                               Grid3 g, int cin, int kp, int cout, int relu,
-                                               __bf16* __restrict__ yb, float* __restrict__ yf) {
-    const int M = g.D * g.H * g.W;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int m0 = (blockIdx.x * 4 + wave) * 16 * MT;
-    if (m0 >= M) return;
+// Exact quotients by a divisor fixed over a launch, without a branch: n / d =
+// umulhi(n, ceil(2^32 / d)) while n * d < 2^32 (the launchers check it); d = 1 passes n through
+// the mask.
+struct FastDiv {
+    uint32_t d, mul, one;
+};
+inline FastDiv fast_div(uint32_t d) {
+    return {d, d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u, d > 1 ? 0u : ~0u};
+}
+__device__ __forceinline__ int quot(int n, const FastDiv& f) { return (int)(__umulhi((uint32_t)n, f.mul) + ((uint32_t)n & f.one)); }
+
+// Epilogue of a convolution: bias, then ReLU or the gate, stored as bf16 and/or fp32, for four
+// consecutive channels n .. n + 3 of voxel mm per call.  quad: cout is a multiple of 4 and every
+// pointer is aligned for four values.
+struct Epilogue {
+    const float* bias;
+    const __bf16* gate;
+    __bf16* yb;
+    float* yf;
+    int cout, relu, quad;
+
+    __device__ __forceinline__ f32x4 bias4(int n) const {
+        f32x4 b = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (bias) {
+            if (quad) {
+                if (n < cout) b = *reinterpret_cast<const f32x4*>(bias + n);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (n + j < cout) b[j] = bias[n + j];
+            }
+        }
+        return b;
+    }
+    // the bf16 output of quads: the network's layers
+    template <bool RELU, bool GATE>
+    __device__ __forceinline__ void store_quad(const f32x4& acc, const f32x4& b, int n, int mm) const {
+        if (n >= cout) return;
+        const int64_t at = (int64_t)mm * cout + n;
+        bf16x4 gt, o;
+        if (GATE) gt = *reinterpret_cast<const bf16x4*>(gate + at);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float v = acc[j] + b[j];
+            if (RELU) v = v > 0.f ? v : 0.f;
+            if (GATE && !(bf2f(gt[j]) > 0.f)) v = 0.f;
+            o[j] = (__bf16)v;
+        }
+        *reinterpret_cast<bf16x4*>(yb + at) = o;
+    }
+    __device__ __forceinline__ void store(const f32x4& acc, const f32x4& b, int n, int mm) const {
+        const int64_t at = (int64_t)mm * cout + n;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (n + j >= cout) return;
+            float v = acc[j] + b[j];
+            if (relu) v = v > 0.f ? v : 0.f;
+            if (gate && !(bf2f(gate[at + j]) > 0.f)) v = 0.f;
+            if (yb) yb[at + j] = (__bf16)v;
+            if (yf) yf[at + j] = v;
+        }
+    }
+    // calls put(store) with the store that fits this launch
+    template <class F>
+    __device__ __forceinline__ void each(F&& put) const {
+        if (quad && yb && !yf) {
+            if (gate && relu) put([this](const f32x4& a, const f32x4& b, int n, int mm) { store_quad<true, true>(a, b, n, mm); });
+            else if (gate) put([this](const f32x4& a, const f32x4& b, int n, int mm) { store_quad<false, true>(a, b, n, mm); });
+            else if (relu) put([this](const f32x4& a, const f32x4& b, int n, int mm) { store_quad<true, false>(a, b, n, mm); });
+            else put([this](const f32x4& a, const f32x4& b, int n, int mm) { store_quad<false, false>(a, b, n, mm); });
+        } else if (quad && yf && !yb && !gate && !relu) {
+            put([this](const f32x4& a, const f32x4& b, int n, int mm) {
+                if (n >= cout) return;
+                f32x4 v;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[j] = a[j] + b[j];
+                *reinterpret_cast<f32x4*>(yf + (int64_t)mm * cout + n) = v;
+            });
+        } else {
+            put([this](const f32x4& a, const f32x4& b, int n, int mm) { store(a, b, n, mm); });
+        }
+    }
+};
+
+// Forward / data-gradient convolution on boxes of voxels staged through LDS.  A workgroup of
+// four waves owns tx x ty x tz voxels, numbered x fastest and cut into 16-voxel MFMA tiles,
+// MT of them per wave, and the 16-channel tiles blockIdx.y * NT .. + NT - 1.  It loads its box
+// with a one-voxel halo once, zeros outside the grid, and every tap of every voxel is then an
+// LDS read at the voxel's place plus an offset common to all voxels (s_tab: per 8-channel
+// piece of k).  In LDS a piece is an array over the box's voxels, padded to whole rounds of
+// the banks: a 16-byte read serves 16 lanes at a time, half of them of one k group of the
+// MFMA operand and half of the next, and with even and odd pieces a multiple of 256 bytes
+// apart the 16 neighbours in x meet 16 different bank groups; pairs of pieces are skewed by
+// one unit for the stores.  The weights go through LDS too, four k blocks at a time: each wave
+// loads the operands of one of the four, PF chunks ahead in registers, and all waves read
+// them (loaded by every wave for itself they were the bound: 7-8 TB/s out of L2 at every size).
+// The operands go in as (weights, voxels), so that a lane ends with four consecutive channels
+// of one voxel and stores them as one vector.  Every accumulator sums the k blocks in
+// ascending order, as k_conv3 does.  Measured launch to launch against a wave per one or two
+// tiles that gathered every operand from global memory, in us: 64^3 16 -> 16 channels 28.4 to
+// 11.0, 48 -> 16 73.5 to 25.2; 16^3 192 -> 64 55.5 to 12.7; 8^3 128 -> 128 35.2 to 9.1; 128^3
+// 48 -> 16 555 to 175 (LDS operand reads, 82 us of it, and the load of 2.5 times the input).
+struct ConvTile {
+    int tx, ty, tz, nx, ny;  // box, boxes along x and y
+    int tv, pv;              // voxels of a box; of a loaded box, in whole groups of 16
+    int pu;                  // 16-byte units of one loaded plane
+    FastDiv row, c8, dtx, dty, dnx, dny;  // units of a loaded row, of a voxel; tx, ty, nx, ny
+    FastDiv dboxes;                       // boxes
+};
+
+template <int MT, int NT, int PF>
+__global__ __launch_bounds__(256) void k_conv3_box(const __bf16* __restrict__ X, const __bf16* __restrict__ Wb, Grid3 g,
+                                                   int cin, int kp, int ntw, Epilogue ep, ConvTile t) {
+    // 16 zero bytes, the box, the weights of two chunks, s_tab
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, q = lane >> 4;
-    const int K = 27 * cin;
-    const int tb = blockIdx.y * NT;  // first channel tile of this block
-    // this lane's voxel of each voxel tile and its coordinates (fixed over the k loop)
-    int mv[MT], xv[MT], yv[MT], zv[MT];
+    const int c8 = cin >> 3, K8 = 27 * c8, LX = t.tx + 2, LY = t.ty + 2, LZ = t.tz + 2;
+    auto unit = [&](int ci) { return (ci >> 1) * (2 * t.pv + 1) + (ci & 1) * t.pv; };  // of piece ci, voxel 0
+    unsigned char* s_w = smem + 16 * (1 + (c8 + 1) / 2 * (2 * t.pv + 1));
+    int* s_tab = reinterpret_cast<int*>(s_w + 2 * 4 * NT * 1024);
+    const int nkb = (K8 + 3) >> 2;    // k blocks of 32 = four pieces of 8
+    const int nch = (nkb + 3) >> 2;   // chunks of four k blocks
+    // boxes in launch order, all of them once per channel group (one contiguous run of boxes
+    // per XCD measured up to 6 % slower)
+    int bx, by, bz, tb;
+    {
+        const int grp = quot(blockIdx.x, t.dboxes), b = blockIdx.x - grp * (int)t.dboxes.d, yz = quot(b, t.dnx);
+        tb = grp * NT;
+        bz = quot(yz, t.dny);
+        bx = b - yz * t.nx;
+        by = yz - bz * t.ny;
+    }
+    const int x0 = bx * t.tx, y0 = by * t.ty, z0 = bz * t.tz;
+
+    // first weight operands: in flight while the box loads
+    const __amdgpu_buffer_rsrc_t wbuf = buffer_of(Wb, 32u * ntw * kp);
+    uint32_t wrow[NT];  // byte offset of this lane's operand in this wave's block of chunk 0
+#pragma unroll
+    for (int n = 0; n < NT; ++n) wrow[n] = 2u * ((min(tb + n, ntw - 1) * 16 + r) * kp + 8 * q + 32 * wave);
+    bf16x8 w[PF][NT];
+    auto load_w = [&](int slot, int c) {  // zeros past the last k block
+        const bool in = 4 * c + wave < nkb;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) w[slot][n] = buffer_load16(wbuf, in ? wrow[n] : NOWHERE, 256u * c);
+    };
+    unsigned char* const w_mine = s_w + wave * NT * 1024 + 16 * lane;
+    const unsigned char* const w_all = s_w + 16 * lane;
+    auto keep_w = [&](int slot) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+            *reinterpret_cast<bf16x8*>(w_mine + ((slot & 1) * 4 * NT + n) * 1024) = w[slot][n];
+    };
+#pragma unroll
+    for (int s = 0; s < PF; ++s) load_w(s, s);
+
+    bf16x8 zero;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) zero[j] = (__bf16)0.f;
+    if (tid == 0) *reinterpret_cast<bf16x8*>(smem) = zero;
+    // The box, up to six planes at a time: a thread keeps its place (row, voxel, piece) over the
+    // planes and loads its next place's planes before it stores the present one's.
+    const uint32_t plane = 2u * g.H * g.W * cin;  // bytes
+    constexpr int ZB = 6;
+    for (int lz0 = 0; lz0 < LZ; lz0 += ZB) {
+        bf16x8 v[2][ZB];
+        unsigned char* dst[2];
+        auto fetch = [&](int slot, int i) {
+            const int ly = quot(i, t.row), c = i - ly * (int)t.row.d;
+            const int lx = quot(c, t.c8), ci = c - lx * c8;
+            const int xx = x0 + lx - 1, yy = y0 + ly - 1;
+            const bool in = i < t.pu && xx >= 0 && yy >= 0 && xx < g.W && yy < g.H;
+            const uint32_t src = in ? 2u * ((yy * g.W + xx) * cin + 8 * ci) : NOWHERE;
+            dst[slot] = smem + 16 * (1 + ly * LX + lx + unit(ci));
+#pragma unroll
+            for (int m = 0; m < ZB; ++m) {
+                const int zz = z0 + lz0 + m - 1;
+                const bool zin = lz0 + m < LZ && zz >= 0 && zz < g.D;
+                v[slot][m] = buffer_load16(buffer_of(X + (int64_t)(zin ? zz : 0) * (plane >> 1), zin ? plane : 0u), src, 0);
+            }
+        };
+        auto keep = [&](int slot, int i) {
+            if (i < t.pu) {
+#pragma unroll
+                for (int m = 0; m < ZB; ++m)
+                    if (lz0 + m < LZ) *reinterpret_cast<bf16x8*>(dst[slot] + 16 * (lz0 + m) * LX * LY) = v[slot][m];
+            }
+        };
+        fetch(0, tid);
+        for (int i0 = 0; i0 < t.pu; i0 += 512) {
+            if (i0 + 256 < t.pu) fetch(1, i0 + 256 + tid);
+            keep(0, i0 + tid);
+            if (i0 + 512 < t.pu) fetch(0, i0 + 512 + tid);
+            if (i0 + 256 < t.pu) keep(1, i0 + 256 + tid);
+        }
+    }
+    // byte offsets of the k pieces, -1 past the last tap
+    for (int c = tid; c < 16 * nch + 16; c += 256) {
+        int off = -1;
+        if (c < K8) {
+            const int tap = quot(c, t.c8), ci = c - tap * c8;
+            const int oz = tap / 9, oy = tap / 3 - 3 * oz, ox = tap % 3;
+            off = 16 * ((oz * LY + oy) * LX + ox + unit(ci));
+        }
+        s_tab[c] = off;
+    }
+    // this lane's voxel of each tile: its place in LDS
+    int base[MT];
 #pragma unroll
     for (int u = 0; u < MT; ++u) {
-        mv[u] = m0 + 16 * u + r;
-        xv[u] = mv[u] % g.W;
-        yv[u] = (mv[u] / g.W) % g.H;
-        zv[u] = mv[u] / (g.W * g.H);
+        const int v = min((wave * MT + u) * 16 + r, t.tv - 1);  // past the box: its last voxel, not stored
+        const int yz = quot(v, t.dtx), lx = v - yz * t.tx, lz = quot(yz, t.dty), ly = yz - lz * t.ty;
+        base[u] = 16 * (1 + (lz * LY + ly) * LX + lx);
     }
     f32x4 acc[MT][NT];
 #pragma unroll
     for (int u = 0; u < MT; ++u)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int n = 0; n < NT; ++n) acc[u][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    keep_w(0);
+    lds_barrier();
+
+    // Operands run one k block ahead of the MFMAs and the voxels' offsets two; the scheduling
+    // barriers keep the reads of the next block in front of the MFMAs of this one (left to
+    // itself the compiler makes every MFMA wait for its own read).  An offset is read before
+    // the operands of its block, so that waiting for it waits for none of them.
+    bf16x8 a[2][MT], b[2][NT];
+    auto read_ab = [&](int slot, int half, int s, int off, bool padded) {
+        const int keep = padded ? ~(off >> 31) : ~0;  // past the last tap: the zeros at 0
+#pragma unroll
+        for (int u = 0; u < MT; ++u) a[slot][u] = *reinterpret_cast<const bf16x8*>(smem + ((base[u] + off) & keep));
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+            b[slot][n] = *reinterpret_cast<const bf16x8*>(w_all + ((half * 4 + s) * NT + n) * 1024);
+    };
+    const int* tab = s_tab + q;
+    int off[2] = {tab[4], tab[8]};  // of the next two blocks
+    read_ab(0, 0, 0, tab[0], true);
+    // block s of the chunk whose weights are in `half` of s_w; tab: the chunk's offsets
+    auto block = [&](int half, int s, const int* tab, bool padded) {
+        if (s == 3) lds_barrier();  // the next chunk's weights are written, this one's are read
+        const int next = tab[4 * (s + 3)];
+        read_ab((s + 1) & 1, s == 3 ? half ^ 1 : half, (s + 1) & 3, off[0], padded);
+        off[0] = off[1];
+        off[1] = next;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < MT; ++u)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                acc[u][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s & 1][n], a[s & 1][u], acc[u][n], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    static_assert(PF % 2 == 0, "slot d's chunk goes to half d & 1");
+    int c0 = 0;
+    for (; c0 + PF < nch; c0 += PF, tab += 16 * PF)
+#pragma unroll
+        for (int d = 0; d < PF; ++d) {
+            // slot d held chunk c0 + d, already in LDS; the next chunk goes to the other half
+            load_w(d, c0 + d + PF);
+            keep_w((d + 1) % PF);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) block(d & 1, s, tab + 16 * d, s == 3);  // only the next chunk may be padded
+        }
+#pragma unroll
+    for (int d = 0; d < PF; ++d)  // the ring holds the chunks left
+        if (c0 + d < nch) {
+            keep_w((d + 1) % PF);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) block(d & 1, s, tab + 16 * d, true);
+        }
+    f32x4 bias4[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) bias4[n] = ep.bias4((tb + n) * 16 + 4 * q);
+    ep.each([&](auto&& store) {
+#pragma unroll
+        for (int u = 0; u < MT; ++u) {
+            const int v = (wave * MT + u) * 16 + r;
+            const int yz = quot(v, t.dtx), lz = quot(yz, t.dty);
+            const int xx = x0 + v - yz * t.tx, yy = y0 + yz - lz * t.ty, zz = z0 + lz;
+            if (v >= t.tv || xx >= g.W || yy >= g.H || zz >= g.D) continue;
+            const int mm = (zz * g.H + yy) * g.W + xx;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) store(acc[u][n], bias4[n], (tb + n) * 16 + 4 * q, mm);
+        }
+    });
+}
+
+// The convolution of channel counts whose boxes do not fit LDS (above about 600 input
+// channels): one wave per 16 voxels and 16 output channels (tile blockIdx.y), every tap
+// gathered from global memory.
+__global__ __launch_bounds__(256) void k_conv3(const __bf16* __restrict__ X, const __bf16* __restrict__ Wb, Grid3 g,
+                                               int cin, int kp, Epilogue ep) {
+    const int M = g.D * g.H * g.W;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int m0 = (blockIdx.x * 4 + wave) * 16;
+    if (m0 >= M) return;
+    const int r = lane & 15, q = lane >> 4;
+    const int K = 27 * cin;
+    const int mv = m0 + r, xv = mv % g.W, yv = (mv / g.W) % g.H, zv = mv / (g.W * g.H);
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int kb = 0; kb < kp; kb += 32) {
         const int k = kb + 8 * q;
         const int tap = k < K ? k / cin : 0, ci = k - tap * cin;
         const int ox = tap % 3 - 1, oy = (tap / 3) % 3 - 1, oz = tap / 9 - 1;
-        bf16x8 b[NT];
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(Wb + (int64_t)(blockIdx.y * 16 + r) * kp + k);
+        bf16x8 a;
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
-            b[t] = *reinterpret_cast<const bf16x8*>(Wb + (int64_t)((tb + t) * 16 + r) * kp + k);
-#pragma unroll
-        for (int u = 0; u < MT; ++u) {
-            bf16x8 a;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) a[j] = (__bf16)0.f;
-            const int xx = xv[u] + ox, yy = yv[u] + oy, zz = zv[u] + oz;
-            if (k < K && mv[u] < M && xx >= 0 && yy >= 0 && zz >= 0 && xx < g.W && yy < g.H && zz < g.D)
-                a = *reinterpret_cast<const bf16x8*>(X + (int64_t)((zz * g.H + yy) * g.W + xx) * cin + ci);
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-                acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[t], acc[u][t], 0, 0, 0);
-        }
+        for (int j = 0; j < 8; ++j) a[j] = (__bf16)0.f;
+        const int xx = xv + ox, yy = yv + oy, zz = zv + oz;
+        if (k < K && mv < M && xx >= 0 && yy >= 0 && zz >= 0 && xx < g.W && yy < g.H && zz < g.D)
+            a = *reinterpret_cast<const bf16x8*>(X + (int64_t)((zz * g.H + yy) * g.W + xx) * cin + ci);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, acc, 0, 0, 0);
     }
-#pragma unroll
-    for (int u = 0; u < MT; ++u)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const int n = (tb + t) * 16 + r;
-            if (n >= cout) continue;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int mm = m0 + 16 * u + 4 * q + j;
-                if (mm >= M) continue;
-                float v = acc[u][t][j] + (bias ? bias[n] : 0.f);
-                if (relu) v = v > 0.f ? v : 0.f;
-                if (gate && !(bf2f(gate[(int64_t)mm * cout + n]) > 0.f)) v = 0.f;
-                if (yb) yb[(int64_t)mm * cout + n] = (__bf16)v;
-                if (yf) yf[(int64_t)mm * cout + n] = v;
-            }
-        }
+    const int n = blockIdx.y * 16 + 4 * q;
+    if (mv < M) ep.store(acc, ep.bias4(n), n, mv);
 }
 
-// Weight gradient partials.  Block (kt, nt, chunk): one wave per 16 x 16·KT block of (output
-// channel n, k) over `chunk` voxels, as KT 16 x 16 MFMA tiles that share the dZ operand;
-// writes part[chunk][n][k] (fp32).  The waves of the first k block also sum the dZ values
+// Weight gradient partials where k_conv3_wgrad_rows would hold few voxels at a time (grids
+// more than about 380 voxels wide).  Block (kt, nt, chunk): one wave per 16 x 16 tile of (output
+// channel n, k) over `chunk` voxels; writes part[chunk][n][k] (fp32).  The waves of the first k block also sum the dZ values
 // they load: the bias gradient partials bpart[chunk][n] (n < cout; null: not wanted).
 // Per step of 32 voxels the operands are staged through LDS: lane (v, h) loads 8 channels
-// (16 bytes) of voxel v -- dZ channels n0 + 8h .., and of each tile the 8 columns
-// k0 + 16t + 8h .. (8 consecutive channels of one tap, since cin is a multiple of 8) at the
+// (16 bytes) of voxel v -- dZ channels n0 + 8h .., and the 8 columns k0 + 8h .. (8 consecutive channels of one tap, since cin is a multiple of 8) at the
 // tap's shifted voxel -- and lane (r, q) then reads column r of voxels 8q .. 8q + 7, the
 // MFMA operand layout.
-template <int KT>
 __global__ __launch_bounds__(64) void k_conv3_wgrad(const __bf16* __restrict__ X, const __bf16* __restrict__ dZ,
                                                     Grid3 g, int cin, int kp, int coutp, int cout, int chunk,
                                                     float* __restrict__ part, float* __restrict__ bpart) {
-    __shared__ __attribute__((aligned(16))) __bf16 sA[32][16];
-    __shared__ __attribute__((aligned(16))) __bf16 sB[KT][32][16];
+    __shared__ __attribute__((aligned(16))) __bf16 sA[32][16], sB[32][16];
     const int M = g.D * g.H * g.W;
     const int lane = threadIdx.x;
-    const int k0 = blockIdx.x * 16 * KT, n0 = blockIdx.y * 16, c = blockIdx.z;
+    const int k0 = blockIdx.x * 16, n0 = blockIdx.y * 16, c = blockIdx.z;
     const int r = lane & 15, q = lane >> 4;  // MFMA role: column r, voxels 8q .. 8q + 7
     const int v = lane >> 1, h = lane & 1;   // loader role: voxel v, 8-channel half h
-    const int K = 27 * cin;
     const int n = n0 + r;
     const bool ain = n0 + 8 * h < cout;  // cout is a multiple of 8: the whole half or none
-    int lci[KT], lox[KT], loy[KT], loz[KT], loff[KT];
-    bool lkin[KT];
-#pragma unroll
-    for (int t = 0; t < KT; ++t) {
-        const int kk = k0 + 16 * t + 8 * h;
-        lkin[t] = kk < K;  // K is a multiple of 8: the whole half or none
-        const int tap = lkin[t] ? kk / cin : 0;
-        lci[t] = lkin[t] ? kk - tap * cin : 0;
-        lox[t] = tap % 3 - 1;
-        loy[t] = (tap / 3) % 3 - 1;
-        loz[t] = tap / 9 - 1;
-        loff[t] = (loz[t] * g.H + loy[t]) * g.W + lox[t];
-    }
-    f32x4 acc[KT];
-#pragma unroll
-    for (int t = 0; t < KT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int kk = k0 + 8 * h;
+    const bool lkin = kk < 27 * cin;  // a multiple of 8: the whole half or none
+    const int tap = lkin ? kk / cin : 0, lci = lkin ? kk - tap * cin : 0;
+    const int lox = tap % 3 - 1, loy = (tap / 3) % 3 - 1, loz = tap / 9 - 1;
+    const int loff = (loz * g.H + loy) * g.W + lox;
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
     float bsum = 0.f;  // this lane's dZ values (row n), in voxel order
     const int mb = c * chunk, me = min(M, mb + chunk);
     bf16x8 zero;
@@ -153,32 +403,25 @@ __global__ __launch_bounds__(64) void k_conv3_wgrad(const __bf16* __restrict__ X
     for (int j = 0; j < 8; ++j) zero[j] = (__bf16)0.f;
     for (int ms = mb; ms < me; ms += 32) {
         const int m = ms + v;
-        bf16x8 la = zero;
+        bf16x8 la = zero, lb = zero;
         if (m < me && ain) la = *reinterpret_cast<const bf16x8*>(dZ + (int64_t)m * cout + n0 + 8 * h);
         *reinterpret_cast<bf16x8*>(&sA[v][8 * h]) = la;
-        const int x = m % g.W, y = (m / g.W) % g.H, z = m / (g.W * g.H);
-#pragma unroll
-        for (int t = 0; t < KT; ++t) {
-            const int xx = x + lox[t], yy = y + loy[t], zz = z + loz[t];
-            const bool in = m < me && lkin[t] && xx >= 0 && yy >= 0 && zz >= 0 && xx < g.W && yy < g.H && zz < g.D;
-            bf16x8 lb = zero;
-            if (in) lb = *reinterpret_cast<const bf16x8*>(X + (int64_t)(m + loff[t]) * cin + lci[t]);
-            *reinterpret_cast<bf16x8*>(&sB[t][v][8 * h]) = lb;
-        }
+        const int xx = m % g.W + lox, yy = (m / g.W) % g.H + loy, zz = m / (g.W * g.H) + loz;
+        const bool in = m < me && lkin && xx >= 0 && yy >= 0 && zz >= 0 && xx < g.W && yy < g.H && zz < g.D;
+        if (in) lb = *reinterpret_cast<const bf16x8*>(X + (int64_t)(m + loff) * cin + lci);
+        *reinterpret_cast<bf16x8*>(&sB[v][8 * h]) = lb;
         __syncthreads();
-        bf16x8 a, b[KT];
+        bf16x8 a, b;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             a[j] = sA[8 * q + j][r];
-#pragma unroll
-            for (int t = 0; t < KT; ++t) b[t][j] = sB[t][8 * q + j][r];
+            b[j] = sB[8 * q + j][r];
         }
         if (bpart && k0 == 0) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) bsum += bf2f(a[j]);
         }
-#pragma unroll
-        for (int t = 0; t < KT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[t], acc[t], 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
         __syncthreads();
     }
     if (bpart && k0 == 0) {
@@ -187,11 +430,228 @@ __global__ __launch_bounds__(64) void k_conv3_wgrad(const __bf16* __restrict__ X
         const float s2 = s1 + __shfl_xor(s1, 32);
         if (q == 0 && n < cout) bpart[(int64_t)c * cout + n] = s2;
     }
-    // tile t: D[row = n0 + 4q + j][col = k0 + 16t + r]
+    // D[row = n0 + 4q + j][col = k0 + r]
 #pragma unroll
-    for (int t = 0; t < KT; ++t)
+    for (int j = 0; j < 4; ++j) part[((int64_t)c * coutp + n0 + 4 * q + j) * kp + k0 + r] = acc[j];
+}
+
+// Weight gradient partials with the operands shared through LDS.  A workgroup owns one chunk of
+// voxels, one plane offset dz of the taps, a slice of 16 input channels (HALF: the last 8 of an
+// odd multiple of 8) and NN 16-channel tiles of the output; its three waves take the three row
+// offsets dy, so that a wave accumulates the three taps of a row (NN x 3 MFMA tiles, NN x 2
+// with two 8-channel taps to a tile).  Up to `sub` voxels at a time, it loads the rows that
+// these voxels' taps reach once, padded by a zero voxel at each end and a zero row above and
+// below each plane, and the voxels' dZ; s_pos holds each voxel's place among the rows, from
+// which every tap is a fixed distance.  The MFMA operands hold eight voxels of one channel per
+// lane: the transposing LDS read (four 16-bit rows per 16 lanes) delivers them from the
+// channels-last rows.  Gathered per tap from global memory and transposed by eight 2-byte LDS
+// reads per operand (k_conv3_wgrad, one wave per tile) the same sums were bound by those reads
+// and by 27-fold loads of the input.  Every accumulator adds the voxel blocks of a chunk in
+// ascending order, as k_conv3_wgrad does.  Measured with the chunk sums against one wave per 16
+// or 32 columns, in us: 64^3 16 -> 16 channels 82.7 to 29.7, 48 -> 16 127 to 61; 32^3 96 -> 32 72
+// to 34.6; 128^3 16 -> 16 317 to 150.  At 64^3 the 64 dependent blocks of a chunk and its four
+// stages of loads bound it, at 128^3 the vector instructions of the staging.
+struct WgradRows {
+    int ci0, sub;        // first channel, voxels staged at a time
+    int lds_dz, lds_pos; // byte offsets of the staged dZ and of s_pos
+    FastDiv row, h2, w, h;  // 16-byte units of a padded row; H + 2, W, H
+};
+
+__device__ __forceinline__ bf16x4 read_transposed(const unsigned char* lds) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                          (__attribute__((address_space(3))) s16x4*)const_cast<unsigned char*>(lds)));
+}
+
+template <int NN, bool HALF>
+__global__ __launch_bounds__(192) void k_conv3_wgrad_rows(const __bf16* __restrict__ X, const __bf16* __restrict__ dZ,
+                                                          Grid3 g, int cin, int kp, int coutp, int cout, int chunk,
+                                                          WgradRows t, float* __restrict__ part,
+                                                          float* __restrict__ bpart) {
+    // 128 zero bytes, the padded rows, the voxels' dZ, the voxels' places
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    constexpr int VB = HALF ? 16 : 32, PU = VB / 16;  // bytes and units of a voxel
+    constexpr int NT = HALF ? 2 : 3;                  // MFMA column tiles of a wave
+    int* s_pos = reinterpret_cast<int*>(smem + t.lds_pos);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int slice = blockIdx.x / 3, dzi = blockIdx.x - 3 * slice, ci0 = t.ci0 + 16 * slice;
+    const int n0 = blockIdx.y * 16 * NN, c = blockIdx.z;
+    const int M = g.D * g.H * g.W, mb = c * chunk, me = min(M, mb + chunk);
+    const int WP = g.W + 2;
+    const bool first = blockIdx.x == 0 && t.ci0 == 0;
+    const bool bias = bpart && first && wave == 0;
+    // this lane's part of the operand reads: voxel r / 4 of four, channels 4 (r % 4) ..; with two
+    // taps to a tile the upper quarters read the next voxel of the row (the tile past the third
+    // tap is not stored)
+    const int lane_off = HALF ? ((r >> 1) & 1) * VB + (r & 1) * 8 : (r & 3) * 8;
+    const int tap_off = ((wave - 1) * WP - 1) * VB + lane_off;  // of the row's first tap from the voxel
+    constexpr int TSTEP = HALF ? 2 * VB : VB;                   // from one column tile to the next
+    f32x4 acc[NN][NT];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) part[((int64_t)c * coutp + n0 + 4 * q + j) * kp + k0 + 16 * t + r] = acc[t][j];
+    for (int n = 0; n < NN; ++n)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) acc[n][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float bsum[NN];
+#pragma unroll
+    for (int n = 0; n < NN; ++n) bsum[n] = 0.f;
+    bf16x8 zero;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) zero[j] = (__bf16)0.f;
+    if (tid < 8) *reinterpret_cast<bf16x8*>(smem + 16 * tid) = zero;
+
+    // One stage: the padded rows and the dZ of voxels s0 .. e - 1.  The first PX and PD units of
+    // a thread are loaded into registers while the stage before is computed; wider rows load
+    // the rest when it is stored.
+    constexpr int PX = 10, PD = 6;
+    bf16x8 vx[PX], vd[PD];
+    int s0, e, xa, ya, za, units, vox, dunits;
+    auto stage = [&](int from) {
+        s0 = from;
+        e = min(me, s0 + t.sub);
+        const int ra = s0 / g.W, rb = (e - 1) / g.W, zb = rb / g.H;
+        za = ra / g.H;
+        xa = s0 - ra * g.W;
+        ya = ra - za * g.H;
+        units = (rb - ra + 2 * (zb - za) + 3) * WP * PU;
+        vox = (e - s0 + 31) & ~31;
+        dunits = vox * NN * 2;
+    };
+    // unit i of the padded rows: its row, and its byte offset in a row of the input (NOWHERE for
+    // the padding); fixed over the stages
+    auto place = [&](int i, int& row, uint32_t& col) {
+        row = quot(i, t.row);
+        const int u = i - row * WP * PU, x = u / PU - 1;
+        col = x >= 0 && x < g.W ? 2u * (x * cin + ci0 + 8 * (u % PU)) : NOWHERE;
+    };
+    const __amdgpu_buffer_rsrc_t xbuf = buffer_of(X, 2u * M * cin), dbuf = buffer_of(dZ, 2u * M * cout);
+    auto row_unit = [&](int i, int row, uint32_t col) {
+        const int yp = ya + row, zo = quot(yp, t.h2), y = yp - zo * (g.H + 2) - 1, z = za + zo + dzi - 1;
+        const uint32_t from = __umul24(__umul24(z, g.H) + y, 2u * g.W * cin) + col;
+        return buffer_load16(xbuf, i < units && (unsigned)y < (unsigned)g.H && (unsigned)z < (unsigned)g.D ? from : NOWHERE, 0);
+    };
+    auto dz_unit = [&](int i) {
+        const int mv = s0 + i / (2 * NN), n = n0 + 8 * (i % (2 * NN));
+        return buffer_load16(dbuf, mv < e && n < cout ? 2u * (mv * cout + n) : NOWHERE, 0);
+    };
+    int prow[PX];
+    uint32_t pcol[PX];
+#pragma unroll
+    for (int m = 0; m < PX; ++m) place(tid + 192 * m, prow[m], pcol[m]);
+    auto fetch = [&]() {
+#pragma unroll
+        for (int m = 0; m < PX; ++m) vx[m] = row_unit(tid + 192 * m, prow[m], pcol[m]);
+#pragma unroll
+        for (int m = 0; m < PD; ++m) vd[m] = dz_unit(tid + 192 * m);
+    };
+    auto keep = [&]() {
+        bf16x8 *rows = reinterpret_cast<bf16x8*>(smem + 128), *ds = reinterpret_cast<bf16x8*>(smem + t.lds_dz);
+#pragma unroll
+        for (int m = 0; m < PX; ++m)
+            if (tid + 192 * m < units) rows[tid + 192 * m] = vx[m];
+#pragma unroll
+        for (int m = 0; m < PD; ++m)
+            if (tid + 192 * m < dunits) ds[tid + 192 * m] = vd[m];
+        for (int i = tid + 192 * PX; i < units; i += 192) {
+            int row;
+            uint32_t col;
+            place(i, row, col);
+            rows[i] = row_unit(i, row, col);
+        }
+        for (int i = tid + 192 * PD; i < dunits; i += 192) ds[i] = dz_unit(i);
+        for (int v = tid; v < vox; v += 192) {
+            const int row = quot(xa + v, t.w), zo = quot(ya + row, t.h);  // rows and planes below voxel s0's
+            s_pos[v] = s0 + v < e ? 128 + ((row + 2 * zo + 1) * WP + xa + v - row * g.W + 1) * VB : -1;
+        }
+    };
+    const int v0 = 8 * q + (r >> 2);  // and v0 + 4: the voxels this lane reads for its group
+    bf16x8 a[2][NN], b[2][NT];
+    const unsigned char* const dz_lane = smem + t.lds_dz + v0 * NN * 32 + (r & 3) * 8;
+    auto read_ab = [&](int slot, int ms, int p0, int p1) {
+        const unsigned char* d = dz_lane + ms * NN * 32;
+#pragma unroll
+        for (int n = 0; n < NN; ++n) {
+            const bf16x4 lo = read_transposed(d + n * 32), hi = read_transposed(d + (4 * NN + n) * 32);
+            a[slot][n] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+        // a voxel past the grid reads the zeros at 0
+        const unsigned char *x0 = smem + (p0 >= 0 ? p0 + tap_off : lane_off), *x1 = smem + (p1 >= 0 ? p1 + tap_off : lane_off);
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const bf16x4 lo = read_transposed(x0 + u * TSTEP), hi = read_transposed(x1 + u * TSTEP);
+            b[slot][u] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+    };
+    stage(mb);
+    fetch();
+    for (;;) {
+        keep();
+        __syncthreads();
+        const int blocks = vox >> 5;
+        const bool more = e < me;
+        if (more) {
+            stage(e);
+            fetch();
+        }
+        // operands run one block of 32 voxels ahead of the MFMAs, places two
+        const int* pos = s_pos + v0;
+        int p0 = pos[0], p1 = pos[4];
+        read_ab(0, 0, p0, p1);
+        p0 = blocks > 1 ? pos[32] : -1;
+        p1 = blocks > 1 ? pos[36] : -1;
+        auto block = [&](int slot, int i) {
+            const int n0_ = p0, n1_ = p1;
+            const int at = min(i + 2, blocks - 1) * 32;
+            p0 = pos[at];
+            p1 = pos[at + 4];
+            read_ab(slot ^ 1, min(i + 1, blocks - 1) * 32, n0_, n1_);
+            __builtin_amdgcn_sched_barrier(0);
+            if (bias) {
+#pragma unroll
+                for (int n = 0; n < NN; ++n)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) bsum[n] += bf2f(a[slot][n][j]);
+            }
+#pragma unroll
+            for (int n = 0; n < NN; ++n)
+#pragma unroll
+                for (int u = 0; u < NT; ++u)
+                    acc[n][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[slot][n], b[slot][u], acc[n][u], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        for (int i = 0; i < blocks; i += 2) {
+            block(0, i);
+            if (i + 1 < blocks) block(1, i + 1);
+        }
+        if (!more) break;
+        lds_barrier();  // every wave is done with the stage; the loads of the next stay in flight
+    }
+#pragma unroll
+    for (int n = 0; n < NN; ++n) {
+        const int row0 = n0 + 16 * n;
+        if (row0 >= coutp) break;
+        if (bias) {
+            // lanes r, r + 16, r + 32, r + 48 hold row r: fixed pairing order
+            const float s1 = bsum[n] + __shfl_xor(bsum[n], 16);
+            const float s2 = s1 + __shfl_xor(s1, 32);
+            if (q == 0 && row0 + r < cout) bpart[(int64_t)c * cout + row0 + r] = s2;
+        }
+        // column r of tile u: its tap's channel
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const int dx = HALF ? 2 * u + (r >> 3) : u;
+            if (dx > 2) continue;
+            const int k = ((dzi * 3 + wave) * 3 + dx) * cin + ci0 + (HALF ? r & 7 : r);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) part[((int64_t)c * coutp + row0 + 4 * q + j) * kp + k] = acc[n][u][j];
+        }
+        // the padding columns
+        if (first)
+            for (int i = tid; i < 16 * (kp - 27 * cin); i += 192) {
+                const int pad = kp - 27 * cin, row = i / pad;
+                part[((int64_t)c * coutp + row0 + row) * kp + 27 * cin + i - row * pad] = 0.f;
+            }
+    }
 }
 
 // dW[i] (+)= sum over chunks of part[chunk][i], i < n, and in the blocks after those,
@@ -357,6 +817,113 @@ __global__ void k_adam(float* __restrict__ w, const float* __restrict__ g, float
 
 inline unsigned nblk(int64_t n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
+// Channel tiles a wave may hold beside mt voxel tiles (registers).
+inline int conv_max_nt(int mt) { return mt >= 8 ? 2 : mt >= 4 ? 3 : 4; }
+
+// Box and tile counts of one k_conv3_box launch.
+struct ConvPlan {
+    ConvTile t;
+    int mt, nt;
+    size_t lds;
+    unsigned boxes;
+};
+
+// Box of a convolution: the equal splits of the axes with rows of up to 32 voxels are priced in
+// cycles of a CU -- one per loaded 16-byte unit, the weights' 64 per channel tile and k block
+// among them; per k block its MFMAs (16 each, a wave on each SIMD) and its operand reads (4 per
+// wave and operand), at least the 70 of one block's dependent chain for a workgroup alone on
+// its CU; load and MFMAs of two workgroups overlap where LDS holds both; whole rounds over the
+// 256 CUs.
+bool conv_plan(const Grid3& g, int cin, int ntw, ConvPlan& best) {
+    const int c8 = cin / 8;
+    const int nkb = (27 * c8 + 3) / 4;
+    const size_t tab = (size_t)((nkb + 3) / 4 * 16 + 16) * 4;
+    constexpr size_t LDS_MAX = 160 * 1024;
+    double best_cost = 0.0;
+    bool found = false;
+    auto parts = [](int n, int lo, int hi, int* out, int cap) {  // distinct ceil(n / p) in [lo, hi]
+        int cnt = 0;
+        for (int p = (n + hi - 1) / hi; p <= n && cnt < cap; ++p) {
+            const int v = (n + p - 1) / p;
+            if (v < lo && cnt) break;
+            if (cnt && out[cnt - 1] == v) continue;
+            out[cnt++] = v;
+        }
+        return cnt;
+    };
+    int xs[6], ys[8], zs[6];
+    const int nxs = parts(g.W, 4, 32, xs, 6), nys = parts(g.H, 1, 8, ys, 8), nzs = parts(g.D, 1, 8, zs, 6);
+    for (int a = 0; a < nxs; ++a)
+        for (int b = 0; b < nys; ++b)
+            for (int c = 0; c < nzs; ++c) {
+                const int tx = xs[a], ty = ys[b], tz = zs[c], tv = tx * ty * tz;
+                if (tv > 512) continue;
+                const int mt = tv > 256 ? 8 : tv > 128 ? 4 : tv > 64 ? 2 : 1;
+                const int64_t loaded = (int64_t)(tx + 2) * (ty + 2) * (tz + 2);
+                const size_t lds_box = 16 * (1 + (size_t)((c8 + 1) / 2) * (2 * ((loaded + 15) / 16 * 16) + 1)) + tab;
+                const int64_t boxes = (int64_t)((g.W + tx - 1) / tx) * ((g.H + ty - 1) / ty) * ((g.D + tz - 1) / tz);
+                for (int nt = 1; nt <= 4 && nt <= ntw; ++nt) {
+                    if (nt > conv_max_nt(mt)) continue;
+                    const size_t lds = lds_box + 8192 * nt;
+                    if (lds > LDS_MAX) continue;
+                    const int64_t wgs = boxes * ((ntw + nt - 1) / nt);
+                    const double load = (double)loaded * c8, fixed = 2000.0 + 250.0 * mt * nt;
+                    const double block = std::max(std::max(16.0 * mt * nt, 16.0 * (mt + nt)), 64.0 * nt) + 24.0;
+                    const double alone = load + nkb * std::max(block, 70.0) + fixed;
+                    const double rounds = (double)((wgs + 255) / 256);
+                    const double each = 2 * lds > LDS_MAX ? alone
+                                                          : std::max(load, nkb * block) +
+                                                                0.5 * std::min(load, nkb * block) + 0.5 * fixed;
+                    const double cost = std::max(alone, rounds * each);
+                    if (!found || cost < best_cost) {
+                        found = true;
+                        best_cost = cost;
+                        best.t.tx = tx; best.t.ty = ty; best.t.tz = tz;
+                        best.mt = mt; best.nt = nt; best.lds = lds; best.boxes = (unsigned)boxes;
+                    }
+                }
+            }
+    if (!found) return false;
+    ConvTile& t = best.t;
+    const int LX = t.tx + 2, LY = t.ty + 2;
+    t.nx = (g.W + t.tx - 1) / t.tx;
+    t.ny = (g.H + t.ty - 1) / t.ty;
+    t.tv = t.tx * t.ty * t.tz;
+    t.pv = (LX * LY * (t.tz + 2) + 15) / 16 * 16;
+    t.pu = LX * LY * c8;
+    t.row = fast_div(LX * c8); t.c8 = fast_div(c8);
+    const unsigned groups = (ntw + best.nt - 1) / best.nt;
+    t.dboxes = fast_div(best.boxes);
+    t.dtx = fast_div(t.tx); t.dty = fast_div(t.ty); t.dnx = fast_div(t.nx); t.dny = fast_div(t.ny);
+    // the quotients are exact while numerator * divisor < 2^32
+    return (uint64_t)best.boxes * best.boxes * groups < (1ull << 32) && (uint64_t)t.pu * LX * c8 < (1ull << 32) &&
+           2ull * g.H * g.W * cin < NOWHERE;
+}
+
+int conv_launch(const __bf16* X, const __bf16* Wb, const float* bias, const __bf16* gate, const Grid3& g, int cin, int kp,
+                int cout, int relu, __bf16* yb, float* yf, hipStream_t s) {
+    const int ntw = (cout + 15) / 16;
+    const bool quad = cout % 4 == 0 && (uintptr_t)bias % 16 == 0 && (uintptr_t)gate % 8 == 0 && (uintptr_t)yb % 8 == 0 &&
+                     (uintptr_t)yf % 16 == 0;
+    const Epilogue ep{bias, gate, yb, yf, cout, relu, quad};
+    ConvPlan p;
+    if (!conv_plan(g, cin, ntw, p)) {
+        k_conv3<<<dim3(nblk((int64_t)g.D * g.H * g.W, 64), ntw), 256, 0, s>>>(X, Wb, g, cin, kp, ep);
+        return hipGetLastError() == hipSuccess ? 0 : -2;
+    }
+    const unsigned grid = p.boxes * ((ntw + p.nt - 1) / p.nt);
+    switch (10 * p.mt + p.nt) {
+#define MFNN_BOX(m, n, pf) \
+    case 10 * m + n: k_conv3_box<m, n, pf><<<grid, 256, p.lds, s>>>(X, Wb, g, cin, kp, ntw, ep, p.t); break;
+        MFNN_BOX(1, 1, 8) MFNN_BOX(1, 2, 4) MFNN_BOX(1, 3, 4) MFNN_BOX(1, 4, 4)
+        MFNN_BOX(2, 1, 4) MFNN_BOX(2, 2, 4) MFNN_BOX(2, 3, 2) MFNN_BOX(2, 4, 2)
+        MFNN_BOX(4, 1, 4) MFNN_BOX(4, 2, 2) MFNN_BOX(4, 3, 2)
+        MFNN_BOX(8, 1, 2) MFNN_BOX(8, 2, 2)
+#undef MFNN_BOX
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
 }  // namespace
 
 extern "C" {
@@ -390,42 +957,8 @@ int mfnn_conv3(const void* x, const void* w, const float* bias, const void* gate
                int32_t cin, int32_t kp, int32_t cout, int32_t relu, void* yb, float* yf, void* stream) {
     if (cin % 8 || kp % 32 || kp < 27 * cin || cout <= 0 || cout > 192 || D <= 0 || H <= 0 || W <= 0) return -1;
     if ((uintptr_t)x % 16 || (uintptr_t)w % 16) return -1;  // 16-byte operand loads
-    const Grid3 g{D, H, W};
-    const int64_t M = (int64_t)D * H * W;
-    const unsigned vblocks = nblk(M, 64);
-    hipStream_t s = (hipStream_t)stream;
-    // channel tiles the weight rows cover: ceil(cout / 16), or 12 (192 rows) above 128 channels
-    const int ntw = cout > 128 ? 12 : (cout + 15) / 16;
-    const __bf16* X = (const __bf16*)x;
-    const __bf16* Wb = (const __bf16*)w;
-    const __bf16* G = (const __bf16*)gate;
-    __bf16* Y = (__bf16*)yb;
-    if (vblocks < 256) {
-        // fewer voxel blocks than CUs: one channel tile per block, the tiles over grid.y
-        k_conv3<1, 1><<<dim3(vblocks, ntw), 256, 0, s>>>(X, Wb, bias, G, g, cin, kp, cout, relu, Y, yf);
-        return hipGetLastError() == hipSuccess ? 0 : -2;
-    }
-    const unsigned grid = vblocks;
-    switch (ntw) {
-        // one or two channel tiles on grids of 65536 voxels and more: two voxel tiles per wave
-        // share each weight load (on smaller grids the halved block count costs more)
-        case 1:
-            if (M >= 65536) k_conv3<1, 2><<<nblk(M, 128), 256, 0, s>>>(X, Wb, bias, G, g, cin, kp, cout, relu, Y, yf);
-            else k_conv3<1, 1><<<grid, 256, 0, s>>>(X, Wb, bias, G, g, cin, kp, cout, relu, Y, yf);
-            break;
-        case 2:
-            if (M >= 65536) k_conv3<2, 2><<<nblk(M, 128), 256, 0, s>>>(X, Wb, bias, G, g, cin, kp, cout, relu, Y, yf);
-            else k_conv3<2, 1><<<grid, 256, 0, s>>>(X, Wb, bias, G, g, cin, kp, cout, relu, Y, yf);
-            break;
-        case 3: k_conv3<3, 1><<<grid, 256, 0, s>>>(X, Wb, bias, G, g, cin, kp, cout, relu, Y, yf); break;
-        case 4: k_conv3<4, 1><<<grid, 256, 0, s>>>(X, Wb, bias, G, g, cin, kp, cout, relu, Y, yf); break;
-        case 5: k_conv3<5, 1><<<grid, 256, 0, s>>>(X, Wb, bias, G, g, cin, kp, cout, relu, Y, yf); break;
-        case 6: k_conv3<6, 1><<<grid, 256, 0, s>>>(X, Wb, bias, G, g, cin, kp, cout, relu, Y, yf); break;
-        case 7: k_conv3<7, 1><<<grid, 256, 0, s>>>(X, Wb, bias, G, g, cin, kp, cout, relu, Y, yf); break;
-        case 8: k_conv3<8, 1><<<grid, 256, 0, s>>>(X, Wb, bias, G, g, cin, kp, cout, relu, Y, yf); break;
-        default: k_conv3<12, 1><<<grid, 256, 0, s>>>(X, Wb, bias, G, g, cin, kp, cout, relu, Y, yf); break;
-    }
-    return hipGetLastError() == hipSuccess ? 0 : -2;
+    return conv_launch((const __bf16*)x, (const __bf16*)w, bias, (const __bf16*)gate, Grid3{D, H, W}, cin, kp, cout, relu,
+                       (__bf16*)yb, yf, (hipStream_t)stream);
 }
 
 int64_t mfnn_wgrad_workspace(int32_t D, int32_t H, int32_t W, int32_t kp, int32_t cout, int32_t chunk) {
@@ -445,6 +978,52 @@ bool wgrad_args_ok(const void* x, const void* dz, int32_t D, int32_t H, int32_t 
     return (uintptr_t)x % 16 == 0 && (uintptr_t)dz % 16 == 0;  // 16-byte operand loads
 }
 
+// Launches k_conv3_wgrad_rows over all chunks; false where its rows do not fit LDS.
+bool wgrad_rows(const __bf16* X, const __bf16* dZ, const Grid3& g, int cin, int kp, int coutp, int cout, int chunk,
+                int nchunk, float* part, float* bpart, hipStream_t s) {
+    const int full = cin / 16, ntiles = coutp / 16;
+    // two output tiles per wave share the input operands; with fewer than 512 workgroups that
+    // way (two per CU) the tiles go to workgroups of their own
+    const int nn = (int64_t)3 * std::max(full, 1) * ((ntiles + 1) / 2) * nchunk >= 512 && ntiles > 1 ? 2 : 1;
+    auto launch = [&](bool half) {
+        const int64_t vb = half ? 16 : 32, WP = g.W + 2, WH = (int64_t)g.W * g.H;
+        WgradRows t;
+        t.ci0 = half ? 16 * full : 0;
+        // as many voxels at a time as 48 KB hold (three workgroups per CU); wide rows take more
+        // LDS, down to 128 voxels at a time
+        int64_t lds = 0;
+        for (t.sub = nn == 2 ? 256 : 512;; t.sub /= 2) {
+            const int64_t rows = (t.sub + g.W - 2) / g.W + 2 * ((t.sub + WH - 2) / WH) + 3;
+            t.lds_dz = (int)(128 + std::min<int64_t>(rows * WP * vb, 1 << 20));
+            t.lds_pos = t.lds_dz + t.sub * nn * 32;
+            lds = t.lds_pos + 4 * t.sub;
+            if (lds <= 48 * 1024 || t.sub == 128) break;
+        }
+        // exact quotients; 24-bit products and 31-bit offsets of the loads
+        const int64_t M = WH * g.D;
+        if (lds > 80 * 1024 || (int64_t)(g.H + 2) * (g.H + 600) >= (1ll << 32) || (int64_t)(g.W + 600) * g.W >= (1ll << 32) ||
+            (int64_t)g.D * g.H >= (1 << 24) || 2ll * g.W * cin >= (1 << 24) || 2 * M * std::max(cin, cout) >= NOWHERE)
+            return false;
+        t.row = fast_div((uint32_t)(WP * vb / 16));
+        t.h2 = fast_div(g.H + 2);
+        t.w = fast_div(g.W);
+        t.h = fast_div(g.H);
+        const dim3 grid(3 * (half ? 1 : full), (ntiles + nn - 1) / nn, nchunk);
+#define MFNN_ROWS(n, h) k_conv3_wgrad_rows<n, h><<<grid, 192, lds, s>>>(X, dZ, g, cin, kp, coutp, cout, chunk, t, part, bpart)
+        if (half) {
+            if (nn == 2) MFNN_ROWS(2, true);
+            else MFNN_ROWS(1, true);
+        } else {
+            if (nn == 2) MFNN_ROWS(2, false);
+            else MFNN_ROWS(1, false);
+        }
+#undef MFNN_ROWS
+        return true;
+    };
+    if (full && !launch(false)) return false;
+    return cin % 16 == 0 || launch(true);
+}
+
 // The weight-gradient launches of valid arguments: partials into `work`, then the chunk sums.
 int wgrad_launch(const void* x, const void* dz, int32_t D, int32_t H, int32_t W, int32_t cin, int32_t kp, int32_t cout,
                  int32_t chunk, float* work, float* dw, float* db, int32_t accumulate, void* stream) {
@@ -455,14 +1034,9 @@ int wgrad_launch(const void* x, const void* dz, int32_t D, int32_t H, int32_t W,
     hipStream_t s = (hipStream_t)stream;
     const int64_t n = (int64_t)coutp * kp;
     float* bpart = db ? work + nchunk * n : nullptr;
-    // two k tiles per wave halve the dZ loads, one keeps twice the waves: the second wins
-    // when the single-tile grid has fewer than 3072 waves (three per SIMD)
-    if ((int64_t)(kp / 16) * (coutp / 16) * nchunk >= 3072)  // kp is a multiple of 32
-        k_conv3_wgrad<2><<<dim3(kp / 32, coutp / 16, nchunk), 64, 0, s>>>((const __bf16*)x, (const __bf16*)dz, g,
-                                                                          cin, kp, coutp, cout, chunk, work, bpart);
-    else
-        k_conv3_wgrad<1><<<dim3(kp / 16, coutp / 16, nchunk), 64, 0, s>>>((const __bf16*)x, (const __bf16*)dz, g,
-                                                                          cin, kp, coutp, cout, chunk, work, bpart);
+    const __bf16 *X = (const __bf16*)x, *dZ = (const __bf16*)dz;
+    if (!wgrad_rows(X, dZ, g, cin, kp, coutp, cout, chunk, nchunk, work, bpart, s))
+        k_conv3_wgrad<<<dim3(kp / 16, coutp / 16, nchunk), 64, 0, s>>>(X, dZ, g, cin, kp, coutp, cout, chunk, work, bpart);
     const unsigned sblocks = nblk(n, 32) + (db ? nblk(cout, 32) : 0);
     k_sum_chunks<<<sblocks, 256, 0, s>>>(work, nchunk, n, bpart, db ? cout : 0, accumulate, dw, db);
     return hipGetLastError() == hipSuccess ? 0 : -2;

@@ -71,6 +71,12 @@ struct mflbm_handle {
     // fused gradient chain
     int32_t* tag = nullptr;     // S4 node tags (lattice.h GradArgs)
     int grad_shape = 0, tiles_x = 0, tiles_y = 0, kchunk = 0, box_order = 0;
+    // work lists of the two-pass chain's boxes (lattice.h TileLists)
+    TileDesc *ndesc = nullptr, *fdesc = nullptr;
+    uint32_t *l3 = nullptr, *l6 = nullptr;
+    uint16_t *l4 = nullptr, *l7 = nullptr;
+    int32_t* r7 = nullptr;
+    uint8_t* tile_fluid = nullptr;
     bool split_gradient = false;
     bool grad_dirty = false;    // dense phi / cn / c_norm / curv behind the step state
     // monitor scratch
@@ -158,6 +164,7 @@ GradArgs<T> grad_args(const mflbm_handle* h) {
     A.cnp = (T*)h->cnp;
     A.shape = h->grad_shape; A.tiles_x = h->tiles_x; A.tiles_y = h->tiles_y; A.kchunk = h->kchunk;
     A.tiles_z = 1; A.box_order = h->box_order;
+    A.lists = TileLists{h->ndesc, h->fdesc, h->l3, h->l4, h->l6, h->l7, h->r7, h->tile_fluid};
     return A;
 }
 
@@ -254,6 +261,46 @@ void pack_solid_normals(mflbm_handle* h) {
                              h->stream);
 }
 
+// The work lists of the two-pass gradient chain, from the node tags.
+template <typename T>
+int build_tile_lists(mflbm_handle* h) {
+    size_t boxes[2];
+    for (int f = 0; f < 2; ++f) {
+        int t[3];
+        Launch<T>::tile_grid(h->d, f == 1, t);
+        boxes[f] = (size_t)t[0] * t[1] * t[2];
+    }
+    TileDesc** dev[2] = {&h->ndesc, &h->fdesc};
+    for (int f = 0; f < 2; ++f) HIPCHK(h, hipMalloc(dev[f], boxes[f] * sizeof(TileDesc)));
+    Launch<T>::tile_counts(grad_args<T>(h), h->ndesc, h->fdesc, h->stream);
+    HIPCHK(h, hipGetLastError());
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    int64_t na[2], nb[2];
+    for (int f = 0; f < 2; ++f) {
+        std::vector<TileDesc> td(boxes[f]);
+        HIPCHK(h, hipMemcpy(td.data(), *dev[f], td.size() * sizeof(TileDesc), hipMemcpyDeviceToHost));
+        na[f] = nb[f] = 0;
+        for (TileDesc& x : td) {
+            x.a = (int32_t)na[f];
+            x.b = (int32_t)nb[f];
+            na[f] += x.na;
+            nb[f] += x.nb;
+        }
+        if (na[f] > INT32_MAX || nb[f] > INT32_MAX) return fail(h, "too many nodes for the gradient work lists");
+        HIPCHK(h, hipMemcpy(*dev[f], td.data(), td.size() * sizeof(TileDesc), hipMemcpyHostToDevice));
+    }
+    auto room = [](int64_t n) { return (size_t)std::max<int64_t>(1, n); };
+    HIPCHK(h, hipMalloc(&h->l3, room(na[0]) * sizeof(uint32_t)));
+    HIPCHK(h, hipMalloc(&h->l4, room(nb[0]) * sizeof(uint16_t)));
+    HIPCHK(h, hipMalloc(&h->l6, room(na[1]) * sizeof(uint32_t)));
+    HIPCHK(h, hipMalloc(&h->l7, room(nb[1]) * sizeof(uint16_t)));
+    HIPCHK(h, hipMalloc(&h->r7, room(nb[1]) * sizeof(int32_t)));
+    HIPCHK(h, hipMalloc(&h->tile_fluid, boxes[1] * Launch<T>::tile_columns()));
+    Launch<T>::tile_fill(grad_args<T>(h), h->l3, h->l4, h->l6, h->l7, h->r7, h->tile_fluid, h->stream);
+    HIPCHK(h, hipGetLastError());
+    return 0;
+}
+
 void free_all(mflbm_handle* h) {
     for (int g = 0; g < 4; ++g)
         if (h->graph[g]) { (void)hipGraphExecDestroy(h->graph[g]); h->graph[g] = nullptr; }
@@ -261,7 +308,7 @@ void free_all(mflbm_handle* h) {
                     h->walls, h->wtype, h->l_fluid, h->l_fluid_ext, h->l_sb, h->mon_part, h->mon_out, h->vprev, h->vpart,
                     h->cells, h->aux, h->nb, h->nb16, h->nbb, h->pairs[0], h->pairs[1], h->zmap, h->pmap, h->w_in, h->conv,
                     h->ext_node, h->ext_off, h->zstart,
-                    h->tag, h->macro_buf};
+                    h->tag, h->macro_buf, h->ndesc, h->fdesc, h->l3, h->l4, h->l6, h->l7, h->r7, h->tile_fluid};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     h->pdf = h->phi = h->cnx = h->cny = h->cnz = h->cnorm = h->cnp = h->snp = h->curv = h->snx = h->sny = h->snz = nullptr;
@@ -275,6 +322,11 @@ void free_all(mflbm_handle* h) {
     h->nb = h->pairs[0] = h->pairs[1] = h->zmap = h->pmap = h->ext_node = h->ext_off = h->zstart = nullptr;
     h->w_in = h->conv = nullptr;
     h->tag = nullptr;
+    h->ndesc = h->fdesc = nullptr;
+    h->l3 = h->l6 = nullptr;
+    h->l4 = h->l7 = nullptr;
+    h->r7 = nullptr;
+    h->tile_fluid = nullptr;
     if (h->stream) { (void)hipStreamDestroy(h->stream); h->stream = nullptr; }
 }
 
@@ -579,6 +631,7 @@ int mflbm_create(const mflbm_params* params, const int8_t* geometry, mflbm_handl
         if (h->grad_shape == GRAD_SHAPE_TILES) {
             HIPCHK(h, hipMalloc(&h->cnp, 4 * d.S2 * esize(h)));
             HIPCHK(h, hipMemsetAsync(h->cnp, 0, 4 * d.S2 * esize(h), h->stream));
+            if (h->prec == MFLBM_FP64 ? build_tile_lists<double>(h) : build_tile_lists<float>(h)) return -1;
         }
     }
 

@@ -133,6 +133,24 @@ struct Sparse {
     }
 };
 
+// The two work lists of one box of the two-pass gradient chain: runs [a, a + na) and
+// [b, b + nb) of the chain's list arrays.
+struct TileDesc {
+    int32_t a, na, b, nb;
+};
+
+// Work lists of the two-pass chain, built once from the geometry (k_tile_lists).  A box entry
+// is its position in the loaded box, x | y << 5 | z << 9.
+struct TileLists {
+    const TileDesc *ndesc, *fdesc;      // per box of k_grad_normals and of k_grad_force
+    const uint32_t* __restrict__ l3;    // K3: entry | written back << 12 | fluid-neighbour mask << 13
+    const uint16_t* __restrict__ l4;    // K4: entry | wetting << 12
+    const uint32_t* __restrict__ l6;    // K6: entry | fluid-neighbour mask << 12
+    const uint16_t* __restrict__ l7;    // K7: entry
+    const int32_t* __restrict__ r7;     // K7: force-record index
+    const uint8_t* __restrict__ fluid;  // k_grad_force: per box and column, the fluid nodes of the loaded box (bit z)
+};
+
 // Inputs of the fused gradient-chain kernel (gradient.inl).  `tag` holds, for every node of
 // the four-ghost-layer grid, (t << 2) | (walls_type & 3) with walls_type 0 -> 0, 1 -> 1,
 // 2 -> 2, -1 -> 3, where t is the fluid-list index (force-record index) of an interior
@@ -157,6 +175,7 @@ struct GradArgs {
     // two-pass chain: boxes along z, and the order in which the workgroups walk the boxes
     // (0: x fastest, then y, then z; 1: x fastest, then z, then y)
     int tiles_z, box_order;
+    TileLists lists;
 };
 
 // Workgroup shapes of the fused gradient kernel: owned nodes in x and y, threads.

@@ -21,6 +21,13 @@ struct Launch {
     static void normal_extrap(const Fields<T>& F, const NodeLists& L, hipStream_t s);
     static void curvature(const Fields<T>& F, const StepConst<T>& P, const NodeLists& L, T* aux, hipStream_t s);
     static void gradient(const GradArgs<T>& A, const StepConst<T>& P, hipStream_t s);
+    // Boxes of the two-pass chain's kernels, and its work lists: first their sizes (na and nb of
+    // the descriptors), then, with the descriptors complete, the lists.
+    static void tile_grid(const Dims& d, bool force, int (&tiles)[3]);
+    static int tile_columns();
+    static void tile_counts(const GradArgs<T>& A, TileDesc* ndesc, TileDesc* fdesc, hipStream_t s);
+    static void tile_fill(const GradArgs<T>& A, uint32_t* l3, uint16_t* l4, uint32_t* l6, uint16_t* l7, int32_t* r7,
+                          uint8_t* fluid, hipStream_t s);
     static void aux_refresh(const Fields<T>& F, const StepConst<T>& P, const NodeLists& L, T* aux, hipStream_t s);
     static void cells(const Sparse<T>& S, T* dense, const Dims& d, const int32_t* ext_node, const int32_t* ext_off,
                       int n_ext, bool to_dense, hipStream_t s);

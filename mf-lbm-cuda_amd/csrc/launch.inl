@@ -95,21 +95,63 @@ void Launch<T>::curvature(const Fields<T>& F, const StepConst<T>& P, const NodeL
 }
 
 template <typename T>
+void Launch<T>::tile_grid(const Dims& d, bool force, int (&tiles)[3]) {
+    const int n[3] = {d.nx, d.ny, d.nz};
+    // normals over [-1, n+2]^3, forces over [1, n]^3
+    for (int a = 0; a < 3; ++a) {
+        const int t = force ? GradTiles<T>::F[a] : GradTiles<T>::N[a];
+        tiles[a] = (n[a] + (force ? 0 : 4) + t - 1) / t;
+    }
+}
+
+template <typename T>
+int Launch<T>::tile_columns() { return (GradTiles<T>::F[0] + 4) * (GradTiles<T>::F[1] + 4); }
+
+namespace {
+// Sets the box counts of one of the two kernels; returns its grid.
+template <typename T>
+unsigned box_grid(GradArgs<T>& A, bool force) {
+    int t[3];
+    Launch<T>::tile_grid(A.d, force, t);
+    A.tiles_x = t[0]; A.tiles_y = t[1]; A.tiles_z = t[2];
+    return (unsigned)(t[0] * t[1] * t[2]);
+}
+}  // namespace
+
+template <typename T>
+void Launch<T>::tile_counts(const GradArgs<T>& A, TileDesc* ndesc, TileDesc* fdesc, hipStream_t s) {
+    constexpr int NX = GradTiles<T>::N[0], NY = GradTiles<T>::N[1], NZ = GradTiles<T>::N[2];
+    constexpr int FX = GradTiles<T>::F[0], FY = GradTiles<T>::F[1], FZ = GradTiles<T>::F[2];
+    GradArgs<T> B = A;
+    const unsigned gn = box_grid(B, false);
+    dev::k_tile_lists<T, NX, NY, NZ, false, false><<<gn, 64, 0, s>>>(B, ndesc, nullptr, nullptr, nullptr, nullptr);
+    const unsigned gf = box_grid(B, true);
+    dev::k_tile_lists<T, FX, FY, FZ, true, false><<<gf, 64, 0, s>>>(B, fdesc, nullptr, nullptr, nullptr, nullptr);
+}
+
+template <typename T>
+void Launch<T>::tile_fill(const GradArgs<T>& A, uint32_t* l3, uint16_t* l4, uint32_t* l6, uint16_t* l7, int32_t* r7,
+                          uint8_t* fluid, hipStream_t s) {
+    constexpr int NX = GradTiles<T>::N[0], NY = GradTiles<T>::N[1], NZ = GradTiles<T>::N[2];
+    constexpr int FX = GradTiles<T>::F[0], FY = GradTiles<T>::F[1], FZ = GradTiles<T>::F[2];
+    GradArgs<T> B = A;
+    const unsigned gn = box_grid(B, false);
+    dev::k_tile_lists<T, NX, NY, NZ, false, true>
+        <<<gn, 64, 0, s>>>(B, const_cast<TileDesc*>(A.lists.ndesc), l3, l4, nullptr, nullptr);
+    const unsigned gf = box_grid(B, true);
+    dev::k_tile_lists<T, FX, FY, FZ, true, true>
+        <<<gf, 64, 0, s>>>(B, const_cast<TileDesc*>(A.lists.fdesc), l6, l7, r7, fluid);
+}
+
+template <typename T>
 void Launch<T>::gradient(const GradArgs<T>& A, const StepConst<T>& P, hipStream_t s) {
     if (A.shape == GRAD_SHAPE_TILES) {
         constexpr int NX = GradTiles<T>::N[0], NY = GradTiles<T>::N[1], NZ = GradTiles<T>::N[2];
         constexpr int FX = GradTiles<T>::F[0], FY = GradTiles<T>::F[1], FZ = GradTiles<T>::F[2];
         GradArgs<T> B = A;
-        // normals over [-1, n+2]^3, forces over [1, n]^3
-        B.tiles_x = (A.d.nx + 4 + NX - 1) / NX;
-        B.tiles_y = (A.d.ny + 4 + NY - 1) / NY;
-        B.tiles_z = (A.d.nz + 4 + NZ - 1) / NZ;
-        const unsigned gn = (unsigned)(B.tiles_x * B.tiles_y * B.tiles_z);
+        const unsigned gn = box_grid(B, false);
         dev::k_grad_normals<T, NX, NY, NZ><<<gn, (NX + 4) * (NY + 4), 0, s>>>(B, P);
-        B.tiles_x = (A.d.nx + FX - 1) / FX;
-        B.tiles_y = (A.d.ny + FY - 1) / FY;
-        B.tiles_z = (A.d.nz + FZ - 1) / FZ;
-        const unsigned gf = (unsigned)(B.tiles_x * B.tiles_y * B.tiles_z);
+        const unsigned gf = box_grid(B, true);
         dev::k_grad_force<T, FX, FY, FZ><<<gf, (FX + 4) * (FY + 4), 0, s>>>(B, P);
         return;
     }

@@ -1,0 +1,55 @@
+"""GPU parity of the step at the geometries where its boxes can go wrong: boxes with no node to
+compute, boxes without solid, a single box, rows just past a box edge.  FP64, so the state
+must equal the oracle's bit for bit."""
+import numpy as np
+import pytest
+
+import oracle as O
+from helpers import assert_same, small_drainage
+from mflbm import gpu
+
+pytestmark = pytest.mark.gpu
+
+
+def solid_block(n, seed, jper=1):
+    """a sphere pack whose middle third along z and lower half along y are solid, except for one
+    channel that keeps the ends connected"""
+    geo, p = small_drainage(n=n, seed=seed, radius=3.0, porosity=0.6, jper=jper, buffer=2)
+    nz, ny, nx = geo.shape
+    geo[nz // 3:2 * nz // 3] = 1
+    geo[2:-2, :ny // 2] = 1
+    geo[2:-2, ny // 2 + 1:ny // 2 + 4, nx // 2:nx // 2 + 3] = 0
+    return geo, p
+
+
+def no_solid(n, seed):
+    geo, p = small_drainage(n=n, seed=seed, radius=3.0, porosity=0.95, jper=1, buffer=2)
+    return np.zeros_like(geo), p
+
+
+CASES = {
+    "solid_boxes": lambda: solid_block((40, 36, 33), 3),
+    "solid_boxes_ywalls": lambda: solid_block((35, 33, 30), 4, jper=0),
+    "no_solid": lambda: no_solid((18, 17, 13), 5),
+    "one_box": lambda: small_drainage(n=(12, 8, 5), seed=2, radius=2.0, porosity=0.6, jper=1, buffer=1),
+    "one_past_a_box": lambda: small_drainage(n=(17, 9, 9), seed=4, radius=2.5, porosity=0.55, jper=1, buffer=2),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_steps_bitwise(name):
+    geo, p = CASES[name]()
+    print(f"[gpu-step-tiles] {name} {geo.shape}", flush=True)
+    o, g = O.Oracle(p, geo), gpu.Solver(p, geo, gpu.FP64)
+    assert g.gradient_path() == "tiles"
+    o.setup()
+    g.setup()
+    for t in range(1, 4):
+        o.step(t)
+        g.step(t)
+        for field in ("pdf", "phi", "cn_x", "cn_y", "cn_z", "c_norm"):
+            assert_same(g.download(field), o.array(field), 0.0, what=f"{name} step {t} {field}")
+    o.run(4, 30)
+    g.run(4, 30)
+    for field in ("pdf", "phi"):
+        assert_same(g.download(field), o.array(field), 0.0, what=f"{name} step 33 {field}")

@@ -60,6 +60,7 @@ struct mflbm_handle {
     int32_t* pairs[2] = {nullptr, nullptr};
     int npairs[2] = {0, 0};
     int32_t* zmap = nullptr;
+    int32_t* bcp = nullptr;     // periodic copies of odd steps that the open boundaries make
     int32_t* pmap = nullptr;    // porous-plate plane map
     int in_bc = 0, out_bc = 0;  // open z: 1 velocity inlet / convective outlet, 2 Zou-He
     int plate_z = 0, plate_blocked = 0;
@@ -188,12 +189,17 @@ void enqueue_step(mflbm_handle* h, bool odd, hipEvent_t* ev) {
     auto mark = [&]() { if (ev) (void)hipEventRecord(ev[e++], s); };
     Launch<T>::collide(S, F.phi, h->d, P, odd, s);
     mark();
-    if (h->p.kper || h->p.jper) {
-        Launch<T>::periodic_pdf(S, h->pairs[odd ? 1 : 0], h->npairs[odd ? 1 : 0], s);
-        Launch<T>::periodic_phi(F.phi, h->d, h->p.kper, h->p.jper, s);
+    {
+        BoundaryArgs<T> B{};
+        if (h->open_z) {
+            B.in_bc = h->in_bc;
+            B.out_bc = h->out_bc;
+        }
+        B.zmap = h->zmap; B.w_in = (const T*)h->w_in; B.conv = (T*)h->conv; B.bcp = h->bcp;
+        B.pairs = h->pairs[odd ? 1 : 0]; B.npairs = h->npairs[odd ? 1 : 0];
+        B.kper = h->p.kper; B.jper = h->p.jper;
+        Launch<T>::boundary(S, F, P, B, odd, s);
     }
-    if (h->open_z && (h->in_bc || h->out_bc))
-        Launch<T>::open_bc(S, F, P, h->zmap, h->in_bc, h->out_bc, (const T*)h->w_in, (T*)h->conv, odd, s);
     if (h->plate_z) Launch<T>::porous_plate(S, h->d, P, h->pmap, h->plate_z, h->plate_blocked, odd, s);
     mark();
     if (h->split_gradient) {
@@ -306,7 +312,7 @@ void free_all(mflbm_handle* h) {
         if (h->graph[g]) { (void)hipGraphExecDestroy(h->graph[g]); h->graph[g] = nullptr; }
     void* ptrs[] = {h->pdf, h->phi, h->cnx, h->cny, h->cnz, h->cnorm, h->cnp, h->snp, h->curv, h->snx, h->sny, h->snz,
                     h->walls, h->wtype, h->l_fluid, h->l_fluid_ext, h->l_sb, h->mon_part, h->mon_out, h->vprev, h->vpart,
-                    h->cells, h->aux, h->nb, h->nb16, h->nbb, h->pairs[0], h->pairs[1], h->zmap, h->pmap, h->w_in, h->conv,
+                    h->cells, h->aux, h->nb, h->nb16, h->nbb, h->pairs[0], h->pairs[1], h->zmap, h->bcp, h->pmap, h->w_in, h->conv,
                     h->ext_node, h->ext_off, h->zstart,
                     h->tag, h->macro_buf, h->ndesc, h->fdesc, h->l3, h->l4, h->l6, h->l7, h->r7, h->tile_fluid};
     for (void* p : ptrs)
@@ -319,7 +325,7 @@ void free_all(mflbm_handle* h) {
     h->cells = h->aux = nullptr;
     h->nb16 = nullptr;
     h->nbb = nullptr;
-    h->nb = h->pairs[0] = h->pairs[1] = h->zmap = h->pmap = h->ext_node = h->ext_off = h->zstart = nullptr;
+    h->nb = h->pairs[0] = h->pairs[1] = h->zmap = h->bcp = h->pmap = h->ext_node = h->ext_off = h->zstart = nullptr;
     h->w_in = h->conv = nullptr;
     h->tag = nullptr;
     h->ndesc = h->fdesc = nullptr;
@@ -671,6 +677,7 @@ int mflbm_create(const mflbm_params* params, const int8_t* geometry, mflbm_handl
     h->npairs[0] = (int)(lay.pairs[0].size() / 3);
     h->npairs[1] = (int)(lay.pairs[1].size() / 3);
     HIPCHK(h, upload_i32(&h->zmap, lay.zmap));
+    if (!lay.bcp.empty()) HIPCHK(h, upload_i32(&h->bcp, lay.bcp));
     if (h->plate_z) HIPCHK(h, upload_i32(&h->pmap, lay.pmap));
     {
         const int64_t P2 = (int64_t)d.X1 * d.Y1;

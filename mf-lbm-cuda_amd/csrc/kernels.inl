@@ -5,9 +5,9 @@
 //
 // Reference correspondence (src/main_iteration_GPU.cu):
 //   k_collide<ODD>     kernel_odd_color_GPU / kernel_even_color_GPU   (56-388 / 395-726)
-//   k_periodic_pdf     perioidc_BC_{Z,Y,ZY}_{odd,even}                (1529-1689)
-//   k_periodic_phi     periodic_phi_{Z,Y,ZY}                          (1691-1733)
-//   k_open_bc<AFTER>   inlet/outlet_Zou_He_pressure_BC_{before,after}_odd_GPU (1085-1524),
+//   k_boundary<AFTER>  perioidc_BC_{Z,Y,ZY}_{odd,even}                (1529-1689)
+//                      periodic_phi_{Z,Y,ZY}                          (1691-1733)
+//                      inlet/outlet_Zou_He_pressure_BC_{before,after}_odd_GPU (1085-1524),
 //                      inlet_bounce_back_velocity_BC_* (1008-1077), outlet_convective_BC_* (1245-1357)
 //   k_porous_plate     porous_plate_BC_{before,after}_odd (1744-1882)
 //   k_phi_extrap       extrapolate_phi_toSolid                        (732-755)
@@ -401,58 +401,6 @@ __global__ __launch_bounds__(MFLBM_COLLIDE_THREADS) void k_collide(Sparse<T> S, 
     }
 }
 
-// Periodic population copies, precomputed as (slot, destination cell, source cell) in the
-// reference's kernel order with repeated destinations resolved to the last writer
-// (perioidc_BC_{Z,Y,ZY}_{odd,even}, src/main_iteration_GPU.cu:1529-1689).
-template <typename T>
-__global__ __launch_bounds__(256) void k_periodic_pdf(Sparse<T> S, const int32_t* __restrict__ pairs, int n) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= n) return;
-    const int slot = pairs[3 * t], dst = pairs[3 * t + 1], src = pairs[3 * t + 2];
-    S.f[S.at(slot, dst)] = S.f[S.at(slot, src)];
-    S.f[S.at(slot + 19, dst)] = S.f[S.at(slot + 19, src)];
-}
-
-// Periodic ghost layers of phi (periodic_phi_{Z,Y,ZY}, src/main_iteration_GPU.cu:1691-1733);
-// the three groups read interior cells and write disjoint ghost cells.
-template <typename T>
-__global__ __launch_bounds__(256) void k_periodic_phi(T* __restrict__ phi, Dims d, int kper, int jper) {
-    const int nx = d.nx, ny = d.ny, nz = d.nz;
-    int t = blockIdx.x * 256 + threadIdx.x;
-    auto P = [&](int a, int b, int c) -> T& { return phi[i4(d, a, b, c)]; };
-    const int nzf = kper ? nx * ny : 0, nyf = jper ? nx * nz : 0, ne = (kper && jper) ? nx : 0;
-    if (t < nzf) {
-        const int i = t % nx + 1, j = t / nx + 1;
-#pragma unroll
-        for (int kk = 1; kk <= 4; ++kk) {
-            P(i, j, kk + nz) = P(i, j, kk);
-            P(i, j, kk - 4) = P(i, j, nz + kk - 4);
-        }
-        return;
-    }
-    t -= nzf;
-    if (t < nyf) {
-        const int i = t % nx + 1, k = t / nx + 1;
-#pragma unroll
-        for (int jj = 1; jj <= 4; ++jj) {
-            P(i, jj + ny, k) = P(i, jj, k);
-            P(i, jj - 4, k) = P(i, ny + jj - 4, k);
-        }
-        return;
-    }
-    t -= nyf;
-    if (t < ne) {
-        const int i = t + 1;
-        for (int kk = 1; kk <= 4; ++kk)
-            for (int jj = 1; jj <= 4; ++jj) {
-                P(i, jj - 4, kk - 4) = P(i, ny + jj - 4, nz + kk - 4);
-                P(i, jj + ny, kk - 4) = P(i, jj, nz + kk - 4);
-                P(i, jj + ny, kk + nz) = P(i, jj, kk);
-                P(i, jj - 4, kk + nz) = P(i, ny + jj - 4, kk);
-            }
-    }
-}
-
 // One colour population of a cell in shifted storage (colour 1 and the total's deviation
 // from the rest state), read and written as the plain colour value; writing colour 1 keeps
 // colour 2 unchanged.
@@ -492,38 +440,118 @@ __device__ __forceinline__ void with_cells(const Sparse<T>& S, T rho_ref, CellOf
     }
 }
 
+// Periodic population copies, precomputed as (slot, destination cell, source cell) in the
+// reference's kernel order with repeated destinations resolved to the last writer
+// (perioidc_BC_{Z,Y,ZY}_{odd,even}, src/main_iteration_GPU.cu:1529-1689).
+template <typename T>
+__device__ __forceinline__ void copy_cell(const Sparse<T>& S, int slot, int dst, int src) {
+    S.f[S.at(slot, dst)] = S.f[S.at(slot, src)];
+    S.f[S.at(slot + 19, dst)] = S.f[S.at(slot + 19, src)];
+}
+
+// Periodic ghost layers of phi (periodic_phi_{Z,Y,ZY}, src/main_iteration_GPU.cu:1691-1733);
+// the three groups read interior cells and write disjoint ghost cells.
+template <typename T>
+__device__ __forceinline__ void periodic_phi(T* __restrict__ phi, const Dims& d, int kper, int jper, int t) {
+    const int nx = d.nx, ny = d.ny, nz = d.nz;
+    auto P = [&](int a, int b, int c) -> T& { return phi[i4(d, a, b, c)]; };
+    const int nzf = kper ? nx * ny : 0, nyf = jper ? nx * nz : 0, ne = (kper && jper) ? nx : 0;
+    if (t < nzf) {
+        const int i = t % nx + 1, j = t / nx + 1;
+#pragma unroll
+        for (int kk = 1; kk <= 4; ++kk) {
+            P(i, j, kk + nz) = P(i, j, kk);
+            P(i, j, kk - 4) = P(i, j, nz + kk - 4);
+        }
+        return;
+    }
+    t -= nzf;
+    if (t < nyf) {
+        const int i = t % nx + 1, k = t / nx + 1;
+#pragma unroll
+        for (int jj = 1; jj <= 4; ++jj) {
+            P(i, jj + ny, k) = P(i, jj, k);
+            P(i, jj - 4, k) = P(i, ny + jj - 4, k);
+        }
+        return;
+    }
+    t -= nyf;
+    if (t < ne) {
+        const int i = t + 1;
+        for (int kk = 1; kk <= 4; ++kk)
+            for (int jj = 1; jj <= 4; ++jj) {
+                P(i, jj - 4, kk - 4) = P(i, ny + jj - 4, nz + kk - 4);
+                P(i, jj + ny, kk - 4) = P(i, jj, nz + kk - 4);
+                P(i, jj + ny, kk + nz) = P(i, jj, kk);
+                P(i, jj - 4, kk + nz) = P(i, ny + jj - 4, kk);
+            }
+    }
+}
+
+// The boundary updates between the collision and the gradient chain in one launch: open
+// inlet/outlet columns, periodic population copies, periodic phi, each in workgroups of its
+// own (nbc, then npair, then the rest).  The reference copies the periodic populations first
+// and the open boundaries then read and write some of the copied cells; here the order is
+// kept without a launch between them:
+//   after an even step the open boundaries read, of the copied cells, ghost cells only, and
+//   write none of the copies' cells; zmap gives, for a copied ghost cell, the cell it is
+//   copied from, which holds the same value;
+//   after an odd step a column's open boundary touches cells of its own column only, so the
+//   thread of a column at j = 1 or ny makes the copies into the planes its boundary touches
+//   (bcp) before it, and the list of copies leaves them out.
+// phi: the open boundaries write ghost planes in z of interior columns, the periodic copies
+// read and write planes 1 .. nz.
+// On domains of 32^3 to 64^3 a launch costs 4.5 us whatever it does: three of them took 18 of a
+// step's 39 to 45 us, the merged one 9.
+//
 // Open inlet/outlet, one thread per (i, j): in_bc / out_bc 2 = Zou-He, 1 = velocity inlet /
 // convective outlet.  zmap[plane][slot][b * (nx+2) + a] gives the cell of (a, b, k) for the
 // six planes k = 0, 1, 2, nz-1, nz, nz+1.  w_in: the inlet velocity plane (X1 * Y1);
 // conv: the convective-outlet state, 38 planes of populations [g][e] then phi.
 template <typename T, bool AFTER_ODD>
-__global__ __launch_bounds__(256) void k_open_bc(Sparse<T> S, Fields<T> F, StepConst<T> P, const int32_t* __restrict__ zmap,
-                                                 int in_bc, int out_bc, const T* __restrict__ w_in, T* __restrict__ conv,
-                                                 int split) {
+__global__ __launch_bounds__(256) void k_boundary(Sparse<T> S, Fields<T> F, StepConst<T> P, BoundaryArgs<T> B) {
     const Dims& d = F.d;
-    int t = blockIdx.x * 256 + threadIdx.x;
+    if ((int)blockIdx.x >= B.nbc) {
+        int t = ((int)blockIdx.x - B.nbc) * 256 + threadIdx.x;
+        if ((int)blockIdx.x < B.nbc + B.npair) {
+            if (t < B.npairs) copy_cell(S, B.pairs[3 * t], B.pairs[3 * t + 1], B.pairs[3 * t + 2]);
+        } else {
+            periodic_phi(F.phi, d, B.kper, B.jper, t - B.npair * 256);
+        }
+        return;
+    }
+    int t = blockIdx.x * 256 + threadIdx.x, in_bc = B.in_bc, out_bc = B.out_bc;
     // split: the inlet columns and the outlet columns on threads of their own (the two
     // planes share no cell); otherwise one thread does both ends of its column
-    if (t >= (split ? 2 : 1) * d.nx * d.ny) return;
-    if (split) {
+    if (t >= (B.split ? 2 : 1) * d.nx * d.ny) return;
+    if (B.split) {
         if (t < d.nx * d.ny) out_bc = 0;
         else { in_bc = 0; t -= d.nx * d.ny; }
     }
     const int i = t % d.nx + 1, j = t / d.nx + 1, nz = d.nz;
     const int64_t P2 = (int64_t)d.X1 * d.Y1, plane = 19 * P2;
+    if (AFTER_ODD && B.bcp && (j == 1 || j == d.ny)) {
+        // planes 1 (inlet), nz - 1 and nz (outlet); five slots each, (slot, dst, src)
+        for (int p = in_bc ? 0 : 1; p < (out_bc ? 3 : 1); ++p)
+#pragma unroll
+            for (int m = 0; m < 5; ++m) {
+                const int32_t* c = B.bcp + 3 * ((((int64_t)p * 2 + (j == 1 ? 0 : 1)) * 5 + m) * d.nx + i - 1);
+                copy_cell(S, c[0], c[1], c[2]);
+            }
+    }
     auto cell_of = [&](int a, int b, int c, int e) -> int64_t {
         const int pl = c <= 2 ? c : 3 + (c - (nz - 1));
-        return zmap[pl * plane + (int64_t)e * P2 + b * d.X1 + a];
+        return B.zmap[pl * plane + (int64_t)e * P2 + b * d.X1 + a];
     };
     auto wall = [&](int a, int b, int c) -> int { return F.walls[i2(d, a, b, c)]; };
     auto ph = [&](int a, int b, int c) -> T& { return F.phi[i4(d, a, b, c)]; };
     const int64_t col = (int64_t)j * d.X1 + i;
     with_cells<T>(S, P.rho_ref, cell_of, [&](auto&& f) {
-        if (in_bc == 1) velocity_inlet_column<T, AFTER_ODD>(P, i, j, w_in[col], f, wall, ph);
+        if (in_bc == 1) velocity_inlet_column<T, AFTER_ODD>(P, i, j, B.w_in[col], f, wall, ph);
         if (in_bc == 2 || out_bc == 2) zou_he_column<T, AFTER_ODD>(P, i, j, nz, in_bc == 2, out_bc == 2, f, wall, ph);
         if (out_bc == 1) {
-            auto cs = [&](int e, int g) -> T& { return conv[(int64_t)(e + 19 * g) * P2 + col]; };
-            auto cp = [&]() -> T& { return conv[38 * P2 + col]; };
+            auto cs = [&](int e, int g) -> T& { return B.conv[(int64_t)(e + 19 * g) * P2 + col]; };
+            auto cp = [&]() -> T& { return B.conv[38 * P2 + col]; };
             convective_outlet_column<T, AFTER_ODD>(P, i, j, nz, f, wall, ph, cs, cp);
         }
     });

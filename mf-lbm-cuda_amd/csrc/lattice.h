@@ -77,6 +77,19 @@ struct StepConst {
     int mrt;    // collision model 1-4 (mflbm_params::mrt)
 };
 
+// One boundary launch (k_boundary): workgroups and inputs of its three parts.
+template <typename T>
+struct BoundaryArgs {
+    int nbc, npair;                      // workgroups of the open boundaries, of the periodic copies
+    const int32_t* __restrict__ zmap;    // open boundaries
+    int in_bc, out_bc, split;
+    const T* __restrict__ w_in;
+    T* __restrict__ conv;
+    const int32_t* __restrict__ bcp;     // copies made by the open boundaries' threads (odd steps)
+    const int32_t* __restrict__ pairs;   // (slot, dst, src) of the other periodic copies
+    int npairs, kper, jper;
+};
+
 struct NodeLists {
     const uint32_t* fluid;      // walls == 0 in [1,n]^3        : collide, curvature
     int n_fluid;

@@ -41,24 +41,18 @@ void Launch<T>::collide(const Sparse<T>& S, T* phi, const Dims& d, const StepCon
 }
 
 template <typename T>
-void Launch<T>::periodic_pdf(const Sparse<T>& S, const int32_t* pairs, int npairs, hipStream_t s) {
-    if (npairs > 0) dev::k_periodic_pdf<T><<<blocks(npairs), 256, 0, s>>>(S, pairs, npairs);
-}
-
-template <typename T>
-void Launch<T>::periodic_phi(T* phi, const Dims& d, int kper, int jper, hipStream_t s) {
-    const int64_t n = (kper ? (int64_t)d.nx * d.ny : 0) + (jper ? (int64_t)d.nx * d.nz : 0) + ((kper && jper) ? d.nx : 0);
-    if (n > 0) dev::k_periodic_phi<T><<<blocks(n), 256, 0, s>>>(phi, d, kper, jper);
-}
-
-template <typename T>
-void Launch<T>::open_bc(const Sparse<T>& S, const Fields<T>& F, const StepConst<T>& P, const int32_t* zmap, int in_bc,
-                        int out_bc, const T* w_in, T* conv, bool after_odd, hipStream_t s) {
+void Launch<T>::boundary(const Sparse<T>& S, const Fields<T>& F, const StepConst<T>& P, BoundaryArgs<T> B, bool after_odd,
+                         hipStream_t s) {
+    const Dims& d = F.d;
     // inlet and outlet on separate threads when both are set and their planes are apart
-    const int split = in_bc && out_bc && F.d.nz >= 6;
-    const int n = (split ? 2 : 1) * F.d.nx * F.d.ny;
-    if (after_odd) dev::k_open_bc<T, true><<<blocks(n), 256, 0, s>>>(S, F, P, zmap, in_bc, out_bc, w_in, conv, split);
-    else dev::k_open_bc<T, false><<<blocks(n), 256, 0, s>>>(S, F, P, zmap, in_bc, out_bc, w_in, conv, split);
+    B.split = B.in_bc && B.out_bc && d.nz >= 6;
+    B.nbc = B.in_bc || B.out_bc ? (int)blocks((int64_t)(B.split ? 2 : 1) * d.nx * d.ny) : 0;
+    B.npair = (int)blocks(B.npairs);
+    const int64_t nphi = (B.kper ? (int64_t)d.nx * d.ny : 0) + (B.jper ? (int64_t)d.nx * d.nz : 0) + ((B.kper && B.jper) ? d.nx : 0);
+    const unsigned grid = (unsigned)(B.nbc + B.npair) + blocks(nphi);
+    if (grid == 0) return;
+    if (after_odd) dev::k_boundary<T, true><<<grid, 256, 0, s>>>(S, F, P, B);
+    else dev::k_boundary<T, false><<<grid, 256, 0, s>>>(S, F, P, B);
 }
 
 template <typename T>

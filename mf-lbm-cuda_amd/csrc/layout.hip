@@ -152,7 +152,14 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
             out.n_escaped += e;
         }
     }
-    // periodic pairs, last writer wins
+    // periodic pairs, last writer wins; on odd steps without the copies into the planes the open
+    // boundaries touch (inlet 1, outlet nz-1 and nz), which their threads make (bcp)
+    const bool zmapped = open_z && (in_bc || out_bc);
+    auto bc_plane = [&](int64_t n) {
+        if (!zmapped || !jper) return false;
+        const int k = (int)(n / ((int64_t)d.X1 * d.Y1));
+        return (in_bc && k == 1) || (out_bc && (k == d.nz - 1 || k == d.nz));
+    };
     for (int odd = 0; odd < 2; ++odd) {
         const std::vector<int32_t>& r = raw[odd];
         const size_t n = r.size() / 3;
@@ -163,7 +170,7 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
         for (size_t m = 0; m + 1 < n; ++m)
             if (key[m].first == key[m + 1].first) keep[key[m].second] = 0;  // a later copy overwrites it
         for (size_t m = 0; m < n; ++m) {
-            if (!keep[m]) continue;
+            if (!keep[m] || (odd && bc_plane(r[3 * m + 1]))) continue;
             const int s = r[3 * m];
             const int32_t cd = cell(r[3 * m + 1], s), cs = cell(r[3 * m + 2], s);
             if (cd < 0 || cs < 0) { err = "periodic copy of an untracked cell"; return false; }
@@ -183,7 +190,7 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
                         out.pmap[((size_t)p * 19 + s) * P2 + (size_t)b * d.X1 + a] = cell(i1(d, a, b, plate_z - 1 + p), s);
     }
     // open-boundary plane maps
-    if (open_z && (in_bc || out_bc)) {
+    if (zmapped) {
         const int64_t P2 = (int64_t)d.X1 * d.Y1;
         out.zmap.assign((size_t)6 * 19 * P2, -1);
         const int kk[6] = {0, 1, 2, d.nz - 1, d.nz, d.nz + 1};
@@ -192,9 +199,41 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
                 for (int b = 0; b < d.Y1; ++b)
                     for (int a = 0; a < d.X1; ++a)
                         out.zmap[((size_t)p * 19 + s) * P2 + (size_t)b * d.X1 + a] = cell(i1(d, a, b, kk[p]), s);
+        if (jper) {
+            // copied ghost cells of the planes 1 .. nz read the cell they are copied from
+            for (size_t m = 0; m + 2 < raw[0].size(); m += 3) {
+                const int64_t dst = raw[0][m + 1], n2 = dst % P2;
+                const int k = (int)(dst / P2);
+                for (int p = 0; p < 6; ++p)
+                    if (kk[p] == k) out.zmap[((size_t)p * 19 + raw[0][m]) * P2 + n2] = cell(raw[0][m + 2], raw[0][m]);
+            }
+            out.bcp.assign((size_t)3 * 2 * 5 * d.nx * 3, -1);
+            const int bk[3] = {1, d.nz - 1, d.nz};
+            int count[3][2] = {};
+            std::vector<int> filled((size_t)3 * 2 * d.nx, 0);
+            for (size_t m = 0; m + 2 < raw[1].size(); m += 3) {
+                const int64_t dst = raw[1][m + 1];
+                const int k = (int)(dst / P2), j = (int)(dst % P2 / d.X1), i = (int)(dst % d.X1);
+                for (int p = 0; p < 3; ++p) {
+                    if (bk[p] != k) continue;
+                    const int side = j == 1 ? 0 : 1;
+                    int& at = filled[((size_t)p * 2 + side) * d.nx + i - 1];
+                    if (at >= 5) { err = "periodic copies of an open boundary column"; return false; }
+                    int32_t* c = &out.bcp[3 * ((((size_t)p * 2 + side) * 5 + at++) * d.nx + i - 1)];
+                    c[0] = raw[1][m];
+                    c[1] = cell(raw[1][m + 1], raw[1][m]);
+                    c[2] = cell(raw[1][m + 2], raw[1][m]);
+                    if (c[1] < 0 || c[2] < 0) { err = "periodic copy of an untracked cell"; return false; }
+                    ++count[p][side];
+                }
+            }
+            for (int p = 0; p < 3; ++p)
+                for (int side = 0; side < 2; ++side)
+                    if (count[p][side] != 5 * d.nx) { err = "periodic copies of an open boundary plane"; return false; }
+        }
     }
     // every access of the boundary kernels resolves through its plane map, looked up exactly as
-    // the kernels do (k_open_bc, k_porous_plate), to a cell of the layout
+    // the kernels do (k_boundary, k_porous_plate), to a cell of the layout
     {
         const int64_t P2 = (int64_t)d.X1 * d.Y1;
         StepConst<double> P{};
@@ -222,7 +261,6 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
         auto ph = [&](int, int, int) -> double& { return dummy; };
         auto cs = [&](int, int) -> double& { return dummy; };
         auto cp = [&]() -> double& { return dummy; };
-        const bool zmapped = open_z && (in_bc || out_bc);
         for (int j = 1; j <= d.ny && !bad; ++j)
             for (int i = 1; i <= d.nx; ++i) {
                 if (zmapped && in_bc == 1) {

@@ -1,6 +1,8 @@
-"""GPU parity of the step at the geometries where its boxes can go wrong: boxes with no node to
-compute, boxes without solid, a single box, rows just past a box edge.  FP64, so the state
-must equal the oracle's bit for bit."""
+"""GPU parity of the step at the geometries where its boxes can go wrong (boxes with no node to
+compute, boxes without solid, a single box, rows just past a box edge) and where its one
+boundary launch can (open boundaries of every kind on a periodic y axis, whose copies share
+cells with them, down to four planes).  FP64, so the state must equal the oracle's bit for
+bit."""
 import numpy as np
 import pytest
 
@@ -32,6 +34,11 @@ CASES = {
     "solid_boxes_ywalls": lambda: solid_block((35, 33, 30), 4, jper=0),
     "no_solid": lambda: no_solid((18, 17, 13), 5),
     "one_box": lambda: small_drainage(n=(12, 8, 5), seed=2, radius=2.0, porosity=0.6, jper=1, buffer=1),
+    "velocity_in_convective_out_yper": lambda: small_drainage(n=(11, 9, 14), seed=6, radius=2.5, porosity=0.55, jper=1,
+                                                              buffer=2, inlet=1, outlet=1),
+    "four_planes_convective_yper": lambda: small_drainage(n=(10, 6, 4), seed=2, radius=1.5, porosity=0.7, jper=1,
+                                                          buffer=1, inlet=1, outlet=1),
+    "four_planes_zouhe_yper": lambda: small_drainage(n=(9, 5, 4), seed=3, radius=1.5, porosity=0.7, jper=1, buffer=1),
     "one_past_a_box": lambda: small_drainage(n=(17, 9, 9), seed=4, radius=2.5, porosity=0.55, jper=1, buffer=2),
 }
 
@@ -51,5 +58,5 @@ def test_steps_bitwise(name):
             assert_same(g.download(field), o.array(field), 0.0, what=f"{name} step {t} {field}")
     o.run(4, 30)
     g.run(4, 30)
-    for field in ("pdf", "phi"):
+    for field in ("pdf", "phi") + (("convec",) if p["outlet_bc"] == 1 else ()):
         assert_same(g.download(field), o.array(field), 0.0, what=f"{name} step 33 {field}")

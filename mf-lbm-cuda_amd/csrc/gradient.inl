@@ -407,8 +407,10 @@ __global__ __launch_bounds__(GRAD_THREADS) void k_gradient(GradArgs<T> A, StepCo
 // classifies nothing (TileLists).  Classified by ballots in every step, 40 % of the vector
 // instructions went into the lists and 4 bytes of tag per loaded node; k_grad_force also
 // loaded the normals of solid nodes.  At 256^3 (drainage, porosity 0.40) the lists took
-// k_grad_force from 416 to 273 us in FP64 and 180 to 150 in FP32, k_grad_normals from 241 to 210
-// and 168 to 142.
+// k_grad_force from 416 to 268 us in FP64 and 180 to 145 in FP32, k_grad_normals from 241 to 205
+// and 168 to 135.  Leaving out the entries that no fluid node of the box reads (a box recomputes
+// the solid-boundary nodes of its halo) and loading the normals through a buffer descriptor, which
+// needs no branch per node, took k_grad_force to 257 and 133 us.
 
 // Owned box (i0, j0, k0) + [0, TX) x [0, TY) x [0, TZ) of this workgroup: boxes laid out x
 // fastest, `tx_n` x `ty_n` per z layer, the first at (org, org, org).
@@ -425,15 +427,43 @@ __device__ __forceinline__ void box_origin(int tx_n, int ty_n, int tz_n, int ord
     }
 }
 
+// K3/K6 weight sums (see k_gradient), evaluated at compile time in the same order.
+template <typename T>
+struct WeightSums {
+    T v[7 * 13];
+    constexpr WeightSums() : v() {
+        for (int a = 0; a < 7; ++a)
+            for (int dd = 0; dd < 13; ++dd) {
+                T ws = T(0);
+                for (int m = 0; m < a; ++m) ws += W<T>::w1;
+                for (int m = 0; m < dd; ++m) ws += W<T>::w2;
+                v[a * 13 + dd] = ws;
+            }
+    }
+};
+template <typename T>
+__device__ const WeightSums<T> weight_sums{};
 template <typename T>
 __device__ __forceinline__ void ws_table(T (*s_ws)[13], int tid) {
-    if (tid < 7 * 13) {
-        const int a = tid / 13, dd = tid % 13;
-        T ws = T(0);
-        for (int m = 0; m < a; ++m) ws += W<T>::w1;
-        for (int m = 0; m < dd; ++m) ws += W<T>::w2;
-        s_ws[a][dd] = ws;
-    }
+    if (tid < 7 * 13) s_ws[tid / 13][tid % 13] = weight_sums<T>.v[tid];
+}
+
+// The three normal components of the 4-vector `offset` bytes after p (up to 2^31 - 1), or zeros
+// for NOWHERE: the load goes through a buffer descriptor, whose bounds check drops the lane
+// without a branch.
+constexpr uint32_t NOWHERE = 0x80000000u;
+__device__ __forceinline__ void load_normal(const float* p, uint32_t offset, float& x, float& y, float& z) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, 0x7FFFFFFF, 0x00027000);
+    const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)offset, 0, 0));
+    x = v.x; y = v.y; z = v.z;
+}
+__device__ __forceinline__ void load_normal(const double* p, uint32_t offset, double& x, double& y, double& z) {
+    typedef double f64x2 __attribute__((ext_vector_type(2)));
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(p), 0, 0x7FFFFFFF, 0x00027000);
+    const f64x2 v = __builtin_bit_cast(f64x2, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)offset, 0, 0));
+    x = v.x; y = v.y;
+    z = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)offset, 16, 0));
 }
 
 // Box entries: position x | y << 5 | z << 9 in the loaded box of LX x LY x LZ nodes.
@@ -448,7 +478,8 @@ struct BoxEntry {
 
 // Work lists of the boxes of k_grad_normals (FORCE = false) or k_grad_force, one wave per box:
 // the sizes (FILL = false), then the entries in box order at the places the descriptor gives.
-// First list: solid-boundary nodes of the box and its 1-halo; second: its fluid nodes.
+// First list: the solid-boundary nodes of the box and its 1-halo that a fluid node of the box
+// reads (or, in k_grad_normals, that are written back); second: its fluid nodes.
 template <typename T, int TX, int TY, int TZ, bool FORCE, bool FILL>
 __global__ __launch_bounds__(64) void k_tile_lists(GradArgs<T> A, TileDesc* __restrict__ desc, uint32_t* __restrict__ la,
                                                    uint16_t* __restrict__ lb, int32_t* __restrict__ rec,
@@ -475,15 +506,24 @@ __global__ __launch_bounds__(64) void k_tile_lists(GradArgs<T> A, TileDesc* __re
         if (e < NL && i <= d.nx + loaded && j <= d.ny + loaded && k <= d.nz + loaded) t = A.tag[i4(d, i, j, k)];
         const bool halo = x >= 1 && x < ox + 3 && y >= 1 && y < oy + 3 && z >= 1 && z < oz + 3;
         const bool own = x >= 2 && x < ox + 2 && y >= 2 && y < oy + 2 && z >= 2 && z < oz + 2;
-        const bool fa = halo && (t & 3) == TAG_SOLID_BND, fb = own && tag_fluid(t & 3);
+        const bool fb = own && tag_fluid(t & 3);
+        // K3 writes the solid-boundary phi of [1, nx] x [1, ny] x [0, nz+1] back
+        const bool wb = !FORCE && own && i >= 1 && i <= d.nx && j >= 1 && j <= d.ny && k >= 0 && k <= d.nz + 1;
+        bool fa = halo && (t & 3) == TAG_SOLID_BND;
+        if (fa && !wb) {
+            // only what the stencil of one of the box's own fluid nodes reads
+            bool read = false;
+            for (int q = 1; q < 19; ++q) {
+                const int nx = x + EX[q], ny = y + EY[q], nz = z + EZ[q];
+                if (nx >= 2 && nx < ox + 2 && ny >= 2 && ny < oy + 2 && nz >= 2 && nz < oz + 2)
+                    read |= tag_fluid(A.tag[i4(d, i + EX[q], j + EY[q], k + EZ[q])] & 3);
+            }
+            fa = read;
+        }
         const uint64_t ma = __ballot(fa), mb = __ballot(fb);
         if (FILL) {
             const uint32_t at = Entry::pack(x, y, z), mask = (uint32_t)t >> 2;
-            if (fa) {
-                // K3 writes the solid-boundary phi of [1, nx] x [1, ny] x [0, nz+1] back
-                const bool wb = own && i >= 1 && i <= d.nx && j >= 1 && j <= d.ny && k >= 0 && k <= d.nz + 1;
-                la[na + below(ma)] = FORCE ? at | mask << 12 : at | (uint32_t)wb << 12 | mask << 13;
-            }
+            if (fa) la[na + below(ma)] = FORCE ? at | mask << 12 : at | (uint32_t)wb << 12 | mask << 13;
             if (fb) {
                 lb[nb + below(mb)] = (uint16_t)(FORCE ? at : at | (uint32_t)((t & 3) == TAG_WET) << 12);
                 if (FORCE) rec[nb + below(mb)] = t >> 2;
@@ -495,8 +535,7 @@ __global__ __launch_bounds__(64) void k_tile_lists(GradArgs<T> A, TileDesc* __re
     }
     if (!FILL) {
         if (lane == 0) {
-            desc[b].na = na;
-            desc[b].nb = nb;
+            desc[b] = TileDesc{0, na, 0, nb, i0, j0, k0, 0};
         }
         return;
     }
@@ -518,8 +557,7 @@ __global__ __launch_bounds__((TX + 4) * (TY + 4)) void k_grad_normals(GradArgs<T
     const int tid = threadIdx.x;
     const TileDesc td = A.lists.ndesc[xcd_block()];
     if ((td.na | td.nb) == 0) return;
-    int i0, j0, k0;
-    box_origin(A.tiles_x, A.tiles_y, A.tiles_z, A.box_order, -1, TX, TY, TZ, i0, j0, k0);
+    const int i0 = td.i0, j0 = td.j0, k0 = td.k0;
 
     // this thread's column; beyond n+4 it loads a clamped address (no list entry reads it)
     const int x = tid % LX, y = tid / LX;
@@ -607,8 +645,7 @@ __global__ __launch_bounds__((TX + 4) * (TY + 4)) void k_grad_force(GradArgs<T> 
     const int b = xcd_block();
     const TileDesc td = A.lists.fdesc[b];
     if (td.nb == 0) return;  // no record to write
-    int i0, j0, k0;
-    box_origin(A.tiles_x, A.tiles_y, A.tiles_z, A.box_order, 1, TX, TY, TZ, i0, j0, k0);
+    const int i0 = td.i0, j0 = td.j0, k0 = td.k0;
 
     // the fluid normals of the box with its 2-halo (inside [-1, n+2], where K4 wrote them):
     // only fluid entries are read before K6 writes the solid-boundary ones, so the lines of
@@ -628,18 +665,13 @@ __global__ __launch_bounds__((TX + 4) * (TY + 4)) void k_grad_force(GradArgs<T> 
         rec[m] = i < td.nb ? r7[i] : 0;
     }
     const int x = tid % LX, y = tid / LX;
-    const Vec4<T>* cnp = reinterpret_cast<const Vec4<T>*>(A.cnp);
     const int corner = i2(d, i0 - 2, j0 - 2, k0 - 2);
-    const int64_t n0 = corner + x + d.X2 * y, P2 = (int64_t)d.X2 * d.Y2;
+    const int64_t P2 = (int64_t)d.X2 * d.Y2;
+    const uint32_t col = (uint32_t)(x + d.X2 * y) * sizeof(Vec4<T>);
     T cv[LZ][3];
 #pragma unroll
-    for (int z = 0; z < LZ; ++z) {
-        cv[z][0] = cv[z][1] = cv[z][2] = T(0);
-        if ((fl >> z) & 1u) {
-            const Vec4<T> v = cnp[n0 + z * P2];
-            cv[z][0] = v.x; cv[z][1] = v.y; cv[z][2] = v.z;
-        }
-    }
+    for (int z = 0; z < LZ; ++z)
+        load_normal(A.cnp + 4 * (corner + z * P2), (fl >> z) & 1u ? col : NOWHERE, cv[z][0], cv[z][1], cv[z][2]);
     ws_table<T>(s_ws, tid);
 #pragma unroll
     for (int z = 0; z < LZ; ++z) {

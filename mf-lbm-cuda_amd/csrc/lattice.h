@@ -146,10 +146,11 @@ struct Sparse {
     }
 };
 
-// The two work lists of one box of the two-pass gradient chain: runs [a, a + na) and
-// [b, b + nb) of the chain's list arrays.
+// One box of the two-pass gradient chain: its two work lists, runs [a, a + na) and [b, b + nb)
+// of the chain's list arrays, and its first owned node.
 struct TileDesc {
     int32_t a, na, b, nb;
+    int32_t i0, j0, k0, pad;
 };
 
 // Work lists of the two-pass chain, built once from the geometry (k_tile_lists).  A box entry
@@ -201,14 +202,17 @@ constexpr int GRAD_SHAPE_DEFAULT = 0, GRAD_SHAPE_FP32 = 3;
 // the two-pass chain on 3-D tiles (k_grad_normals, k_grad_force): the shape after the
 // march shapes
 constexpr int GRAD_SHAPE_TILES = GRAD_NSHAPES;
-// owned nodes (x, y, z) of a workgroup of k_grad_normals (N) and k_grad_force (F), per precision
+// owned nodes (x, y, z) of a workgroup of k_grad_normals (N) and k_grad_force (F), per precision;
+// us per launch at 256^3, drainage: force FP64 16x8x4 268, 16x6x4 273, 12x12x4 279, FP32 12x8x4
+// 136, 12x12x4 137, 16x8x4 145; boxes of more than 256 threads 420 to 470; normals 16x8x4 204 and
+// 135, the other shapes up to 223 and 147 (28x8x4 131 in FP32)
 template <typename T>
 struct GradTiles {
     static constexpr int N[3] = {16, 8, 4}, F[3] = {16, 8, 4};
 };
 template <>
 struct GradTiles<float> {
-    static constexpr int N[3] = {16, 8, 4}, F[3] = {16, 8, 4};
+    static constexpr int N[3] = {16, 8, 4}, F[3] = {12, 8, 4};
 };
 
 // Uniform deviate in [0, 1) of lattice node n under a seed, for the random initial phase

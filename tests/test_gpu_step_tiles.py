@@ -60,3 +60,18 @@ def test_steps_bitwise(name):
     g.run(4, 30)
     for field in ("pdf", "phi") + (("convec",) if p["outlet_bc"] == 1 else ()):
         assert_same(g.download(field), o.array(field), 0.0, what=f"{name} step 33 {field}")
+
+
+@pytest.mark.parametrize("n", [(11, 7, 6), (12, 8, 9), (13, 17, 8), (25, 9, 13)])
+def test_fp32_boxes_match_the_split_chain(n):
+    """FP32 at the edges of its 12 x 8 x 4 and 16 x 8 x 4 boxes, against the kernels of one stage
+    each.  Contraction is allowed in FP32, so the two round differently; the bound is that of the
+    parity test of the two paths."""
+    geo, p = small_drainage(n=n, seed=7, radius=2.0, porosity=0.6, jper=1, buffer=1)
+    print(f"[gpu-step-tiles] fp32 {n}", flush=True)
+    a, b = gpu.Solver(p, geo, gpu.FP32), gpu.Solver(p, geo, gpu.FP32, split_gradient=True)
+    for s in (a, b):
+        s.setup()
+        s.run(1, 30)
+    for field in ("pdf", "phi"):
+        assert_same(a.download(field), b.download(field), 1e-5, what=f"{n} {field}")

@@ -60,7 +60,7 @@ struct mflbm_handle {
     int32_t* pairs[2] = {nullptr, nullptr};
     int npairs[2] = {0, 0};
     int32_t* zmap = nullptr;
-    int32_t* bcp = nullptr;     // periodic copies of odd steps that the open boundaries make
+    int32_t* zread[2] = {nullptr, nullptr};  // the map as read after even and odd steps (null: zmap)
     int32_t* pmap = nullptr;    // porous-plate plane map
     int in_bc = 0, out_bc = 0;  // open z: 1 velocity inlet / convective outlet, 2 Zou-He
     int plate_z = 0, plate_blocked = 0;
@@ -195,7 +195,8 @@ void enqueue_step(mflbm_handle* h, bool odd, hipEvent_t* ev) {
             B.in_bc = h->in_bc;
             B.out_bc = h->out_bc;
         }
-        B.zmap = h->zmap; B.w_in = (const T*)h->w_in; B.conv = (T*)h->conv; B.bcp = h->bcp;
+        B.zread = h->zread[odd ? 1 : 0] ? h->zread[odd ? 1 : 0] : h->zmap;
+        B.zmap = h->zmap; B.w_in = (const T*)h->w_in; B.conv = (T*)h->conv;
         B.pairs = h->pairs[odd ? 1 : 0]; B.npairs = h->npairs[odd ? 1 : 0];
         B.kper = h->p.kper; B.jper = h->p.jper;
         Launch<T>::boundary(S, F, P, B, odd, s);
@@ -312,7 +313,7 @@ void free_all(mflbm_handle* h) {
         if (h->graph[g]) { (void)hipGraphExecDestroy(h->graph[g]); h->graph[g] = nullptr; }
     void* ptrs[] = {h->pdf, h->phi, h->cnx, h->cny, h->cnz, h->cnorm, h->cnp, h->snp, h->curv, h->snx, h->sny, h->snz,
                     h->walls, h->wtype, h->l_fluid, h->l_fluid_ext, h->l_sb, h->mon_part, h->mon_out, h->vprev, h->vpart,
-                    h->cells, h->aux, h->nb, h->nb16, h->nbb, h->pairs[0], h->pairs[1], h->zmap, h->bcp, h->pmap, h->w_in, h->conv,
+                    h->cells, h->aux, h->nb, h->nb16, h->nbb, h->pairs[0], h->pairs[1], h->zmap, h->zread[0], h->zread[1], h->pmap, h->w_in, h->conv,
                     h->ext_node, h->ext_off, h->zstart,
                     h->tag, h->macro_buf, h->ndesc, h->fdesc, h->l3, h->l4, h->l6, h->l7, h->r7, h->tile_fluid};
     for (void* p : ptrs)
@@ -325,7 +326,7 @@ void free_all(mflbm_handle* h) {
     h->cells = h->aux = nullptr;
     h->nb16 = nullptr;
     h->nbb = nullptr;
-    h->nb = h->pairs[0] = h->pairs[1] = h->zmap = h->bcp = h->pmap = h->ext_node = h->ext_off = h->zstart = nullptr;
+    h->nb = h->pairs[0] = h->pairs[1] = h->zmap = h->zread[0] = h->zread[1] = h->pmap = h->ext_node = h->ext_off = h->zstart = nullptr;
     h->w_in = h->conv = nullptr;
     h->tag = nullptr;
     h->ndesc = h->fdesc = nullptr;
@@ -677,7 +678,8 @@ int mflbm_create(const mflbm_params* params, const int8_t* geometry, mflbm_handl
     h->npairs[0] = (int)(lay.pairs[0].size() / 3);
     h->npairs[1] = (int)(lay.pairs[1].size() / 3);
     HIPCHK(h, upload_i32(&h->zmap, lay.zmap));
-    if (!lay.bcp.empty()) HIPCHK(h, upload_i32(&h->bcp, lay.bcp));
+    for (int o = 0; o < 2; ++o)
+        if (!lay.zread[o].empty()) HIPCHK(h, upload_i32(&h->zread[o], lay.zread[o]));
     if (h->plate_z) HIPCHK(h, upload_i32(&h->pmap, lay.pmap));
     {
         const int64_t P2 = (int64_t)d.X1 * d.Y1;

@@ -488,26 +488,79 @@ __device__ __forceinline__ void periodic_phi(T* __restrict__ phi, const Dims& d,
     }
 }
 
+// A population cell of both colours in registers: get, set as ColourRef reads and writes them in
+// shifted storage, put stores.
+template <typename T>
+struct ColourCell {
+    T* p1;
+    T* p2;
+    T a, b, rest;
+    __device__ __forceinline__ T get(int g) const {
+        if (ShiftedStorage<T>::value) return g == 0 ? a : (b + rest) - a;
+        return g == 0 ? a : b;
+    }
+    __device__ __forceinline__ void set(int g, T v) {
+        if (!ShiftedStorage<T>::value) {
+            if (g == 0) a = v;
+            else b = v;
+        } else if (g == 0) {
+            const T g2 = (b + rest) - a;
+            a = v;
+            b = (v + g2) - rest;
+        } else {
+            b = (a + v) - rest;
+        }
+    }
+    __device__ __forceinline__ void put() const {
+        *p1 = a;
+        *p2 = b;
+    }
+};
+
+// Cells of the open boundaries, through the plane maps zread and zmap ([plane][slot][b * (nx+2)
+// + a], planes k = 0, 1, 2, nz-1, nz, nz+1).
+template <typename T>
+struct OpenCells {
+    const Sparse<T>& S;
+    const int32_t* __restrict__ zread;
+    const int32_t* __restrict__ zmap;
+    int64_t P2;
+    int X1, nz;
+    T rho_ref;
+    __device__ __forceinline__ int64_t at(int a, int b, int c, int e) const {
+        return (int64_t)((c <= 2 ? c : 3 + (c - (nz - 1))) * 19 + e) * P2 + b * X1 + a;
+    }
+    __device__ __forceinline__ ColourCell<T> rd(int a, int b, int c, int e) const {
+        const int64_t r = zread[at(a, b, c, e)];
+        T *p1 = S.f + S.at(e, r), *p2 = S.f + S.at(e + 19, r);
+        return {p1, p2, *p1, *p2, rho_ref * (T)rest_weight(e)};
+    }
+    __device__ __forceinline__ ColourCell<T> rw(int a, int b, int c, int e) const {
+        ColourCell<T> x = rd(a, b, c, e);
+        const int64_t w = zmap[at(a, b, c, e)];
+        x.p1 = S.f + S.at(e, w);
+        x.p2 = S.f + S.at(e + 19, w);
+        return x;
+    }
+};
+
 // The boundary updates between the collision and the gradient chain in one launch: open
 // inlet/outlet columns, periodic population copies, periodic phi, each in workgroups of its
 // own (nbc, then npair, then the rest).  The reference copies the periodic populations first
-// and the open boundaries then read and write some of the copied cells; here the order is
-// kept without a launch between them:
-//   after an even step the open boundaries read, of the copied cells, ghost cells only, and
-//   write none of the copies' cells; zmap gives, for a copied ghost cell, the cell it is
-//   copied from, which holds the same value;
-//   after an odd step a column's open boundary touches cells of its own column only, so the
-//   thread of a column at j = 1 or ny makes the copies into the planes its boundary touches
-//   (bcp) before it, and the list of copies leaves them out.
+// and the open boundaries then read and write some of the copied cells; here the order needs
+// no launch between them:
+//   the open boundaries read a copy's destination where it is copied from (zread), a cell that
+//   neither they nor another copy writes;
+//   after an even step they write none of the copies' cells; after an odd step they write, of
+//   the copies' destinations, slots 17, 18 of plane 1 and 15, 16 of plane nz, and the list of
+//   copies leaves those out.
 // phi: the open boundaries write ghost planes in z of interior columns, the periodic copies
 // read and write planes 1 .. nz.
-// On domains of 32^3 to 64^3 a launch costs 4.5 us whatever it does: three of them took 18 of a
-// step's 39 to 45 us, the merged one 9.
+// On domains of 32^3 to 64^3 a launch costs 4.5 us whatever it does: as three launches they took
+// 18 of a step's 39 to 45 us, now 8 of 25 to 30.
 //
 // Open inlet/outlet, one thread per (i, j): in_bc / out_bc 2 = Zou-He, 1 = velocity inlet /
-// convective outlet.  zmap[plane][slot][b * (nx+2) + a] gives the cell of (a, b, k) for the
-// six planes k = 0, 1, 2, nz-1, nz, nz+1.  w_in: the inlet velocity plane (X1 * Y1);
-// conv: the convective-outlet state, 38 planes of populations [g][e] then phi.
+// convective outlet.  w_in: the inlet velocity plane (X1 * Y1); conv: the convective-outlet state, 38 planes of populations [g][e] then phi.
 template <typename T, bool AFTER_ODD>
 __global__ __launch_bounds__(256) void k_boundary(Sparse<T> S, Fields<T> F, StepConst<T> P, BoundaryArgs<T> B) {
     const Dims& d = F.d;
@@ -529,32 +582,17 @@ __global__ __launch_bounds__(256) void k_boundary(Sparse<T> S, Fields<T> F, Step
         else { in_bc = 0; t -= d.nx * d.ny; }
     }
     const int i = t % d.nx + 1, j = t / d.nx + 1, nz = d.nz;
-    const int64_t P2 = (int64_t)d.X1 * d.Y1, plane = 19 * P2;
-    if (AFTER_ODD && B.bcp && (j == 1 || j == d.ny)) {
-        // planes 1 (inlet), nz - 1 and nz (outlet); five slots each, (slot, dst, src)
-        for (int p = in_bc ? 0 : 1; p < (out_bc ? 3 : 1); ++p)
-#pragma unroll
-            for (int m = 0; m < 5; ++m) {
-                const int32_t* c = B.bcp + 3 * ((((int64_t)p * 2 + (j == 1 ? 0 : 1)) * 5 + m) * d.nx + i - 1);
-                copy_cell(S, c[0], c[1], c[2]);
-            }
-    }
-    auto cell_of = [&](int a, int b, int c, int e) -> int64_t {
-        const int pl = c <= 2 ? c : 3 + (c - (nz - 1));
-        return B.zmap[pl * plane + (int64_t)e * P2 + b * d.X1 + a];
-    };
     auto wall = [&](int a, int b, int c) -> int { return F.walls[i2(d, a, b, c)]; };
     auto ph = [&](int a, int b, int c) -> T& { return F.phi[i4(d, a, b, c)]; };
-    const int64_t col = (int64_t)j * d.X1 + i;
-    with_cells<T>(S, P.rho_ref, cell_of, [&](auto&& f) {
-        if (in_bc == 1) velocity_inlet_column<T, AFTER_ODD>(P, i, j, B.w_in[col], f, wall, ph);
-        if (in_bc == 2 || out_bc == 2) zou_he_column<T, AFTER_ODD>(P, i, j, nz, in_bc == 2, out_bc == 2, f, wall, ph);
-        if (out_bc == 1) {
-            auto cs = [&](int e, int g) -> T& { return B.conv[(int64_t)(e + 19 * g) * P2 + col]; };
-            auto cp = [&]() -> T& { return B.conv[38 * P2 + col]; };
-            convective_outlet_column<T, AFTER_ODD>(P, i, j, nz, f, wall, ph, cs, cp);
-        }
-    });
+    const int64_t P2 = (int64_t)d.X1 * d.Y1, col = (int64_t)j * d.X1 + i;
+    const OpenCells<T> f{S, B.zread, B.zmap, P2, d.X1, nz, P.rho_ref};
+    if (in_bc == 1) velocity_inlet_column<T, AFTER_ODD>(P, i, j, B.w_in[col], f, wall, ph);
+    if (in_bc == 2 || out_bc == 2) zou_he_column<T, AFTER_ODD>(P, i, j, nz, in_bc == 2, out_bc == 2, f, wall, ph);
+    if (out_bc == 1) {
+        auto cs = [&](int e, int g) -> T& { return B.conv[(int64_t)(e + 19 * g) * P2 + col]; };
+        auto cp = [&]() -> T& { return B.conv[38 * P2 + col]; };
+        convective_outlet_column<T, AFTER_ODD>(P, i, j, nz, f, wall, ph, cs, cp);
+    }
 }
 
 // Porous plate at k = zp, one thread per (i, j); pmap as zmap for the planes zp-1, zp, zp+1.

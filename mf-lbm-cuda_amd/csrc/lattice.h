@@ -81,12 +81,12 @@ struct StepConst {
 template <typename T>
 struct BoundaryArgs {
     int nbc, npair;                      // workgroups of the open boundaries, of the periodic copies
-    const int32_t* __restrict__ zmap;    // open boundaries
+    const int32_t* __restrict__ zread;   // open boundaries: cells as read and as written
+    const int32_t* __restrict__ zmap;
     int in_bc, out_bc, split;
     const T* __restrict__ w_in;
     T* __restrict__ conv;
-    const int32_t* __restrict__ bcp;     // copies made by the open boundaries' threads (odd steps)
-    const int32_t* __restrict__ pairs;   // (slot, dst, src) of the other periodic copies
+    const int32_t* __restrict__ pairs;   // (slot, dst, src) of the periodic copies
     int npairs, kper, jper;
 };
 

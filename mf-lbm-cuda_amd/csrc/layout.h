@@ -20,13 +20,10 @@ struct LayoutHost {
     std::vector<int32_t> ext_node;  // s1 node of every extra cell, grouped by slot
     std::vector<int32_t> ext_off;   // 20 offsets into ext_node
     std::vector<int32_t> pairs[2];  // periodic copies (slot, dst, src) for [0] even, [1] odd steps
-    // open z only: 6 planes * 19 slots * X1 * Y1 cells; a y-periodic ghost cell that the even
-    // steps copy is given as the cell it is copied from
-    std::vector<int32_t> zmap;
-    // open z, periodic y: the odd steps' copies into the planes the open boundaries touch, made
-    // by their threads instead of by pairs[1]: (slot, dst, src) of [plane 1, nz-1, nz][j = 1,
-    // ny][5 slots][nx]
-    std::vector<int32_t> bcp;
+    std::vector<int32_t> zmap;      // 6 planes * 19 slots * X1 * Y1 (open z only)
+    // open z, periodic y: zmap as the open boundaries read it after even and odd steps, where a
+    // periodic copy's destination is given as the cell it is copied from
+    std::vector<int32_t> zread[2];
     std::vector<int32_t> pmap;      // porous plate: 3 planes (zp-1, zp, zp+1) * 19 slots * X1 * Y1
     std::vector<int32_t> zstart;    // nz + 1 offsets of the z-slices in the fluid list
 };

@@ -57,10 +57,9 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
         StepConst<double> P{};
         double dummy = 0.0;
         bool bad = false;
-        auto rec = [&](int a, int b, int c, int e, int) -> double& {
+        CellRecorder rec{[&](int a, int b, int c, int e, bool) {
             if (!note(i1(d, a, b, c), e)) bad = true;
-            return dummy;
-        };
+        }};
         auto wall = [&](int, int, int) -> int { return 0; };
         auto ph = [&](int, int, int) -> double& { return dummy; };
         for (int j = 1; j <= d.ny; ++j)
@@ -75,7 +74,10 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
         StepConst<double> P{};
         double dummy = 0.0;
         bool bad = false;
-        auto rec = [&](int a, int b, int c, int e, int) -> double& {
+        CellRecorder rec{[&](int a, int b, int c, int e, bool) {
+            if (!note(i1(d, a, b, c), e)) bad = true;
+        }};
+        auto prec = [&](int a, int b, int c, int e, int) -> double& {
             if (!note(i1(d, a, b, c), e)) bad = true;
             return dummy;
         };
@@ -94,10 +96,10 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
                     convective_outlet_column<double, true>(P, i, j, d.nz, rec, wall, ph, cs, cp);
                 }
                 if (plate_z >= 1 && plate_z <= d.nz) {
-                    porous_plate_column<false>(i, j, plate_z, 0, rec);
-                    porous_plate_column<true>(i, j, plate_z, 0, rec);
-                    porous_plate_column<false>(i, j, plate_z, 1, rec);
-                    porous_plate_column<true>(i, j, plate_z, 1, rec);
+                    porous_plate_column<false>(i, j, plate_z, 0, prec);
+                    porous_plate_column<true>(i, j, plate_z, 0, prec);
+                    porous_plate_column<false>(i, j, plate_z, 1, prec);
+                    porous_plate_column<true>(i, j, plate_z, 1, prec);
                 }
             }
         if (bad) { err = "boundary access outside the population array"; return false; }
@@ -152,13 +154,13 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
             out.n_escaped += e;
         }
     }
-    // periodic pairs, last writer wins; on odd steps without the copies into the planes the open
-    // boundaries touch (inlet 1, outlet nz-1 and nz), which their threads make (bcp)
+    // periodic pairs, last writer wins; on odd steps without the copies into cells that the open
+    // boundaries write (their threads read the copy's source instead)
     const bool zmapped = open_z && (in_bc || out_bc);
-    auto bc_plane = [&](int64_t n) {
+    auto bc_writes = [&](int64_t n, int slot) {
         if (!zmapped || !jper) return false;
         const int k = (int)(n / ((int64_t)d.X1 * d.Y1));
-        return (in_bc && k == 1) || (out_bc && (k == d.nz - 1 || k == d.nz));
+        return (in_bc && k == 1 && (slot == 17 || slot == 18)) || (out_bc && k == d.nz && (slot == 15 || slot == 16));
     };
     for (int odd = 0; odd < 2; ++odd) {
         const std::vector<int32_t>& r = raw[odd];
@@ -170,7 +172,7 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
         for (size_t m = 0; m + 1 < n; ++m)
             if (key[m].first == key[m + 1].first) keep[key[m].second] = 0;  // a later copy overwrites it
         for (size_t m = 0; m < n; ++m) {
-            if (!keep[m] || (odd && bc_plane(r[3 * m + 1]))) continue;
+            if (!keep[m] || (odd && bc_writes(r[3 * m + 1], r[3 * m]))) continue;
             const int s = r[3 * m];
             const int32_t cd = cell(r[3 * m + 1], s), cs = cell(r[3 * m + 2], s);
             if (cd < 0 || cs < 0) { err = "periodic copy of an untracked cell"; return false; }
@@ -199,37 +201,17 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
                 for (int b = 0; b < d.Y1; ++b)
                     for (int a = 0; a < d.X1; ++a)
                         out.zmap[((size_t)p * 19 + s) * P2 + (size_t)b * d.X1 + a] = cell(i1(d, a, b, kk[p]), s);
-        if (jper) {
-            // copied ghost cells of the planes 1 .. nz read the cell they are copied from
-            for (size_t m = 0; m + 2 < raw[0].size(); m += 3) {
-                const int64_t dst = raw[0][m + 1], n2 = dst % P2;
+        // read maps: a periodic copy's destination reads the cell it is copied from
+        for (int odd = 0; odd < 2; ++odd) {
+            if (!jper) break;
+            out.zread[odd] = out.zmap;
+            for (size_t m = 0; m + 2 < raw[odd].size(); m += 3) {
+                const int64_t dst = raw[odd][m + 1], n2 = dst % P2;
                 const int k = (int)(dst / P2);
                 for (int p = 0; p < 6; ++p)
-                    if (kk[p] == k) out.zmap[((size_t)p * 19 + raw[0][m]) * P2 + n2] = cell(raw[0][m + 2], raw[0][m]);
+                    if (kk[p] == k)
+                        out.zread[odd][((size_t)p * 19 + raw[odd][m]) * P2 + n2] = cell(raw[odd][m + 2], raw[odd][m]);
             }
-            out.bcp.assign((size_t)3 * 2 * 5 * d.nx * 3, -1);
-            const int bk[3] = {1, d.nz - 1, d.nz};
-            int count[3][2] = {};
-            std::vector<int> filled((size_t)3 * 2 * d.nx, 0);
-            for (size_t m = 0; m + 2 < raw[1].size(); m += 3) {
-                const int64_t dst = raw[1][m + 1];
-                const int k = (int)(dst / P2), j = (int)(dst % P2 / d.X1), i = (int)(dst % d.X1);
-                for (int p = 0; p < 3; ++p) {
-                    if (bk[p] != k) continue;
-                    const int side = j == 1 ? 0 : 1;
-                    int& at = filled[((size_t)p * 2 + side) * d.nx + i - 1];
-                    if (at >= 5) { err = "periodic copies of an open boundary column"; return false; }
-                    int32_t* c = &out.bcp[3 * ((((size_t)p * 2 + side) * 5 + at++) * d.nx + i - 1)];
-                    c[0] = raw[1][m];
-                    c[1] = cell(raw[1][m + 1], raw[1][m]);
-                    c[2] = cell(raw[1][m + 2], raw[1][m]);
-                    if (c[1] < 0 || c[2] < 0) { err = "periodic copy of an untracked cell"; return false; }
-                    ++count[p][side];
-                }
-            }
-            for (int p = 0; p < 3; ++p)
-                for (int side = 0; side < 2; ++side)
-                    if (count[p][side] != 5 * d.nx) { err = "periodic copies of an open boundary plane"; return false; }
         }
     }
     // every access of the boundary kernels resolves through its plane map, looked up exactly as
@@ -239,15 +221,16 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
         StepConst<double> P{};
         double dummy = 0.0;
         bool bad = false;
-        auto zrec = [&](int a, int b, int c, int e, int) -> double& {
+        int odd = 0;
+        CellRecorder zrec{[&](int a, int b, int c, int e, bool written) {
             const int pl = c <= 2 ? c : 3 + (c - (d.nz - 1));
             if (pl < 0 || pl > 5 || a < 0 || a >= d.X1 || b < 0 || b >= d.Y1 || e < 0 || e >= 19) bad = true;
             else {
-                const int32_t c2 = out.zmap[((size_t)pl * 19 + e) * P2 + (size_t)b * d.X1 + a];
-                if (c2 < 0 || c2 >= out.ns) bad = true;
+                const size_t at = ((size_t)pl * 19 + e) * P2 + (size_t)b * d.X1 + a;
+                const int32_t r2 = jper ? out.zread[odd][at] : out.zmap[at], w2 = written ? out.zmap[at] : r2;
+                if (r2 < 0 || r2 >= out.ns || w2 < 0 || w2 >= out.ns) bad = true;
             }
-            return dummy;
-        };
+        }};
         auto prec = [&](int a, int b, int c, int e, int) -> double& {
             const int pl = c - (plate_z - 1);
             if (pl < 0 || pl > 2 || a < 0 || a >= d.X1 || b < 0 || b >= d.Y1 || e < 0 || e >= 19) bad = true;
@@ -263,18 +246,14 @@ bool build_layout(const Dims& d, const std::vector<uint32_t>& fluid, int kper, i
         auto cp = [&]() -> double& { return dummy; };
         for (int j = 1; j <= d.ny && !bad; ++j)
             for (int i = 1; i <= d.nx; ++i) {
-                if (zmapped && in_bc == 1) {
-                    velocity_inlet_column<double, false>(P, i, j, 0.0, zrec, wall, ph);
-                    velocity_inlet_column<double, true>(P, i, j, 0.0, zrec, wall, ph);
-                }
-                if (zmapped && (zou_in || zou_out)) {
-                    zou_he_column<double, false>(P, i, j, d.nz, zou_in, zou_out, zrec, wall, ph);
-                    zou_he_column<double, true>(P, i, j, d.nz, zou_in, zou_out, zrec, wall, ph);
-                }
-                if (zmapped && out_bc == 1) {
-                    convective_outlet_column<double, false>(P, i, j, d.nz, zrec, wall, ph, cs, cp);
-                    convective_outlet_column<double, true>(P, i, j, d.nz, zrec, wall, ph, cs, cp);
-                }
+                odd = 0;
+                if (zmapped && in_bc == 1) velocity_inlet_column<double, false>(P, i, j, 0.0, zrec, wall, ph);
+                if (zmapped && (zou_in || zou_out)) zou_he_column<double, false>(P, i, j, d.nz, zou_in, zou_out, zrec, wall, ph);
+                if (zmapped && out_bc == 1) convective_outlet_column<double, false>(P, i, j, d.nz, zrec, wall, ph, cs, cp);
+                odd = 1;
+                if (zmapped && in_bc == 1) velocity_inlet_column<double, true>(P, i, j, 0.0, zrec, wall, ph);
+                if (zmapped && (zou_in || zou_out)) zou_he_column<double, true>(P, i, j, d.nz, zou_in, zou_out, zrec, wall, ph);
+                if (zmapped && out_bc == 1) convective_outlet_column<double, true>(P, i, j, d.nz, zrec, wall, ph, cs, cp);
                 if (plate_z >= 1 && plate_z <= d.nz)
                     for (int blocked = 0; blocked < 2; ++blocked) {
                         porous_plate_column<false>(i, j, plate_z, blocked, prec);

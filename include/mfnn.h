@@ -78,6 +78,21 @@ int mfnn_pool2(const void* x, int32_t D, int32_t H, int32_t W, int32_t C, void* 
 int mfnn_up2(const void* x, int32_t D, int32_t H, int32_t W, int32_t C, int32_t ct, int32_t c0, void* y,
              int32_t backward, void* stream);
 
+/* up2 of `low` (cl channels) and the cs channels of `skip` (D x H x W x cs) beside it, into
+ * channels [c0, c0 + cl + cs) of a ct-channel tensor in one pass. */
+int mfnn_up2_cat(const void* low, int32_t cl, const void* skip, int32_t cs, int32_t D, int32_t H, int32_t W, int32_t ct,
+                 int32_t c0, void* y, void* stream);
+
+/* Adjoint of up2 on channels [c0, c0 + C) of dy (D x H x W x ct), times [gate > 0] (gate: the
+ * coarse activation; optional). */
+int mfnn_up2_split(const void* dy, int32_t D, int32_t H, int32_t W, int32_t C, int32_t ct, int32_t c0, const void* gate,
+                   void* dx, void* stream);
+
+/* (a + adjoint of pool2 on dy) * [gate > 0] on the D x H x W grid: a is channels [ca0, ca0 + C) of a
+ * ca-channel tensor; a and gate optional. */
+int mfnn_pool2_merge(const void* dy, int32_t D, int32_t H, int32_t W, int32_t C, const void* a, int32_t ca, int32_t ca0,
+                     const void* gate, void* out, void* stream);
+
 /* copy channels [c0, c0 + C) between a C-channel and a ct-channel tensor of nvox voxels
  * (into_wide != 0: narrow -> wide, else wide -> narrow). */
 int mfnn_channels(const void* src, int64_t nvox, int32_t C, int32_t ct, int32_t c0, int32_t into_wide, void* dst,

@@ -43,6 +43,9 @@ SIGNATURES = {
     "mfnn_to_bf16": [_vp, _i64, _vp, _vp],
     "mfnn_pool2": [_vp, _i32, _i32, _i32, _i32, _vp, _i32, _vp],
     "mfnn_up2": [_vp, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _i32, _vp],
+    "mfnn_up2_cat": [_vp, _i32, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp],
+    "mfnn_up2_split": [_vp, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp],
+    "mfnn_pool2_merge": [_vp, _i32, _i32, _i32, _i32, _vp, _i32, _i32, _vp, _vp, _vp],
     "mfnn_channels": [_vp, _i64, _i32, _i32, _i32, _i32, _vp, _vp],
     "mfnn_add_gate": [_vp, _vp, _vp, _i64, _vp, _vp],
     "mfnn_mse_partials": [_i64, _i32],
@@ -296,8 +299,7 @@ class UNet:
 
         def cat(name, low, lowC, skip, skipC, shape):
             out = self._t(name, shape + (lowC + skipC,))
-            _chk(L.mfnn_up2(ptr(low), *shape, lowC, lowC + skipC, 0, ptr(out), 0, stream), "up")
-            _chk(L.mfnn_channels(ptr(skip), int(np.prod(shape)), skipC, lowC + skipC, lowC, 1, ptr(out), stream), "cat")
+            _chk(L.mfnn_up2_cat(ptr(low), lowC, ptr(skip), skipC, *shape, lowC + skipC, 0, ptr(out), stream), "cat")
             a[name] = out
             return out
 
@@ -333,52 +335,46 @@ class UNet:
         cv = self.conv
         g = lambda name, shape, C_: self._t("g_" + name, shape + (C_,))
 
-        def split_up(gcat, lowC, skipC, shape_fine, name_low, name_skip, gate_low):
-            # gradient of the upsampled part -> coarse grid (then the ReLU of the coarse
-            # activation), gradient of the skip part -> its own buffer
+        def split_up(gcat, lowC, skipC, shape_fine, name_low, gate_low):
+            # gradient of the upsampled part -> coarse grid, then the ReLU of the coarse
+            # activation; the skip part is read from gcat where it meets the pooled branch
             shape_c = (shape_fine[0] // 2, shape_fine[1] // 2, shape_fine[2] // 2)
-            glow = g(name_low + "_u", shape_c, lowC)
-            _chk(L.mfnn_up2(ptr(gcat), *shape_fine, lowC, lowC + skipC, 0, ptr(glow), 1, stream), "up bwd")
-            glow_g = g(name_low, shape_c, lowC)
-            _chk(L.mfnn_add_gate(ptr(glow), None, ptr(gate_low), glow.numel(), ptr(glow_g), stream), "gate")
-            gskip = g(name_skip + "_s", shape_fine, skipC)
-            _chk(L.mfnn_channels(ptr(gcat), int(np.prod(shape_fine)), skipC, lowC + skipC, lowC, 0, ptr(gskip), stream),
-                 "split")
-            return glow_g, gskip
+            glow = g(name_low, shape_c, lowC)
+            _chk(L.mfnn_up2_split(ptr(gcat), *shape_fine, lowC, lowC + skipC, 0, ptr(gate_low), ptr(glow), stream), "split")
+            return glow
 
-        def merge_pool(gskip, gpooled, shape_fine, C_, gate, name):
-            gp = g(name + "_p", shape_fine, C_)
-            _chk(L.mfnn_pool2(ptr(gpooled), *shape_fine, C_, ptr(gp), 1, stream), "pool bwd")
+        def merge_pool(gcat, lowC, gpooled, shape_fine, C_, gate, name):
             out = g(name, shape_fine, C_)
-            _chk(L.mfnn_add_gate(ptr(gskip), ptr(gp), ptr(gate), out.numel(), ptr(out), stream), "merge")
+            _chk(L.mfnn_pool2_merge(ptr(gpooled), *shape_fine, C_, ptr(gcat), lowC + C_, lowC, ptr(gate), ptr(out),
+                                    stream), "merge")
             return out
 
         gd11 = g("d11", s0, c0)
         cv["head"].backward(a["d11"], gy, s0, work, acc, dx=gd11, gate=a["d11"], stream=stream)
         gc3 = g("c3", s0, c1 + c0)
         cv["d11"].backward(a["c3"], gd11, s0, work, acc, dx=gc3, stream=stream)
-        gd10, ge2_a = split_up(gc3, c1, c0, s0, "d10", "e2", a["d10"])
+        gd10 = split_up(gc3, c1, c0, s0, "d10", a["d10"])
         gc2 = g("c2", s1, c2 + c1)
         cv["d10"].backward(a["c2"], gd10, s1, work, acc, dx=gc2, stream=stream)
-        gd9, ge4_a = split_up(gc2, c2, c1, s1, "d9", "e4", a["d9"])
+        gd9 = split_up(gc2, c2, c1, s1, "d9", a["d9"])
         gc1 = g("c1", s2, c3 + c2)
         cv["d9"].backward(a["c1"], gd9, s2, work, acc, dx=gc1, stream=stream)
-        ge8, ge6_a = split_up(gc1, c3, c2, s2, "e8", "e6", a["e8"])
+        ge8 = split_up(gc1, c3, c2, s2, "e8", a["e8"])
         ge7 = g("e7", s3, c3)
         cv["e8"].backward(a["e7"], ge8, s3, work, acc, dx=ge7, gate=a["e7"], stream=stream)
         gp3 = g("p3", s3, c2)
         cv["e7"].backward(a["p3"], ge7, s3, work, acc, dx=gp3, stream=stream)
-        ge6 = merge_pool(ge6_a, gp3, s2, c2, a["e6"], "e6")
+        ge6 = merge_pool(gc1, c3, gp3, s2, c2, a["e6"], "e6")
         ge5 = g("e5", s2, c2)
         cv["e6"].backward(a["e5"], ge6, s2, work, acc, dx=ge5, gate=a["e5"], stream=stream)
         gp2 = g("p2", s2, c1)
         cv["e5"].backward(a["p2"], ge5, s2, work, acc, dx=gp2, stream=stream)
-        ge4 = merge_pool(ge4_a, gp2, s1, c1, a["e4"], "e4")
+        ge4 = merge_pool(gc2, c2, gp2, s1, c1, a["e4"], "e4")
         ge3 = g("e3", s1, c1)
         cv["e4"].backward(a["e3"], ge4, s1, work, acc, dx=ge3, gate=a["e3"], stream=stream)
         gp1 = g("p1", s1, c0)
         cv["e3"].backward(a["p1"], ge3, s1, work, acc, dx=gp1, stream=stream)
-        ge2 = merge_pool(ge2_a, gp1, s0, c0, a["e2"], "e2")
+        ge2 = merge_pool(gc3, c1, gp1, s0, c0, a["e2"], "e2")
         ge1 = g("e1", s0, c0)
         cv["e2"].backward(a["e1"], ge2, s0, work, acc, dx=ge1, gate=a["e1"], stream=stream)
         cv["e1"].backward(a["x"], ge1, s0, work, acc, stream=stream)

@@ -66,6 +66,12 @@ int mfnn_conv3_wgrad_static(const void* x, const void* dz, int32_t D, int32_t H,
 int mfnn_flip_weights(const void* w, int32_t cin, int32_t kp, int32_t cout, int32_t kp2, int32_t cinp, void* wt,
                       void* stream);
 
+/* mfnn_conv3_wgrad, and mfnn_flip_weights(w, ..., wt) for the data gradient that follows, in one
+ * launch fewer. */
+int mfnn_conv3_wgrad_flip(const void* x, const void* dz, int32_t D, int32_t H, int32_t W, int32_t cin, int32_t kp,
+                          int32_t cout, int32_t chunk, float* work, float* dw, float* db, int32_t accumulate, const void* w,
+                          int32_t kp2, int32_t cinp, void* wt, void* stream);
+
 /* fp32 -> bf16 copy of n values */
 int mfnn_to_bf16(const float* x, int64_t n, void* y, void* stream);
 
@@ -112,6 +118,17 @@ int mfnn_mse(const float* y, const float* t, const float* mask, int64_t M, int32
  * m1, m2; writes the bf16 copy wb when not null. */
 int mfnn_adam(float* w, const float* g, float* m1, float* m2, int64_t n, float lr, float b1, float b2, float eps,
               int32_t step, void* wb, void* stream);
+
+/* The same step on `count` tensors (no two sharing memory) in as few launches as they need. */
+typedef struct {
+    float* w;
+    const float* g;
+    float *m1, *m2;
+    int64_t n;
+    void* wb;
+} mfnn_adam_tensor;
+int mfnn_adam_many(const mfnn_adam_tensor* list, int32_t count, float lr, float b1, float b2, float eps, int32_t step,
+                   void* stream);
 
 #ifdef __cplusplus
 }

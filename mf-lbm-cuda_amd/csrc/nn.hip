@@ -655,13 +655,40 @@ __global__ __launch_bounds__(192) void k_conv3_wgrad_rows(const __bf16* __restri
     }
 }
 
+// W'[ci][tap' * cout + co] = W[co][(26 - tap') * cin + ci]  (bf16, padded: ci to 16, k' to 32)
+struct Flip {
+    const __bf16* W;
+    int cin, kp, cout, kp2, cinp;
+    __bf16* Wt;
+
+    __device__ __forceinline__ void entry(int64_t i) const {
+        if (i >= (int64_t)cinp * kp2) return;
+        const int ci = (int)(i / kp2), k2 = (int)(i - (int64_t)ci * kp2);
+        __bf16 v = (__bf16)0.f;
+        if (ci < cin && k2 < 27 * cout) {
+            const int tp = k2 / cout, co = k2 - tp * cout;
+            v = W[(int64_t)co * kp + (26 - tp) * cin + ci];
+        }
+        Wt[i] = v;
+    }
+};
+
+__global__ void k_flip_weights(Flip f) { f.entry((int64_t)blockIdx.x * blockDim.x + threadIdx.x); }
+
 // dW[i] (+)= sum over chunks of part[chunk][i], i < n, and in the blocks after those,
 // db[i] (+)= the same over bpart[chunk][i], i < nb (bpart null: no bias).  A block covers
 // 32 entries with 8 groups of 32 threads: group g adds chunks g, g + 8, g + 16, ... in order,
 // then the 8 group sums are added in group order (a fixed order for every launch).
+// The last blocks flip the layer's weights for the data gradient that follows: on the layers of
+// a 64^3 training step the sums take 5 us and the flip took 3.5 as a launch of its own, both
+// little more than the launch; together they take 5.7.
 __global__ __launch_bounds__(256) void k_sum_chunks(const float* __restrict__ part, int nchunk, int64_t n,
                                                     const float* __restrict__ bpart, int nb, int accumulate,
-                                                    float* __restrict__ dw, float* __restrict__ db) {
+                                                    float* __restrict__ dw, float* __restrict__ db, int64_t sums, Flip flip) {
+    if ((int64_t)blockIdx.x >= sums) {
+        flip.entry(((int64_t)blockIdx.x - sums) * 256 + threadIdx.x);
+        return;
+    }
     __shared__ float red[8][32];
     const int x = threadIdx.x & 31, grp = threadIdx.x >> 5;
     const int64_t wblocks = (n + 31) / 32;
@@ -681,20 +708,6 @@ __global__ __launch_bounds__(256) void k_sum_chunks(const float* __restrict__ pa
         for (int g = 1; g < 8; ++g) t += red[g][x];
         dst[i] = accumulate ? dst[i] + t : t;
     }
-}
-
-// W'[ci][tap' * cout + co] = W[co][(26 - tap') * cin + ci]  (bf16, padded: ci to 16, k' to 32)
-__global__ void k_flip_weights(const __bf16* __restrict__ W, int cin, int kp, int cout, int kp2, int cinp,
-                               __bf16* __restrict__ Wt) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)cinp * kp2) return;
-    const int ci = (int)(i / kp2), k2 = (int)(i % kp2);
-    __bf16 v = (__bf16)0.f;
-    if (ci < cin && k2 < 27 * cout) {
-        const int tp = k2 / cout, co = k2 - tp * cout;
-        v = W[(int64_t)co * kp + (26 - tp) * cin + ci];
-    }
-    Wt[i] = v;
 }
 
 __global__ void k_to_bf16(const float* __restrict__ x, int64_t n, __bf16* __restrict__ y) {
@@ -865,20 +878,32 @@ __global__ __launch_bounds__(256) void k_mse(const float* __restrict__ y, const 
     if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
-// Adam step on fp32 master weights; refreshes the bf16 copy.
-__global__ void k_adam(float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m1,
-                       float* __restrict__ m2, int64_t n, float lr, float b1, float b2, float eps, float c1,
-                       float c2, __bf16* __restrict__ wb) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float a = b1 * m1[i] + (1.f - b1) * gi;
-    const float b = b2 * m2[i] + (1.f - b2) * gi * gi;
-    m1[i] = a;
-    m2[i] = b;
-    const float v = w[i] - lr * (a * c1) / (sqrtf(b * c2) + eps);
-    w[i] = v;
-    if (wb) wb[i] = (__bf16)v;
+// Adam step on fp32 master weights; refreshes the bf16 copies.  One launch for up to ADAM_MAX
+// tensors, the launch's blocks split between them in order (first[t]: the first block of tensor
+// t): a network's weights are many small tensors, and a launch apiece took 24 x 2.2 us of a 64^3
+// training step, one takes 9.7.
+constexpr int ADAM_MAX = 48;  // at most a wave's lanes, and 4 KiB of kernel arguments
+struct AdamList {
+    mfnn_adam_tensor t[ADAM_MAX];
+    uint32_t first[ADAM_MAX];
+    int count;
+};
+
+__global__ __launch_bounds__(256) void k_adam(AdamList list, float lr, float b1, float b2, float eps, float c1, float c2) {
+    const int lane = threadIdx.x & 63;
+    const int k = __builtin_amdgcn_readfirstlane(
+        (int)__popcll(__ballot(lane < list.count && blockIdx.x >= list.first[lane < ADAM_MAX ? lane : 0])) - 1);
+    const mfnn_adam_tensor& t = list.t[k];
+    const int64_t i = (int64_t)(blockIdx.x - list.first[k]) * 256 + threadIdx.x;
+    if (i >= t.n) return;
+    const float gi = t.g[i];
+    const float a = b1 * t.m1[i] + (1.f - b1) * gi;
+    const float b = b2 * t.m2[i] + (1.f - b2) * gi * gi;
+    t.m1[i] = a;
+    t.m2[i] = b;
+    const float v = t.w[i] - lr * (a * c1) / (sqrtf(b * c2) + eps);
+    t.w[i] = v;
+    if (t.wb) static_cast<__bf16*>(t.wb)[i] = (__bf16)v;
 }
 
 inline unsigned nblk(int64_t n, int b = 256) { return (unsigned)((n + b - 1) / b); }
@@ -1113,9 +1138,14 @@ bool wgrad_rows(const __bf16* X, const __bf16* dZ, const Grid3& g, int cin, int 
     return cin % 16 == 0 || launch(true);
 }
 
-// The weight-gradient launches of valid arguments: partials into `work`, then the chunk sums.
+bool flip_args_ok(int32_t cin, int32_t cout, int32_t kp2, int32_t cinp) {
+    return kp2 >= 27 * cout && kp2 % 32 == 0 && cinp >= cin && cinp % 16 == 0;
+}
+
+// The weight-gradient launches of valid arguments: partials into `work`, then the chunk sums and,
+// with flip.Wt, the flipped weights.
 int wgrad_launch(const void* x, const void* dz, int32_t D, int32_t H, int32_t W, int32_t cin, int32_t kp, int32_t cout,
-                 int32_t chunk, float* work, float* dw, float* db, int32_t accumulate, void* stream) {
+                 int32_t chunk, float* work, float* dw, float* db, int32_t accumulate, const Flip& flip, void* stream) {
     const Grid3 g{D, H, W};
     const int64_t M = (int64_t)D * H * W;
     const int nchunk = (int)((M + chunk - 1) / chunk);
@@ -1127,7 +1157,8 @@ int wgrad_launch(const void* x, const void* dz, int32_t D, int32_t H, int32_t W,
     if (!wgrad_rows(X, dZ, g, cin, kp, coutp, cout, chunk, nchunk, work, bpart, s))
         k_conv3_wgrad<<<dim3(kp / 16, coutp / 16, nchunk), 64, 0, s>>>(X, dZ, g, cin, kp, coutp, cout, chunk, work, bpart);
     const unsigned sblocks = nblk(n, 32) + (db ? nblk(cout, 32) : 0);
-    k_sum_chunks<<<sblocks, 256, 0, s>>>(work, nchunk, n, bpart, db ? cout : 0, accumulate, dw, db);
+    const unsigned fblocks = flip.Wt ? nblk((int64_t)flip.cinp * flip.kp2) : 0;
+    k_sum_chunks<<<sblocks + fblocks, 256, 0, s>>>(work, nchunk, n, bpart, db ? cout : 0, accumulate, dw, db, sblocks, flip);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -1160,7 +1191,7 @@ extern "C" {
 int mfnn_conv3_wgrad(const void* x, const void* dz, int32_t D, int32_t H, int32_t W, int32_t cin, int32_t kp,
                      int32_t cout, int32_t chunk, float* work, float* dw, float* db, int32_t accumulate, void* stream) {
     if (!wgrad_args_ok(x, dz, D, H, W, cin, kp, cout, chunk)) return -1;
-    return wgrad_launch(x, dz, D, H, W, cin, kp, cout, chunk, work, dw, db, accumulate, stream);
+    return wgrad_launch(x, dz, D, H, W, cin, kp, cout, chunk, work, dw, db, accumulate, Flip{}, stream);
 }
 
 int mfnn_conv3_wgrad_static(const void* x, const void* dz, int32_t D, int32_t H, int32_t W, int32_t cin, int32_t kp,
@@ -1169,14 +1200,22 @@ int mfnn_conv3_wgrad_static(const void* x, const void* dz, int32_t D, int32_t H,
     if (mfnn_wgrad_workspace(D, H, W, kp, cout, chunk) > (int64_t)MFNN_WGRAD_SCRATCH_FLOATS) return -3;
     float* work = scratch_address();
     if (!work) return -2;
-    return wgrad_launch(x, dz, D, H, W, cin, kp, cout, chunk, work, dw, db, accumulate, stream);
+    return wgrad_launch(x, dz, D, H, W, cin, kp, cout, chunk, work, dw, db, accumulate, Flip{}, stream);
+}
+
+int mfnn_conv3_wgrad_flip(const void* x, const void* dz, int32_t D, int32_t H, int32_t W, int32_t cin, int32_t kp,
+                          int32_t cout, int32_t chunk, float* work, float* dw, float* db, int32_t accumulate, const void* w,
+                          int32_t kp2, int32_t cinp, void* wt, void* stream) {
+    if (!wgrad_args_ok(x, dz, D, H, W, cin, kp, cout, chunk) || !flip_args_ok(cin, cout, kp2, cinp) || !w || !wt) return -1;
+    return wgrad_launch(x, dz, D, H, W, cin, kp, cout, chunk, work, dw, db, accumulate,
+                        Flip{(const __bf16*)w, cin, kp, cout, kp2, cinp, (__bf16*)wt}, stream);
 }
 
 int mfnn_flip_weights(const void* w, int32_t cin, int32_t kp, int32_t cout, int32_t kp2, int32_t cinp, void* wt,
                       void* stream) {
-    if (kp2 < 27 * cout || kp2 % 32 || cinp < cin || cinp % 16) return -1;
+    if (!flip_args_ok(cin, cout, kp2, cinp)) return -1;
     const int64_t n = (int64_t)cinp * kp2;
-    k_flip_weights<<<nblk(n), 256, 0, (hipStream_t)stream>>>((const __bf16*)w, cin, kp, cout, kp2, cinp, (__bf16*)wt);
+    k_flip_weights<<<nblk(n), 256, 0, (hipStream_t)stream>>>(Flip{(const __bf16*)w, cin, kp, cout, kp2, cinp, (__bf16*)wt});
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -1257,13 +1296,33 @@ int mfnn_mse(const float* y, const float* t, const float* mask, int64_t M, int32
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-int mfnn_adam(float* w, const float* g, float* m1, float* m2, int64_t n, float lr, float b1, float b2, float eps,
-              int32_t step, void* wb, void* stream) {
-    if (step < 1) return -1;
+int mfnn_adam_many(const mfnn_adam_tensor* list, int32_t count, float lr, float b1, float b2, float eps, int32_t step,
+                   void* stream) {
+    if (step < 1 || count < 0) return -1;
     const float c1 = 1.f / (1.f - powf(b1, (float)step));
     const float c2 = 1.f / (1.f - powf(b2, (float)step));
-    k_adam<<<nblk(n), 256, 0, (hipStream_t)stream>>>(w, g, m1, m2, n, lr, b1, b2, eps, c1, c2, (__bf16*)wb);
-    return hipGetLastError() == hipSuccess ? 0 : -2;
+    for (int at = 0; at < count;) {
+        AdamList l;
+        int64_t blocks = 0;
+        for (l.count = 0; l.count < ADAM_MAX && at < count; ++l.count, ++at) {
+            const int64_t b = (list[at].n + 255) / 256;
+            if (l.count && blocks + b > 1 << 23) break;  // a launch holds fewer than 2^32 threads
+            l.t[l.count] = list[at];
+            l.first[l.count] = (uint32_t)blocks;
+            blocks += b;
+        }
+        if (!blocks) continue;
+        k_adam<<<(unsigned)blocks, 256, 0, (hipStream_t)stream>>>(l, lr, b1, b2, eps, c1, c2);
+        if (hipGetLastError() != hipSuccess) return -2;
+    }
+    return 0;
+}
+
+int mfnn_adam(float* w, const float* g, float* m1, float* m2, int64_t n, float lr, float b1, float b2, float eps,
+              int32_t step, void* wb, void* stream) {
+    if (n <= 0) return step < 1 ? -1 : -2;
+    const mfnn_adam_tensor t{w, g, m1, m2, n, wb};
+    return mfnn_adam_many(&t, 1, lr, b1, b2, eps, step, stream);
 }
 
 }  // extern "C"

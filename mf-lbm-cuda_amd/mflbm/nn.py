@@ -39,6 +39,8 @@ SIGNATURES = {
     "mfnn_wgrad_workspace": [_i32, _i32, _i32, _i32, _i32, _i32],
     "mfnn_conv3_wgrad": [_vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp],
     "mfnn_conv3_wgrad_static": [_vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _i32, _vp],
+    "mfnn_conv3_wgrad_flip": [_vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _i32, _i32,
+                              _vp, _vp],
     "mfnn_flip_weights": [_vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp],
     "mfnn_to_bf16": [_vp, _i64, _vp, _vp],
     "mfnn_pool2": [_vp, _i32, _i32, _i32, _i32, _vp, _i32, _vp],
@@ -50,6 +52,7 @@ SIGNATURES = {
     "mfnn_add_gate": [_vp, _vp, _vp, _i64, _vp, _vp],
     "mfnn_mse_partials": [_i64, _i32],
     "mfnn_mse": [_vp, _vp, _vp, _i64, _i32, _fp, _vp, _vp, _vp],
+    "mfnn_adam_many": [_vp, _i32, _fp, _fp, _fp, _fp, _i32, _vp],
     "mfnn_adam": [_vp, _vp, _vp, _vp, _i64, _fp, _fp, _fp, _fp, _i32, _vp, _vp],
 }
 
@@ -103,6 +106,11 @@ def bf16_bits(a):
 
 def bf16_values(bits):
     return (bits.astype(np.uint32) << 16).view(np.float32)
+
+
+class AdamTensor(C.Structure):
+    """mfnn_adam_tensor: a parameter tensor with its gradient, moments and bf16 copy"""
+    _fields_ = [("w", _vp), ("g", _vp), ("m1", _vp), ("m2", _vp), ("n", _i64), ("wb", _vp)]
 
 
 class DevArray:
@@ -213,20 +221,28 @@ class Conv:
         (times [gate > 0] when gate is given)."""
         D, H, W = shape
         L = lib()
-        _chk(L.mfnn_conv3_wgrad(ptr(x), ptr(dz), D, H, W, self.cin, self.kp, self.cout, wgrad_chunk(D, H, W),
-                                ptr(work), ptr(self.dw), ptr(self.db), int(accumulate), stream), "wgrad")
-        if dx is not None:
-            _chk(L.mfnn_flip_weights(ptr(self.wb), self.cin, self.kp, self.cout, self.kp2, self.wt.shape[0],
-                                     ptr(self.wt), stream), "flip")
+        args = (ptr(x), ptr(dz), D, H, W, self.cin, self.kp, self.cout, wgrad_chunk(D, H, W), ptr(work), ptr(self.dw),
+                ptr(self.db), int(accumulate))
+        if dx is None:
+            _chk(L.mfnn_conv3_wgrad(*args, stream), "wgrad")
+        else:
+            _chk(L.mfnn_conv3_wgrad_flip(*args, ptr(self.wb), self.kp2, self.wt.shape[0], ptr(self.wt), stream), "wgrad")
             _chk(L.mfnn_conv3(ptr(dz), ptr(self.wt), None, ptr(gate), D, H, W, self.cout, self.kp2, self.cin, 0,
                               ptr(dx), None, stream), "dgrad")
 
+    def adam_tensors(self):
+        return [AdamTensor(self.w.data_ptr(), self.dw.data_ptr(), self.m[0].data_ptr(), self.m[1].data_ptr(),
+                           self.w.numel(), self.wb.data_ptr()),
+                AdamTensor(self.b.data_ptr(), self.db.data_ptr(), self.m[2].data_ptr(), self.m[3].data_ptr(),
+                           self.b.numel(), None)]
+
     def adam(self, step, lr, stream=None, b1=0.9, b2=0.999, eps=1e-8):
-        L = lib()
-        _chk(L.mfnn_adam(ptr(self.w), ptr(self.dw), ptr(self.m[0]), ptr(self.m[1]), self.w.numel(), lr, b1, b2, eps,
-                         step, ptr(self.wb), stream), "adam w")
-        _chk(L.mfnn_adam(ptr(self.b), ptr(self.db), ptr(self.m[2]), ptr(self.m[3]), self.b.numel(), lr, b1, b2, eps,
-                         step, None, stream), "adam b")
+        adam_many(self.adam_tensors(), step, lr, stream, b1, b2, eps)
+
+
+def adam_many(tensors, step, lr, stream=None, b1=0.9, b2=0.999, eps=1e-8):
+    """One Adam step of a list of AdamTensor."""
+    _chk(lib().mfnn_adam_many((AdamTensor * len(tensors))(*tensors), len(tensors), lr, b1, b2, eps, step, stream), "adam")
 
 
 class UNet:
@@ -393,8 +409,7 @@ class UNet:
 
     def adam(self, lr, stream=None):
         self.step_count += 1
-        for c in self.conv.values():
-            c.adam(self.step_count, lr, stream)
+        adam_many([t for c in self.conv.values() for t in c.adam_tensors()], self.step_count, lr, stream)
 
     def params_numpy(self):
         return {k: c.get_numpy() for k, c in self.conv.items()}

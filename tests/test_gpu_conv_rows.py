@@ -93,3 +93,25 @@ def test_row_passes(shape, cl, cs, shift):
         assert np.array_equal(out["merge"].numpy(), np.where(fgate > 0, rnd(wide[..., cl:] + adj), f32(0)), equal_nan=True)
         assert L.mfnn_pool2(b["skip"].ptr(), *shape, cs, out["pool"].ptr(), 0, None) == 0
         assert np.array_equal(out["pool"].numpy(), rnd(f32(0.125) * sum8(skip)), equal_nan=True)
+
+
+def test_adam_many_matches_one_by_one():
+    """more tensors than one launch holds, empty and odd sizes among them: the same bits as a call
+    per tensor"""
+    rng = np.random.default_rng(5)
+    sizes = [1, 255, 256, 257, 0, 1000] * 9
+    print(f"[gpu-conv-rows] adam {len(sizes)} tensors", flush=True)
+    full = [[np.asarray(rng.normal(size=n + 1), f32) for n in sizes] for _ in range(4)]
+    full[3] = [np.abs(m) for m in full[3]]
+    a, b = [[[nn.DevArray.from_numpy(v) for v in part] for part in full] + [[nn.DevArray((n + 1,), "bf16", zero=True) for n in sizes]]
+            for _ in range(2)]
+    nn.adam_many([nn.AdamTensor(*(a[j][i].data_ptr() for j in range(4)), n, a[4][i].data_ptr() if i % 3 else None)
+                  for i, n in enumerate(sizes)], 3, 1e-2)
+    for i, n in enumerate(sizes):
+        if n:
+            assert nn.lib().mfnn_adam(*(nn.ptr(b[j][i]) for j in range(4)), n, 1e-2, 0.9, 0.999, 1e-8, 3,
+                                      nn.ptr(b[4][i]) if i % 3 else None, None) == 0
+    nn.sync()
+    for j in (0, 2, 3, 4):
+        for i in range(len(sizes)):
+            assert np.array_equal(a[j][i].numpy(), b[j][i].numpy()), (j, i)

@@ -23,6 +23,7 @@
 #include "geometry.h"
 #include "lattice.h"
 #include "launch.h"
+#include "copy_out.h"
 #include "device_lock.h"
 #include "layout.h"
 
@@ -84,6 +85,7 @@ struct mflbm_handle {
     double *mon_part = nullptr, *mon_out = nullptr;
     int mon_nsplit = 0;
     double *vprev = nullptr, *vpart = nullptr;  // mflbm_velocity_change: 3 nf previous velocity, block sums
+    HostStaging staging;                       // large copies to the host
     double* macro_buf = nullptr;               // mflbm_macro: one s1 field
     bool vprev_valid = false;
     // captured step graphs: [0] even step, [1] odd step
@@ -323,6 +325,7 @@ void free_all(mflbm_handle* h) {
     h->mon_part = h->mon_out = nullptr;
     h->vprev = h->vpart = nullptr;
     h->macro_buf = nullptr;
+    h->staging.release();
     h->cells = h->aux = nullptr;
     h->nb16 = nullptr;
     h->nbb = nullptr;
@@ -877,8 +880,7 @@ int mflbm_download(mflbm_handle* h, int32_t field, void* dst, size_t bytes) {
         cells_transfer(h, true);
         HIPCHK(h, hipGetLastError());
     }
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    HIPCHK(h, hipMemcpy(dst, ptr, bytes, hipMemcpyDeviceToHost));
+    HIPCHK(h, h->staging.copy(dst, ptr, bytes, h->stream));
     if (field == MFLBM_PDF && h->prec == MFLBM_FP32) shifted_to_colours((float*)dst, h->d.S1, h->rho_ref);
     return 0;
 }
@@ -927,8 +929,7 @@ int mflbm_macro(mflbm_handle* h, double* rho, double* u, double* v, double* w) {
             Launch<double>::macro(sparse<double>(h), consts<double>(h), h->d, dv[0], dv[1], dv[2], dv[3], h->stream);
         else Launch<float>::macro(sparse<float>(h), consts<float>(h), h->d, dv[0], dv[1], dv[2], dv[3], h->stream);
         HIPCHK(h, hipGetLastError());
-        HIPCHK(h, hipMemcpyAsync(host[a], h->macro_buf, n * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(h, hipStreamSynchronize(h->stream));
+        HIPCHK(h, h->staging.copy(host[a], h->macro_buf, n * sizeof(double), h->stream));
     }
     return 0;
 }

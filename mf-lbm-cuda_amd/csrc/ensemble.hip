@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../include/mflbm.h"
+#include "copy_out.h"
 #include "device_lock.h"
 #include "kernels.inl"
 #include "layout.h"
@@ -197,6 +198,7 @@ struct mflbm_ensemble {
     std::vector<int32_t> taken, checks;
     std::vector<double> perm, change;
     std::vector<double> rho_d;  // rest density of each domain
+    HostStaging staging;        // large copies to the host
     std::string err;
 };
 
@@ -231,6 +233,7 @@ EnsDev dev_view(const mflbm_ensemble* e) {
 void free_all(mflbm_ensemble* e) {
     if (e->graph) (void)hipGraphExecDestroy(e->graph);
     e->graph = nullptr;
+    e->staging.release();
     void* p[] = {e->f, e->nb, e->nb16, e->nbb, e->blk_dom, e->dom_start, e->dom_count, e->active, e->loc, e->ux, e->uy, e->uz,
                  e->drho, e->part, e->red};
     for (void* x : p)
@@ -560,8 +563,7 @@ int mflbm_ensemble_fields(mflbm_ensemble* e, int32_t first, int32_t count, float
                                                                                 e->npt, buf);
         r = hipGetLastError();
     }
-    if (r == hipSuccess) r = hipStreamSynchronize(e->stream);
-    if (r == hipSuccess) r = hipMemcpy(out, buf, bytes, hipMemcpyDeviceToHost);
+    if (r == hipSuccess) r = e->staging.copy(out, buf, bytes, e->stream);
     (void)hipFree(buf);
     if (r != hipSuccess) return fail(e, "ensemble fields: %s", hipGetErrorString(r));
     return 0;

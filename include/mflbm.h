@@ -85,7 +85,10 @@ typedef struct mflbm_monitor_out {
 
 /* Device time of the kernel groups of a profiled run (milliseconds, summed over steps;
  * divide collide_odd_ms by n_odd, collide_even_ms by n_even, the others by n_odd + n_even).
- * boundary = periodic copies + Zou-He; gradient = the colour-gradient chain. */
+ * boundary = periodic copies + open boundaries, gradient = the colour-gradient chain.  Where the
+ * boundary updates have no launch of their own (the default chain on boxes, periodic axes of 8
+ * nodes or more) their time is in the collisions (phi) and the gradient (populations), and
+ * boundary is the gap between two events. */
 typedef struct mflbm_kernel_times {
     double collide_odd_ms, collide_even_ms, boundary_ms, gradient_ms;
     int32_t n_odd, n_even;

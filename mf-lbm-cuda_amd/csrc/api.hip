@@ -189,23 +189,39 @@ void enqueue_step(mflbm_handle* h, bool odd, hipEvent_t* ev) {
     hipStream_t s = h->stream;
     int e = 0;
     auto mark = [&]() { if (ev) (void)hipEventRecord(ev[e++], s); };
-    Launch<T>::collide(S, F.phi, h->d, P, odd, s);
-    mark();
-    {
-        BoundaryArgs<T> B{};
-        if (h->open_z) {
-            B.in_bc = h->in_bc;
-            B.out_bc = h->out_bc;
-        }
-        B.zread = h->zread[odd ? 1 : 0] ? h->zread[odd ? 1 : 0] : h->zmap;
-        B.zmap = h->zmap; B.w_in = (const T*)h->w_in; B.conv = (T*)h->conv;
-        B.pairs = h->pairs[odd ? 1 : 0]; B.npairs = h->npairs[odd ? 1 : 0];
-        B.kper = h->p.kper; B.jper = h->p.jper;
-        Launch<T>::boundary(S, F, P, B, odd, s);
+    BoundaryArgs<T> B{};
+    if (h->open_z) {
+        B.in_bc = h->in_bc;
+        B.out_bc = h->out_bc;
     }
-    if (h->plate_z) Launch<T>::porous_plate(S, h->d, P, h->pmap, h->plate_z, h->plate_blocked, odd, s);
+    B.zread = h->zread[odd ? 1 : 0] ? h->zread[odd ? 1 : 0] : h->zmap;
+    B.zmap = h->zmap; B.w_in = (const T*)h->w_in; B.conv = (T*)h->conv;
+    B.pairs = h->pairs[odd ? 1 : 0]; B.npairs = h->npairs[odd ? 1 : 0];
+    B.kper = h->p.kper; B.jper = h->p.jper;
+    // With the gradient chain on boxes a step needs no boundary launch: the collision writes the
+    // ghost phi that k_grad_normals reads, and the populations' part runs beside k_grad_force.
+    // A node then has one periodic image per axis, which takes 8 nodes (the ghost layers are 4
+    // deep); shorter axes and the other chains keep the launch.  us a step with the launch and
+    // without: 32^3 FP64 25.0 and 20.3, 64^3 FP32 30.0 and 25.9, periodic 96^3 FP64 101.8 and 87.1,
+    // 128^3 FP32 104.6 and 99.5, 256^3 FP32 781.3 and 777.8, FP64 1435 and 1437 (there the
+    // boundary planes' bytes cost the same in either place).
+    const bool merged = !h->split_gradient && h->grad_shape == GRAD_SHAPE_TILES && h->n_fluid > 0 &&
+                        (!B.jper || h->d.ny >= 8) && (!B.kper || h->d.nz >= 8);
+    const PhiGhosts<T> G{0, B.kper, B.jper, B.in_bc, B.out_bc, F.walls, B.conv ? B.conv + 38 * (int64_t)h->d.X1 * h->d.Y1 : nullptr};
+    Launch<T>::collide(S, F.phi, h->d, P, odd, merged ? &G : nullptr, s);
     mark();
-    if (h->split_gradient) {
+    auto plate = [&]() {
+        if (h->plate_z) Launch<T>::porous_plate(S, h->d, P, h->pmap, h->plate_z, h->plate_blocked, odd, s);
+    };
+    if (!merged) {
+        Launch<T>::boundary(S, F, P, B, odd, s);
+        plate();
+    }
+    mark();
+    if (merged) {
+        Launch<T>::gradient_boundary(grad_args<T>(h), S, F, P, B, odd, s);
+        plate();
+    } else if (h->split_gradient) {
         Launch<T>::phi_extrap(F, L, s);
         Launch<T>::normals(F, P, L, s);
         Launch<T>::normal_extrap(F, L, s);

@@ -634,15 +634,24 @@ __global__ __launch_bounds__((TX + 4) * (TY + 4)) void k_grad_normals(GradArgs<T
 // K6 + K7 on the box of owned nodes inside [1, n]^3: normals of the solid-boundary nodes of
 // the box and its 1-halo from the fluid normals around them, then the curvature and the
 // force record of the fluid nodes of the box.
-template <typename T, int TX, int TY, int TZ>
-__global__ __launch_bounds__((TX + 4) * (TY + 4)) void k_grad_force(GradArgs<T> A, StepConst<T> P) {
+//
+// CELLS: the first B.blocks workgroups make the population updates of the open boundaries and the
+// periodic copies after an odd (1) or even (2) collision instead (boundary_cells): they touch
+// nothing that this chain reads or writes, and the step is a launch shorter.
+template <typename T, int TX, int TY, int TZ, int CELLS>
+__global__ __launch_bounds__((TX + 4) * (TY + 4)) void k_grad_force(GradArgs<T> A, StepConst<T> P, Sparse<T> S, Fields<T> F,
+                                                                    BoundaryArgs<T> B) {
     constexpr int LX = TX + 4, LY = TY + 4, LZ = TZ + 4, NC = LX * LY, NL = NC * LZ, THREADS = NC;
     using Entry = BoxEntry<LX, LY, LZ>;
     __shared__ T s_cn[3][NL];
     __shared__ T s_ws[7][13];
     const Dims& d = A.d;
     const int tid = threadIdx.x;
-    const int b = xcd_block();
+    if (CELLS && (int)blockIdx.x < B.blocks) {
+        if ((int)blockIdx.x < B.nbc + B.npair) boundary_cells<T, CELLS == 1, false>(S, F, P, B, blockIdx.x, THREADS);
+        return;
+    }
+    const int b = CELLS ? xcd_block(gridDim.x - B.blocks, blockIdx.x - B.blocks) : xcd_block();
     const TileDesc td = A.lists.fdesc[b];
     if (td.nb == 0) return;  // no record to write
     const int i0 = td.i0, j0 = td.j0, k0 = td.k0;

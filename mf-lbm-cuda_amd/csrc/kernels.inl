@@ -31,11 +31,11 @@ namespace dev {
 // Workgroups are dispatched round-robin over the 8 XCDs of the MI355X.  Remap the
 // hardware block index so that each XCD works on one contiguous range of the node list:
 // neighbouring nodes (which share cache lines and stencil data) then meet in the same L2.
-__device__ __forceinline__ int xcd_block() {
-    const int nb = gridDim.x, b = blockIdx.x;
+__device__ __forceinline__ int xcd_block(int nb, int b) {
     const int q = nb >> 3, r = nb & 7, x = b & 7;
     return x * q + (x < r ? x : r) + (b >> 3);
 }
+__device__ __forceinline__ int xcd_block() { return xcd_block(gridDim.x, blockIdx.x); }
 
 // FP64 block reductions as wavefront-shuffle trees.  Each wave combines its 64 lanes with
 // xor shuffles at distances 32, 16, ..., 1 (the two lanes of a pair compute the same
@@ -335,13 +335,141 @@ __device__ __forceinline__ void odd_links(const int32_t* __restrict__ nbb, const
     }
 }
 
+// Periodic ghost layers of phi (periodic_phi_{Z,Y,ZY}, src/main_iteration_GPU.cu:1691-1733);
+// the three groups read interior cells and write disjoint ghost cells.
+template <typename T>
+__device__ __forceinline__ void periodic_phi(T* __restrict__ phi, const Dims& d, int kper, int jper, int t) {
+    const int nx = d.nx, ny = d.ny, nz = d.nz;
+    auto P = [&](int a, int b, int c) -> T& { return phi[i4(d, a, b, c)]; };
+    const int nzf = kper ? nx * ny : 0, nyf = jper ? nx * nz : 0, ne = (kper && jper) ? nx : 0;
+    if (t < nzf) {
+        const int i = t % nx + 1, j = t / nx + 1;
+#pragma unroll
+        for (int kk = 1; kk <= 4; ++kk) {
+            P(i, j, kk + nz) = P(i, j, kk);
+            P(i, j, kk - 4) = P(i, j, nz + kk - 4);
+        }
+        return;
+    }
+    t -= nzf;
+    if (t < nyf) {
+        const int i = t % nx + 1, k = t / nx + 1;
+#pragma unroll
+        for (int jj = 1; jj <= 4; ++jj) {
+            P(i, jj + ny, k) = P(i, jj, k);
+            P(i, jj - 4, k) = P(i, ny + jj - 4, k);
+        }
+        return;
+    }
+    t -= nyf;
+    if (t < ne) {
+        const int i = t + 1;
+        for (int kk = 1; kk <= 4; ++kk)
+            for (int jj = 1; jj <= 4; ++jj) {
+                P(i, jj - 4, kk - 4) = P(i, ny + jj - 4, nz + kk - 4);
+                P(i, jj + ny, kk - 4) = P(i, jj, nz + kk - 4);
+                P(i, jj + ny, kk + nz) = P(i, jj, kk);
+                P(i, jj - 4, kk + nz) = P(i, ny + jj - 4, kk);
+            }
+    }
+}
+
+// Ghost phi of fluid node (i, j, k) whose new phi is v: its periodic images and, at k = nz, the
+// planes behind the outlet.  Axes of at least 8 nodes, so that a node has one image per axis.
+template <typename T>
+__device__ __forceinline__ void ghost_phi(const PhiGhosts<T>& G, const StepConst<T>& P, T* __restrict__ phi, const Dims& d,
+                                          int i, int j, int k, T v) {
+    const bool yg = G.jper && (j <= 4 || j > d.ny - 4), zg = G.kper && (k <= 4 || k > d.nz - 4);
+    const int jg = j <= 4 ? j + d.ny : j - d.ny, kg = k <= 4 ? k + d.nz : k - d.nz;
+    if (yg) phi[i4(d, i, jg, k)] = v;
+    if (zg) phi[i4(d, i, j, kg)] = v;
+    if (yg && zg) phi[i4(d, i, jg, kg)] = v;
+    if (G.out_bc && k == d.nz) {
+        auto ph = [&](int a, int b, int c) -> T& { return phi[i4(d, a, b, c)]; };
+        if (G.out_bc == 1) {
+            convective_phi<T>(P, i, j, k, 0, v, ph, [&]() -> T& { return G.conv[(int64_t)j * d.X1 + i]; });
+        } else {
+            for (int m = 1; m <= 4; ++m) ph(i, j, k + m) = v;
+        }
+    }
+}
+
+// The rest of the ghost phi, one thread per t: both inlets' planes, the outlet's planes behind
+// solid nodes, the periodic images of solid nodes.  Reads and writes no phi of a fluid node
+// or of one of its images, so it may run beside the collision.
+template <typename T>
+__device__ __forceinline__ void ghost_phi_rest(const PhiGhosts<T>& G, const StepConst<T>& P, T* __restrict__ phi,
+                                               const Dims& d, int t) {
+    const int n = d.nx * d.ny, nz = d.nz;
+    auto ph = [&](int a, int b, int c) -> T& { return phi[i4(d, a, b, c)]; };
+    if (G.in_bc) {
+        if (t < n) {
+            const int i = t % d.nx + 1, j = t / d.nx + 1;
+            inlet_phi<T>(P, i, j, G.walls[i2(d, i, j, 1)], ph);
+            return;
+        }
+        t -= n;
+    }
+    if (G.out_bc) {
+        if (t < n) {
+            const int i = t % d.nx + 1, j = t / d.nx + 1;
+            if (!G.walls[i2(d, i, j, nz)]) return;
+            if (G.out_bc == 1) {
+                convective_phi<T>(P, i, j, nz, 1, ph(i, j, nz), ph, [&]() -> T& { return G.conv[(int64_t)j * d.X1 + i]; });
+            } else {
+                const T v = ph(i, j, nz);
+                for (int m = 1; m <= 4; ++m) ph(i, j, nz + m) = v;
+            }
+            return;
+        }
+        t -= n;
+    }
+    // the eight images of a column's ends per thread, all read before the first is written (a load
+    // and a store in turn took 16 us at 96^3), and the edges' one by one
+    const int ny = d.ny, zf = G.kper ? n : 0, yf = G.jper ? d.nx * nz : 0, ef = G.kper && G.jper ? 64 * d.nx : 0;
+    auto ends = [&](int len, auto&& node, auto&& wall) {
+        uint8_t w[8];
+        T v[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) w[m] = G.walls[wall(m < 4 ? len + m - 3 : m - 3)];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) v[m] = w[m] ? phi[node(m < 4 ? len + m - 3 : m - 3)] : T(0);
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+            if (w[m]) phi[node(m < 4 ? m - 3 : len + m - 3)] = v[m];
+    };
+    if (t < zf) {
+        const int i = t % d.nx + 1, j = t / d.nx + 1;
+        ends(nz, [&](int k) { return i4(d, i, j, k); }, [&](int k) { return i2(d, i, j, k); });
+    } else if ((t -= zf) < yf) {
+        const int i = t % d.nx + 1, k = t / d.nx + 1;
+        ends(ny, [&](int j) { return i4(d, i, j, k); }, [&](int j) { return i2(d, i, j, k); });
+    } else if ((t -= yf) < ef) {
+        const int m = t / d.nx, i = t - m * d.nx + 1, my = m & 7, mz = m >> 3;
+        const int sj = my < 4 ? ny + my - 3 : my - 3, sk = mz < 4 ? nz + mz - 3 : mz - 3;
+        if (G.walls[i2(d, i, sj, sk)])
+            phi[i4(d, i, my < 4 ? my - 3 : ny + my - 3, mz < 4 ? mz - 3 : nz + mz - 3)] = phi[i4(d, i, sj, sk)];
+    }
+}
+
+// Threads of ghost_phi_rest.
+template <typename T>
+inline int64_t ghost_phi_threads(const PhiGhosts<T>& G, const Dims& d) {
+    return (int64_t)((G.in_bc ? 1 : 0) + (G.out_bc ? 1 : 0) + (G.kper ? 1 : 0)) * d.nx * d.ny +
+           (G.jper ? (int64_t)d.nx * d.nz : 0) + (G.kper && G.jper ? 64 * d.nx : 0);
+}
+
 #ifndef MFLBM_COLLIDE_THREADS
 #define MFLBM_COLLIDE_THREADS 256  // threads per collide workgroup (tuning: 128, 256, 512)
 #endif
 template <typename T, bool ODD, bool ORIG = true>
 __global__ __launch_bounds__(MFLBM_COLLIDE_THREADS) void k_collide(Sparse<T> S, T* __restrict__ phi, Dims d,
-                                                                   StepConst<T> P) {
-    const int t = xcd_block() * MFLBM_COLLIDE_THREADS + threadIdx.x;
+                                                                   StepConst<T> P, PhiGhosts<T> G) {
+    if ((int)blockIdx.x < G.rest) {
+        ghost_phi_rest<T>(G, P, phi, d, (int)blockIdx.x * MFLBM_COLLIDE_THREADS + threadIdx.x);
+        return;
+    }
+    const int t = xcd_block(gridDim.x - G.rest, blockIdx.x - G.rest) * MFLBM_COLLIDE_THREADS + threadIdx.x;
     if (t >= S.nf) return;
     // The neighbour row, force record and phi of the odd step are touched once; nontemporal
     // accesses leave the cache to the shared lines of the scattered cells (6 % faster; in
@@ -399,6 +527,9 @@ __global__ __launch_bounds__(MFLBM_COLLIDE_THREADS) void k_collide(Sparse<T> S, 
             __builtin_nontemporal_store(o2[q], S.f + S.at(slot + 19, dst));
         }
     }
+    // last: a branch in front of the stores keeps all 38 populations alive across it (even
+    // collide 61 -> 111 VGPRs in FP32, 134 -> 189 in FP64)
+    if (G.rest) ghost_phi<T>(G, P, phi, d, i, j, k, ph);
 }
 
 // One colour population of a cell in shifted storage (colour 1 and the total's deviation
@@ -443,49 +574,29 @@ __device__ __forceinline__ void with_cells(const Sparse<T>& S, T rho_ref, CellOf
 // Periodic population copies, precomputed as (slot, destination cell, source cell) in the
 // reference's kernel order with repeated destinations resolved to the last writer
 // (perioidc_BC_{Z,Y,ZY}_{odd,even}, src/main_iteration_GPU.cu:1529-1689).
+// PAIRS of them per thread, all read before the first is written (no copy reads a cell that another
+// writes): one per thread is 2700 workgroups of three round trips to memory each at 256^3.
+constexpr int PAIRS = 4;
 template <typename T>
-__device__ __forceinline__ void copy_cell(const Sparse<T>& S, int slot, int dst, int src) {
-    S.f[S.at(slot, dst)] = S.f[S.at(slot, src)];
-    S.f[S.at(slot + 19, dst)] = S.f[S.at(slot + 19, src)];
-}
-
-// Periodic ghost layers of phi (periodic_phi_{Z,Y,ZY}, src/main_iteration_GPU.cu:1691-1733);
-// the three groups read interior cells and write disjoint ghost cells.
-template <typename T>
-__device__ __forceinline__ void periodic_phi(T* __restrict__ phi, const Dims& d, int kper, int jper, int t) {
-    const int nx = d.nx, ny = d.ny, nz = d.nz;
-    auto P = [&](int a, int b, int c) -> T& { return phi[i4(d, a, b, c)]; };
-    const int nzf = kper ? nx * ny : 0, nyf = jper ? nx * nz : 0, ne = (kper && jper) ? nx : 0;
-    if (t < nzf) {
-        const int i = t % nx + 1, j = t / nx + 1;
+__device__ __forceinline__ void copy_cells(const Sparse<T>& S, const int32_t* __restrict__ pairs, int npairs, int first,
+                                           int stride) {
+    int32_t p[PAIRS][3];
+    T v[PAIRS][2];
 #pragma unroll
-        for (int kk = 1; kk <= 4; ++kk) {
-            P(i, j, kk + nz) = P(i, j, kk);
-            P(i, j, kk - 4) = P(i, j, nz + kk - 4);
-        }
-        return;
-    }
-    t -= nzf;
-    if (t < nyf) {
-        const int i = t % nx + 1, k = t / nx + 1;
+    for (int m = 0; m < PAIRS; ++m)
 #pragma unroll
-        for (int jj = 1; jj <= 4; ++jj) {
-            P(i, jj + ny, k) = P(i, jj, k);
-            P(i, jj - 4, k) = P(i, ny + jj - 4, k);
+        for (int c = 0; c < 3; ++c) p[m][c] = pairs[3 * min(first + m * stride, npairs - 1) + c];
+#pragma unroll
+    for (int m = 0; m < PAIRS; ++m) {
+        v[m][0] = S.f[S.at(p[m][0], p[m][2])];
+        v[m][1] = S.f[S.at(p[m][0] + 19, p[m][2])];
+    }
+#pragma unroll
+    for (int m = 0; m < PAIRS; ++m)
+        if (first + m * stride < npairs) {
+            S.f[S.at(p[m][0], p[m][1])] = v[m][0];
+            S.f[S.at(p[m][0] + 19, p[m][1])] = v[m][1];
         }
-        return;
-    }
-    t -= nyf;
-    if (t < ne) {
-        const int i = t + 1;
-        for (int kk = 1; kk <= 4; ++kk)
-            for (int jj = 1; jj <= 4; ++jj) {
-                P(i, jj - 4, kk - 4) = P(i, ny + jj - 4, nz + kk - 4);
-                P(i, jj + ny, kk - 4) = P(i, jj, nz + kk - 4);
-                P(i, jj + ny, kk + nz) = P(i, jj, kk);
-                P(i, jj - 4, kk + nz) = P(i, ny + jj - 4, kk);
-            }
-    }
 }
 
 // A population cell of both colours in registers: get, set as ColourRef reads and writes them in
@@ -544,11 +655,11 @@ struct OpenCells {
     }
 };
 
-// The boundary updates between the collision and the gradient chain in one launch: open
-// inlet/outlet columns, periodic population copies, periodic phi, each in workgroups of its
-// own (nbc, then npair, then the rest).  The reference copies the periodic populations first
-// and the open boundaries then read and write some of the copied cells; here the order needs
-// no launch between them:
+// The boundary updates after a collision: open inlet/outlet columns, periodic population copies
+// and, with PHI, periodic phi and the open boundaries' ghost phi, each in workgroups of its own
+// (nbc, then npair, then the rest), as a launch (k_boundary) or, without PHI, as workgroups of
+// k_grad_force.  The reference copies the periodic populations first and the open boundaries then
+// read and write some of the copied cells; here the order needs no launch between them:
 //   the open boundaries read a copy's destination where it is copied from (zread), a cell that
 //   neither they nor another copy writes;
 //   after an even step they write none of the copies' cells; after an odd step they write, of
@@ -556,24 +667,24 @@ struct OpenCells {
 //   copies leaves those out.
 // phi: the open boundaries write ghost planes in z of interior columns, the periodic copies
 // read and write planes 1 .. nz.
-// On domains of 32^3 to 64^3 a launch costs 4.5 us whatever it does: as three launches they took
-// 18 of a step's 39 to 45 us, now 8 of 25 to 30.
+// On domains of 32^3 to 64^3 a launch costs 4.5 us whatever it does: as three launches the updates
+// took 18 of a step's 39 to 45 us, as one 8 of 25 to 30, inside the launches around them 3.5.
 //
 // Open inlet/outlet, one thread per (i, j): in_bc / out_bc 2 = Zou-He, 1 = velocity inlet /
-// convective outlet.  w_in: the inlet velocity plane (X1 * Y1); conv: the convective-outlet state, 38 planes of populations [g][e] then phi.
-template <typename T, bool AFTER_ODD>
-__global__ __launch_bounds__(256) void k_boundary(Sparse<T> S, Fields<T> F, StepConst<T> P, BoundaryArgs<T> B) {
+// convective outlet.  w_in: the inlet velocity plane (X1 * Y1); conv: the convective-outlet state,
+// 38 planes of populations [g][e] then phi.
+template <typename T, bool AFTER_ODD, bool PHI>
+__device__ __forceinline__ void boundary_cells(const Sparse<T>& S, const Fields<T>& F, const StepConst<T>& P,
+                                               const BoundaryArgs<T>& B, int block, int threads) {
     const Dims& d = F.d;
-    if ((int)blockIdx.x >= B.nbc) {
-        int t = ((int)blockIdx.x - B.nbc) * 256 + threadIdx.x;
-        if ((int)blockIdx.x < B.nbc + B.npair) {
-            if (t < B.npairs) copy_cell(S, B.pairs[3 * t], B.pairs[3 * t + 1], B.pairs[3 * t + 2]);
-        } else {
-            periodic_phi(F.phi, d, B.kper, B.jper, t - B.npair * 256);
-        }
+    if (block >= B.nbc) {
+        if (block < B.nbc + B.npair)
+            copy_cells(S, B.pairs, B.npairs, (block - B.nbc) * threads * PAIRS + threadIdx.x, threads);
+        else if (PHI)
+            periodic_phi<T>(F.phi, d, B.kper, B.jper, (block - B.nbc - B.npair) * threads + threadIdx.x);
         return;
     }
-    int t = blockIdx.x * 256 + threadIdx.x, in_bc = B.in_bc, out_bc = B.out_bc;
+    int t = block * threads + threadIdx.x, in_bc = B.in_bc, out_bc = B.out_bc;
     // split: the inlet columns and the outlet columns on threads of their own (the two
     // planes share no cell); otherwise one thread does both ends of its column
     if (t >= (B.split ? 2 : 1) * d.nx * d.ny) return;
@@ -586,13 +697,18 @@ __global__ __launch_bounds__(256) void k_boundary(Sparse<T> S, Fields<T> F, Step
     auto ph = [&](int a, int b, int c) -> T& { return F.phi[i4(d, a, b, c)]; };
     const int64_t P2 = (int64_t)d.X1 * d.Y1, col = (int64_t)j * d.X1 + i;
     const OpenCells<T> f{S, B.zread, B.zmap, P2, d.X1, nz, P.rho_ref};
-    if (in_bc == 1) velocity_inlet_column<T, AFTER_ODD>(P, i, j, B.w_in[col], f, wall, ph);
-    if (in_bc == 2 || out_bc == 2) zou_he_column<T, AFTER_ODD>(P, i, j, nz, in_bc == 2, out_bc == 2, f, wall, ph);
+    if (in_bc == 1) velocity_inlet_column<T, AFTER_ODD, PHI>(P, i, j, B.w_in[col], f, wall, ph);
+    if (in_bc == 2 || out_bc == 2) zou_he_column<T, AFTER_ODD, PHI>(P, i, j, nz, in_bc == 2, out_bc == 2, f, wall, ph);
     if (out_bc == 1) {
         auto cs = [&](int e, int g) -> T& { return B.conv[(int64_t)(e + 19 * g) * P2 + col]; };
         auto cp = [&]() -> T& { return B.conv[38 * P2 + col]; };
-        convective_outlet_column<T, AFTER_ODD>(P, i, j, nz, f, wall, ph, cs, cp);
+        convective_outlet_column<T, AFTER_ODD, PHI>(P, i, j, nz, f, wall, ph, cs, cp);
     }
+}
+
+template <typename T, bool AFTER_ODD>
+__global__ __launch_bounds__(256) void k_boundary(Sparse<T> S, Fields<T> F, StepConst<T> P, BoundaryArgs<T> B) {
+    boundary_cells<T, AFTER_ODD, true>(S, F, P, B, blockIdx.x, 256);
 }
 
 // Porous plate at k = zp, one thread per (i, j); pmap as zmap for the planes zp-1, zp, zp+1.

@@ -81,6 +81,7 @@ struct StepConst {
 template <typename T>
 struct BoundaryArgs {
     int nbc, npair;                      // workgroups of the open boundaries, of the periodic copies
+    int blocks;                          // both, in whole rounds of the XCDs (k_grad_force)
     const int32_t* __restrict__ zread;   // open boundaries: cells as read and as written
     const int32_t* __restrict__ zmap;
     int in_bc, out_bc, split;
@@ -88,6 +89,17 @@ struct BoundaryArgs {
     T* __restrict__ conv;
     const int32_t* __restrict__ pairs;   // (slot, dst, src) of the periodic copies
     int npairs, kper, jper;
+};
+
+// Ghost phi written by the collision launch (k_collide): by the threads of the nodes it is copied
+// from, and, where those are solid or the value comes from elsewhere, by its first `rest`
+// workgroups (a multiple of the XCDs).  rest = 0: not by this launch.
+template <typename T>
+struct PhiGhosts {
+    int rest;
+    int kper, jper, in_bc, out_bc;
+    const uint8_t* __restrict__ walls;
+    T* conv;  // phi of the convective outlet's state, [j * X1 + i]
 };
 
 struct NodeLists {

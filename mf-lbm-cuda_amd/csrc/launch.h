@@ -8,8 +8,10 @@ namespace mflbm {
 
 template <typename T>
 struct Launch {
-    static void collide(const Sparse<T>& S, T* phi, const Dims& d, const StepConst<T>& P, bool odd, hipStream_t s);
-    // Periodic copies and open boundaries of one step; B without nbc, npair and split.
+    // ghosts: the ghost phi to write as well (its `rest` is set here), or null
+    static void collide(const Sparse<T>& S, T* phi, const Dims& d, const StepConst<T>& P, bool odd, const PhiGhosts<T>* ghosts,
+                        hipStream_t s);
+    // Periodic copies and open boundaries of one step; B without nbc, npair, blocks and split.
     static void boundary(const Sparse<T>& S, const Fields<T>& F, const StepConst<T>& P, BoundaryArgs<T> B, bool after_odd,
                          hipStream_t s);
     static void porous_plate(const Sparse<T>& S, const Dims& d, const StepConst<T>& P, const int32_t* pmap, int zp,
@@ -20,6 +22,9 @@ struct Launch {
     static void normal_extrap(const Fields<T>& F, const NodeLists& L, hipStream_t s);
     static void curvature(const Fields<T>& F, const StepConst<T>& P, const NodeLists& L, T* aux, hipStream_t s);
     static void gradient(const GradArgs<T>& A, const StepConst<T>& P, hipStream_t s);
+    // The two-pass chain with, in its second launch, the populations' part of boundary().
+    static void gradient_boundary(const GradArgs<T>& A, const Sparse<T>& S, const Fields<T>& F, const StepConst<T>& P,
+                                  BoundaryArgs<T> B, bool after_odd, hipStream_t s);
     // Boxes of the two-pass chain's kernels, and its work lists: first their sizes (na and nb of
     // the descriptors), then, with the descriptors complete, the lists.
     static void tile_grid(const Dims& d, bool force, int (&tiles)[3]);

@@ -9,6 +9,21 @@ namespace mflbm {
 namespace {
 inline unsigned blocks(int64_t n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
+// Threads of periodic_phi.
+int64_t periodic_threads(const Dims& d, int kper, int jper) {
+    return (kper ? (int64_t)d.nx * d.ny : 0) + (jper ? (int64_t)d.nx * d.nz : 0) + (kper && jper ? d.nx : 0);
+}
+
+// Workgroups of the open boundaries and the periodic copies.
+template <typename T>
+void boundary_groups(BoundaryArgs<T>& B, const Dims& d, int threads) {
+    // inlet and outlet on separate threads when both are set and their planes are apart
+    B.split = B.in_bc && B.out_bc && d.nz >= 6;
+    B.nbc = B.in_bc || B.out_bc ? (int)blocks((int64_t)(B.split ? 2 : 1) * d.nx * d.ny, threads) : 0;
+    B.npair = (int)blocks(B.npairs, threads * dev::PAIRS);
+    B.blocks = (B.nbc + B.npair + 7) / 8 * 8;
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void k_pack4(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z,
                                                T* __restrict__ dst, int64_t n) {
@@ -28,28 +43,31 @@ __global__ __launch_bounds__(256) void k_to_real(const double* __restrict__ src,
 }  // namespace
 
 template <typename T>
-void Launch<T>::collide(const Sparse<T>& S, T* phi, const Dims& d, const StepConst<T>& P, bool odd, hipStream_t s) {
+void Launch<T>::collide(const Sparse<T>& S, T* phi, const Dims& d, const StepConst<T>& P, bool odd,
+                        const PhiGhosts<T>* ghosts, hipStream_t s) {
     if (S.nf <= 0) return;
     constexpr int b = MFLBM_COLLIDE_THREADS;
+    unsigned grid = blocks(S.nf, b);
+    PhiGhosts<T> G{};
+    if (ghosts) {
+        G = *ghosts;
+        G.rest = (int)((blocks(dev::ghost_phi_threads(G, d), b) + 7) / 8 * 8);
+        grid += G.rest;
+    }
     if (P.mrt == 2) {
-        if (odd) dev::k_collide<T, true><<<blocks(S.nf, b), b, 0, s>>>(S, phi, d, P);
-        else dev::k_collide<T, false><<<blocks(S.nf, b), b, 0, s>>>(S, phi, d, P);
+        if (odd) dev::k_collide<T, true><<<grid, b, 0, s>>>(S, phi, d, P, G);
+        else dev::k_collide<T, false><<<grid, b, 0, s>>>(S, phi, d, P, G);
     } else {  // collision models 1, 3, 4
-        if (odd) dev::k_collide<T, true, false><<<blocks(S.nf, b), b, 0, s>>>(S, phi, d, P);
-        else dev::k_collide<T, false, false><<<blocks(S.nf, b), b, 0, s>>>(S, phi, d, P);
+        if (odd) dev::k_collide<T, true, false><<<grid, b, 0, s>>>(S, phi, d, P, G);
+        else dev::k_collide<T, false, false><<<grid, b, 0, s>>>(S, phi, d, P, G);
     }
 }
 
 template <typename T>
 void Launch<T>::boundary(const Sparse<T>& S, const Fields<T>& F, const StepConst<T>& P, BoundaryArgs<T> B, bool after_odd,
                          hipStream_t s) {
-    const Dims& d = F.d;
-    // inlet and outlet on separate threads when both are set and their planes are apart
-    B.split = B.in_bc && B.out_bc && d.nz >= 6;
-    B.nbc = B.in_bc || B.out_bc ? (int)blocks((int64_t)(B.split ? 2 : 1) * d.nx * d.ny) : 0;
-    B.npair = (int)blocks(B.npairs);
-    const int64_t nphi = (B.kper ? (int64_t)d.nx * d.ny : 0) + (B.jper ? (int64_t)d.nx * d.nz : 0) + ((B.kper && B.jper) ? d.nx : 0);
-    const unsigned grid = (unsigned)(B.nbc + B.npair) + blocks(nphi);
+    boundary_groups(B, F.d, 256);
+    const unsigned grid = (unsigned)(B.nbc + B.npair) + blocks(periodic_threads(F.d, B.kper, B.jper));
     if (grid == 0) return;
     if (after_odd) dev::k_boundary<T, true><<<grid, 256, 0, s>>>(S, F, P, B);
     else dev::k_boundary<T, false><<<grid, 256, 0, s>>>(S, F, P, B);
@@ -138,15 +156,24 @@ void Launch<T>::tile_fill(const GradArgs<T>& A, uint32_t* l3, uint16_t* l4, uint
 }
 
 template <typename T>
+void Launch<T>::gradient_boundary(const GradArgs<T>& A, const Sparse<T>& S, const Fields<T>& F, const StepConst<T>& P,
+                                  BoundaryArgs<T> B, bool after_odd, hipStream_t s) {
+    constexpr int NX = GradTiles<T>::N[0], NY = GradTiles<T>::N[1], NZ = GradTiles<T>::N[2];
+    constexpr int FX = GradTiles<T>::F[0], FY = GradTiles<T>::F[1], FZ = GradTiles<T>::F[2], threads = (FX + 4) * (FY + 4);
+    GradArgs<T> G = A;
+    const unsigned gn = box_grid(G, false);
+    dev::k_grad_normals<T, NX, NY, NZ><<<gn, (NX + 4) * (NY + 4), 0, s>>>(G, P);
+    const unsigned gf = box_grid(G, true);
+    boundary_groups(B, F.d, threads);
+    if (B.blocks == 0) dev::k_grad_force<T, FX, FY, FZ, 0><<<gf, threads, 0, s>>>(G, P, S, F, B);
+    else if (after_odd) dev::k_grad_force<T, FX, FY, FZ, 1><<<gf + B.blocks, threads, 0, s>>>(G, P, S, F, B);
+    else dev::k_grad_force<T, FX, FY, FZ, 2><<<gf + B.blocks, threads, 0, s>>>(G, P, S, F, B);
+}
+
+template <typename T>
 void Launch<T>::gradient(const GradArgs<T>& A, const StepConst<T>& P, hipStream_t s) {
     if (A.shape == GRAD_SHAPE_TILES) {
-        constexpr int NX = GradTiles<T>::N[0], NY = GradTiles<T>::N[1], NZ = GradTiles<T>::N[2];
-        constexpr int FX = GradTiles<T>::F[0], FY = GradTiles<T>::F[1], FZ = GradTiles<T>::F[2];
-        GradArgs<T> B = A;
-        const unsigned gn = box_grid(B, false);
-        dev::k_grad_normals<T, NX, NY, NZ><<<gn, (NX + 4) * (NY + 4), 0, s>>>(B, P);
-        const unsigned gf = box_grid(B, true);
-        dev::k_grad_force<T, FX, FY, FZ><<<gf, (FX + 4) * (FY + 4), 0, s>>>(B, P);
+        gradient_boundary(A, Sparse<T>{}, Fields<T>{}, P, BoundaryArgs<T>{}, false, s);
         return;
     }
     const int chunks = (A.d.nz + A.kchunk - 1) / A.kchunk;

@@ -21,7 +21,32 @@
 
 namespace mflbm {
 
-template <typename T, bool AFTER_ODD, class Acc, class Wall, class Phi>
+// PHI = false leaves out the ghost planes of phi, which a caller may fill separately: inlet_phi
+// for either inlet, four copies of phi(i, j, nz) for the Zou-He outlet, convective_phi.
+template <typename T, class Phi>
+MFLBM_HD void inlet_phi(const StepConst<T>& P, int i, int j, int w, Phi&& ph) {
+    T& p0 = ph(i, j, 0);
+    const T pv = P.phi_inlet * (1 - w) + p0 * w;
+    p0 = pv;
+    ph(i, j, -1) = pv;
+    ph(i, j, -2) = pv;
+    ph(i, j, -3) = pv;
+}
+
+// phi_nz: phi(i, j, nz) of this step
+template <typename T, class Phi, class CP>
+MFLBM_HD void convective_phi(const StepConst<T>& P, int i, int j, int nz, int w, T phi_nz, Phi&& ph, CP&& cphi) {
+    const T u = P.uin_avg, tmp = T(1.0) / (T(1.0) + u);
+    T& pg = ph(i, j, nz + 1);
+    const T pv = ((cphi() + u * phi_nz) * tmp) * (1 - w) + pg * w;
+    pg = pv;
+    cphi() = pv;
+    ph(i, j, nz + 2) = pv;
+    ph(i, j, nz + 3) = pv;
+    ph(i, j, nz + 4) = pv;
+}
+
+template <typename T, bool AFTER_ODD, bool PHI = true, class Acc, class Wall, class Phi>
 MFLBM_HD void zou_he_column(const StepConst<T>& P, int i, int j, int nz, int do_in, int do_out, Acc&& f, Wall&& wall,
                             Phi&& ph) {
     const T c3 = T(0.333333333333333333), c6 = T(0.166666666666666667);
@@ -31,8 +56,6 @@ MFLBM_HD void zou_he_column(const StepConst<T>& P, int i, int j, int nz, int do_
         rT[1] = P.rho_in;
         rT[0] = P.rho_in * P.sa_inject;
         rT[1] = rT[1] - rT[0];
-        T& p0 = ph(i, j, 0);
-        const T pv = P.phi_inlet * (1 - w) + p0 * w;
         if (!AFTER_ODD) {
             auto f0 = f.rd(i, j, 1, 0), f1 = f.rd(i - 1, j, 1, 1), f2 = f.rd(i + 1, j, 1, 2), f3 = f.rd(i, j - 1, 1, 3),
                  f4 = f.rd(i, j + 1, 1, 4), f7 = f.rd(i - 1, j - 1, 1, 7), f8 = f.rd(i + 1, j - 1, 1, 8),
@@ -77,10 +100,7 @@ MFLBM_HD void zou_he_column(const StepConst<T>& P, int i, int j, int nz, int do_
             }
             d6.put(); d13.put(); d14.put(); d17.put(); d18.put();
         }
-        p0 = pv;
-        ph(i, j, -1) = pv;
-        ph(i, j, -2) = pv;
-        ph(i, j, -3) = pv;
+        if (PHI) inlet_phi<T>(P, i, j, w, ph);
     }
     if (do_out) {
         const int w = wall(i, j, nz);
@@ -137,18 +157,17 @@ MFLBM_HD void zou_he_column(const StepConst<T>& P, int i, int j, int nz, int do_
             }
             d5.put(); d11.put(); d12.put(); d15.put(); d16.put();
         }
-        for (int m = 1; m <= 4; ++m) ph(i, j, nz + m) = phv;
+        if (PHI)
+            for (int m = 1; m <= 4; ++m) ph(i, j, nz + m) = phv;
     }
 }
 
 // Velocity inlet at k = 1 by bounce-back with the injected momentum of the column's inlet
 // velocity w_in, split between the colours by the injected saturation
 // (src/main_iteration_GPU.cu:1008-1077, inlet_bounce_back_velocity_BC_{before,after}_odd).
-template <typename T, bool AFTER_ODD, class Acc, class Wall, class Phi>
+template <typename T, bool AFTER_ODD, bool PHI = true, class Acc, class Wall, class Phi>
 MFLBM_HD void velocity_inlet_column(const StepConst<T>& P, int i, int j, T w_in, Acc&& f, Wall&& wall, Phi&& ph) {
     const int w = wall(i, j, 1);
-    T& p0 = ph(i, j, 0);
-    const T pv = P.phi_inlet * (1 - w) + p0 * w;
     T t2 = w_in * P.relaxation;
     const T t1 = t2 * P.sa_inject;  // fluid 1
     t2 = t2 - t1;                   // fluid 2
@@ -182,24 +201,19 @@ MFLBM_HD void velocity_inlet_column(const StepConst<T>& P, int i, int j, T w_in,
         }
         d6.put(); d13.put(); d14.put(); d17.put(); d18.put();
     }
-    p0 = pv;
-    ph(i, j, -1) = pv;
-    ph(i, j, -2) = pv;
-    ph(i, j, -3) = pv;
+    if (PHI) inlet_phi<T>(P, i, j, w, ph);
 }
 
 // Convective outlet at k = nz: the unknown populations and the ghost phi follow
 // d/dt + u d/dz = 0 with u = P.uin_avg, from the values stored for the column at the last
 // step (cs(e, g) populations, cphi() phi), which are then replaced
 // (src/main_iteration_GPU.cu:1245-1357, outlet_convective_BC_{before,after}_odd).
-template <typename T, bool AFTER_ODD, class Acc, class Wall, class Phi, class CS, class CP>
+template <typename T, bool AFTER_ODD, bool PHI = true, class Acc, class Wall, class Phi, class CS, class CP>
 MFLBM_HD void convective_outlet_column(const StepConst<T>& P, int i, int j, int nz, Acc&& f, Wall&& wall, Phi&& ph,
                                        CS&& cs, CP&& cphi) {
     const T u = P.uin_avg;
     const T tmp = T(1.0) / (T(1.0) + u);
     const int w = wall(i, j, nz);
-    T& pg = ph(i, j, nz + 1);
-    const T pv = ((cphi() + u * ph(i, j, nz)) * tmp) * (1 - w) + pg * w;
     if (!AFTER_ODD) {
         auto f6 = f.rd(i, j, nz, 6), f13 = f.rd(i - 1, j, nz, 13), f14 = f.rd(i + 1, j, nz, 14), f17 = f.rd(i, j - 1, nz, 17),
              f18 = f.rd(i, j + 1, nz, 18);
@@ -241,11 +255,7 @@ MFLBM_HD void convective_outlet_column(const StepConst<T>& P, int i, int j, int 
             cs(17, g) = d16.get(g);
         }
     }
-    pg = pv;
-    cphi() = pv;
-    ph(i, j, nz + 2) = pv;
-    ph(i, j, nz + 3) = pv;
-    ph(i, j, nz + 4) = pv;
+    if (PHI) convective_phi<T>(P, i, j, nz, w, ph(i, j, nz), ph, cphi);
 }
 
 // Recording accessor of the host passes: note(a, b, c, e) for every cell.

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from helpers import assert_same, small_drainage
+from helpers import assert_same, periodic_drop, small_drainage
 from mflbm import gpu
 
 pytestmark = pytest.mark.gpu
@@ -39,6 +39,10 @@ CASES = {
     "four_planes_convective_yper": lambda: small_drainage(n=(10, 6, 4), seed=2, radius=1.5, porosity=0.7, jper=1,
                                                           buffer=1, inlet=1, outlet=1),
     "four_planes_zouhe_yper": lambda: small_drainage(n=(9, 5, 4), seed=3, radius=1.5, porosity=0.7, jper=1, buffer=1),
+    # periodic axes of 8 nodes, the fewest whose ghost phi the collision writes, and of 7
+    "periodic_8_8": lambda: periodic_drop(n=(12, 8, 8), radius=3.0, geo_seed=3),
+    "periodic_7_8": lambda: periodic_drop(n=(12, 7, 8), radius=3.0, geo_seed=4),
+    "periodic_8_7": lambda: periodic_drop(n=(12, 8, 7), radius=3.0, geo_seed=5),
     "one_past_a_box": lambda: small_drainage(n=(17, 9, 9), seed=4, radius=2.5, porosity=0.55, jper=1, buffer=2),
 }
 

@@ -244,7 +244,7 @@ void Launch<T>::monitor(const Sparse<T>& S, const StepConst<T>& P, const T* phi,
                         int nsplit, double* part, double* out, hipStream_t s) {
     dim3 grid(nsplit, d.nz);
     dev::k_monitor_partial<T><<<grid, 256, 0, s>>>(S, P, phi, d, zstart, part);
-    dev::k_monitor_combine<T><<<blocks(d.nz, 64), 64, 0, s>>>(part, nsplit, d.nz, out);
+    dev::k_monitor_combine<T><<<blocks((int64_t)d.nz * dev::MON_VALUES, 64), 64, 0, s>>>(part, nsplit, d.nz, out);
 }
 
 template <typename T>

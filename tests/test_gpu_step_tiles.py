@@ -79,3 +79,19 @@ def test_fp32_boxes_match_the_split_chain(n):
         s.run(1, 30)
     for field in ("pdf", "phi"):
         assert_same(a.download(field), b.download(field), 1e-5, what=f"{n} {field}")
+
+
+def test_phi_read_first_leaves_the_normals_to_bring_up():
+    """a read of phi brings up phi alone; a read of the normals after it still matches the oracle"""
+    geo, p = CASES["one_past_a_box"]()
+    o, g = O.Oracle(p, geo), gpu.Solver(p, geo, gpu.FP64)
+    print("[gpu-step-tiles] phi before normals", flush=True)
+    for s in (o, g):
+        s.setup()
+        s.run(1, 7)
+    for field in ("phi", "cn_x", "phi", "c_norm", "cn_z"):
+        assert_same(g.download(field), o.array(field), 0.0, what=field)
+    o.run(8, 5)
+    g.run(8, 5)
+    for field in ("phi", "pdf"):
+        assert_same(g.download(field), o.array(field), 0.0, what=field)

@@ -438,9 +438,10 @@ __global__ __launch_bounds__(64) void k_conv3_wgrad(const __bf16* __restrict__ X
 
 // Weight gradient partials with the operands shared through LDS.  A workgroup owns one chunk of
 // voxels, one plane offset dz of the taps, a slice of 16 input channels (HALF: the last 8 of an
-// odd multiple of 8) and NN 16-channel tiles of the output; its three waves take the three row
-// offsets dy, so that a wave accumulates the three taps of a row (NN x 3 MFMA tiles, NN x 2
-// with two 8-channel taps to a tile).  Up to `sub` voxels at a time, it loads the rows that
+// odd multiple of 8) and a 16-channel tile of the output; its three waves take the three row
+// offsets dy, so that a wave accumulates the three taps of a row (three MFMA tiles, two with two
+// 8-channel taps to a tile).  With G = 2 a second group of three waves takes every other block of
+// 32 voxels.  Up to `sub` voxels at a time, it loads the rows that
 // these voxels' taps reach once, padded by a zero voxel at each end and a zero row above and
 // below each plane, and the voxels' dZ; s_pos holds each voxel's place among the rows, from
 // which every tap is a fixed distance.  The MFMA operands hold eight voxels of one channel per
@@ -448,15 +449,26 @@ __global__ __launch_bounds__(64) void k_conv3_wgrad(const __bf16* __restrict__ X
 // channels-last rows.  Gathered per tap from global memory and transposed by eight 2-byte LDS
 // reads per operand (k_conv3_wgrad, one wave per tile) the same sums were bound by those reads
 // and by 27-fold loads of the input.  Every accumulator adds the voxel blocks of a chunk in
-// ascending order, as k_conv3_wgrad does.  Measured with the chunk sums against one wave per 16
-// or 32 columns, in us: 64^3 16 -> 16 channels 82.7 to 29.7, 48 -> 16 127 to 61; 32^3 96 -> 32 72
-// to 34.6; 128^3 16 -> 16 317 to 150.  At 64^3 the 64 dependent blocks of a chunk and its four
-// stages of loads bound it, at 128^3 the vector instructions of the staging.
+// ascending order (of each group, whose sums are then added).  Measured with the chunk sums
+// against one wave per 16 or 32 columns, in us: 64^3 16 -> 16 channels 82.7 to 25.2, 48 -> 16 127
+// to 48; 32^3 96 -> 32 72 to 31.9; 128^3 16 -> 16 317 to 142.  At 64^3 the 64 dependent blocks of a
+// chunk and its four stages of loads bound it, at 128^3 the vector instructions of the staging.
+// Two output tiles to a workgroup, sharing the rows, measured no faster on any of 17 shapes but
+// one once a chunk's workgroups share an XCD (128^3 32 -> 32 390 against 402), and slower on others
+// (128^3 16 -> 48 384 against 311, 96^3 24 -> 40 315 against 220).
 struct WgradRows {
+    int gx, gy, per_xcd; // workgroups of a chunk along the input and the output channels; their order
     int ci0, sub;        // first channel, voxels staged at a time
     int lds_dz, lds_pos; // byte offsets of the staged dZ and of s_pos
     FastDiv row, h2, w, h;  // 16-byte units of a padded row; H + 2, W, H
 };
+
+// Place of workgroup b in an order where each of the 8 XCDs takes one contiguous run (workgroups
+// go to the XCDs in turn).
+__device__ __forceinline__ int contiguous_per_xcd(int total, int b) {
+    const int per = total >> 3, rem = total & 7, xcd = b & 7;
+    return xcd * per + min(xcd, rem) + (b >> 3);
+}
 
 __device__ __forceinline__ bf16x4 read_transposed(const unsigned char* lds) {
     typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -464,8 +476,8 @@ __device__ __forceinline__ bf16x4 read_transposed(const unsigned char* lds) {
                                           (__attribute__((address_space(3))) s16x4*)const_cast<unsigned char*>(lds)));
 }
 
-template <int NN, bool HALF>
-__global__ __launch_bounds__(192) void k_conv3_wgrad_rows(const __bf16* __restrict__ X, const __bf16* __restrict__ dZ,
+template <bool HALF, int G>
+__global__ __launch_bounds__(192 * G) void k_conv3_wgrad_rows(const __bf16* __restrict__ X, const __bf16* __restrict__ dZ,
                                                           Grid3 g, int cin, int kp, int coutp, int cout, int chunk,
                                                           WgradRows t, float* __restrict__ part,
                                                           float* __restrict__ bpart) {
@@ -474,13 +486,23 @@ __global__ __launch_bounds__(192) void k_conv3_wgrad_rows(const __bf16* __restri
     constexpr int VB = HALF ? 16 : 32, PU = VB / 16;  // bytes and units of a voxel
     constexpr int NT = HALF ? 2 : 3;                  // MFMA column tiles of a wave
     int* s_pos = reinterpret_cast<int*>(smem + t.lds_pos);
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int TH = 192 * G;
+    const int tid = threadIdx.x, lane = tid & 63, wave6 = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = wave6 / 3, wave = wave6 - 3 * grp;
     const int r = lane & 15, q = lane >> 4;
-    const int slice = blockIdx.x / 3, dzi = blockIdx.x - 3 * slice, ci0 = t.ci0 + 16 * slice;
-    const int n0 = blockIdx.y * 16 * NN, c = blockIdx.z;
+    int slice, dzi, n0, c;
+    {
+        const int per = t.gx * t.gy, l = t.per_xcd ? contiguous_per_xcd(gridDim.x, blockIdx.x) : blockIdx.x;
+        c = l / per;
+        const int xy = l - c * per, by = xy / t.gx, bx = xy - by * t.gx;
+        n0 = by * 16;
+        slice = bx / 3;
+        dzi = bx - 3 * slice;
+    }
+    const int ci0 = t.ci0 + 16 * slice;
     const int M = g.D * g.H * g.W, mb = c * chunk, me = min(M, mb + chunk);
     const int WP = g.W + 2;
-    const bool first = blockIdx.x == 0 && t.ci0 == 0;
+    const bool first = slice == 0 && dzi == 0 && t.ci0 == 0;
     const bool bias = bpart && first && wave == 0;
     // this lane's part of the operand reads: voxel r / 4 of four, channels 4 (r % 4) ..; with two
     // taps to a tile the upper quarters read the next voxel of the row (the tile past the third
@@ -488,14 +510,10 @@ __global__ __launch_bounds__(192) void k_conv3_wgrad_rows(const __bf16* __restri
     const int lane_off = HALF ? ((r >> 1) & 1) * VB + (r & 1) * 8 : (r & 3) * 8;
     const int tap_off = ((wave - 1) * WP - 1) * VB + lane_off;  // of the row's first tap from the voxel
     constexpr int TSTEP = HALF ? 2 * VB : VB;                   // from one column tile to the next
-    f32x4 acc[NN][NT];
+    f32x4 acc[NT];
 #pragma unroll
-    for (int n = 0; n < NN; ++n)
-#pragma unroll
-        for (int u = 0; u < NT; ++u) acc[n][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float bsum[NN];
-#pragma unroll
-    for (int n = 0; n < NN; ++n) bsum[n] = 0.f;
+    for (int u = 0; u < NT; ++u) acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float bsum = 0.f;
     bf16x8 zero;
 #pragma unroll
     for (int j = 0; j < 8; ++j) zero[j] = (__bf16)0.f;
@@ -504,7 +522,7 @@ __global__ __launch_bounds__(192) void k_conv3_wgrad_rows(const __bf16* __restri
     // One stage: the padded rows and the dZ of voxels s0 .. e - 1.  The first PX and PD units of
     // a thread are loaded into registers while the stage before is computed; wider rows load
     // the rest when it is stored.
-    constexpr int PX = 10, PD = 6;
+    constexpr int PX = 10 / G, PD = 6 / G;
     bf16x8 vx[PX], vd[PD];
     int s0, e, xa, ya, za, units, vox, dunits;
     auto stage = [&](int from) {
@@ -516,7 +534,7 @@ __global__ __launch_bounds__(192) void k_conv3_wgrad_rows(const __bf16* __restri
         ya = ra - za * g.H;
         units = (rb - ra + 2 * (zb - za) + 3) * WP * PU;
         vox = (e - s0 + 31) & ~31;
-        dunits = vox * NN * 2;
+        dunits = vox * 2;
     };
     // unit i of the padded rows: its row, and its byte offset in a row of the input (NOWHERE for
     // the padding); fixed over the stages
@@ -532,49 +550,46 @@ __global__ __launch_bounds__(192) void k_conv3_wgrad_rows(const __bf16* __restri
         return buffer_load16(xbuf, i < units && (unsigned)y < (unsigned)g.H && (unsigned)z < (unsigned)g.D ? from : NOWHERE, 0);
     };
     auto dz_unit = [&](int i) {
-        const int mv = s0 + i / (2 * NN), n = n0 + 8 * (i % (2 * NN));
+        const int mv = s0 + i / 2, n = n0 + 8 * (i % 2);
         return buffer_load16(dbuf, mv < e && n < cout ? 2u * (mv * cout + n) : NOWHERE, 0);
     };
     int prow[PX];
     uint32_t pcol[PX];
 #pragma unroll
-    for (int m = 0; m < PX; ++m) place(tid + 192 * m, prow[m], pcol[m]);
+    for (int m = 0; m < PX; ++m) place(tid + TH * m, prow[m], pcol[m]);
     auto fetch = [&]() {
 #pragma unroll
-        for (int m = 0; m < PX; ++m) vx[m] = row_unit(tid + 192 * m, prow[m], pcol[m]);
+        for (int m = 0; m < PX; ++m) vx[m] = row_unit(tid + TH * m, prow[m], pcol[m]);
 #pragma unroll
-        for (int m = 0; m < PD; ++m) vd[m] = dz_unit(tid + 192 * m);
+        for (int m = 0; m < PD; ++m) vd[m] = dz_unit(tid + TH * m);
     };
     auto keep = [&]() {
         bf16x8 *rows = reinterpret_cast<bf16x8*>(smem + 128), *ds = reinterpret_cast<bf16x8*>(smem + t.lds_dz);
 #pragma unroll
         for (int m = 0; m < PX; ++m)
-            if (tid + 192 * m < units) rows[tid + 192 * m] = vx[m];
+            if (tid + TH * m < units) rows[tid + TH * m] = vx[m];
 #pragma unroll
         for (int m = 0; m < PD; ++m)
-            if (tid + 192 * m < dunits) ds[tid + 192 * m] = vd[m];
-        for (int i = tid + 192 * PX; i < units; i += 192) {
+            if (tid + TH * m < dunits) ds[tid + TH * m] = vd[m];
+        for (int i = tid + TH * PX; i < units; i += TH) {
             int row;
             uint32_t col;
             place(i, row, col);
             rows[i] = row_unit(i, row, col);
         }
-        for (int i = tid + 192 * PD; i < dunits; i += 192) ds[i] = dz_unit(i);
-        for (int v = tid; v < vox; v += 192) {
+        for (int i = tid + TH * PD; i < dunits; i += TH) ds[i] = dz_unit(i);
+        for (int v = tid; v < vox; v += TH) {
             const int row = quot(xa + v, t.w), zo = quot(ya + row, t.h);  // rows and planes below voxel s0's
             s_pos[v] = s0 + v < e ? 128 + ((row + 2 * zo + 1) * WP + xa + v - row * g.W + 1) * VB : -1;
         }
     };
     const int v0 = 8 * q + (r >> 2);  // and v0 + 4: the voxels this lane reads for its group
-    bf16x8 a[2][NN], b[2][NT];
-    const unsigned char* const dz_lane = smem + t.lds_dz + v0 * NN * 32 + (r & 3) * 8;
+    bf16x8 a[2], b[2][NT];
+    const unsigned char* const dz_lane = smem + t.lds_dz + v0 * 32 + (r & 3) * 8;
     auto read_ab = [&](int slot, int ms, int p0, int p1) {
-        const unsigned char* d = dz_lane + ms * NN * 32;
-#pragma unroll
-        for (int n = 0; n < NN; ++n) {
-            const bf16x4 lo = read_transposed(d + n * 32), hi = read_transposed(d + (4 * NN + n) * 32);
-            a[slot][n] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        }
+        const unsigned char* d = dz_lane + ms * 32;
+        const bf16x4 dlo = read_transposed(d), dhi = read_transposed(d + 4 * 32);
+        a[slot] = __builtin_shufflevector(dlo, dhi, 0, 1, 2, 3, 4, 5, 6, 7);
         // a voxel past the grid reads the zeros at 0
         const unsigned char *x0 = smem + (p0 >= 0 ? p0 + tap_off : lane_off), *x1 = smem + (p1 >= 0 ? p1 + tap_off : lane_off);
 #pragma unroll
@@ -594,65 +609,74 @@ __global__ __launch_bounds__(192) void k_conv3_wgrad_rows(const __bf16* __restri
             stage(e);
             fetch();
         }
-        // operands run one block of 32 voxels ahead of the MFMAs, places two
+        // group grp takes blocks grp, grp + G, ..; operands run one of its blocks of 32 voxels
+        // ahead of the MFMAs, places two
+        const int mine = (blocks - grp + G - 1) / G, last = blocks - 1;
         const int* pos = s_pos + v0;
-        int p0 = pos[0], p1 = pos[4];
-        read_ab(0, 0, p0, p1);
-        p0 = blocks > 1 ? pos[32] : -1;
-        p1 = blocks > 1 ? pos[36] : -1;
+        auto nth = [&](int i) { return min(grp + G * i, last) * 32; };
+        int p0 = pos[nth(0)], p1 = pos[nth(0) + 4];
+        read_ab(0, nth(0), p0, p1);
+        p0 = pos[nth(1)];
+        p1 = pos[nth(1) + 4];
         auto block = [&](int slot, int i) {
             const int n0_ = p0, n1_ = p1;
-            const int at = min(i + 2, blocks - 1) * 32;
-            p0 = pos[at];
-            p1 = pos[at + 4];
-            read_ab(slot ^ 1, min(i + 1, blocks - 1) * 32, n0_, n1_);
+            p0 = pos[nth(i + 2)];
+            p1 = pos[nth(i + 2) + 4];
+            read_ab(slot ^ 1, nth(i + 1), n0_, n1_);
             __builtin_amdgcn_sched_barrier(0);
             if (bias) {
 #pragma unroll
-                for (int n = 0; n < NN; ++n)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) bsum[n] += bf2f(a[slot][n][j]);
+                for (int j = 0; j < 8; ++j) bsum += bf2f(a[slot][j]);
             }
 #pragma unroll
-            for (int n = 0; n < NN; ++n)
-#pragma unroll
-                for (int u = 0; u < NT; ++u)
-                    acc[n][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[slot][n], b[slot][u], acc[n][u], 0, 0, 0);
+            for (int u = 0; u < NT; ++u)
+                acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[slot], b[slot][u], acc[u], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         };
-        for (int i = 0; i < blocks; i += 2) {
+        for (int i = 0; i < mine; i += 2) {
             block(0, i);
-            if (i + 1 < blocks) block(1, i + 1);
+            if (i + 1 < mine) block(1, i + 1);
         }
         if (!more) break;
         lds_barrier();  // every wave is done with the stage; the loads of the next stay in flight
     }
+    if (G > 1) {
+        // the second group's sums are added to the first's
+        __syncthreads();
+        f32x4* const sum = reinterpret_cast<f32x4*>(smem) + wave * 64 * NT + lane;
+        float* const bs = reinterpret_cast<float*>(smem + 3 * 64 * NT * 16) + lane;
+        if (grp == 1) {
 #pragma unroll
-    for (int n = 0; n < NN; ++n) {
-        const int row0 = n0 + 16 * n;
-        if (row0 >= coutp) break;
-        if (bias) {
-            // lanes r, r + 16, r + 32, r + 48 hold row r: fixed pairing order
-            const float s1 = bsum[n] + __shfl_xor(bsum[n], 16);
-            const float s2 = s1 + __shfl_xor(s1, 32);
-            if (q == 0 && row0 + r < cout) bpart[(int64_t)c * cout + row0 + r] = s2;
+            for (int u = 0; u < NT; ++u) sum[u * 64] = acc[u];
+            if (bias) bs[0] = bsum;
         }
-        // column r of tile u: its tap's channel
+        __syncthreads();
+        if (grp == 1) return;
 #pragma unroll
-        for (int u = 0; u < NT; ++u) {
-            const int dx = HALF ? 2 * u + (r >> 3) : u;
-            if (dx > 2) continue;
-            const int k = ((dzi * 3 + wave) * 3 + dx) * cin + ci0 + (HALF ? r & 7 : r);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) part[((int64_t)c * coutp + row0 + 4 * q + j) * kp + k] = acc[n][u][j];
-        }
-        // the padding columns
-        if (first)
-            for (int i = tid; i < 16 * (kp - 27 * cin); i += 192) {
-                const int pad = kp - 27 * cin, row = i / pad;
-                part[((int64_t)c * coutp + row0 + row) * kp + 27 * cin + i - row * pad] = 0.f;
-            }
+        for (int u = 0; u < NT; ++u) acc[u] += sum[u * 64];
+        if (bias) bsum += bs[0];
     }
+    if (bias) {
+        // lanes r, r + 16, r + 32, r + 48 hold row r: fixed pairing order
+        const float s1 = bsum + __shfl_xor(bsum, 16);
+        const float s2 = s1 + __shfl_xor(s1, 32);
+        if (q == 0 && n0 + r < cout) bpart[(int64_t)c * cout + n0 + r] = s2;
+    }
+    // column r of tile u: its tap's channel
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+        const int dx = HALF ? 2 * u + (r >> 3) : u;
+        if (dx > 2) continue;
+        const int k = ((dzi * 3 + wave) * 3 + dx) * cin + ci0 + (HALF ? r & 7 : r);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[((int64_t)c * coutp + n0 + 4 * q + j) * kp + k] = acc[u][j];
+    }
+    // the padding columns
+    if (first)
+        for (int i = tid; i < 16 * (kp - 27 * cin); i += 192) {
+            const int pad = kp - 27 * cin, row = i / pad;
+            part[((int64_t)c * coutp + n0 + row) * kp + 27 * cin + i - row * pad] = 0.f;
+        }
 }
 
 // W'[ci][tap' * cout + co] = W[co][(26 - tap') * cin + ci]  (bf16, padded: ci to 16, k' to 32)
@@ -1096,9 +1120,6 @@ bool wgrad_args_ok(const void* x, const void* dz, int32_t D, int32_t H, int32_t 
 bool wgrad_rows(const __bf16* X, const __bf16* dZ, const Grid3& g, int cin, int kp, int coutp, int cout, int chunk,
                 int nchunk, float* part, float* bpart, hipStream_t s) {
     const int full = cin / 16, ntiles = coutp / 16;
-    // two output tiles per wave share the input operands; with fewer than 512 workgroups that
-    // way (two per CU) the tiles go to workgroups of their own
-    const int nn = (int64_t)3 * std::max(full, 1) * ((ntiles + 1) / 2) * nchunk >= 512 && ntiles > 1 ? 2 : 1;
     auto launch = [&](bool half) {
         const int64_t vb = half ? 16 : 32, WP = g.W + 2, WH = (int64_t)g.W * g.H;
         WgradRows t;
@@ -1106,30 +1127,43 @@ bool wgrad_rows(const __bf16* X, const __bf16* dZ, const Grid3& g, int cin, int 
         // as many voxels at a time as 48 KB hold (three workgroups per CU); wide rows take more
         // LDS, down to 128 voxels at a time
         int64_t lds = 0;
-        for (t.sub = nn == 2 ? 256 : 512;; t.sub /= 2) {
+        for (t.sub = 512;; t.sub /= 2) {
             const int64_t rows = (t.sub + g.W - 2) / g.W + 2 * ((t.sub + WH - 2) / WH) + 3;
             t.lds_dz = (int)(128 + std::min<int64_t>(rows * WP * vb, 1 << 20));
-            t.lds_pos = t.lds_dz + t.sub * nn * 32;
-            lds = t.lds_pos + 4 * t.sub;
+            t.lds_pos = t.lds_dz + t.sub * 32;
+            lds = std::max<int64_t>(t.lds_pos + 4 * t.sub, 3 * 64 * 3 * 16 + 64 * 4);  // and the second group's sums
             if (lds <= 48 * 1024 || t.sub == 128) break;
         }
-        // exact quotients; 24-bit products and 31-bit offsets of the loads
-        const int64_t M = WH * g.D;
+        t.gx = 3 * (half ? 1 : full);
+        t.gy = ntiles;
+        const int64_t M = WH * g.D, wgs = (int64_t)t.gx * t.gy * nchunk;
+        // exact quotients; 24-bit products and 31-bit offsets of the loads; threads of the launch
         if (lds > 80 * 1024 || (int64_t)(g.H + 2) * (g.H + 600) >= (1ll << 32) || (int64_t)(g.W + 600) * g.W >= (1ll << 32) ||
-            (int64_t)g.D * g.H >= (1 << 24) || 2ll * g.W * cin >= (1 << 24) || 2 * M * std::max(cin, cout) >= NOWHERE)
+            (int64_t)g.D * g.H >= (1 << 24) || 2ll * g.W * cin >= (1 << 24) || 2 * M * std::max(cin, cout) >= NOWHERE ||
+            wgs >= 1 << 23)
             return false;
+        // The workgroups of a chunk read the same rows and the same dZ.  On inputs that an XCD's
+        // 4 MB L2 holds a good part of, they may lie anywhere; beyond, they go to one XCD (us, in
+        // turn and contiguous: 16^3 192 -> 64 22.1 and 23.7, 32^3 96 -> 32 31.9 and 32.8, 64^3
+        // 16 -> 16 29.1 and 29.0, 48 -> 16 59.3 and 48.3, 128^3 48 -> 16 528 and 323).
+        t.per_xcd = 2 * M * (cin + cout) > 16 << 20;
+        // Up to two workgroups per CU the staging and the operand latency bound a workgroup, and a
+        // second group of waves halves both (us with one and two: 64^3 16 -> 16 29.1 and 25.2, 16^3
+        // 32 -> 64 9.3 and 8.4); beyond, more workgroups per CU do better (32^3 32 -> 32 16.0 and
+        // 16.9, 128^3 16 -> 16 142 and 183).
+        const bool two = wgs <= 512;
         t.row = fast_div((uint32_t)(WP * vb / 16));
         t.h2 = fast_div(g.H + 2);
         t.w = fast_div(g.W);
         t.h = fast_div(g.H);
-        const dim3 grid(3 * (half ? 1 : full), (ntiles + nn - 1) / nn, nchunk);
-#define MFNN_ROWS(n, h) k_conv3_wgrad_rows<n, h><<<grid, 192, lds, s>>>(X, dZ, g, cin, kp, coutp, cout, chunk, t, part, bpart)
+#define MFNN_ROWS(h, gr) \
+    k_conv3_wgrad_rows<h, gr><<<(unsigned)wgs, 192 * gr, lds, s>>>(X, dZ, g, cin, kp, coutp, cout, chunk, t, part, bpart)
         if (half) {
-            if (nn == 2) MFNN_ROWS(2, true);
-            else MFNN_ROWS(1, true);
+            if (two) MFNN_ROWS(true, 2);
+            else MFNN_ROWS(true, 1);
         } else {
-            if (nn == 2) MFNN_ROWS(2, false);
-            else MFNN_ROWS(1, false);
+            if (two) MFNN_ROWS(false, 2);
+            else MFNN_ROWS(false, 1);
         }
 #undef MFNN_ROWS
         return true;

@@ -451,7 +451,7 @@ __global__ __launch_bounds__(64) void k_conv3_wgrad(const __bf16* __restrict__ X
 // and by 27-fold loads of the input.  Every accumulator adds the voxel blocks of a chunk in
 // ascending order (of each group, whose sums are then added).  Measured with the chunk sums
 // against one wave per 16 or 32 columns, in us: 64^3 16 -> 16 channels 82.7 to 25.2, 48 -> 16 127
-// to 48; 32^3 96 -> 32 72 to 31.9; 128^3 16 -> 16 317 to 142.  At 64^3 the 64 dependent blocks of a
+// to 47; 32^3 96 -> 32 72 to 31.7; 128^3 16 -> 16 317 to 132.  At 64^3 the 64 dependent blocks of a
 // chunk and its four stages of loads bound it, at 128^3 the vector instructions of the staging.
 // Two output tiles to a workgroup, sharing the rows, measured no faster on any of 17 shapes but
 // one once a chunk's workgroups share an XCD (128^3 32 -> 32 390 against 402), and slower on others
@@ -459,6 +459,7 @@ __global__ __launch_bounds__(64) void k_conv3_wgrad(const __bf16* __restrict__ X
 struct WgradRows {
     int gx, gy, per_xcd; // workgroups of a chunk along the input and the output channels; their order
     int ci0, sub;        // first channel, voxels staged at a time
+    int planes;          // a plane holds a stage, and there are several
     int lds_dz, lds_pos; // byte offsets of the staged dZ and of s_pos
     FastDiv row, h2, w, h;  // 16-byte units of a padded row; H + 2, W, H
 };
@@ -524,7 +525,8 @@ __global__ __launch_bounds__(192 * G) void k_conv3_wgrad_rows(const __bf16* __re
     // the rest when it is stored.
     constexpr int PX = 10 / G, PD = 6 / G;
     bf16x8 vx[PX], vd[PD];
-    int s0, e, xa, ya, za, units, vox, dunits;
+    int s0, e, xa, ya, za, units, vox, dunits, ylast;
+    bool flat;  // every voxel of the stage is in plane za, and the rows' last is ylast - 1
     auto stage = [&](int from) {
         s0 = from;
         e = min(me, s0 + t.sub);
@@ -532,12 +534,14 @@ __global__ __launch_bounds__(192 * G) void k_conv3_wgrad_rows(const __bf16* __re
         za = ra / g.H;
         xa = s0 - ra * g.W;
         ya = ra - za * g.H;
+        flat = t.planes && zb == za;
+        ylast = min(g.H, ya + rb - ra + 2);
         units = (rb - ra + 2 * (zb - za) + 3) * WP * PU;
         vox = (e - s0 + 31) & ~31;
         dunits = vox * 2;
     };
     // unit i of the padded rows: its row, and its byte offset in a row of the input (NOWHERE for
-    // the padding); fixed over the stages
+    // the padding)
     auto place = [&](int i, int& row, uint32_t& col) {
         row = quot(i, t.row);
         const int u = i - row * WP * PU, x = u / PU - 1;
@@ -553,13 +557,50 @@ __global__ __launch_bounds__(192 * G) void k_conv3_wgrad_rows(const __bf16* __re
         const int mv = s0 + i / 2, n = n0 + 8 * (i % 2);
         return buffer_load16(dbuf, mv < e && n < cout ? 2u * (mv * cout + n) : NOWHERE, 0);
     };
-    int prow[PX];
-    uint32_t pcol[PX];
+    // Within a plane the rows of a stage are one run of the input: a unit's offset from the row of
+    // the first voxel is fixed over the stages, and one compare says whether the run holds it (the
+    // general address takes 20 instructions; 128^3 16 -> 16 142 to 133 us, 48 -> 16 323 to 308).
+    // Two groups of waves have half the units each and keep the general places in registers.
+    const uint32_t rowbytes = 2u * g.W * cin;
+    uint32_t at[PX];
+    int prow[G == 1 ? 1 : PX];
+    uint32_t pcol[G == 1 ? 1 : PX];
+    if (G > 1) {
 #pragma unroll
-    for (int m = 0; m < PX; ++m) place(tid + TH * m, prow[m], pcol[m]);
+        for (int m = 0; m < PX; ++m) place(tid + TH * m, prow[G == 1 ? 0 : m], pcol[G == 1 ? 0 : m]);
+    } else if (t.planes) {
+#pragma unroll
+        for (int m = 0; m < PX; ++m) {
+            int row;
+            uint32_t col;
+            place(tid + TH * m, row, col);
+            at[m] = col == NOWHERE ? NOWHERE : (row - 1) * rowbytes + col;
+        }
+    }
     auto fetch = [&]() {
+        if (G > 1) {
 #pragma unroll
-        for (int m = 0; m < PX; ++m) vx[m] = row_unit(tid + TH * m, prow[m], pcol[m]);
+            for (int m = 0; m < PX; ++m) vx[m] = row_unit(tid + TH * m, prow[G == 1 ? 0 : m], pcol[G == 1 ? 0 : m]);
+        } else if (flat) {
+            const int z = za + dzi - 1;
+            const bool in = (unsigned)z < (unsigned)g.D;
+            const uint32_t first = ya * rowbytes, end = in ? ylast * rowbytes : 0, plane = in ? z * g.H * rowbytes : 0;
+#pragma unroll
+            for (int m = 0; m < PX; ++m) {
+                const uint32_t o = first + at[m];
+                vx[m] = buffer_load16(xbuf, o < end ? o : NOWHERE, plane);
+            }
+        } else {
+            int i = tid;
+            asm volatile("" : "+v"(i));  // computed here, not kept over the stages in 20 registers
+#pragma unroll
+            for (int m = 0; m < PX; ++m) {
+                int row;
+                uint32_t col;
+                place(i + TH * m, row, col);
+                vx[m] = row_unit(i + TH * m, row, col);
+            }
+        }
 #pragma unroll
         for (int m = 0; m < PD; ++m) vd[m] = dz_unit(tid + TH * m);
     };
@@ -1152,6 +1193,7 @@ bool wgrad_rows(const __bf16* X, const __bf16* dZ, const Grid3& g, int cin, int 
         // 32 -> 64 9.3 and 8.4); beyond, more workgroups per CU do better (32^3 32 -> 32 16.0 and
         // 16.9, 128^3 16 -> 16 142 and 183).
         const bool two = wgs <= 512;
+        t.planes = WH >= t.sub && chunk > t.sub;
         t.row = fast_div((uint32_t)(WP * vb / 16));
         t.h2 = fast_div(g.H + 2);
         t.w = fast_div(g.W);

@@ -140,3 +140,11 @@ def test_bad_values_stay_local(nn, bad):
     finite = np.isfinite(dw.numpy()[:, :27 * cin].reshape(16, 27, cin)).all(axis=(0, 1))
     assert list(finite) == [c != 5 for c in range(cin)]
     assert np.all(np.isfinite(db.numpy()))
+
+
+@pytest.mark.parametrize("shape,cin,cout,chunk", [
+    ((40, 33, 30), 48, 32, 1024), ((40, 66, 70), 32, 16, 2048), ((40, 66, 70), 40, 8, 2048), ((6, 11, 150), 96, 64, 1024)])
+def test_weight_gradient_many_stages(nn, shape, cin, cout, chunk):
+    """chunks of several stages with one group of waves per workgroup (more than 512 workgroups),
+    stages inside a plane and across two, and inputs above 16 MB, whose chunks go to one XCD"""
+    test_weight_gradient(nn, shape, cin, cout, chunk)

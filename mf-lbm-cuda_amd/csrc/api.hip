@@ -42,10 +42,11 @@ struct mflbm_handle {
     // the two-pass gradient chain's intermediate: (cn_x, cn_y, cn_z, c_norm) of each S2 node
     // side by side (4 * S2 elements), written by its first kernel and read by its second
     void* cnp = nullptr;
-    // the solid normals as 4-vectors (snx, sny, snz, 0) per S4 node: what the two-pass
-    // gradient chain reads at wetting nodes (one vector load); rebuilt whenever snx/sny/snz
-    // change
+    // the solid normals of its wetting nodes in the order it reads them (3 * n_wet); rebuilt
+    // whenever snx/sny/snz change
     void* snp = nullptr;
+    int32_t* wet = nullptr;  // S4 index of those nodes
+    int n_wet = 0;
     uint8_t* walls = nullptr;
     int8_t* wtype = nullptr;
     uint32_t *l_fluid = nullptr, *l_fluid_ext = nullptr, *l_sb = nullptr;
@@ -75,8 +76,8 @@ struct mflbm_handle {
     int grad_shape = 0, tiles_x = 0, tiles_y = 0, kchunk = 0, box_order = 0;
     // work lists of the two-pass chain's boxes (lattice.h TileLists)
     TileDesc *ndesc = nullptr, *fdesc = nullptr;
-    uint32_t *l3 = nullptr, *l6 = nullptr;
-    uint16_t *l4 = nullptr, *l7 = nullptr;
+    uint32_t *l3 = nullptr, *l4 = nullptr, *l6 = nullptr;
+    uint16_t* l7 = nullptr;
     int32_t* r7 = nullptr;
     uint8_t* tile_fluid = nullptr;
     bool split_gradient = false;
@@ -162,11 +163,13 @@ GradArgs<T> grad_args(const mflbm_handle* h) {
     A.tag = h->tag;
     A.snx = (const T*)h->snx; A.sny = (const T*)h->sny; A.snz = (const T*)h->snz;
     A.snp = (const T*)h->snp;
+    A.nwet = h->n_wet;
     A.aux = (T*)h->aux;
     A.cnx = (T*)h->cnx; A.cny = (T*)h->cny; A.cnz = (T*)h->cnz; A.cnorm = (T*)h->cnorm;
     A.cnp = (T*)h->cnp;
     A.shape = h->grad_shape; A.tiles_x = h->tiles_x; A.tiles_y = h->tiles_y; A.kchunk = h->kchunk;
     A.tiles_z = 1; A.box_order = h->box_order;
+    A.jper = h->p.jper; A.kper = h->p.kper;
     A.lists = TileLists{h->ndesc, h->fdesc, h->l3, h->l4, h->l6, h->l7, h->r7, h->tile_fluid};
     return A;
 }
@@ -288,14 +291,14 @@ int materialize_phi(mflbm_handle* h) {
     return 0;
 }
 
-// The gradient chain's copy of the solid normals, (snx, sny, snz, 0) per S4 node.
+// The two-pass gradient chain's copy of the solid normals.
 void pack_solid_normals(mflbm_handle* h) {
     if (h->prec == MFLBM_FP64)
-        Launch<double>::pack4((const double*)h->snx, (const double*)h->sny, (const double*)h->snz, (double*)h->snp,
-                              h->d.S4, h->stream);
+        Launch<double>::pack_solid_normals((const double*)h->snx, (const double*)h->sny, (const double*)h->snz, h->wet,
+                                           h->n_wet, (double*)h->snp, h->stream);
     else
-        Launch<float>::pack4((const float*)h->snx, (const float*)h->sny, (const float*)h->snz, (float*)h->snp, h->d.S4,
-                             h->stream);
+        Launch<float>::pack_solid_normals((const float*)h->snx, (const float*)h->sny, (const float*)h->snz, h->wet,
+                                          h->n_wet, (float*)h->snp, h->stream);
 }
 
 // The work lists of the two-pass gradient chain, from the node tags.
@@ -312,7 +315,7 @@ int build_tile_lists(mflbm_handle* h) {
     Launch<T>::tile_counts(grad_args<T>(h), h->ndesc, h->fdesc, h->stream);
     HIPCHK(h, hipGetLastError());
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    int64_t na[2], nb[2];
+    int64_t na[2], nb[2], nw = 0;
     for (int f = 0; f < 2; ++f) {
         std::vector<TileDesc> td(boxes[f]);
         HIPCHK(h, hipMemcpy(td.data(), *dev[f], td.size() * sizeof(TileDesc), hipMemcpyDeviceToHost));
@@ -322,18 +325,26 @@ int build_tile_lists(mflbm_handle* h) {
             x.b = (int32_t)nb[f];
             na[f] += x.na;
             nb[f] += x.nb;
+            const int32_t wet = x.wet;
+            x.wet = (int32_t)nw;
+            nw += wet;
         }
         if (na[f] > INT32_MAX || nb[f] > INT32_MAX) return fail(h, "too many nodes for the gradient work lists");
         HIPCHK(h, hipMemcpy(*dev[f], td.data(), td.size() * sizeof(TileDesc), hipMemcpyHostToDevice));
     }
     auto room = [](int64_t n) { return (size_t)std::max<int64_t>(1, n); };
     HIPCHK(h, hipMalloc(&h->l3, room(na[0]) * sizeof(uint32_t)));
-    HIPCHK(h, hipMalloc(&h->l4, room(nb[0]) * sizeof(uint16_t)));
+    HIPCHK(h, hipMalloc(&h->l4, room(nb[0]) * sizeof(uint32_t)));
     HIPCHK(h, hipMalloc(&h->l6, room(na[1]) * sizeof(uint32_t)));
     HIPCHK(h, hipMalloc(&h->l7, room(nb[1]) * sizeof(uint16_t)));
     HIPCHK(h, hipMalloc(&h->r7, room(nb[1]) * sizeof(int32_t)));
     HIPCHK(h, hipMalloc(&h->tile_fluid, boxes[1] * Launch<T>::tile_columns()));
-    Launch<T>::tile_fill(grad_args<T>(h), h->l3, h->l4, h->l6, h->l7, h->r7, h->tile_fluid, h->stream);
+    h->n_wet = (int)nw;
+    HIPCHK(h, hipMalloc(&h->wet, room(nw) * sizeof(int32_t)));
+    HIPCHK(h, hipMalloc(&h->snp, room(nw) * 3 * sizeof(T)));
+    Launch<T>::tile_fill(grad_args<T>(h), TileFill{h->l3, h->l4, h->l6, h->l7, h->r7, h->wet, h->tile_fluid}, h->stream);
+    HIPCHK(h, hipGetLastError());
+    pack_solid_normals(h);
     HIPCHK(h, hipGetLastError());
     return 0;
 }
@@ -345,7 +356,7 @@ void free_all(mflbm_handle* h) {
                     h->walls, h->wtype, h->l_fluid, h->l_fluid_ext, h->l_sb, h->mon_part, h->mon_out, h->vprev, h->vpart,
                     h->cells, h->aux, h->nb, h->nb16, h->nbb, h->pairs[0], h->pairs[1], h->zmap, h->zread[0], h->zread[1], h->pmap, h->w_in, h->conv,
                     h->ext_node, h->ext_off, h->zstart,
-                    h->tag, h->macro_buf, h->ndesc, h->fdesc, h->l3, h->l4, h->l6, h->l7, h->r7, h->tile_fluid};
+                    h->tag, h->macro_buf, h->ndesc, h->fdesc, h->l3, h->l4, h->l6, h->l7, h->r7, h->tile_fluid, h->wet};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     h->pdf = h->phi = h->cnx = h->cny = h->cnz = h->cnorm = h->cnp = h->snp = h->curv = h->snx = h->sny = h->snz = nullptr;
@@ -361,9 +372,9 @@ void free_all(mflbm_handle* h) {
     h->w_in = h->conv = nullptr;
     h->tag = nullptr;
     h->ndesc = h->fdesc = nullptr;
-    h->l3 = h->l6 = nullptr;
-    h->l4 = h->l7 = nullptr;
-    h->r7 = nullptr;
+    h->l3 = h->l4 = h->l6 = nullptr;
+    h->l7 = nullptr;
+    h->r7 = h->wet = nullptr;
     h->tile_fluid = nullptr;
     if (h->stream) { (void)hipStreamDestroy(h->stream); h->stream = nullptr; }
 }
@@ -573,8 +584,6 @@ int mflbm_create(const mflbm_params* params, const int8_t* geometry, mflbm_handl
         HIPCHK(h, hipStreamSynchronize(h->stream));
         (void)hipFree(sx); (void)hipFree(sy); (void)hipFree(sz);
     }
-    HIPCHK(h, hipMalloc(&h->snp, 4 * d.S4 * es));
-    pack_solid_normals(h);
 
     // node lists from the classified geometry
     std::vector<uint8_t> walls(d.S2);
@@ -775,6 +784,11 @@ static int init_populations(mflbm_handle* h, const double* rho, const double* u,
     std::lock_guard<std::recursive_mutex> lock(device_lock());
     if (!h) return -1;
     h->vprev_valid = false;
+    // after a step: the boxes leave the phi of solid nodes behind, which the solid cells start from
+    if (h->grad_dirty) {
+        if (h->prec == MFLBM_FP64) Launch<double>::phi_extrap(fields<double>(h), lists(h), h->stream, true);
+        else Launch<float>::phi_extrap(fields<float>(h), lists(h), h->stream, true);
+    }
     const int64_t n = h->d.S1;
     const double* src[4] = {rho, u, v, w};
     double* dv[4] = {nullptr, nullptr, nullptr, nullptr};

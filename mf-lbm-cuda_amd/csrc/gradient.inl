@@ -481,10 +481,11 @@ struct BoxEntry {
 // First list: the solid-boundary nodes of the box and its 1-halo that a fluid node of the box
 // reads (or, in k_grad_normals, that are written back); second: its fluid nodes.
 template <typename T, int TX, int TY, int TZ, bool FORCE, bool FILL>
-__global__ __launch_bounds__(64) void k_tile_lists(GradArgs<T> A, TileDesc* __restrict__ desc, uint32_t* __restrict__ la,
-                                                   uint16_t* __restrict__ lb, int32_t* __restrict__ rec,
-                                                   uint8_t* __restrict__ fluid) {
+__global__ __launch_bounds__(64) void k_tile_lists(GradArgs<T> A, TileDesc* __restrict__ desc, TileFill out) {
     constexpr int LX = TX + 4, LY = TY + 4, LZ = TZ + 4, NC = LX * LY, NL = NC * LZ;
+    // K3's results that a later kernel of the step reads: the planes next to the open boundaries
+    // (whose ghost phi wall columns keep) and what the periodic images are copied from
+    const int zl = A.kper ? 4 : 1, yl = A.jper ? 4 : 0;
     using Entry = BoxEntry<LX, LY, LZ>;
     __shared__ unsigned s_fluid[NC];
     const Dims& d = A.d;
@@ -495,7 +496,9 @@ __global__ __launch_bounds__(64) void k_tile_lists(GradArgs<T> A, TileDesc* __re
     const int ox = min(TX, d.nx + last + 1 - i0), oy = min(TY, d.ny + last + 1 - j0), oz = min(TZ, d.nz + last + 1 - k0);
     for (int c = lane; c < NC; c += 64) s_fluid[c] = 0;
     __syncthreads();
-    int na = FILL ? desc[b].a : 0, nb = FILL ? desc[b].b : 0;
+    int na = FILL ? desc[b].a : 0, nb = FILL ? desc[b].b : 0, nw = 0;
+    const int w0 = FILL ? desc[b].wet : 0;
+    static_assert(TX * TY * TZ <= 1 << 16, "entries keep a place among the box's wetting nodes in 16 bits");
     auto below = [](uint64_t m) {
         return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
     };
@@ -507,8 +510,8 @@ __global__ __launch_bounds__(64) void k_tile_lists(GradArgs<T> A, TileDesc* __re
         const bool halo = x >= 1 && x < ox + 3 && y >= 1 && y < oy + 3 && z >= 1 && z < oz + 3;
         const bool own = x >= 2 && x < ox + 2 && y >= 2 && y < oy + 2 && z >= 2 && z < oz + 2;
         const bool fb = own && tag_fluid(t & 3);
-        // K3 writes the solid-boundary phi of [1, nx] x [1, ny] x [0, nz+1] back
-        const bool wb = !FORCE && own && i >= 1 && i <= d.nx && j >= 1 && j <= d.ny && k >= 0 && k <= d.nz + 1;
+        const bool wb = !FORCE && own && i >= 1 && i <= d.nx && j >= 1 && j <= d.ny && k >= 0 && k <= d.nz + 1 &&
+                        (k <= zl || k > d.nz - zl || j <= yl || j > d.ny - yl);
         bool fa = halo && (t & 3) == TAG_SOLID_BND;
         if (fa && !wb) {
             // only what the stencil of one of the box's own fluid nodes reads
@@ -520,33 +523,45 @@ __global__ __launch_bounds__(64) void k_tile_lists(GradArgs<T> A, TileDesc* __re
             }
             fa = read;
         }
-        const uint64_t ma = __ballot(fa), mb = __ballot(fb);
+        const bool fw = !FORCE && fb && (t & 3) == TAG_WET;
+        const uint64_t ma = __ballot(fa), mb = __ballot(fb), mw = __ballot(fw);
         if (FILL) {
             const uint32_t at = Entry::pack(x, y, z), mask = (uint32_t)t >> 2;
-            if (fa) la[na + below(ma)] = FORCE ? at | mask << 12 : at | (uint32_t)wb << 12 | mask << 13;
+            if (fa) (FORCE ? out.l6 : out.l3)[na + below(ma)] = FORCE ? at | mask << 12 : at | (uint32_t)wb << 12 | mask << 13;
             if (fb) {
-                lb[nb + below(mb)] = (uint16_t)(FORCE ? at : at | (uint32_t)((t & 3) == TAG_WET) << 12);
-                if (FORCE) rec[nb + below(mb)] = t >> 2;
+                if (FORCE) {
+                    out.l7[nb + below(mb)] = (uint16_t)at;
+                    out.r7[nb + below(mb)] = t >> 2;
+                } else {
+                    out.l4[nb + below(mb)] = at | (uint32_t)fw << 12 | (uint32_t)(fw ? nw + below(mw) : 0) << 13;
+                }
             }
+            if (fw) out.wet[w0 + nw + below(mw)] = i4(d, i, j, k);
             if (FORCE && e < NL && tag_fluid(t & 3)) atomicOr(&s_fluid[x + LX * y], 1u << z);
         }
         na += __popcll(ma);
         nb += __popcll(mb);
+        nw += __popcll(mw);
     }
     if (!FILL) {
         if (lane == 0) {
-            desc[b] = TileDesc{0, na, 0, nb, i0, j0, k0, 0};
+            desc[b] = TileDesc{0, na, 0, nb, i0, j0, k0, nw};
         }
         return;
     }
     if (FORCE) {
         __syncthreads();
-        for (int c = lane; c < NC; c += 64) fluid[(int64_t)b * NC + c] = (uint8_t)s_fluid[c];
+        for (int c = lane; c < NC; c += 64) out.fluid[(int64_t)b * NC + c] = (uint8_t)s_fluid[c];
     }
 }
 
 // K3 + K4/K5 on the box of owned nodes inside [-1, n+2]^3: phi of the solid-boundary nodes
 // of the box and its 1-halo, then normals and c_norm of the fluid nodes of the box.
+// What it moved beside phi and the normals bounded it at 256^3: the solid normals of the wetting
+// nodes, a 128-byte line each from an array over all nodes, come packed in list order, and K3 writes
+// back only what a later kernel reads.  256^3 drainage: 226 -> 195 us FP64, 154 -> 124 FP32 (in a
+// profiled run of a few steps); with the normals packed by fluid node too it took 190 and 118, but
+// k_grad_force, whose loads then go through a table of rows, up to 10 us more.
 template <typename T, int TX, int TY, int TZ>
 __global__ __launch_bounds__((TX + 4) * (TY + 4)) void k_grad_normals(GradArgs<T> A, StepConst<T> P) {
     constexpr int LX = TX + 4, LY = TY + 4, LZ = TZ + 4, NC = LX * LY, NL = NC * LZ, THREADS = NC;
@@ -569,7 +584,7 @@ __global__ __launch_bounds__((TX + 4) * (TY + 4)) void k_grad_normals(GradArgs<T
     for (int z = 0; z < LZ; ++z) pv[z] = A.phi[c0 + (int64_t)min(z, zmax) * P4];
     // this thread's list entries
     const uint32_t* l3 = A.lists.l3 + td.a;
-    const uint16_t* l4 = A.lists.l4 + td.b;
+    const uint32_t* l4 = A.lists.l4 + td.b;
     constexpr int M4 = (TX * TY * TZ + THREADS - 1) / THREADS;
     const uint32_t first3 = tid < td.na ? l3[tid] : 0u;
     uint32_t v4[M4];
@@ -585,9 +600,8 @@ __global__ __launch_bounds__((TX + 4) * (TY + 4)) void k_grad_normals(GradArgs<T
     for (int m = 0; m < M4; ++m) {
         wn[m][0] = wn[m][1] = wn[m][2] = T(0);
         if ((v4[m] >> 12) & 1u) {
-            const Entry e(v4[m]);
-            const Vec4<T> sn = reinterpret_cast<const Vec4<T>*>(A.snp)[corner4 + e.x + d.X4 * (e.y + d.Y4 * e.z)];
-            wn[m][0] = sn.x; wn[m][1] = sn.y; wn[m][2] = sn.z;
+            const T* sn = A.snp + td.wet + (v4[m] >> 13);
+            wn[m][0] = sn[0]; wn[m][1] = sn[A.nwet]; wn[m][2] = sn[2 * (int64_t)A.nwet];
         }
     }
     lds_barrier();

@@ -878,12 +878,14 @@ __device__ __forceinline__ T curvature_of(NX&& nx, NY&& ny, NZ&& nz) {
 
 // K3: phi at solid-boundary nodes = D3Q19-weighted mean over fluid neighbours, [-2, n+3].
 template <typename T>
-__global__ __launch_bounds__(256) void k_phi_extrap(Fields<T> F, const uint32_t* __restrict__ list, int n) {
+__global__ __launch_bounds__(256) void k_phi_extrap(Fields<T> F, const uint32_t* __restrict__ list, int n,
+                                                    bool inner) {
     const int t = xcd_block() * 256 + threadIdx.x;
     if (t >= n) return;
     int i, j, k;
     unpack_ijk(list[t], i, j, k);
     const Dims& d = F.d;
+    if (inner && (i < 1 || i > d.nx || j < 1 || j > d.ny || k < 0 || k > d.nz + 1)) return;
     const int c = i4(d, i, j, k);
     T ps = T(0), ws = T(0);
 #pragma unroll

@@ -159,10 +159,11 @@ struct Sparse {
 };
 
 // One box of the two-pass gradient chain: its two work lists, runs [a, a + na) and [b, b + nb)
-// of the chain's list arrays, and its first owned node.
+// of the chain's list arrays, its first owned node, and (k_grad_normals) the place of its first
+// wetting node among the packed solid normals.
 struct TileDesc {
     int32_t a, na, b, nb;
-    int32_t i0, j0, k0, pad;
+    int32_t i0, j0, k0, wet;
 };
 
 // Work lists of the two-pass chain, built once from the geometry (k_tile_lists).  A box entry
@@ -170,11 +171,19 @@ struct TileDesc {
 struct TileLists {
     const TileDesc *ndesc, *fdesc;      // per box of k_grad_normals and of k_grad_force
     const uint32_t* __restrict__ l3;    // K3: entry | written back << 12 | fluid-neighbour mask << 13
-    const uint16_t* __restrict__ l4;    // K4: entry | wetting << 12
+    const uint32_t* __restrict__ l4;    // K4: entry | wetting << 12 | place among the box's wetting nodes << 13
     const uint32_t* __restrict__ l6;    // K6: entry | fluid-neighbour mask << 12
     const uint16_t* __restrict__ l7;    // K7: entry
     const int32_t* __restrict__ r7;     // K7: force-record index
     const uint8_t* __restrict__ fluid;  // k_grad_force: per box and column, the fluid nodes of the loaded box (bit z)
+};
+
+// Where k_tile_lists writes them; wet: the S4 index of the wetting nodes in the order of the lists.
+struct TileFill {
+    uint32_t *l3, *l4, *l6;
+    uint16_t* l7;
+    int32_t *r7, *wet;
+    uint8_t* fluid;
 };
 
 // Inputs of the fused gradient-chain kernel (gradient.inl).  `tag` holds, for every node of
@@ -190,7 +199,8 @@ struct GradArgs {
     const T* __restrict__ snx;        // S4 solid normals, read at fluid-boundary nodes
     const T* __restrict__ sny;
     const T* __restrict__ snz;
-    const T* __restrict__ snp;        // 4 * S4: (snx, sny, snz, 0) side by side (two-pass chain)
+    const T* __restrict__ snp;        // 3 * nwet: x, y, z solid normals of the wetting nodes in box order (two-pass chain)
+    int nwet;
     T* aux;                           // 4 * nf force records
     T* cnx;                           // S2 dense normals and c_norm
     T* cny;
@@ -201,6 +211,7 @@ struct GradArgs {
     // two-pass chain: boxes along z, and the order in which the workgroups walk the boxes
     // (0: x fastest, then y, then z; 1: x fastest, then z, then y)
     int tiles_z, box_order;
+    int jper, kper;
     TileLists lists;
 };
 

@@ -17,7 +17,8 @@ struct Launch {
     static void porous_plate(const Sparse<T>& S, const Dims& d, const StepConst<T>& P, const int32_t* pmap, int zp,
                              int blocked, bool after_odd, hipStream_t s);
     static void conv_init(const Fields<T>& F, T rho_ref, T* conv, hipStream_t s);
-    static void phi_extrap(const Fields<T>& F, const NodeLists& L, hipStream_t s);
+    // inner: only of the nodes [1, nx] x [1, ny] x [0, nz+1]
+    static void phi_extrap(const Fields<T>& F, const NodeLists& L, hipStream_t s, bool inner = false);
     static void normals(const Fields<T>& F, const StepConst<T>& P, const NodeLists& L, hipStream_t s);
     static void normal_extrap(const Fields<T>& F, const NodeLists& L, hipStream_t s);
     static void curvature(const Fields<T>& F, const StepConst<T>& P, const NodeLists& L, T* aux, hipStream_t s);
@@ -30,8 +31,7 @@ struct Launch {
     static void tile_grid(const Dims& d, bool force, int (&tiles)[3]);
     static int tile_columns();
     static void tile_counts(const GradArgs<T>& A, TileDesc* ndesc, TileDesc* fdesc, hipStream_t s);
-    static void tile_fill(const GradArgs<T>& A, uint32_t* l3, uint16_t* l4, uint32_t* l6, uint16_t* l7, int32_t* r7,
-                          uint8_t* fluid, hipStream_t s);
+    static void tile_fill(const GradArgs<T>& A, const TileFill& out, hipStream_t s);
     static void aux_refresh(const Fields<T>& F, const StepConst<T>& P, const NodeLists& L, T* aux, hipStream_t s);
     static void cells(const Sparse<T>& S, T* dense, const Dims& d, const int32_t* ext_node, const int32_t* ext_off,
                       int n_ext, bool to_dense, hipStream_t s);
@@ -47,8 +47,8 @@ struct Launch {
     static void monitor(const Sparse<T>& S, const StepConst<T>& P, const T* phi, const Dims& d, const int32_t* zstart,
                         int nsplit, double* part, double* out, hipStream_t s);
     static void to_real(const double* src, T* dst, int64_t n, hipStream_t s);
-    // dst[4 i .. 4 i + 3] = (x[i], y[i], z[i], 0)
-    static void pack4(const T* x, const T* y, const T* z, T* dst, int64_t n, hipStream_t s);
+    // dst[c * n + w] = component c of the solid normal at S4 node wet[w].
+    static void pack_solid_normals(const T* x, const T* y, const T* z, const int32_t* wet, int n, T* dst, hipStream_t s);
 };
 
 extern template struct Launch<double>;

@@ -25,14 +25,15 @@ void boundary_groups(BoundaryArgs<T>& B, const Dims& d, int threads) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_pack4(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z,
-                                               T* __restrict__ dst, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    dst[4 * i] = x[i];
-    dst[4 * i + 1] = y[i];
-    dst[4 * i + 2] = z[i];
-    dst[4 * i + 3] = T(0);
+__global__ __launch_bounds__(256) void k_pack_solid_normals(const T* __restrict__ x, const T* __restrict__ y,
+                                                            const T* __restrict__ z, const int32_t* __restrict__ wet,
+                                                            int n, T* __restrict__ dst) {
+    const int w = blockIdx.x * 256 + threadIdx.x;
+    if (w >= n) return;
+    const int c = wet[w];
+    dst[w] = x[c];
+    dst[(int64_t)n + w] = y[c];
+    dst[2 * (int64_t)n + w] = z[c];
 }
 
 template <typename T>
@@ -87,8 +88,9 @@ void Launch<T>::conv_init(const Fields<T>& F, T rho_ref, T* conv, hipStream_t s)
 }
 
 template <typename T>
-void Launch<T>::phi_extrap(const Fields<T>& F, const NodeLists& L, hipStream_t s) {
-    if (L.n_solid_bnd > 0) dev::k_phi_extrap<T><<<blocks(L.n_solid_bnd), 256, 0, s>>>(F, L.solid_bnd, L.n_solid_bnd);
+void Launch<T>::phi_extrap(const Fields<T>& F, const NodeLists& L, hipStream_t s, bool inner) {
+    if (L.n_solid_bnd > 0)
+        dev::k_phi_extrap<T><<<blocks(L.n_solid_bnd), 256, 0, s>>>(F, L.solid_bnd, L.n_solid_bnd, inner);
 }
 
 template <typename T>
@@ -116,9 +118,6 @@ void Launch<T>::tile_grid(const Dims& d, bool force, int (&tiles)[3]) {
     }
 }
 
-template <typename T>
-int Launch<T>::tile_columns() { return (GradTiles<T>::F[0] + 4) * (GradTiles<T>::F[1] + 4); }
-
 namespace {
 // Sets the box counts of one of the two kernels; returns its grid.
 template <typename T>
@@ -131,28 +130,28 @@ unsigned box_grid(GradArgs<T>& A, bool force) {
 }  // namespace
 
 template <typename T>
+int Launch<T>::tile_columns() { return (GradTiles<T>::F[0] + 4) * (GradTiles<T>::F[1] + 4); }
+
+template <typename T>
 void Launch<T>::tile_counts(const GradArgs<T>& A, TileDesc* ndesc, TileDesc* fdesc, hipStream_t s) {
     constexpr int NX = GradTiles<T>::N[0], NY = GradTiles<T>::N[1], NZ = GradTiles<T>::N[2];
     constexpr int FX = GradTiles<T>::F[0], FY = GradTiles<T>::F[1], FZ = GradTiles<T>::F[2];
     GradArgs<T> B = A;
     const unsigned gn = box_grid(B, false);
-    dev::k_tile_lists<T, NX, NY, NZ, false, false><<<gn, 64, 0, s>>>(B, ndesc, nullptr, nullptr, nullptr, nullptr);
+    dev::k_tile_lists<T, NX, NY, NZ, false, false><<<gn, 64, 0, s>>>(B, ndesc, TileFill{});
     const unsigned gf = box_grid(B, true);
-    dev::k_tile_lists<T, FX, FY, FZ, true, false><<<gf, 64, 0, s>>>(B, fdesc, nullptr, nullptr, nullptr, nullptr);
+    dev::k_tile_lists<T, FX, FY, FZ, true, false><<<gf, 64, 0, s>>>(B, fdesc, TileFill{});
 }
 
 template <typename T>
-void Launch<T>::tile_fill(const GradArgs<T>& A, uint32_t* l3, uint16_t* l4, uint32_t* l6, uint16_t* l7, int32_t* r7,
-                          uint8_t* fluid, hipStream_t s) {
+void Launch<T>::tile_fill(const GradArgs<T>& A, const TileFill& out, hipStream_t s) {
     constexpr int NX = GradTiles<T>::N[0], NY = GradTiles<T>::N[1], NZ = GradTiles<T>::N[2];
     constexpr int FX = GradTiles<T>::F[0], FY = GradTiles<T>::F[1], FZ = GradTiles<T>::F[2];
     GradArgs<T> B = A;
     const unsigned gn = box_grid(B, false);
-    dev::k_tile_lists<T, NX, NY, NZ, false, true>
-        <<<gn, 64, 0, s>>>(B, const_cast<TileDesc*>(A.lists.ndesc), l3, l4, nullptr, nullptr);
+    dev::k_tile_lists<T, NX, NY, NZ, false, true><<<gn, 64, 0, s>>>(B, const_cast<TileDesc*>(A.lists.ndesc), out);
     const unsigned gf = box_grid(B, true);
-    dev::k_tile_lists<T, FX, FY, FZ, true, true>
-        <<<gf, 64, 0, s>>>(B, const_cast<TileDesc*>(A.lists.fdesc), l6, l7, r7, fluid);
+    dev::k_tile_lists<T, FX, FY, FZ, true, true><<<gf, 64, 0, s>>>(B, const_cast<TileDesc*>(A.lists.fdesc), out);
 }
 
 template <typename T>
@@ -248,8 +247,8 @@ void Launch<T>::monitor(const Sparse<T>& S, const StepConst<T>& P, const T* phi,
 }
 
 template <typename T>
-void Launch<T>::pack4(const T* x, const T* y, const T* z, T* dst, int64_t n, hipStream_t s) {
-    k_pack4<T><<<blocks(n), 256, 0, s>>>(x, y, z, dst, n);
+void Launch<T>::pack_solid_normals(const T* x, const T* y, const T* z, const int32_t* wet, int n, T* dst, hipStream_t s) {
+    if (n > 0) k_pack_solid_normals<T><<<blocks(n), 256, 0, s>>>(x, y, z, wet, n, dst);
 }
 
 template <typename T>

@@ -304,12 +304,8 @@ void pack_solid_normals(mflbm_handle* h) {
 // The work lists of the two-pass gradient chain, from the node tags.
 template <typename T>
 int build_tile_lists(mflbm_handle* h) {
-    size_t boxes[2];
-    for (int f = 0; f < 2; ++f) {
-        int t[3];
-        Launch<T>::tile_grid(h->d, f == 1, t);
-        boxes[f] = (size_t)t[0] * t[1] * t[2];
-    }
+    int columns = 0;
+    const size_t boxes[2] = {(size_t)Launch<T>::tile_boxes(h->d, false), (size_t)Launch<T>::tile_boxes(h->d, true, &columns)};
     TileDesc** dev[2] = {&h->ndesc, &h->fdesc};
     for (int f = 0; f < 2; ++f) HIPCHK(h, hipMalloc(dev[f], boxes[f] * sizeof(TileDesc)));
     Launch<T>::tile_counts(grad_args<T>(h), h->ndesc, h->fdesc, h->stream);
@@ -338,7 +334,7 @@ int build_tile_lists(mflbm_handle* h) {
     HIPCHK(h, hipMalloc(&h->l6, room(na[1]) * sizeof(uint32_t)));
     HIPCHK(h, hipMalloc(&h->l7, room(nb[1]) * sizeof(uint16_t)));
     HIPCHK(h, hipMalloc(&h->r7, room(nb[1]) * sizeof(int32_t)));
-    HIPCHK(h, hipMalloc(&h->tile_fluid, boxes[1] * Launch<T>::tile_columns()));
+    HIPCHK(h, hipMalloc(&h->tile_fluid, boxes[1] * columns));
     h->n_wet = (int)nw;
     HIPCHK(h, hipMalloc(&h->wet, room(nw) * sizeof(int32_t)));
     HIPCHK(h, hipMalloc(&h->snp, room(nw) * 3 * sizeof(T)));

@@ -459,17 +459,14 @@ inline int64_t ghost_phi_threads(const PhiGhosts<T>& G, const Dims& d) {
            (G.jper ? (int64_t)d.nx * d.nz : 0) + (G.kper && G.jper ? 64 * d.nx : 0);
 }
 
-#ifndef MFLBM_COLLIDE_THREADS
-#define MFLBM_COLLIDE_THREADS 256  // threads per collide workgroup (tuning: 128, 256, 512)
-#endif
-template <typename T, bool ODD, bool ORIG = true>
-__global__ __launch_bounds__(MFLBM_COLLIDE_THREADS) void k_collide(Sparse<T> S, T* __restrict__ phi, Dims d,
-                                                                   StepConst<T> P, PhiGhosts<T> G) {
+template <typename T, bool ODD, bool ORIG, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_collide(Sparse<T> S, T* __restrict__ phi, Dims d, StepConst<T> P,
+                                                     PhiGhosts<T> G) {
     if ((int)blockIdx.x < G.rest) {
-        ghost_phi_rest<T>(G, P, phi, d, (int)blockIdx.x * MFLBM_COLLIDE_THREADS + threadIdx.x);
+        ghost_phi_rest<T>(G, P, phi, d, (int)blockIdx.x * THREADS + threadIdx.x);
         return;
     }
-    const int t = xcd_block(gridDim.x - G.rest, blockIdx.x - G.rest) * MFLBM_COLLIDE_THREADS + threadIdx.x;
+    const int t = xcd_block(gridDim.x - G.rest, blockIdx.x - G.rest) * THREADS + threadIdx.x;
     if (t >= S.nf) return;
     // The neighbour row, force record and phi of the odd step are touched once; nontemporal
     // accesses leave the cache to the shared lines of the scattered cells (6 % faster; in

@@ -237,6 +237,10 @@ template <>
 struct GradTiles<float> {
     static constexpr int N[3] = {16, 8, 4}, F[3] = {12, 8, 4};
 };
+// of domains with fewer boxes than CUs
+struct SmallGradTiles {
+    static constexpr int N[3] = {8, 4, 4}, F[3] = {8, 4, 4};
+};
 
 // Uniform deviate in [0, 1) of lattice node n under a seed, for the random initial phase
 // distribution: the splitmix64 output function (Steele, Lea and Flood, OOPSLA 2014) of

@@ -28,8 +28,8 @@ struct Launch {
                                   BoundaryArgs<T> B, bool after_odd, hipStream_t s);
     // Boxes of the two-pass chain's kernels, and its work lists: first their sizes (na and nb of
     // the descriptors), then, with the descriptors complete, the lists.
-    static void tile_grid(const Dims& d, bool force, int (&tiles)[3]);
-    static int tile_columns();
+    // boxes of one of the kernels; columns: loaded columns of a box of k_grad_force
+    static int tile_boxes(const Dims& d, bool force, int* columns = nullptr);
     static void tile_counts(const GradArgs<T>& A, TileDesc* ndesc, TileDesc* fdesc, hipStream_t s);
     static void tile_fill(const GradArgs<T>& A, const TileFill& out, hipStream_t s);
     static void aux_refresh(const Fields<T>& F, const StepConst<T>& P, const NodeLists& L, T* aux, hipStream_t s);

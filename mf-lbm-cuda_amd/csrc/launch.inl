@@ -43,25 +43,37 @@ __global__ __launch_bounds__(256) void k_to_real(const double* __restrict__ src,
 }
 }  // namespace
 
+namespace {
+template <typename T, int THREADS>
+void launch_collide(const Sparse<T>& S, T* phi, const Dims& d, const StepConst<T>& P, bool odd, const PhiGhosts<T>* ghosts,
+                    hipStream_t s) {
+    unsigned grid = blocks(S.nf, THREADS);
+    PhiGhosts<T> G{};
+    if (ghosts) {
+        G = *ghosts;
+        G.rest = (int)((blocks(dev::ghost_phi_threads(G, d), THREADS) + 7) / 8 * 8);
+        grid += G.rest;
+    }
+    if (P.mrt == 2) {
+        if (odd) dev::k_collide<T, true, true, THREADS><<<grid, THREADS, 0, s>>>(S, phi, d, P, G);
+        else dev::k_collide<T, false, true, THREADS><<<grid, THREADS, 0, s>>>(S, phi, d, P, G);
+    } else {  // collision models 1, 3, 4
+        if (odd) dev::k_collide<T, true, false, THREADS><<<grid, THREADS, 0, s>>>(S, phi, d, P, G);
+        else dev::k_collide<T, false, false, THREADS><<<grid, THREADS, 0, s>>>(S, phi, d, P, G);
+    }
+}
+}  // namespace
+
 template <typename T>
 void Launch<T>::collide(const Sparse<T>& S, T* phi, const Dims& d, const StepConst<T>& P, bool odd,
                         const PhiGhosts<T>* ghosts, hipStream_t s) {
     if (S.nf <= 0) return;
-    constexpr int b = MFLBM_COLLIDE_THREADS;
-    unsigned grid = blocks(S.nf, b);
-    PhiGhosts<T> G{};
-    if (ghosts) {
-        G = *ghosts;
-        G.rest = (int)((blocks(dev::ghost_phi_threads(G, d), b) + 7) / 8 * 8);
-        grid += G.rest;
-    }
-    if (P.mrt == 2) {
-        if (odd) dev::k_collide<T, true><<<grid, b, 0, s>>>(S, phi, d, P, G);
-        else dev::k_collide<T, false><<<grid, b, 0, s>>>(S, phi, d, P, G);
-    } else {  // collision models 1, 3, 4
-        if (odd) dev::k_collide<T, true, false><<<grid, b, 0, s>>>(S, phi, d, P, G);
-        else dev::k_collide<T, false, false><<<grid, b, 0, s>>>(S, phi, d, P, G);
-    }
+    // One wave to a workgroup where workgroups of 256 nodes would leave half of the 256 CUs without
+    // one.  us, odd / even, 256 and 64 threads: 32^3 FP64 8.5 / 5.9 and 6.3 / 5.0, 40^3 FP32 6.8 / 4.6
+    // and 6.4 / 4.5; 48^3 level; 64^3 FP32 14.1 / 7.1 and 14.7 / 7.4, 256^3 FP64 1127 / 752 and 1138 /
+    // 770 (128 threads: 1128 / 758).
+    if (S.nf < 128 * 256) launch_collide<T, 64>(S, phi, d, P, odd, ghosts, s);
+    else launch_collide<T, 256>(S, phi, d, P, odd, ghosts, s);
 }
 
 template <typename T>
@@ -108,65 +120,89 @@ void Launch<T>::curvature(const Fields<T>& F, const StepConst<T>& P, const NodeL
     if (L.n_fluid > 0) dev::k_curvature<T><<<blocks(L.n_fluid), 256, 0, s>>>(F, P, L.fluid, L.n_fluid, aux);
 }
 
-template <typename T>
-void Launch<T>::tile_grid(const Dims& d, bool force, int (&tiles)[3]) {
+namespace {
+unsigned boxes(const Dims& d, bool force, const int (&t)[3], int (&tiles)[3]) {
     const int n[3] = {d.nx, d.ny, d.nz};
     // normals over [-1, n+2]^3, forces over [1, n]^3
-    for (int a = 0; a < 3; ++a) {
-        const int t = force ? GradTiles<T>::F[a] : GradTiles<T>::N[a];
-        tiles[a] = (n[a] + (force ? 0 : 4) + t - 1) / t;
-    }
+    for (int a = 0; a < 3; ++a) tiles[a] = (n[a] + (force ? 0 : 4) + t[a] - 1) / t[a];
+    return (unsigned)(tiles[0] * tiles[1] * tiles[2]);
 }
 
-namespace {
+// Calls f with the box shapes of a domain: the small ones where a CU would have less than one box
+// of k_grad_force.  us, normals / force, large and small boxes: 32^3 FP64 6.6 / 6.8 and 5.6 / 6.2, 40^3
+// FP64 7.0 / 7.2 and 6.2 / 7.4, FP32 6.3 / 5.7 and 5.6 / 5.6; beyond, 54^3 FP64 7.5 / 9.1 and 8.9 / 9.8,
+// FP32 6.2 / 6.7 and 7.0 / 7.1 (the halos of small boxes are more than half of what they load).
+template <typename T, class Fn>
+void with_boxes(const Dims& d, Fn&& f) {
+    int t[3];
+    if (boxes(d, true, GradTiles<T>::F, t) < 256) f(SmallGradTiles{});
+    else f(GradTiles<T>{});
+}
+
 // Sets the box counts of one of the two kernels; returns its grid.
-template <typename T>
+template <typename T, class Shape>
 unsigned box_grid(GradArgs<T>& A, bool force) {
     int t[3];
-    Launch<T>::tile_grid(A.d, force, t);
+    const unsigned n = boxes(A.d, force, force ? Shape::F : Shape::N, t);
     A.tiles_x = t[0]; A.tiles_y = t[1]; A.tiles_z = t[2];
-    return (unsigned)(t[0] * t[1] * t[2]);
+    return n;
 }
 }  // namespace
 
 template <typename T>
-int Launch<T>::tile_columns() { return (GradTiles<T>::F[0] + 4) * (GradTiles<T>::F[1] + 4); }
+int Launch<T>::tile_boxes(const Dims& d, bool force, int* columns) {
+    int n = 0;
+    with_boxes<T>(d, [&](auto shape) {
+        using S = decltype(shape);
+        int t[3];
+        n = (int)boxes(d, force, force ? S::F : S::N, t);
+        if (columns) *columns = (S::F[0] + 4) * (S::F[1] + 4);
+    });
+    return n;
+}
 
 template <typename T>
 void Launch<T>::tile_counts(const GradArgs<T>& A, TileDesc* ndesc, TileDesc* fdesc, hipStream_t s) {
-    constexpr int NX = GradTiles<T>::N[0], NY = GradTiles<T>::N[1], NZ = GradTiles<T>::N[2];
-    constexpr int FX = GradTiles<T>::F[0], FY = GradTiles<T>::F[1], FZ = GradTiles<T>::F[2];
-    GradArgs<T> B = A;
-    const unsigned gn = box_grid(B, false);
-    dev::k_tile_lists<T, NX, NY, NZ, false, false><<<gn, 64, 0, s>>>(B, ndesc, TileFill{});
-    const unsigned gf = box_grid(B, true);
-    dev::k_tile_lists<T, FX, FY, FZ, true, false><<<gf, 64, 0, s>>>(B, fdesc, TileFill{});
+    with_boxes<T>(A.d, [&](auto shape) {
+        using S = decltype(shape);
+        GradArgs<T> B = A;
+        const unsigned gn = box_grid<T, S>(B, false);
+        dev::k_tile_lists<T, S::N[0], S::N[1], S::N[2], false, false><<<gn, 64, 0, s>>>(B, ndesc, TileFill{});
+        const unsigned gf = box_grid<T, S>(B, true);
+        dev::k_tile_lists<T, S::F[0], S::F[1], S::F[2], true, false><<<gf, 64, 0, s>>>(B, fdesc, TileFill{});
+    });
 }
 
 template <typename T>
 void Launch<T>::tile_fill(const GradArgs<T>& A, const TileFill& out, hipStream_t s) {
-    constexpr int NX = GradTiles<T>::N[0], NY = GradTiles<T>::N[1], NZ = GradTiles<T>::N[2];
-    constexpr int FX = GradTiles<T>::F[0], FY = GradTiles<T>::F[1], FZ = GradTiles<T>::F[2];
-    GradArgs<T> B = A;
-    const unsigned gn = box_grid(B, false);
-    dev::k_tile_lists<T, NX, NY, NZ, false, true><<<gn, 64, 0, s>>>(B, const_cast<TileDesc*>(A.lists.ndesc), out);
-    const unsigned gf = box_grid(B, true);
-    dev::k_tile_lists<T, FX, FY, FZ, true, true><<<gf, 64, 0, s>>>(B, const_cast<TileDesc*>(A.lists.fdesc), out);
+    with_boxes<T>(A.d, [&](auto shape) {
+        using S = decltype(shape);
+        GradArgs<T> B = A;
+        const unsigned gn = box_grid<T, S>(B, false);
+        dev::k_tile_lists<T, S::N[0], S::N[1], S::N[2], false, true>
+            <<<gn, 64, 0, s>>>(B, const_cast<TileDesc*>(A.lists.ndesc), out);
+        const unsigned gf = box_grid<T, S>(B, true);
+        dev::k_tile_lists<T, S::F[0], S::F[1], S::F[2], true, true>
+            <<<gf, 64, 0, s>>>(B, const_cast<TileDesc*>(A.lists.fdesc), out);
+    });
 }
 
 template <typename T>
 void Launch<T>::gradient_boundary(const GradArgs<T>& A, const Sparse<T>& S, const Fields<T>& F, const StepConst<T>& P,
                                   BoundaryArgs<T> B, bool after_odd, hipStream_t s) {
-    constexpr int NX = GradTiles<T>::N[0], NY = GradTiles<T>::N[1], NZ = GradTiles<T>::N[2];
-    constexpr int FX = GradTiles<T>::F[0], FY = GradTiles<T>::F[1], FZ = GradTiles<T>::F[2], threads = (FX + 4) * (FY + 4);
-    GradArgs<T> G = A;
-    const unsigned gn = box_grid(G, false);
-    dev::k_grad_normals<T, NX, NY, NZ><<<gn, (NX + 4) * (NY + 4), 0, s>>>(G, P);
-    const unsigned gf = box_grid(G, true);
-    boundary_groups(B, F.d, threads);
-    if (B.blocks == 0) dev::k_grad_force<T, FX, FY, FZ, 0><<<gf, threads, 0, s>>>(G, P, S, F, B);
-    else if (after_odd) dev::k_grad_force<T, FX, FY, FZ, 1><<<gf + B.blocks, threads, 0, s>>>(G, P, S, F, B);
-    else dev::k_grad_force<T, FX, FY, FZ, 2><<<gf + B.blocks, threads, 0, s>>>(G, P, S, F, B);
+    with_boxes<T>(A.d, [&](auto shape) {
+        using H = decltype(shape);
+        constexpr int NX = H::N[0], NY = H::N[1], NZ = H::N[2];
+        constexpr int FX = H::F[0], FY = H::F[1], FZ = H::F[2], threads = (FX + 4) * (FY + 4);
+        GradArgs<T> G = A;
+        const unsigned gn = box_grid<T, H>(G, false);
+        dev::k_grad_normals<T, NX, NY, NZ><<<gn, (NX + 4) * (NY + 4), 0, s>>>(G, P);
+        const unsigned gf = box_grid<T, H>(G, true);
+        boundary_groups(B, F.d, threads);
+        if (B.blocks == 0) dev::k_grad_force<T, FX, FY, FZ, 0><<<gf, threads, 0, s>>>(G, P, S, F, B);
+        else if (after_odd) dev::k_grad_force<T, FX, FY, FZ, 1><<<gf + B.blocks, threads, 0, s>>>(G, P, S, F, B);
+        else dev::k_grad_force<T, FX, FY, FZ, 2><<<gf + B.blocks, threads, 0, s>>>(G, P, S, F, B);
+    });
 }
 
 template <typename T>

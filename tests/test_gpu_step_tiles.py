@@ -110,3 +110,22 @@ def test_populations_started_anew_from_the_phi_of_a_run(name):
         s.init_equilibrium()
     inside = (..., slice(1, -1), slice(1, -1), slice(1, -1))
     assert_same(a.download("pdf")[inside], b.download("pdf")[inside], 0.0, what=f"{name} pdf")
+
+
+@pytest.mark.parametrize("n, precision", [((49, 41, 45), gpu.FP64), ((50, 39, 46), gpu.FP32), ((33, 41, 44), gpu.FP64),
+                                          ((37, 33, 41), gpu.FP32)])
+def test_domains_around_the_change_of_box_and_workgroup_sizes(n, precision):
+    """the last sizes with small boxes and with one-wave collide workgroups and the first beyond them:
+    FP64 against the oracle, FP32 against the kernels of one stage each (as above)"""
+    geo, p = small_drainage(n=n, seed=9, radius=3.5, porosity=0.55, jper=1, buffer=2)
+    print(f"[gpu-step-tiles] sizes {n} {precision}", flush=True)
+    g = gpu.Solver(p, geo, precision)
+    o = O.Oracle(p, geo) if precision == gpu.FP64 else gpu.Solver(p, geo, precision, split_gradient=True)
+    for s in (o, g):
+        s.setup()
+        s.run(1, 30)
+    for field in ("pdf", "phi"):
+        if precision == gpu.FP64:
+            assert_same(g.download(field), o.array(field), 0.0, what=f"{n} {field}")
+        else:
+            assert_same(g.download(field), o.download(field), 1e-5, what=f"{n} {field}")

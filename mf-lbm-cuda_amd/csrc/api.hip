@@ -82,6 +82,7 @@ struct mflbm_handle {
     uint8_t* tile_fluid = nullptr;
     bool split_gradient = false;
     bool grad_dirty = false;    // dense phi / cn / c_norm / curv behind the step state
+    bool phi_behind = false;    // phi of solid nodes [1, nx] x [1, ny] x [0, nz+1] behind the step state's
     // monitor scratch
     double *mon_part = nullptr, *mon_out = nullptr;
     int mon_nsplit = 0;
@@ -266,6 +267,13 @@ void step_dispatch(mflbm_handle* h, bool odd, hipEvent_t* ev) {
     else enqueue_step<float>(h, odd, ev);
 }
 
+// After steps: the fused chains leave the dense fields behind, the one on boxes also the phi of
+// most solid nodes.
+void stepped(mflbm_handle* h) {
+    h->grad_dirty = !h->split_gradient;
+    h->phi_behind = h->grad_dirty && h->grad_shape == GRAD_SHAPE_TILES;
+}
+
 // Brings the dense phi (solid-boundary nodes of the ghost layers), cn, c_norm and curv up
 // to the step state with the split kernels.  The fused step leaves them behind; they are
 // functions of phi alone, and the split kernels also rewrite the force records with the
@@ -274,7 +282,7 @@ int materialize_gradient(mflbm_handle* h) {
     if (!h->grad_dirty) return 0;
     if (h->prec == MFLBM_FP64) enqueue_gradient<double>(h);
     else enqueue_gradient<float>(h);
-    h->grad_dirty = false;
+    h->grad_dirty = h->phi_behind = false;
     HIPCHK(h, hipGetLastError());
     return 0;
 }
@@ -287,6 +295,7 @@ int materialize_phi(mflbm_handle* h) {
     if (h->prec != MFLBM_FP64) return materialize_gradient(h);
     if (!h->grad_dirty) return 0;
     Launch<double>::phi_extrap(fields<double>(h), lists(h), h->stream);
+    h->phi_behind = false;
     HIPCHK(h, hipGetLastError());
     return 0;
 }
@@ -753,6 +762,7 @@ void mflbm_destroy(mflbm_handle* h) {
 
 static int init_phi(mflbm_handle* h, int option, double interface_z0, double sa_target, uint64_t seed) {
     const double pin = h->p.phi_inlet;
+    h->phi_behind = false;  // every node's is set
     if (h->prec == MFLBM_FP64)
         Launch<double>::init_phi(fields<double>(h), option, interface_z0, pin, h->open_z, sa_target, seed, h->stream);
     else Launch<float>::init_phi(fields<float>(h), option, interface_z0, pin, h->open_z, sa_target, seed, h->stream);
@@ -780,10 +790,12 @@ static int init_populations(mflbm_handle* h, const double* rho, const double* u,
     std::lock_guard<std::recursive_mutex> lock(device_lock());
     if (!h) return -1;
     h->vprev_valid = false;
-    // after a step: the boxes leave the phi of solid nodes behind, which the solid cells start from
-    if (h->grad_dirty) {
+    // the solid cells start from the phi of solid nodes: that of the last step where steps left it
+    // behind, untouched where mflbm_init_phi has set it since
+    if (h->phi_behind) {
         if (h->prec == MFLBM_FP64) Launch<double>::phi_extrap(fields<double>(h), lists(h), h->stream, true);
         else Launch<float>::phi_extrap(fields<float>(h), lists(h), h->stream, true);
+        h->phi_behind = false;
     }
     const int64_t n = h->d.S1;
     const double* src[4] = {rho, u, v, w};
@@ -832,7 +844,7 @@ int mflbm_color_gradient(mflbm_handle* h) {
     if (!h) return -1;
     if (h->prec == MFLBM_FP64) enqueue_gradient<double>(h);
     else enqueue_gradient<float>(h);
-    h->grad_dirty = false;
+    h->grad_dirty = h->phi_behind = false;
     HIPCHK(h, hipGetLastError());
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return 0;
@@ -841,7 +853,7 @@ int mflbm_color_gradient(mflbm_handle* h) {
 int mflbm_step(mflbm_handle* h, int32_t ntime) {
     if (!h) return -1;
     step_dispatch(h, (ntime % 2) != 0, nullptr);
-    h->grad_dirty = !h->split_gradient;
+    stepped(h);
     HIPCHK(h, hipGetLastError());
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return 0;
@@ -855,7 +867,7 @@ int mflbm_run(mflbm_handle* h, int32_t ntime0, int32_t nsteps) {
     int32_t t = ntime0;
     for (; end - t >= GRAPH_BLOCK; t += GRAPH_BLOCK) HIPCHK(h, hipGraphLaunch(h->graph[2 + ((t % 2) != 0)], h->stream));
     for (; t < end; ++t) HIPCHK(h, hipGraphLaunch(h->graph[(t % 2) != 0], h->stream));
-    h->grad_dirty = !h->split_gradient;
+    stepped(h);
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return 0;
 }
@@ -878,7 +890,7 @@ int mflbm_profile(mflbm_handle* h, int32_t ntime0, int32_t nsteps, mflbm_kernel_
         out->boundary_ms += ms[1];
         out->gradient_ms += ms[2];
     }
-    h->grad_dirty = !h->split_gradient;
+    stepped(h);
     for (int e = 0; e < NE; ++e) (void)hipEventDestroy(ev[e]);
     HIPCHK(h, hipGetLastError());
     return 0;

@@ -41,6 +41,7 @@ struct EnsDev {
     const uint32_t* nb16;      // the same links as 16-bit rows against per-wave bases (Sparse<T>)
     const int32_t* nbb;
     const int32_t* blk_dom;    // domain of each block
+    const int32_t* blk_end;    // end of its domain's fluid cells, 0 while the domain is not stepped
     const int32_t* dom_start;  // first fluid cell of each domain
     const int32_t* dom_count;  // fluid nodes of each domain
     const int32_t* active;     // 1 while the domain is being stepped
@@ -48,14 +49,15 @@ struct EnsDev {
     int mrt;                   // collision model (mflbm_params::mrt)
 };
 
-// AA step of one fluid node (the access pattern of k_collide, one colour).
-template <bool ODD>
-__global__ __launch_bounds__(EB) void k_ens_collide(EnsDev E) {
-    const int b = dev::xcd_block();
-    const int d = E.blk_dom[b];
-    if (!E.active[d]) return;
-    const int64_t t = (int64_t)b * EB + threadIdx.x;
-    if (t >= (int64_t)E.dom_start[d] + E.dom_count[d]) return;
+// AA step of one fluid node (the access pattern of k_collide, one colour).  One load says what a
+// workgroup has to do: through the block's domain and the domain's flag, start and count the first
+// loads of a node waited for two more (us a step of a solve, with the workgroups of solve(): one
+// domain of 40^3 4.86 to 4.21, of 48^3 5.17 to 4.91, two 6.5 to 6.2, four 9.2 to 8.8, eight of 56^3 22.5 to
+// 22.2, 48 of 64^3 172.2 to 171.4).
+template <bool ODD, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_ens_collide(EnsDev E) {
+    const int64_t t0 = (int64_t)dev::xcd_block() * THREADS, t = t0 + threadIdx.x;
+    if (t >= E.blk_end[t0 / EB]) return;
     const int64_t NS = E.ns, NF = E.nf;
     float ft[19];
     int64_t nb[19];
@@ -186,7 +188,7 @@ struct mflbm_ensemble {
     uint32_t* nb16 = nullptr;
     int32_t* nbb = nullptr;
     int n_escaped = 0;  // waves on the 32-bit rows
-    int32_t *nb = nullptr, *blk_dom = nullptr, *dom_start = nullptr, *dom_count = nullptr, *active = nullptr;
+    int32_t *nb = nullptr, *blk_dom = nullptr, *blk_end = nullptr, *dom_start = nullptr, *dom_count = nullptr, *active = nullptr;
     int32_t* loc = nullptr;
     float *ux = nullptr, *uy = nullptr, *uz = nullptr, *drho = nullptr;
     double *part = nullptr, *red = nullptr;
@@ -223,23 +225,31 @@ int fail(mflbm_ensemble* e, const char* fmt, ...) {
 EnsDev dev_view(const mflbm_ensemble* e) {
     EnsDev E;
     E.f = e->f; E.ns = e->ns; E.nf = e->nf; E.nb = e->nb; E.nb16 = e->nb16; E.nbb = e->nbb; E.blk_dom = e->blk_dom;
-    E.dom_start = e->dom_start; E.dom_count = e->dom_count; E.active = e->active;
+    E.blk_end = e->blk_end; E.dom_start = e->dom_start; E.dom_count = e->dom_count; E.active = e->active;
     E.nui = (float)(1.0 / e->nu);
     E.force = (float)e->force;
     E.mrt = e->mrt;
     return E;
 }
 
+// EnsDev::blk_end for the domains whose flag is set.
+std::vector<int32_t> block_ends(const mflbm_ensemble* e, const std::vector<int32_t>& active) {
+    std::vector<int32_t> ends((size_t)(e->nf / EB), 0);
+    for (int d = 0; d < e->nd; ++d)
+        for (int t = e->start[d]; active[d] && t < e->start[d] + e->count[d]; t += EB) ends[t / EB] = e->start[d] + e->count[d];
+    return ends;
+}
+
 void free_all(mflbm_ensemble* e) {
     if (e->graph) (void)hipGraphExecDestroy(e->graph);
     e->graph = nullptr;
     e->staging.release();
-    void* p[] = {e->f, e->nb, e->nb16, e->nbb, e->blk_dom, e->dom_start, e->dom_count, e->active, e->loc, e->ux, e->uy, e->uz,
-                 e->drho, e->part, e->red};
+    void* p[] = {e->f, e->nb, e->nb16, e->nbb, e->blk_dom, e->blk_end, e->dom_start, e->dom_count, e->active, e->loc,
+                 e->ux, e->uy, e->uz, e->drho, e->part, e->red};
     for (void* x : p)
         if (x) (void)hipFree(x);
     e->f = nullptr; e->nb16 = nullptr; e->nbb = nullptr;
-    e->nb = e->blk_dom = e->dom_start = e->dom_count = e->active = e->loc = nullptr;
+    e->nb = e->blk_dom = e->blk_end = e->dom_start = e->dom_count = e->active = e->loc = nullptr;
     e->ux = e->uy = e->uz = e->drho = nullptr; e->part = e->red = nullptr;
     if (e->stream) (void)hipStreamDestroy(e->stream);
     e->stream = nullptr;
@@ -411,6 +421,7 @@ int mflbm_ensemble_create(const mflbm_params* params, const int8_t* geometries, 
     std::vector<int32_t> act(nd);
     for (int d = 0; d < nd; ++d) act[d] = e->count[d] > 0;
     ECHK(e, up(&e->active, act));
+    ECHK(e, up(&e->blk_end, block_ends(e, act)));
     ECHK(e, hipMalloc(&e->f, (size_t)19 * e->ns * sizeof(float)));
     ECHK(e, hipMemset(e->f, 0, (size_t)19 * e->ns * sizeof(float)));  // rest state: zero deviations
     for (float** u : {&e->ux, &e->uy, &e->uz, &e->drho}) {
@@ -445,14 +456,18 @@ int mflbm_ensemble_solve(mflbm_ensemble* e, int32_t check, double tol, int32_t m
     const int nd = e->nd;
     const EnsDev E = dev_view(e);
     const int nblk = (int)(e->nf / EB);
+    // one wave to a workgroup where whole blocks leave half of the 256 CUs without one (as Launch::collide)
+    const bool small = nblk < 128;
     if (!e->graph || e->graph_steps != check) {
         if (e->graph) (void)hipGraphExecDestroy(e->graph);
         e->graph = nullptr;
         hipGraph_t g = nullptr;
         ECHK(e, hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
         for (int s = 0; s < check; ++s) {
-            if (s % 2 == 0) k_ens_collide<true><<<nblk, EB, 0, e->stream>>>(E);
-            else k_ens_collide<false><<<nblk, EB, 0, e->stream>>>(E);
+            if (small && s % 2 == 0) k_ens_collide<true, 64><<<nblk * (EB / 64), 64, 0, e->stream>>>(E);
+            else if (small) k_ens_collide<false, 64><<<nblk * (EB / 64), 64, 0, e->stream>>>(E);
+            else if (s % 2 == 0) k_ens_collide<true, EB><<<nblk, EB, 0, e->stream>>>(E);
+            else k_ens_collide<false, EB><<<nblk, EB, 0, e->stream>>>(E);
         }
         ECHK(e, hipStreamEndCapture(e->stream, &g));
         hipError_t r = hipGraphInstantiate(&e->graph, g, nullptr, nullptr, 0);
@@ -500,7 +515,11 @@ int mflbm_ensemble_solve(mflbm_ensemble* e, int32_t check, double tol, int32_t m
                 any = true;
             }
         }
-        if (changed) ECHK(e, hipMemcpy(e->active, act.data(), nd * sizeof(int32_t), hipMemcpyHostToDevice));
+        if (changed) {
+            ECHK(e, hipMemcpy(e->active, act.data(), nd * sizeof(int32_t), hipMemcpyHostToDevice));
+            const std::vector<int32_t> ends = block_ends(e, act);
+            ECHK(e, hipMemcpy(e->blk_end, ends.data(), ends.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+        }
     }
     (void)hipEventDestroy(ev0);
     (void)hipEventDestroy(ev1);

@@ -81,7 +81,9 @@ struct mflbm_handle {
     int32_t* r7 = nullptr;
     uint8_t* tile_fluid = nullptr;
     bool split_gradient = false;
-    bool grad_dirty = false;    // dense phi / cn / c_norm / curv behind the step state
+    bool grad_dirty = false;    // dense cn / c_norm / curv behind the step state
+    bool phi_dirty = false;     // dense phi of solid-boundary nodes behind the step state
+    bool phi_set = false;       // phi is the one mflbm_init_phi set: no step since
     bool phi_behind = false;    // phi of solid nodes [1, nx] x [1, ny] x [0, nz+1] behind the step state's
     // monitor scratch
     double *mon_part = nullptr, *mon_out = nullptr;
@@ -270,20 +272,38 @@ void step_dispatch(mflbm_handle* h, bool odd, hipEvent_t* ev) {
 // After steps: the fused chains leave the dense fields behind, the one on boxes also the phi of
 // most solid nodes.
 void stepped(mflbm_handle* h) {
-    h->grad_dirty = !h->split_gradient;
+    h->grad_dirty = h->phi_dirty = !h->split_gradient;
     h->phi_behind = h->grad_dirty && h->grad_shape == GRAD_SHAPE_TILES;
+    h->phi_set = false;
 }
 
 // Brings the dense phi (solid-boundary nodes of the ghost layers), cn, c_norm and curv up
 // to the step state with the split kernels.  The fused step leaves them behind; they are
 // functions of phi alone, and the split kernels also rewrite the force records with the
-// same values.
+// same values.  A phi that mflbm_init_phi set after the steps stays as it is: populations
+// start from it, and the extrapolation into solid nodes is not a reader's to make.
 int materialize_gradient(mflbm_handle* h) {
     if (!h->grad_dirty) return 0;
-    if (h->prec == MFLBM_FP64) enqueue_gradient<double>(h);
-    else enqueue_gradient<float>(h);
-    h->grad_dirty = h->phi_behind = false;
-    HIPCHK(h, hipGetLastError());
+    const size_t bytes = h->d.S4 * esize(h);
+    void* kept = nullptr;
+    if (h->phi_set) {
+        std::lock_guard<std::recursive_mutex> lock(device_lock());
+        HIPCHK(h, hipMalloc(&kept, bytes));
+    }
+    hipError_t e = kept ? hipMemcpyAsync(kept, h->phi, bytes, hipMemcpyDeviceToDevice, h->stream) : hipSuccess;
+    if (e == hipSuccess) {
+        if (h->prec == MFLBM_FP64) enqueue_gradient<double>(h);
+        else enqueue_gradient<float>(h);
+        e = hipGetLastError();
+    }
+    if (kept) {
+        if (e == hipSuccess) e = hipMemcpyAsync(h->phi, kept, bytes, hipMemcpyDeviceToDevice, h->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        std::lock_guard<std::recursive_mutex> lock(device_lock());
+        (void)hipFree(kept);
+    }
+    if (e != hipSuccess) return fail(h, "gradient fields: %s", hipGetErrorString(e));
+    h->grad_dirty = h->phi_dirty = h->phi_behind = false;
     return 0;
 }
 
@@ -292,10 +312,10 @@ int materialize_gradient(mflbm_handle* h) {
 // the split kernels round the force records they rewrite differently from the boxes', and a
 // run that went on after the read would leave the course it had.
 int materialize_phi(mflbm_handle* h) {
+    if (!h->phi_dirty) return 0;
     if (h->prec != MFLBM_FP64) return materialize_gradient(h);
-    if (!h->grad_dirty) return 0;
     Launch<double>::phi_extrap(fields<double>(h), lists(h), h->stream);
-    h->phi_behind = false;
+    h->phi_dirty = h->phi_behind = false;
     HIPCHK(h, hipGetLastError());
     return 0;
 }
@@ -762,7 +782,8 @@ void mflbm_destroy(mflbm_handle* h) {
 
 static int init_phi(mflbm_handle* h, int option, double interface_z0, double sa_target, uint64_t seed) {
     const double pin = h->p.phi_inlet;
-    h->phi_behind = false;  // every node's is set
+    h->phi_dirty = h->phi_behind = false;  // every node's is set
+    h->phi_set = true;
     if (h->prec == MFLBM_FP64)
         Launch<double>::init_phi(fields<double>(h), option, interface_z0, pin, h->open_z, sa_target, seed, h->stream);
     else Launch<float>::init_phi(fields<float>(h), option, interface_z0, pin, h->open_z, sa_target, seed, h->stream);
@@ -844,7 +865,7 @@ int mflbm_color_gradient(mflbm_handle* h) {
     if (!h) return -1;
     if (h->prec == MFLBM_FP64) enqueue_gradient<double>(h);
     else enqueue_gradient<float>(h);
-    h->grad_dirty = h->phi_behind = false;
+    h->grad_dirty = h->phi_dirty = h->phi_behind = false;
     HIPCHK(h, hipGetLastError());
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return 0;

@@ -911,7 +911,7 @@ int mflbm_profile(mflbm_handle* h, int32_t ntime0, int32_t nsteps, mflbm_kernel_
         out->boundary_ms += ms[1];
         out->gradient_ms += ms[2];
     }
-    stepped(h);
+    if (nsteps > 0) stepped(h);
     for (int e = 0; e < NE; ++e) (void)hipEventDestroy(ev[e]);
     HIPCHK(h, hipGetLastError());
     return 0;

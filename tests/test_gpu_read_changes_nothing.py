@@ -33,3 +33,18 @@ def test_reads_between_phi_and_populations(name, precision, read):
         s.run(1, 20)
     for field in ("pdf", "phi"):
         assert_same(a.download(field), b.download(field), 0.0, what=f"{name} step 20 {field}")
+
+
+@pytest.mark.parametrize("precision", [gpu.FP64, gpu.FP32])
+def test_profile_of_no_steps(precision):
+    """no step taken leaves nothing behind: the populations that follow start from the phi as set"""
+    geo, p = CASES["drainage"]()
+    print(f"[gpu-reads] profile of no steps {precision}", flush=True)
+    a, b = gpu.Solver(p, geo, precision), gpu.Solver(p, geo, precision)
+    for s in (a, b):
+        s.init_phi(p["initial_fluid_distribution_option"], p["interface_z0"])
+        if s is a:
+            assert s.profile(1, 0)["n_odd"] == 0
+        s.init_equilibrium()
+    for field in ("pdf", "phi"):
+        assert_same(a.download(field), b.download(field), 0.0, what=field)

@@ -119,7 +119,8 @@ int mfnn_mse(const float* y, const float* t, const float* mask, int64_t M, int32
 int mfnn_adam(float* w, const float* g, float* m1, float* m2, int64_t n, float lr, float b1, float b2, float eps,
               int32_t step, void* wb, void* stream);
 
-/* The same step on `count` tensors (no two sharing memory) in as few launches as they need. */
+/* The same step on `count` tensors (no two sharing memory) in as few launches as they need; empty
+ * tensors are left out, a negative n is refused (-1) before any launch. */
 typedef struct {
     float* w;
     const float* g;

@@ -1374,7 +1374,9 @@ int mfnn_mse(const float* y, const float* t, const float* mask, int64_t M, int32
 
 int mfnn_adam_many(const mfnn_adam_tensor* list, int32_t count, float lr, float b1, float b2, float eps, int32_t step,
                    void* stream) {
-    if (step < 1 || count < 0) return -1;
+    if (step < 1 || count < 0 || (count && !list)) return -1;
+    for (int t = 0; t < count; ++t)
+        if (list[t].n < 0) return -1;
     const float c1 = 1.f / (1.f - powf(b1, (float)step));
     const float c2 = 1.f / (1.f - powf(b2, (float)step));
     for (int at = 0; at < count;) {

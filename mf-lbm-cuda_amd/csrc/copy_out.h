@@ -20,7 +20,9 @@
 namespace mflbm {
 
 // Pinned slots of one handle: made by its first large copy, given back with it.  One copy at a
-// time uses them (mutex).
+// time, of all handles: it holds the library's lock, which callers may hold already and which the
+// slots' allocation needs (a mutex of the slots' own, taken by a copy before that lock and by a
+// caller that held it after, could deadlock two threads).
 class HostStaging {
 public:
     static constexpr int WORKERS = 4;
@@ -31,7 +33,7 @@ public:
     // dst[0, bytes) = src[0, bytes), after the work queued on `stream`; returns when it is there
     hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t stream) {
         if (bytes >= MIN_BYTES) {
-            std::lock_guard<std::mutex> lock(busy_);
+            std::lock_guard<std::recursive_mutex> lock(device_lock());
             int dev = 0;
             if (make() && hipGetDevice(&dev) == hipSuccess) return staged(static_cast<char*>(dst), static_cast<const char*>(src), bytes, stream, dev);
         }
@@ -49,9 +51,8 @@ public:
     }
 
 private:
-    bool make() {
+    bool make() {  // under device_lock
         if (ring_) return true;
-        std::lock_guard<std::recursive_mutex> lock(device_lock());
         void* p = nullptr;
         bool ok = hipHostMalloc(&p, WORKERS * SLOT, hipHostMallocDefault) == hipSuccess;
         ring_ = ok ? static_cast<char*>(p) : nullptr;
@@ -101,7 +102,6 @@ private:
         return static_cast<hipError_t>(error.load());
     }
 
-    std::mutex busy_;
     char* ring_ = nullptr;
     hipEvent_t done_[WORKERS] = {};
 };

@@ -1,0 +1,101 @@
+// Host harness of HostStaging (mf-lbm-cuda_amd/csrc/copy_out.h) for tests/test_copy_out_host.py:
+// the HIP calls that it makes are defined here, on host memory, so that a CPU runs it.  Built with
+// g++; argv[1] names the check, the exit status says whether it held.
+#include <chrono>
+#include <csignal>
+#include <cstdio>
+#include <cstdlib>
+#include <set>
+#include <string>
+#include <unistd.h>
+#include <vector>
+
+#include "copy_out.h"
+
+namespace {
+std::mutex book;
+std::set<std::thread::id> callers;  // threads that made a HIP call
+void called() {
+    std::lock_guard<std::mutex> lock(book);
+    callers.insert(std::this_thread::get_id());
+}
+}  // namespace
+
+extern "C" {
+hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) { called(); *p = std::malloc(bytes); return hipSuccess; }
+hipError_t hipHostFree(void* p) { called(); std::free(p); return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { called(); *e = reinterpret_cast<hipEvent_t>(std::malloc(1)); return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { called(); std::free(reinterpret_cast<void*>(e)); return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { called(); return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { called(); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { called(); return hipSuccess; }
+hipError_t hipGetLastError() { called(); return hipSuccess; }
+hipError_t hipGetDevice(int* d) { called(); *d = 0; return hipSuccess; }
+hipError_t hipSetDevice(int) { called(); return hipSuccess; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { called(); std::memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+    called();
+    std::memcpy(d, s, n);
+    return hipSuccess;
+}
+}
+
+namespace {
+using mflbm::HostStaging;
+
+std::vector<unsigned char> pattern(size_t n) {
+    std::vector<unsigned char> v(n);
+    uint32_t x = 12345u + (uint32_t)n;
+    for (auto& b : v) b = (unsigned char)((x = x * 1664525u + 1013904223u) >> 24);
+    return v;
+}
+
+bool copies(HostStaging& h, size_t n) {
+    const auto src = pattern(n);
+    std::vector<unsigned char> dst(n + 64, 7);
+    if (h.copy(dst.data(), src.data(), n, nullptr) != hipSuccess) return false;
+    if (std::memcmp(dst.data(), src.data(), n) != 0) return false;
+    for (size_t i = n; i < dst.size(); ++i)
+        if (dst[i] != 7) return false;
+    return true;
+}
+
+// sizes around the least staged one, in whole and broken chunks, on one set of slots
+int contents() {
+    HostStaging h;
+    for (size_t n : {(size_t)1, HostStaging::MIN_BYTES - 1, HostStaging::MIN_BYTES, HostStaging::MIN_BYTES + 1,
+                     4 * HostStaging::SLOT, 4 * HostStaging::SLOT + 1, 9 * HostStaging::SLOT + 4097, 25 * HostStaging::SLOT - 1})
+        if (!copies(h, n)) {
+            std::printf("%zu bytes differ\n", n);
+            return 1;
+        }
+    h.release();
+    return 0;
+}
+
+// an entry point that holds the library's lock copies while another thread makes its first copy
+int order() {
+    HostStaging h;
+    bool ok = false;
+    std::thread other;
+    {
+        std::lock_guard<std::recursive_mutex> lock(mflbm::device_lock());
+        other = std::thread([&] { ok = copies(h, HostStaging::MIN_BYTES); });
+        std::this_thread::sleep_for(std::chrono::milliseconds(300));  // the other is where it waits
+        if (!copies(h, HostStaging::MIN_BYTES + 5)) return 1;
+    }
+    other.join();
+    h.release();
+    return ok ? 0 : 1;
+}
+}  // namespace
+
+int main(int argc, char** argv) {
+    if (argc != 2) return 2;
+    std::signal(SIGALRM, [](int) { _exit(3); });  // a deadlock
+    alarm(20);
+    const std::string what = argv[1];
+    if (what == "contents") return contents();
+    if (what == "order") return order();
+    return 2;
+}

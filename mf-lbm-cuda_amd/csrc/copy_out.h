@@ -3,16 +3,19 @@
 // hipMemcpy to pageable memory moves the data through the runtime's own staging buffer with one
 // thread, which also takes the first-touch faults of a fresh destination: 18.5 ms for 200 MB
 // (11 GB/s; 11.4 ms into touched memory), where the link carries 56 GB/s into pinned memory.
-// Here WORKERS threads each hold a pinned slot and take the next chunk in turn: while one copies
-// its slot to the destination, the link fills another's: 6.1 ms for the 201 MB of 48 domains of
-// 64^3 (before: 18.6), 4.0 for 147 MB (15.3), 0.33 for 9 MB (0.56).  Slots of 2 and 1 MB took 6.6
-// and 7.7 ms; 8 threads with 2 MB 5.9.
+// Here the calling thread queues chunks into a ring of pinned slots and waits for them in turn, and
+// WORKERS threads copy the slots that have arrived to the destination while the link fills the next
+// ones.  Every HIP call is the calling thread's: concurrent HIP calls from many host threads have
+// stalled this library's work on the GPU before, and the copies need the threads for memory alone.
+// A phi read into a fresh array, hipMemcpy and this: 147 MB 14.0 and 3.9 ms, 20 MB 1.2 and 0.58, 9 MB
+// 0.53 and 0.30 (with the HIP calls in each thread 4.5, 0.58 and 0.33).  Into touched memory 201 MB
+// take 4.4 ms with 6 or 8 slots of 4 MB, 5.0 with 8 of 2 MB and 6.3 with 12 of 1 MB; 4 slots of 4 MB
+// make fresh memory 5 % slower.
 #pragma once
 #include <hip/hip_runtime.h>
-#include <atomic>
+#include <condition_variable>
 #include <cstring>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 #include "device_lock.h"
@@ -25,7 +28,7 @@ namespace mflbm {
 // caller that held it after, could deadlock two threads).
 class HostStaging {
 public:
-    static constexpr int WORKERS = 4;
+    static constexpr size_t WORKERS = 4, SLOTS = 6;
     static constexpr size_t SLOT = 4 << 20;
     // below this hipMemcpy is as fast
     static constexpr size_t MIN_BYTES = 6 << 20;
@@ -34,15 +37,14 @@ public:
     hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t stream) {
         if (bytes >= MIN_BYTES) {
             std::lock_guard<std::recursive_mutex> lock(device_lock());
-            int dev = 0;
-            if (make() && hipGetDevice(&dev) == hipSuccess) return staged(static_cast<char*>(dst), static_cast<const char*>(src), bytes, stream, dev);
+            if (make()) return staged(static_cast<char*>(dst), static_cast<const char*>(src), bytes, stream);
         }
         const hipError_t r = hipStreamSynchronize(stream);
         return r == hipSuccess ? hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost) : r;
     }
 
     void release() {  // under device_lock, with no copy running
-        for (int w = 0; w < WORKERS; ++w) {
+        for (size_t w = 0; w < SLOTS; ++w) {
             if (done_[w]) (void)hipEventDestroy(done_[w]);
             done_[w] = nullptr;
         }
@@ -54,9 +56,9 @@ private:
     bool make() {  // under device_lock
         if (ring_) return true;
         void* p = nullptr;
-        bool ok = hipHostMalloc(&p, WORKERS * SLOT, hipHostMallocDefault) == hipSuccess;
+        bool ok = hipHostMalloc(&p, SLOTS * SLOT, hipHostMallocDefault) == hipSuccess;
         ring_ = ok ? static_cast<char*>(p) : nullptr;
-        for (int w = 0; ok && w < WORKERS; ++w) ok = hipEventCreateWithFlags(&done_[w], hipEventDisableTiming) == hipSuccess;
+        for (size_t w = 0; ok && w < SLOTS; ++w) ok = hipEventCreateWithFlags(&done_[w], hipEventDisableTiming) == hipSuccess;
         if (!ok) {
             release();
             (void)hipGetLastError();
@@ -64,46 +66,81 @@ private:
         return ok;
     }
 
-    hipError_t staged(char* dst, const char* src, size_t bytes, hipStream_t stream, int dev) {
+    hipError_t staged(char* dst, const char* src, size_t bytes, hipStream_t stream) {
         // a slot at a time, or a share of the whole to each thread
         const size_t share = (bytes / WORKERS + 4096) & ~(size_t)4095, chunk = share < SLOT ? share : SLOT;
         const size_t chunks = (bytes + chunk - 1) / chunk;
-        std::atomic<size_t> next{0};
-        std::atomic<int> error{hipSuccess};
-        auto work = [&](int w) {
-            char* slot = ring_ + w * SLOT;
-            hipError_t r = hipSuccess;
-            while (r == hipSuccess && error.load() == hipSuccess) {
-                const size_t c = next++;
-                if (c >= chunks) return;
-                const size_t at = c * chunk, len = bytes - at < chunk ? bytes - at : chunk;
-                r = hipMemcpyAsync(slot, src + at, len, hipMemcpyDeviceToHost, stream);
-                if (r == hipSuccess) r = hipEventRecord(done_[w], stream);
-                if (r == hipSuccess) r = hipEventSynchronize(done_[w]);
-                if (r == hipSuccess) std::memcpy(dst + at, slot, len);
+        auto slot = [&](size_t c) { return ring_ + c % SLOTS * SLOT; };
+        auto length = [&](size_t c) { return bytes - c * chunk < chunk ? bytes - c * chunk : chunk; };
+        std::mutex m;
+        std::condition_variable ready, freed;
+        size_t issued = 0, arrived = 0, taken = 0;  // chunks queued; in their slots; given to a thread
+        bool full[SLOTS] = {}, stop = false;        // slots in use
+        // copies chunks out of their slots as they arrive, until all are given out
+        auto drain = [&] {
+            std::unique_lock<std::mutex> lock(m);
+            for (;;) {
+                ready.wait(lock, [&] { return taken < arrived || taken == chunks || stop; });
+                if (taken == arrived) return;
+                const size_t c = taken++;
+                if (taken == chunks) ready.notify_all();
+                lock.unlock();
+                std::memcpy(dst + c * chunk, slot(c), length(c));
+                lock.lock();
+                full[c % SLOTS] = false;
+                freed.notify_one();
             }
-            if (r != hipSuccess) error = r;
         };
+        auto issue = [&] {
+            hipError_t r = hipMemcpyAsync(slot(issued), src + issued * chunk, length(issued), hipMemcpyDeviceToHost, stream);
+            if (r == hipSuccess) r = hipEventRecord(done_[issued % SLOTS], stream);
+            full[issued++ % SLOTS] = true;
+            return r;
+        };
+        hipError_t r = hipSuccess;
+        while (issued < chunks && issued < SLOTS && r == hipSuccess) r = issue();
+        // this thread makes the HIP calls and, once all chunks are there, copies with the others
         std::thread other[WORKERS];
-        for (int w = 1; w < WORKERS && (size_t)w < chunks; ++w) {
-            try {
-                other[w] = std::thread([&work, w, dev, &error] {
-                    const hipError_t r = hipSetDevice(dev);
-                    if (r == hipSuccess) work(w);
-                    else error = r;
-                });
-            } catch (const std::system_error&) {
-                break;  // the threads there are take all chunks
+        size_t threads = 0;
+        try {
+            while (threads < WORKERS && threads + 1 < chunks) {
+                other[threads] = std::thread(drain);
+                ++threads;
+            }
+        } catch (...) {  // the threads there are take all chunks
+        }
+        for (size_t c = 0; c < chunks && r == hipSuccess; ++c) {
+            r = hipEventSynchronize(done_[c % SLOTS]);
+            if (r != hipSuccess) break;
+            std::unique_lock<std::mutex> lock(m);
+            arrived = c + 1;
+            if (threads == 0) {
+                std::memcpy(dst + c * chunk, slot(c), length(c));
+                full[taken++ % SLOTS] = false;
+            }
+            ready.notify_one();
+            // refill the slots that are free; wait for one only where nothing else is on its way
+            while (issued < chunks && r == hipSuccess) {
+                if (full[issued % SLOTS]) {
+                    if (issued > c + 1) break;
+                    freed.wait(lock, [&] { return !full[issued % SLOTS]; });
+                }
+                r = issue();
             }
         }
-        work(0);
-        for (std::thread& t : other)
-            if (t.joinable()) t.join();
-        return static_cast<hipError_t>(error.load());
+        if (r != hipSuccess) {
+            std::lock_guard<std::mutex> lock(m);
+            stop = true;
+            ready.notify_all();
+        }
+        drain();
+        for (size_t t = 0; t < threads; ++t) other[t].join();
+        if (r != hipSuccess) (void)hipStreamSynchronize(stream);  // no copy into the slots goes on
+        return r;
     }
 
     char* ring_ = nullptr;
-    hipEvent_t done_[WORKERS] = {};
+    hipEvent_t done_[SLOTS] = {};  // a slot's chunk is there
 };
 
 }  // namespace mflbm

@@ -88,6 +88,16 @@ int order() {
     h.release();
     return ok ? 0 : 1;
 }
+
+// the threads that copy out of the slots leave the HIP calls to the calling thread
+int calls() {
+    HostStaging h;
+    callers.clear();
+    if (!copies(h, 3 * HostStaging::MIN_BYTES) || !copies(h, 25 * HostStaging::SLOT - 1)) return 1;
+    h.release();
+    std::printf("%zu threads made HIP calls\n", callers.size());
+    return callers.size() == 1 && callers.count(std::this_thread::get_id()) ? 0 : 1;
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -97,5 +107,6 @@ int main(int argc, char** argv) {
     const std::string what = argv[1];
     if (what == "contents") return contents();
     if (what == "order") return order();
+    if (what == "calls") return calls();
     return 2;
 }

@@ -35,7 +35,7 @@ public:
 
     // dst[0, bytes) = src[0, bytes), after the work queued on `stream`; returns when it is there
     hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t stream) {
-        if (bytes >= MIN_BYTES) {
+        if (bytes >= MIN_BYTES && pageable(dst)) {
             std::lock_guard<std::recursive_mutex> lock(device_lock());
             if (make()) return staged(static_cast<char*>(dst), static_cast<const char*>(src), bytes, stream);
         }
@@ -53,6 +53,15 @@ public:
     }
 
 private:
+    // Memory that the runtime knows (pinned, managed, a device's) it copies to directly, at the link's
+    // rate: 201 MB into pinned memory 3.5 ms, through the slots 25.
+    static bool pageable(const void* dst) {
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, dst) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+        (void)hipGetLastError();  // what runtimes that do not know ordinary memory return for it
+        return true;
+    }
+
     bool make() {  // under device_lock
         if (ring_) return true;
         void* p = nullptr;

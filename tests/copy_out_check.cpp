@@ -15,6 +15,9 @@
 namespace {
 std::mutex book;
 std::set<std::thread::id> callers;  // threads that made a HIP call
+int queued = 0, direct = 0;         // hipMemcpyAsync and hipMemcpy calls
+hipMemoryType kind = hipMemoryTypeUnregistered;  // of every destination
+hipError_t known = hipSuccess;
 void called() {
     std::lock_guard<std::mutex> lock(book);
     callers.insert(std::this_thread::get_id());
@@ -32,9 +35,11 @@ hipError_t hipStreamSynchronize(hipStream_t) { called(); return hipSuccess; }
 hipError_t hipGetLastError() { called(); return hipSuccess; }
 hipError_t hipGetDevice(int* d) { called(); *d = 0; return hipSuccess; }
 hipError_t hipSetDevice(int) { called(); return hipSuccess; }
-hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { called(); std::memcpy(d, s, n); return hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*) { called(); a->type = kind; return known; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { called(); ++direct; std::memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
     called();
+    ++queued;
     std::memcpy(d, s, n);
     return hipSuccess;
 }
@@ -98,6 +103,24 @@ int calls() {
     std::printf("%zu threads made HIP calls\n", callers.size());
     return callers.size() == 1 && callers.count(std::this_thread::get_id()) ? 0 : 1;
 }
+
+// destinations that the runtime copies to directly are left to it
+int destinations() {
+    HostStaging h;
+    for (hipMemoryType k : {hipMemoryTypeHost, hipMemoryTypeManaged, hipMemoryTypeDevice}) {
+        kind = k;
+        direct = queued = 0;
+        if (!copies(h, 25 * HostStaging::SLOT) || direct != 1 || queued) return 1;
+    }
+    kind = hipMemoryTypeUnregistered;
+    for (hipError_t e : {hipSuccess, hipErrorInvalidValue}) {
+        known = e;
+        direct = queued = 0;
+        if (!copies(h, 25 * HostStaging::SLOT) || direct || !queued) return 1;
+    }
+    h.release();
+    return 0;
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -108,5 +131,6 @@ int main(int argc, char** argv) {
     if (what == "contents") return contents();
     if (what == "order") return order();
     if (what == "calls") return calls();
+    if (what == "destinations") return destinations();
     return 2;
 }

@@ -22,7 +22,7 @@
 
 namespace mflbm {
 
-// Pinned slots of one handle: made by its first large copy, given back with it.  One copy at a
+// Pinned slots of one handle: made once its large copies are worth them, given back with it.  One copy at a
 // time, of all handles: it holds the library's lock, which callers may hold already and which the
 // slots' allocation needs (a mutex of the slots' own, taken by a copy before that lock and by a
 // caller that held it after, could deadlock two threads).
@@ -32,12 +32,18 @@ public:
     static constexpr size_t SLOT = 4 << 20;
     // below this hipMemcpy is as fast
     static constexpr size_t MIN_BYTES = 6 << 20;
+    // The slots take 1.6 ms to make, which the copies of fewer bytes than this do not win back (a
+    // handle's first read, hipMemcpy and staged with the slots' making: 9 MB 0.9 and 2.2 ms, 20 MB
+    // 2.1 and 2.9, 147 MB 15 and 7.4; later reads 0.53 and 0.30, 1.2 and 0.58, 14 and 3.9): until a
+    // handle's large copies come to it they are hipMemcpy's.
+    static constexpr size_t WORTH_BYTES = 48 << 20;
 
     // dst[0, bytes) = src[0, bytes), after the work queued on `stream`; returns when it is there
     hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t stream) {
         if (bytes >= MIN_BYTES && pageable(dst)) {
             std::lock_guard<std::recursive_mutex> lock(device_lock());
-            if (make()) return staged(static_cast<char*>(dst), static_cast<const char*>(src), bytes, stream);
+            copied_ = copied_ < WORTH_BYTES ? copied_ + bytes : copied_;
+            if (copied_ >= WORTH_BYTES && make()) return staged(static_cast<char*>(dst), static_cast<const char*>(src), bytes, stream);
         }
         const hipError_t r = hipStreamSynchronize(stream);
         return r == hipSuccess ? hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost) : r;
@@ -148,6 +154,7 @@ private:
         return r;
     }
 
+    size_t copied_ = 0;  // by large copies, up to WORTH_BYTES
     char* ring_ = nullptr;
     hipEvent_t done_[SLOTS] = {};  // a slot's chunk is there
 };

@@ -15,6 +15,7 @@
 namespace {
 std::mutex book;
 std::set<std::thread::id> callers;  // threads that made a HIP call
+int made = 0;                       // hipHostMalloc calls
 int queued = 0, direct = 0;         // hipMemcpyAsync and hipMemcpy calls
 hipMemoryType kind = hipMemoryTypeUnregistered;  // of every destination
 hipError_t known = hipSuccess;
@@ -25,7 +26,7 @@ void called() {
 }  // namespace
 
 extern "C" {
-hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) { called(); *p = std::malloc(bytes); return hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) { called(); ++made; *p = std::malloc(bytes); return hipSuccess; }
 hipError_t hipHostFree(void* p) { called(); std::free(p); return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { called(); *e = reinterpret_cast<hipEvent_t>(std::malloc(1)); return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { called(); std::free(reinterpret_cast<void*>(e)); return hipSuccess; }
@@ -68,6 +69,7 @@ bool copies(HostStaging& h, size_t n) {
 // sizes around the least staged one, in whole and broken chunks, on one set of slots
 int contents() {
     HostStaging h;
+    if (!copies(h, 25 * HostStaging::SLOT)) return 1;  // makes the slots
     for (size_t n : {(size_t)1, HostStaging::MIN_BYTES - 1, HostStaging::MIN_BYTES, HostStaging::MIN_BYTES + 1,
                      4 * HostStaging::SLOT, 4 * HostStaging::SLOT + 1, 9 * HostStaging::SLOT + 4097, 25 * HostStaging::SLOT - 1})
         if (!copies(h, n)) {
@@ -85,9 +87,9 @@ int order() {
     std::thread other;
     {
         std::lock_guard<std::recursive_mutex> lock(mflbm::device_lock());
-        other = std::thread([&] { ok = copies(h, HostStaging::MIN_BYTES); });
+        other = std::thread([&] { ok = copies(h, 25 * HostStaging::SLOT); });
         std::this_thread::sleep_for(std::chrono::milliseconds(300));  // the other is where it waits
-        if (!copies(h, HostStaging::MIN_BYTES + 5)) return 1;
+        if (!copies(h, 25 * HostStaging::SLOT + 5)) return 1;
     }
     other.join();
     h.release();
@@ -98,7 +100,7 @@ int order() {
 int calls() {
     HostStaging h;
     callers.clear();
-    if (!copies(h, 3 * HostStaging::MIN_BYTES) || !copies(h, 25 * HostStaging::SLOT - 1)) return 1;
+    if (!copies(h, 25 * HostStaging::SLOT - 1) || !copies(h, 3 * HostStaging::MIN_BYTES)) return 1;
     h.release();
     std::printf("%zu threads made HIP calls\n", callers.size());
     return callers.size() == 1 && callers.count(std::this_thread::get_id()) ? 0 : 1;
@@ -121,6 +123,25 @@ int destinations() {
     h.release();
     return 0;
 }
+
+// the slots are made by the copy that is worth them: a first large one, or a later small one
+int worth() {
+    const size_t small = HostStaging::MIN_BYTES + 3000000, large = 36 * HostStaging::SLOT;
+    HostStaging one, many;
+    made = 0;
+    if (!copies(one, large) || made != 1 || !copies(one, small) || !copies(one, large) || made != 1) return 1;
+    made = 0;
+    if (!copies(many, small) || made != 0) return 1;
+    int n = 1;
+    while (made == 0 && n < 100) {
+        if (!copies(many, small)) return 1;
+        ++n;
+    }
+    if (made != 1 || (size_t)n * small < (40 << 20) || (size_t)n * small > (60 << 20)) return 1;
+    one.release();
+    many.release();
+    return 0;
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -131,6 +152,7 @@ int main(int argc, char** argv) {
     if (what == "contents") return contents();
     if (what == "order") return order();
     if (what == "calls") return calls();
+    if (what == "worth") return worth();
     if (what == "destinations") return destinations();
     return 2;
 }

@@ -22,9 +22,12 @@
 #include <type_traits>
 
 #include "../../include/mfnn.h"
+#include "conv_plan.h"
 #include "device_lock.h"
 
 namespace {
+
+using namespace mfnn;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
@@ -36,14 +39,9 @@ __device__ __forceinline__ float bf2f(__bf16 v) { return (float)v; }
 // loads from memory in flight.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-struct Grid3 {
-    int D, H, W;
-};
-
 // 16-byte load through a buffer descriptor: a lane past the descriptor's bytes reads zeros, so
 // the zero padding of a convolution costs no select (num = 0 for a whole plane outside the
 // grid, NOWHERE as the offset of a single lane).  Descriptors address less than 2^31 bytes.
-constexpr uint32_t NOWHERE = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t num) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)num, 0x00027000);
 }
@@ -54,15 +52,6 @@ __device__ __forceinline__ bf16x8 buffer_load16(__amdgpu_buffer_rsrc_t rsrc, uin
 // Taps: 0..26, x fastest (dx = tap % 3 - 1, dy = tap / 3 % 3 - 1, dz = tap / 9 - 1); a tap
 // outside the grid reads zero (zero padding).
 
-// Exact quotients by a divisor fixed over a launch, without a branch: n / d =
-// umulhi(n, ceil(2^32 / d)) while n * d < 2^32 (the launchers check it); d = 1 passes n through
-// the mask.
-struct FastDiv {
-    uint32_t d, mul, one;
-};
-inline FastDiv fast_div(uint32_t d) {
-    return {d, d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u, d > 1 ? 0u : ~0u};
-}
 __device__ __forceinline__ int quot(int n, const FastDiv& f) { return (int)(__umulhi((uint32_t)n, f.mul) + ((uint32_t)n & f.one)); }
 
 // Epilogue of a convolution: bias, then ReLU or the gate, stored as bf16 and/or fp32, for four
@@ -156,14 +145,6 @@ struct Epilogue {
 // tiles that gathered every operand from global memory, in us: 64^3 16 -> 16 channels 28.4 to
 // 11.0, 48 -> 16 73.5 to 25.2; 16^3 192 -> 64 55.5 to 12.7; 8^3 128 -> 128 35.2 to 9.1; 128^3
 // 48 -> 16 555 to 175 (LDS operand reads, 82 us of it, and the load of 2.5 times the input).
-struct ConvTile {
-    int tx, ty, tz, nx, ny;  // box, boxes along x and y
-    int tv, pv;              // voxels of a box; of a loaded box, in whole groups of 16
-    int pu;                  // 16-byte units of one loaded plane
-    FastDiv row, c8, dtx, dty, dnx, dny;  // units of a loaded row, of a voxel; tx, ty, nx, ny
-    FastDiv dboxes;                       // boxes
-};
-
 template <int MT, int NT, int PF>
 __global__ __launch_bounds__(256) void k_conv3_box(const __bf16* __restrict__ X, const __bf16* __restrict__ Wb, Grid3 g,
                                                    int cin, int kp, int ntw, Epilogue ep, ConvTile t) {
@@ -181,8 +162,8 @@ __global__ __launch_bounds__(256) void k_conv3_box(const __bf16* __restrict__ X,
     // per XCD measured up to 6 % slower)
     int bx, by, bz, tb;
     {
-        const int grp = quot(blockIdx.x, t.dboxes), b = blockIdx.x - grp * (int)t.dboxes.d, yz = quot(b, t.dnx);
-        tb = grp * NT;
+        const int b = blockIdx.x, yz = quot(b, t.dnx);
+        tb = blockIdx.y * NT;
         bz = quot(yz, t.dny);
         bx = b - yz * t.nx;
         by = yz - bz * t.ny;
@@ -996,89 +977,6 @@ int rows_of(int64_t D, int64_t H, int64_t W, int C, bool wide, Fn&& launch) {
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-// Channel tiles a wave may hold beside mt voxel tiles (registers).
-inline int conv_max_nt(int mt) { return mt >= 8 ? 2 : mt >= 4 ? 3 : 4; }
-
-// Box and tile counts of one k_conv3_box launch.
-struct ConvPlan {
-    ConvTile t;
-    int mt, nt;
-    size_t lds;
-    unsigned boxes;
-};
-
-// Box of a convolution: the equal splits of the axes with rows of up to 32 voxels are priced in
-// cycles of a CU -- one per loaded 16-byte unit, the weights' 64 per channel tile and k block
-// among them; per k block its MFMAs (16 each, a wave on each SIMD) and its operand reads (4 per
-// wave and operand), at least the 70 of one block's dependent chain for a workgroup alone on
-// its CU; load and MFMAs of two workgroups overlap where LDS holds both; whole rounds over the
-// 256 CUs.
-bool conv_plan(const Grid3& g, int cin, int ntw, ConvPlan& best) {
-    const int c8 = cin / 8;
-    const int nkb = (27 * c8 + 3) / 4;
-    const size_t tab = (size_t)((nkb + 3) / 4 * 16 + 16) * 4;
-    constexpr size_t LDS_MAX = 160 * 1024;
-    double best_cost = 0.0;
-    bool found = false;
-    auto parts = [](int n, int lo, int hi, int* out, int cap) {  // distinct ceil(n / p) in [lo, hi]
-        int cnt = 0;
-        for (int p = (n + hi - 1) / hi; p <= n && cnt < cap; ++p) {
-            const int v = (n + p - 1) / p;
-            if (v < lo && cnt) break;
-            if (cnt && out[cnt - 1] == v) continue;
-            out[cnt++] = v;
-        }
-        return cnt;
-    };
-    int xs[6], ys[8], zs[6];
-    const int nxs = parts(g.W, 4, 32, xs, 6), nys = parts(g.H, 1, 8, ys, 8), nzs = parts(g.D, 1, 8, zs, 6);
-    for (int a = 0; a < nxs; ++a)
-        for (int b = 0; b < nys; ++b)
-            for (int c = 0; c < nzs; ++c) {
-                const int tx = xs[a], ty = ys[b], tz = zs[c], tv = tx * ty * tz;
-                if (tv > 512) continue;
-                const int mt = tv > 256 ? 8 : tv > 128 ? 4 : tv > 64 ? 2 : 1;
-                const int64_t loaded = (int64_t)(tx + 2) * (ty + 2) * (tz + 2);
-                const size_t lds_box = 16 * (1 + (size_t)((c8 + 1) / 2) * (2 * ((loaded + 15) / 16 * 16) + 1)) + tab;
-                const int64_t boxes = (int64_t)((g.W + tx - 1) / tx) * ((g.H + ty - 1) / ty) * ((g.D + tz - 1) / tz);
-                for (int nt = 1; nt <= 4 && nt <= ntw; ++nt) {
-                    if (nt > conv_max_nt(mt)) continue;
-                    const size_t lds = lds_box + 8192 * nt;
-                    if (lds > LDS_MAX) continue;
-                    const int64_t wgs = boxes * ((ntw + nt - 1) / nt);
-                    const double load = (double)loaded * c8, fixed = 2000.0 + 250.0 * mt * nt;
-                    const double block = std::max(std::max(16.0 * mt * nt, 16.0 * (mt + nt)), 64.0 * nt) + 24.0;
-                    const double alone = load + nkb * std::max(block, 70.0) + fixed;
-                    const double rounds = (double)((wgs + 255) / 256);
-                    const double each = 2 * lds > LDS_MAX ? alone
-                                                          : std::max(load, nkb * block) +
-                                                                0.5 * std::min(load, nkb * block) + 0.5 * fixed;
-                    const double cost = std::max(alone, rounds * each);
-                    if (!found || cost < best_cost) {
-                        found = true;
-                        best_cost = cost;
-                        best.t.tx = tx; best.t.ty = ty; best.t.tz = tz;
-                        best.mt = mt; best.nt = nt; best.lds = lds; best.boxes = (unsigned)boxes;
-                    }
-                }
-            }
-    if (!found) return false;
-    ConvTile& t = best.t;
-    const int LX = t.tx + 2, LY = t.ty + 2;
-    t.nx = (g.W + t.tx - 1) / t.tx;
-    t.ny = (g.H + t.ty - 1) / t.ty;
-    t.tv = t.tx * t.ty * t.tz;
-    t.pv = (LX * LY * (t.tz + 2) + 15) / 16 * 16;
-    t.pu = LX * LY * c8;
-    t.row = fast_div(LX * c8); t.c8 = fast_div(c8);
-    const unsigned groups = (ntw + best.nt - 1) / best.nt;
-    t.dboxes = fast_div(best.boxes);
-    t.dtx = fast_div(t.tx); t.dty = fast_div(t.ty); t.dnx = fast_div(t.nx); t.dny = fast_div(t.ny);
-    // the quotients are exact while numerator * divisor < 2^32
-    return (uint64_t)best.boxes * best.boxes * groups < (1ull << 32) && (uint64_t)t.pu * LX * c8 < (1ull << 32) &&
-           2ull * g.H * g.W * cin < NOWHERE;
-}
-
 int conv_launch(const __bf16* X, const __bf16* Wb, const float* bias, const __bf16* gate, const Grid3& g, int cin, int kp,
                 int cout, int relu, __bf16* yb, float* yf, hipStream_t s) {
     const int ntw = (cout + 15) / 16;
@@ -1090,7 +988,7 @@ int conv_launch(const __bf16* X, const __bf16* Wb, const float* bias, const __bf
         k_conv3<<<dim3(nblk((int64_t)g.D * g.H * g.W, 64), ntw), 256, 0, s>>>(X, Wb, g, cin, kp, ep);
         return hipGetLastError() == hipSuccess ? 0 : -2;
     }
-    const unsigned grid = p.boxes * ((ntw + p.nt - 1) / p.nt);
+    const dim3 grid(p.boxes, (ntw + p.nt - 1) / p.nt);
     switch (10 * p.mt + p.nt) {
 #define MFNN_BOX(m, n, pf) \
     case 10 * m + n: k_conv3_box<m, n, pf><<<grid, 256, p.lds, s>>>(X, Wb, g, cin, kp, ntw, ep, p.t); break;

@@ -61,6 +61,15 @@ struct ConvPlan {
     unsigned boxes;
 };
 
+// The gathering kernel (k_conv3) takes one channel tile per block where there are fewer blocks of
+// four voxel tiles than CUs, or five and less per CU with one channel tile each; else all of them (us,
+// one and all: 23040 voxels 1056 -> 32 503 and 587, 20480 720 -> 64 490 and 568, 25600 800 -> 64 785
+// and 510, 32768 800 -> 64 976 and 515).
+inline bool gather_single(const Grid3& g, int ntw) {
+    const int64_t blocks = ((int64_t)g.D * g.H * g.W + 63) / 64;
+    return blocks < 256 || (ntw > 1 && blocks * ntw <= 1280);
+}
+
 // Box of a convolution: the equal splits of the axes with rows of up to 32 voxels are priced in
 // cycles of a CU -- one per loaded 16-byte unit, the weights' 64 per channel tile and k block
 // among them; per k block its MFMAs (16 each, a wave on each SIMD) and its operand reads (4 per

@@ -323,34 +323,64 @@ __global__ __launch_bounds__(256) void k_conv3_box(const __bf16* __restrict__ X,
     });
 }
 
-// The convolution of channel counts whose boxes do not fit LDS (above about 600 input
-// channels): one wave per 16 voxels and 16 output channels (tile blockIdx.y), every tap
-// gathered from global memory.
+// The convolution of planes of 2 GiB and more and of channel counts whose boxes do not fit LDS
+// (conv_plan): every tap gathered from global memory.  One wave per MT tiles of 16 voxels and the
+// NT 16-channel tiles blockIdx.y * NT ..: the voxel tiles share each weight load, the channel
+// tiles each voxel load.
+template <int NT, int MT>
 __global__ __launch_bounds__(256) void k_conv3(const __bf16* __restrict__ X, const __bf16* __restrict__ Wb, Grid3 g,
-                                               int cin, int kp, Epilogue ep) {
+                                               int cin, int kp, int ntw, Epilogue ep) {
     const int M = g.D * g.H * g.W;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int m0 = (blockIdx.x * 4 + wave) * 16;
+    const int m0 = (blockIdx.x * 4 + wave) * 16 * MT;
     if (m0 >= M) return;
     const int r = lane & 15, q = lane >> 4;
-    const int K = 27 * cin;
-    const int mv = m0 + r, xv = mv % g.W, yv = (mv / g.W) % g.H, zv = mv / (g.W * g.H);
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int K = 27 * cin, tb = blockIdx.y * NT;
+    int mv[MT], xv[MT], yv[MT], zv[MT];
+#pragma unroll
+    for (int u = 0; u < MT; ++u) {
+        mv[u] = m0 + 16 * u + r;
+        xv[u] = mv[u] % g.W;
+        yv[u] = (mv[u] / g.W) % g.H;
+        zv[u] = mv[u] / (g.W * g.H);
+    }
+    f32x4 acc[MT][NT];
+#pragma unroll
+    for (int u = 0; u < MT; ++u)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int kb = 0; kb < kp; kb += 32) {
         const int k = kb + 8 * q;
         const int tap = k < K ? k / cin : 0, ci = k - tap * cin;
         const int ox = tap % 3 - 1, oy = (tap / 3) % 3 - 1, oz = tap / 9 - 1;
-        const bf16x8 b = *reinterpret_cast<const bf16x8*>(Wb + (int64_t)(blockIdx.y * 16 + r) * kp + k);
-        bf16x8 a;
+        bf16x8 b[NT];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) a[j] = (__bf16)0.f;
-        const int xx = xv + ox, yy = yv + oy, zz = zv + oz;
-        if (k < K && mv < M && xx >= 0 && yy >= 0 && zz >= 0 && xx < g.W && yy < g.H && zz < g.D)
-            a = *reinterpret_cast<const bf16x8*>(X + (int64_t)((zz * g.H + yy) * g.W + xx) * cin + ci);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, acc, 0, 0, 0);
+        for (int t = 0; t < NT; ++t)
+            b[t] = *reinterpret_cast<const bf16x8*>(Wb + (int64_t)((NT == 1 ? tb : min(tb + t, ntw - 1)) * 16 + r) * kp + k);
+#pragma unroll
+        for (int u = 0; u < MT; ++u) {
+            bf16x8 a;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) a[j] = (__bf16)0.f;
+            const int xx = xv[u] + ox, yy = yv[u] + oy, zz = zv[u] + oz;
+            if (k < K && mv[u] < M && xx >= 0 && yy >= 0 && zz >= 0 && xx < g.W && yy < g.H && zz < g.D)
+                a = *reinterpret_cast<const bf16x8*>(X + (int64_t)((zz * g.H + yy) * g.W + xx) * cin + ci);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[t], a, acc[u][t], 0, 0, 0);
+        }
     }
-    const int n = blockIdx.y * 16 + 4 * q;
-    if (mv < M) ep.store(acc, ep.bias4(n), n, mv);
+    auto store_all = [&](auto&& store) {
+#pragma unroll
+        for (int u = 0; u < MT; ++u)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const int n = (tb + t) * 16 + 4 * q;
+                if (mv[u] < M) store(acc[u][t], ep.bias4(n), n, mv[u]);
+            }
+    };
+    // one tile: its four stores are too few to choose between forms for
+    if (MT * NT == 1) store_all([&ep](const f32x4& a, const f32x4& b, int n, int mm) { ep.store(a, b, n, mm); });
+    else ep.each(store_all);
 }
 
 // Weight gradient partials where k_conv3_wgrad_rows would hold few voxels at a time (grids
@@ -985,7 +1015,26 @@ int conv_launch(const __bf16* X, const __bf16* Wb, const float* bias, const __bf
     const Epilogue ep{bias, gate, yb, yf, cout, relu, quad};
     ConvPlan p;
     if (!conv_plan(g, cin, ntw, p)) {
-        k_conv3<<<dim3(nblk((int64_t)g.D * g.H * g.W, 64), ntw), 256, 0, s>>>(X, Wb, g, cin, kp, ep);
+        const int64_t M = (int64_t)g.D * g.H * g.W;
+        // grids of 65536 voxels and more with one or two channel tiles: two voxel tiles per wave, but not
+        // one channel tile of deep inputs beyond the caches (us, one voxel tile and two: 128^3 48 -> 16
+        // 615 and 530, 448 -> 32 15900 and 10850, 48^3 1104 -> 16 1390 and 1113; 64^3 1104 -> 16 3195 and
+        // 4100)
+        const bool pair = M >= 65536 && !(ntw == 1 && cin > 512 && M >= 1 << 18);
+        switch (gather_single(g, ntw) ? 0 : ntw) {
+#define MFNN_GATHER(n, m) k_conv3<n, m><<<dim3(nblk(M, 64 * m), (ntw + n - 1) / n), 256, 0, s>>>(X, Wb, g, cin, kp, ntw, ep)
+            case 0: MFNN_GATHER(1, 1); break;
+            case 1: if (pair) MFNN_GATHER(1, 2); else MFNN_GATHER(1, 1); break;
+            case 2: if (pair) MFNN_GATHER(2, 2); else MFNN_GATHER(2, 1); break;
+            case 3: MFNN_GATHER(3, 1); break;
+            case 4: MFNN_GATHER(4, 1); break;
+            case 5: MFNN_GATHER(5, 1); break;
+            case 6: MFNN_GATHER(6, 1); break;
+            case 7: MFNN_GATHER(7, 1); break;
+            case 8: MFNN_GATHER(8, 1); break;
+            default: MFNN_GATHER(12, 1); break;
+#undef MFNN_GATHER
+        }
         return hipGetLastError() == hipSuccess ? 0 : -2;
     }
     const dim3 grid(p.boxes, (ntw + p.nt - 1) / p.nt);

@@ -70,12 +70,24 @@ inline bool gather_single(const Grid3& g, int ntw) {
     return blocks < 256 || (ntw > 1 && blocks * ntw <= 1280);
 }
 
+// Its time on more than 512 channels, in cycles: LDS then holds one workgroup of few voxels, whose
+// box may cost more than it saves (us, gathered and on boxes: 32^3 800 -> 64 515 and 1430, 12^3 1056
+// -> 128 395 and 604, 24^3 720 -> 64 381 and 440, 64^3 600 -> 128 5930 and 7360; 32^3 576 -> 64 529 and
+// 480, 20^3 560 -> 128 338 and 227, 8^3 1056 -> 128 391 and 180).  A k block costs the latency of
+// its loads or what the tiles move.
+inline double gather_cycles(const Grid3& g, int cin, int ntw) {
+    const double blocks = (double)(((int64_t)g.D * g.H * g.W + 63) / 64), nkb = (27 * (cin / 8) + 3) / 4;
+    const double tiles = 1.3 * std::min(ntw, 4) + 0.7 * std::max(ntw - 4, 0);
+    return nkb * (gather_single(g, ntw) ? 700.0 + blocks * ntw : std::max(2200.0, tiles * blocks));
+}
+
 // Box of a convolution: the equal splits of the axes with rows of up to 32 voxels are priced in
 // cycles of a CU -- one per loaded 16-byte unit, the weights' 64 per channel tile and k block
 // among them; per k block its MFMAs (16 each, a wave on each SIMD) and its operand reads (4 per
 // wave and operand), at least the 70 of one block's dependent chain for a workgroup alone on
 // its CU; load and MFMAs of two workgroups overlap where LDS holds both; whole rounds over the
-// 256 CUs.  False where no box fits LDS or its launch, or no descriptor a plane.
+// 256 CUs.  False where no box fits LDS or its launch, no descriptor a plane, or the gathering
+// kernel is cheaper.
 inline bool conv_plan(const Grid3& g, int cin, int ntw, ConvPlan& best) {
     const int c8 = cin / 8;
     const int nkb = (27 * c8 + 3) / 4;
@@ -84,21 +96,23 @@ inline bool conv_plan(const Grid3& g, int cin, int ntw, ConvPlan& best) {
     double best_cost = 0.0;
     bool found = false;
     if (2ull * g.H * g.W * cin >= NOWHERE) return false;  // a plane that no descriptor addresses
-    auto parts = [](int n, int lo, int hi, int* out, int cap) {  // distinct ceil(n / p) in [lo, hi]
+    auto parts = [](int n, int lo, int hi, int* out) {  // the values ceil(n / p) in [lo, hi], largest first
         int cnt = 0;
-        for (int p = (n + hi - 1) / hi; p <= n && cnt < cap; ++p) {
-            const int v = (n + p - 1) / p;
-            if (v < lo && cnt) break;
-            if (cnt && out[cnt - 1] == v) continue;
-            out[cnt++] = v;
+        for (int v = std::min(n, hi); v >= 1 && (v >= lo || !cnt); --v) {
+            const int p = (n + v - 1) / v;
+            if ((n + p - 1) / p == v) out[cnt++] = v;
         }
         return cnt;
     };
-    int xs[6], ys[8], zs[6];
-    const int nxs = parts(g.W, 4, 32, xs, 6), nys = parts(g.H, 1, 8, ys, 8), nzs = parts(g.D, 1, 8, zs, 6);
-    for (int a = 0; a < nxs; ++a)
+    int xs[32], ys[8], zs[8];
+    const int nxs = parts(g.W, 4, 32, xs), nys = parts(g.H, 1, 8, ys), nzs = parts(g.D, 1, 8, zs);
+    // The largest splits, and beyond 256 channels, of which LDS holds small boxes only, all of them
+    // (us, gathered, on boxes of the largest splits and of all: 128^3 320 -> 64 18800, none and 6170,
+    // 64^3 448 -> 64 3290, none and 1750, 384 -> 128 5040, 5700 and 2400).
+    const bool all = cin > 256;
+    for (int a = 0; a < (all ? nxs : std::min(nxs, 6)); ++a)
         for (int b = 0; b < nys; ++b)
-            for (int c = 0; c < nzs; ++c) {
+            for (int c = 0; c < (all ? nzs : std::min(nzs, 6)); ++c) {
                 const int tx = xs[a], ty = ys[b], tz = zs[c], tv = tx * ty * tz;
                 if (tv > 512) continue;
                 const int mt = tv > 256 ? 8 : tv > 128 ? 4 : tv > 64 ? 2 : 1;
@@ -127,7 +141,7 @@ inline bool conv_plan(const Grid3& g, int cin, int ntw, ConvPlan& best) {
                     }
                 }
             }
-    if (!found) return false;
+    if (!found || (cin > 512 && best_cost > 0.93 * gather_cycles(g, cin, ntw))) return false;
     ConvTile& t = best.t;
     const int LX = t.tx + 2, LY = t.ty + 2;
     t.nx = (g.W + t.tx - 1) / t.tx;

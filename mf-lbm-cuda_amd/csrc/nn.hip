@@ -323,8 +323,8 @@ __global__ __launch_bounds__(256) void k_conv3_box(const __bf16* __restrict__ X,
     });
 }
 
-// The convolution of planes of 2 GiB and more and of channel counts whose boxes do not fit LDS
-// (conv_plan): every tap gathered from global memory.  One wave per MT tiles of 16 voxels and the
+// The convolution of planes of 2 GiB and more and of channel counts whose boxes do not fit LDS or
+// hold too few voxels to pay (from 512 on; conv_plan): every tap gathered from global memory.  One wave per MT tiles of 16 voxels and the
 // NT 16-channel tiles blockIdx.y * NT ..: the voxel tiles share each weight load, the channel
 // tiles each voxel load.
 template <int NT, int MT>

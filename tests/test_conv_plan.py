@@ -27,10 +27,17 @@ def plan(harness, *args):
     ((256, 256, 256), 48, 16), ((256, 256, 256), 16, 48), ((256, 256, 256), 96, 32), ((256, 256, 256), 192, 64),
     ((192, 192, 192), 192, 64), ((192, 192, 192), 128, 128), ((320, 320, 320), 32, 32), ((512, 512, 512), 16, 16),
     ((800, 1000, 900), 8, 16), ((3, 5, 10000000), 8, 8), ((7, 30000000, 1), 8, 8), ((20000000, 3, 5), 8, 8),
-    ((1, 1, 1), 8, 8), ((33, 34, 35), 16, 48), ((64, 64, 64), 48, 16)])
+    ((1, 1, 1), 8, 8), ((33, 34, 35), 16, 48), ((64, 64, 64), 48, 16),
+    ((128, 128, 128), 320, 64), ((128, 128, 128), 320, 160), ((96, 96, 96), 384, 64), ((64, 64, 64), 448, 192),
+    ((32, 32, 32), 576, 64), ((20, 20, 20), 560, 128), ((8, 8, 8), 1056, 128)])
 def test_grids_have_a_box(harness, shape, cin, cout):
     rc, box = plan(harness, *shape, cin, cout)
     assert rc == 0, box
+
+
+@pytest.mark.parametrize("shape,cin,cout", [((32, 32, 32), 800, 64), ((24, 24, 24), 720, 64), ((64, 64, 64), 600, 128), ((12, 12, 12), 1056, 128), ((3, 2, 5), 1104, 8)])
+def test_deep_inputs_are_left_to_the_gathering_kernel(harness, shape, cin, cout):
+    assert plan(harness, *shape, cin, cout)[0] == 1
 
 
 def test_planes_beyond_a_descriptor_have_none(harness):

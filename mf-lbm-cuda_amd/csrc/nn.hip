@@ -383,31 +383,46 @@ __global__ __launch_bounds__(256) void k_conv3(const __bf16* __restrict__ X, con
     else ep.each(store_all);
 }
 
-// Weight gradient partials where k_conv3_wgrad_rows would hold few voxels at a time (grids
-// more than about 380 voxels wide).  Block (kt, nt, chunk): one wave per 16 x 16 tile of (output
-// channel n, k) over `chunk` voxels; writes part[chunk][n][k] (fp32).  The waves of the first k block also sum the dZ values
-// they load: the bias gradient partials bpart[chunk][n] (n < cout; null: not wanted).
+// Weight gradient partials where k_conv3_wgrad_rows cannot address its operands (2 GiB and more) or
+// would hold few voxels at a time (grids more than about 380 voxels wide).  Block (kt, nt, chunk): one wave per 16 x 16·KT block of (output channel
+// n, k) over `chunk` voxels, as KT 16 x 16 MFMA tiles that share the dZ operand; writes
+// part[chunk][n][k] (fp32).  The waves of the first k block also sum the dZ values they load: the
+// bias gradient partials bpart[chunk][n] (n < cout; null: not wanted).
 // Per step of 32 voxels the operands are staged through LDS: lane (v, h) loads 8 channels
-// (16 bytes) of voxel v -- dZ channels n0 + 8h .., and the 8 columns k0 + 8h .. (8 consecutive channels of one tap, since cin is a multiple of 8) at the
+// (16 bytes) of voxel v -- dZ channels n0 + 8h .., and of each tile the 8 columns
+// k0 + 16t + 8h .. (8 consecutive channels of one tap, since cin is a multiple of 8) at the
 // tap's shifted voxel -- and lane (r, q) then reads column r of voxels 8q .. 8q + 7, the
 // MFMA operand layout.
+template <int KT>
 __global__ __launch_bounds__(64) void k_conv3_wgrad(const __bf16* __restrict__ X, const __bf16* __restrict__ dZ,
                                                     Grid3 g, int cin, int kp, int coutp, int cout, int chunk,
                                                     float* __restrict__ part, float* __restrict__ bpart) {
-    __shared__ __attribute__((aligned(16))) __bf16 sA[32][16], sB[32][16];
+    __shared__ __attribute__((aligned(16))) __bf16 sA[32][16];
+    __shared__ __attribute__((aligned(16))) __bf16 sB[KT][32][16];
     const int M = g.D * g.H * g.W;
     const int lane = threadIdx.x;
-    const int k0 = blockIdx.x * 16, n0 = blockIdx.y * 16, c = blockIdx.z;
+    const int k0 = blockIdx.x * 16 * KT, n0 = blockIdx.y * 16, c = blockIdx.z;
     const int r = lane & 15, q = lane >> 4;  // MFMA role: column r, voxels 8q .. 8q + 7
     const int v = lane >> 1, h = lane & 1;   // loader role: voxel v, 8-channel half h
+    const int K = 27 * cin;
     const int n = n0 + r;
     const bool ain = n0 + 8 * h < cout;  // cout is a multiple of 8: the whole half or none
-    const int kk = k0 + 8 * h;
-    const bool lkin = kk < 27 * cin;  // a multiple of 8: the whole half or none
-    const int tap = lkin ? kk / cin : 0, lci = lkin ? kk - tap * cin : 0;
-    const int lox = tap % 3 - 1, loy = (tap / 3) % 3 - 1, loz = tap / 9 - 1;
-    const int loff = (loz * g.H + loy) * g.W + lox;
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    int lci[KT], lox[KT], loy[KT], loz[KT], loff[KT];
+    bool lkin[KT];
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+        const int kk = k0 + 16 * t + 8 * h;
+        lkin[t] = kk < K;  // K is a multiple of 8: the whole half or none
+        const int tap = lkin[t] ? kk / cin : 0;
+        lci[t] = lkin[t] ? kk - tap * cin : 0;
+        lox[t] = tap % 3 - 1;
+        loy[t] = (tap / 3) % 3 - 1;
+        loz[t] = tap / 9 - 1;
+        loff[t] = (loz[t] * g.H + loy[t]) * g.W + lox[t];
+    }
+    f32x4 acc[KT];
+#pragma unroll
+    for (int t = 0; t < KT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     float bsum = 0.f;  // this lane's dZ values (row n), in voxel order
     const int mb = c * chunk, me = min(M, mb + chunk);
     bf16x8 zero;
@@ -415,25 +430,32 @@ __global__ __launch_bounds__(64) void k_conv3_wgrad(const __bf16* __restrict__ X
     for (int j = 0; j < 8; ++j) zero[j] = (__bf16)0.f;
     for (int ms = mb; ms < me; ms += 32) {
         const int m = ms + v;
-        bf16x8 la = zero, lb = zero;
+        bf16x8 la = zero;
         if (m < me && ain) la = *reinterpret_cast<const bf16x8*>(dZ + (int64_t)m * cout + n0 + 8 * h);
         *reinterpret_cast<bf16x8*>(&sA[v][8 * h]) = la;
-        const int xx = m % g.W + lox, yy = (m / g.W) % g.H + loy, zz = m / (g.W * g.H) + loz;
-        const bool in = m < me && lkin && xx >= 0 && yy >= 0 && zz >= 0 && xx < g.W && yy < g.H && zz < g.D;
-        if (in) lb = *reinterpret_cast<const bf16x8*>(X + (int64_t)(m + loff) * cin + lci);
-        *reinterpret_cast<bf16x8*>(&sB[v][8 * h]) = lb;
+        const int x = m % g.W, y = (m / g.W) % g.H, z = m / (g.W * g.H);
+#pragma unroll
+        for (int t = 0; t < KT; ++t) {
+            const int xx = x + lox[t], yy = y + loy[t], zz = z + loz[t];
+            const bool in = m < me && lkin[t] && xx >= 0 && yy >= 0 && zz >= 0 && xx < g.W && yy < g.H && zz < g.D;
+            bf16x8 lb = zero;
+            if (in) lb = *reinterpret_cast<const bf16x8*>(X + (int64_t)(m + loff[t]) * cin + lci[t]);
+            *reinterpret_cast<bf16x8*>(&sB[t][v][8 * h]) = lb;
+        }
         __syncthreads();
-        bf16x8 a, b;
+        bf16x8 a, b[KT];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             a[j] = sA[8 * q + j][r];
-            b[j] = sB[8 * q + j][r];
+#pragma unroll
+            for (int t = 0; t < KT; ++t) b[t][j] = sB[t][8 * q + j][r];
         }
         if (bpart && k0 == 0) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) bsum += bf2f(a[j]);
         }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < KT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[t], acc[t], 0, 0, 0);
         __syncthreads();
     }
     if (bpart && k0 == 0) {
@@ -442,9 +464,11 @@ __global__ __launch_bounds__(64) void k_conv3_wgrad(const __bf16* __restrict__ X
         const float s2 = s1 + __shfl_xor(s1, 32);
         if (q == 0 && n < cout) bpart[(int64_t)c * cout + n] = s2;
     }
-    // D[row = n0 + 4q + j][col = k0 + r]
+    // tile t: D[row = n0 + 4q + j][col = k0 + 16t + r]
 #pragma unroll
-    for (int j = 0; j < 4; ++j) part[((int64_t)c * coutp + n0 + 4 * q + j) * kp + k0 + r] = acc[j];
+    for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[((int64_t)c * coutp + n0 + 4 * q + j) * kp + k0 + 16 * t + r] = acc[t][j];
 }
 
 // Weight gradient partials with the operands shared through LDS.  A workgroup owns one chunk of
@@ -1104,6 +1128,9 @@ bool wgrad_args_ok(const void* x, const void* dz, int32_t D, int32_t H, int32_t 
     return (uintptr_t)x % 16 == 0 && (uintptr_t)dz % 16 == 0;  // 16-byte operand loads
 }
 
+// Waves of k_conv3_wgrad with one tile each.
+inline int64_t wgrad_waves(int kp, int coutp, int nchunk) { return (int64_t)(kp / 16) * (coutp / 16) * nchunk; }
+
 // Launches k_conv3_wgrad_rows over all chunks; false where its rows do not fit LDS.
 bool wgrad_rows(const __bf16* X, const __bf16* dZ, const Grid3& g, int cin, int kp, int coutp, int cout, int chunk,
                 int nchunk, float* part, float* bpart, hipStream_t s) {
@@ -1177,8 +1204,16 @@ int wgrad_launch(const void* x, const void* dz, int32_t D, int32_t H, int32_t W,
     const int64_t n = (int64_t)coutp * kp;
     float* bpart = db ? work + nchunk * n : nullptr;
     const __bf16 *X = (const __bf16*)x, *dZ = (const __bf16*)dz;
-    if (!wgrad_rows(X, dZ, g, cin, kp, coutp, cout, chunk, nchunk, work, bpart, s))
-        k_conv3_wgrad<<<dim3(kp / 16, coutp / 16, nchunk), 64, 0, s>>>(X, dZ, g, cin, kp, coutp, cout, chunk, work, bpart);
+    if (!wgrad_rows(X, dZ, g, cin, kp, coutp, cout, chunk, nchunk, work, bpart, s)) {
+        // Two k tiles per wave halve the dZ loads, one keeps twice the waves: the second wins where the
+        // grid of single tiles has fewer than 3072 waves (three per SIMD) and on up to 16 channels on both
+        // sides (us, one and two: 8 x 64 x 512 16 -> 16 75 and 87, 48 -> 16 200 and 131, 1 x 38 x 623 16
+        // -> 144 42 and 36, 256^3 64 -> 64 58300 and 46300).  kp is a multiple of 32.
+        if (std::max(cin, cout) > 16 && wgrad_waves(kp, coutp, nchunk) >= 3072)
+            k_conv3_wgrad<2><<<dim3(kp / 32, coutp / 16, nchunk), 64, 0, s>>>(X, dZ, g, cin, kp, coutp, cout, chunk, work, bpart);
+        else
+            k_conv3_wgrad<1><<<dim3(kp / 16, coutp / 16, nchunk), 64, 0, s>>>(X, dZ, g, cin, kp, coutp, cout, chunk, work, bpart);
+    }
     const unsigned sblocks = nblk(n, 32) + (db ? nblk(cout, 32) : 0);
     const unsigned fblocks = flip.Wt ? nblk((int64_t)flip.cinp * flip.kp2) : 0;
     k_sum_chunks<<<sblocks + fblocks, 256, 0, s>>>(work, nchunk, n, bpart, db ? cout : 0, accumulate, dw, db, sblocks, flip);

@@ -384,7 +384,7 @@ __global__ __launch_bounds__(256) void k_conv3(const __bf16* __restrict__ X, con
 }
 
 // Weight gradient partials where k_conv3_wgrad_rows cannot address its operands (2 GiB and more) or
-// would hold few voxels at a time (grids more than about 380 voxels wide).  Block (kt, nt, chunk): one wave per 16 x 16·KT block of (output channel
+// does not pay (rows_pay).  Block (kt, nt, chunk): one wave per 16 x 16·KT block of (output channel
 // n, k) over `chunk` voxels, as KT 16 x 16 MFMA tiles that share the dZ operand; writes
 // part[chunk][n][k] (fp32).  The waves of the first k block also sum the dZ values they load: the
 // bias gradient partials bpart[chunk][n] (n < cout; null: not wanted).
@@ -1131,9 +1131,28 @@ bool wgrad_args_ok(const void* x, const void* dz, int32_t D, int32_t H, int32_t 
 // Waves of k_conv3_wgrad with one tile each.
 inline int64_t wgrad_waves(int kp, int coutp, int nchunk) { return (int64_t)(kp / 16) * (coutp / 16) * nchunk; }
 
-// Launches k_conv3_wgrad_rows over all chunks; false where its rows do not fit LDS.
+// Whether the rows kernel is the faster one.  It loads at least three rows for the voxels that it
+// stages, and LDS holds fewer voxels of wider rows (512 of 90, 256 of 200, 128 beyond), so that wide
+// grids lose on it, the sooner the fewer voxels share its start: us of 12 x 12 rows 32 -> 32, with it
+// and with k_conv3_wgrad, 204 wide 21 and 25, 280 32.1 and 31.8, 360 44 and 34; of 8 x 64 rows 340 wide
+// 0.93 of the time, 360 1.19; of 16 x 200 rows 360 wide level.  Inputs of one slice of channels keep
+// it longer.  A count of channels with 8 over takes it two launches: 24 -> 24 on 165 voxels 11 and 7.5,
+// 72 -> 128 on 2544 18.7 and 24.5.  On fewer than 128 voxels its 16-channel slices are the longer chain:
+// 192 -> 40 on 6 voxels 8.8 and 7.1.
+bool rows_pay(const Grid3& g, int cin, int waves) {
+    const int64_t M = (int64_t)g.D * g.H * g.W;
+    const bool two = cin > 16 && cin % 16;  // launches
+    if (M < 128 && waves >= 500) return false;
+    if (two && waves < (g.W >= 128 ? 2000 : 1200)) return false;
+    if (cin == 8) return M < 65536 || g.W <= 512;
+    if (M < 65536) return g.W <= (two ? 212 : cin == 16 ? 340 : 270);
+    return M >= 1 << 19 || cin == 16 || g.W <= (two ? 230 : 340);
+}
+
+// Launches k_conv3_wgrad_rows over all chunks; false where its rows do not fit LDS or do not pay.
 bool wgrad_rows(const __bf16* X, const __bf16* dZ, const Grid3& g, int cin, int kp, int coutp, int cout, int chunk,
                 int nchunk, float* part, float* bpart, hipStream_t s) {
+    if (!rows_pay(g, cin, (int)std::min<int64_t>(wgrad_waves(kp, coutp, nchunk), 1 << 20))) return false;
     const int full = cin / 16, ntiles = coutp / 16;
     auto launch = [&](bool half) {
         const int64_t vb = half ? 16 : 32, WP = g.W + 2, WH = (int64_t)g.W * g.H;

@@ -3,7 +3,7 @@ below 2^24, exact in bfloat16 operands and float32 sums whatever their order, so
 the exact one.  The shapes take every form of the two kernels: rows with one and two groups of
 waves, whole and half slices of channels, chunks of several stages within a plane and across planes,
 inputs above 16 MB (a chunk's workgroups on one XCD), and the gathering kernel with one and two
-tiles to a wave."""
+tiles to a wave, on both sides of each rule that chooses between them."""
 import numpy as np
 import pytest
 
@@ -41,9 +41,15 @@ def test_stages(shape, cin, cout, chunk):
     check(shape, cin, cout, chunk)
 
 
+# the last width of each rule and the first beyond it, for one slice, several, and a half slice; few
+# waves and many of a half slice; few voxels with a short and a long chain of slices
 @pytest.mark.parametrize("shape,cin,cout,chunk", [
-    ((4, 5, 421), 48, 24, 96), ((4, 15, 421), 16, 16, 96), ((2, 3, 600), 24, 24, 512), ((3, 40, 430), 40, 72, 96)])
-def test_wide_grids(shape, cin, cout, chunk):
+    ((3, 5, 340), 16, 16, 96), ((3, 5, 341), 16, 16, 96), ((3, 4, 270), 32, 16, 96), ((3, 4, 271), 32, 16, 96),
+    ((4, 6, 212), 24, 40, 96), ((4, 6, 213), 24, 40, 96), ((5, 40, 340), 32, 16, 2048), ((5, 40, 341), 32, 16, 2048),
+    ((4, 75, 230), 24, 40, 512), ((4, 75, 231), 24, 40, 512), ((4, 40, 512), 8, 16, 2048), ((4, 40, 513), 8, 16, 2048),
+    ((4, 5, 421), 48, 24, 96), ((4, 15, 421), 16, 16, 96), ((7, 8, 9), 24, 24, 512), ((17, 18, 19), 72, 72, 512),
+    ((1, 2, 3), 192, 40, 512), ((1, 3, 5), 16, 32, 512), ((2, 3, 600), 24, 24, 512), ((3, 40, 430), 40, 72, 96)])
+def test_both_sides_of_the_rules(shape, cin, cout, chunk):
     check(shape, cin, cout, chunk)
 
 

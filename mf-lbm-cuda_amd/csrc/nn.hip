@@ -1037,8 +1037,8 @@ int conv_launch(const __bf16* X, const __bf16* Wb, const float* bias, const __bf
     const bool quad = cout % 4 == 0 && (uintptr_t)bias % 16 == 0 && (uintptr_t)gate % 8 == 0 && (uintptr_t)yb % 8 == 0 &&
                      (uintptr_t)yf % 16 == 0;
     const Epilogue ep{bias, gate, yb, yf, cout, relu, quad};
-    ConvPlan p;
-    if (!conv_plan(g, cin, ntw, p)) {
+    const ConvPlan* const plan = kept_plan(g, cin, ntw);
+    if (!plan) {
         const int64_t M = (int64_t)g.D * g.H * g.W;
         // grids of 65536 voxels and more with one or two channel tiles: two voxel tiles per wave, but not
         // one channel tile of deep inputs beyond the caches (us, one voxel tile and two: 128^3 48 -> 16
@@ -1061,6 +1061,7 @@ int conv_launch(const __bf16* X, const __bf16* Wb, const float* bias, const __bf
         }
         return hipGetLastError() == hipSuccess ? 0 : -2;
     }
+    const ConvPlan& p = *plan;
     const dim3 grid(p.boxes, (ntw + p.nt - 1) / p.nt);
     switch (10 * p.mt + p.nt) {
 #define MFNN_BOX(m, n, pf) \

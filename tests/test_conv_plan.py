@@ -44,3 +44,8 @@ def test_planes_beyond_a_descriptor_have_none(harness):
     """2 GiB and more a plane: the gathering kernel's"""
     assert plan(harness, 2, 8192, 8192, 16, 16)[0] == 1
     assert plan(harness, 2, 8192, 8192, 8, 16)[0] == 0
+
+
+def test_kept_plans(harness):
+    """a size is searched for once while it keeps its place, and gets the plan of a search"""
+    assert subprocess.run([harness, "kept"], timeout=60).returncode == 0

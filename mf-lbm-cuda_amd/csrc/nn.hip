@@ -833,25 +833,42 @@ struct Channels {
     __device__ __forceinline__ void store(__bf16* p, int64_t unit) const { *reinterpret_cast<vec*>(p + unit * V) = v; }
 };
 
-// The D x H rows of the output, a workgroup each (and again beyond the launch), their units
-// walked by its threads: f(plane, row of the plane, row, voxel x, unit of the voxel).
-template <class Fn>
-__device__ __forceinline__ void each_row(int D, int H, int W, FastDiv cu, Fn&& f) {
+// How the rows of an output are walked: a workgroup to a row; `segs` workgroups to a row; a
+// workgroup to the rows that its threads hold at 1 << lanes threads each.
+enum class Rows { WHOLE, CUT, SHARED };
+struct RowSplit {
+    int segs, lanes;
+};
+
+// The D x H rows of the output (and again beyond the launch), their units walked by the threads:
+// f(plane, row of the plane, row, voxel x, unit of the voxel).  The row is uniform but for SHARED.
+template <Rows MODE, class Fn>
+__device__ __forceinline__ void each_row(int D, int H, int W, FastDiv cu, RowSplit sp, Fn&& f) {
     const int n = W * (int)cu.d;
-    for (int row = blockIdx.x; row < D * H; row += gridDim.x) {
+    auto walk = [&](int row, unsigned first, unsigned step) {
         const int z = row / H, y = row - z * H;
-        for (int e = threadIdx.x; e < n; e += blockDim.x) {
-            const int x = cu.mul | cu.one ? quot(e, cu) : (int)((uint32_t)e / cu.d);
-            f(z, y, row, x, e - x * (int)cu.d);
+        for (unsigned e = first; e < (unsigned)n; e += step) {
+            const int x = cu.mul | cu.one ? quot((int)e, cu) : (int)(e / cu.d);
+            f(z, y, row, x, (int)(e - x * cu.d));
         }
+    };
+    if (MODE == Rows::WHOLE) {
+        for (int row = blockIdx.x; row < D * H; row += gridDim.x) walk(row, threadIdx.x, blockDim.x);
+    } else if (MODE == Rows::CUT) {  // few rows, all of them in the launch
+        const int row = blockIdx.x / sp.segs, seg = blockIdx.x - row * sp.segs;
+        walk(row, seg * blockDim.x + threadIdx.x, sp.segs * blockDim.x);
+    } else {
+        const int64_t held = blockDim.x >> sp.lanes;
+        for (int64_t row = blockIdx.x * held + (threadIdx.x >> sp.lanes); row < (int64_t)D * H; row += gridDim.x * held)
+            walk((int)row, threadIdx.x & ((1u << sp.lanes) - 1), 1u << sp.lanes);
     }
 }
 
 // 2x2x2 average pool; C in units
-template <int V>
-__global__ __launch_bounds__(256) void k_pool2(const __bf16* __restrict__ x, Grid3 f, FastDiv C, __bf16* __restrict__ y) {
+template <int V, Rows MODE>
+__global__ __launch_bounds__(256) void k_pool2(const __bf16* __restrict__ x, Grid3 f, FastDiv C, RowSplit sp, __bf16* __restrict__ y) {
     const int Wc = f.W / 2, cu = (int)C.d;
-    each_row(f.D / 2, f.H / 2, Wc, C, [&](int zc, int yc, int row, int xc, int c) {
+    each_row<MODE>(f.D / 2, f.H / 2, Wc, C, sp, [&](int zc, int yc, int row, int xc, int c) {
         const int64_t fine = ((int64_t)2 * zc * f.H + 2 * yc) * f.W;
         Channels<V> in[8], out;
 #pragma unroll
@@ -871,12 +888,12 @@ __global__ __launch_bounds__(256) void k_pool2(const __bf16* __restrict__ x, Gri
 // Adjoint of the pool (dy coarse -> fine), added to the gradient of the other branch (a, null:
 // none; channels [ca0, ca0 + C) of a tensor of Ca) and passed through the ReLU of the layer
 // (gate, null: none):  out = (a + dy / 8) [gate > 0].  All channel counts in units.
-template <int V>
-__global__ __launch_bounds__(256) void k_pool2_bwd(const __bf16* __restrict__ dy, Grid3 f, FastDiv C,
+template <int V, Rows MODE>
+__global__ __launch_bounds__(256) void k_pool2_bwd(const __bf16* __restrict__ dy, Grid3 f, FastDiv C, RowSplit sp,
                                                    const __bf16* __restrict__ a, int Ca, int ca0,
                                                    const __bf16* __restrict__ gate, __bf16* __restrict__ out) {
     const int cu = (int)C.d;
-    each_row(f.D, f.H, f.W, C, [&](int z, int y, int row, int x, int c) {
+    each_row<MODE>(f.D, f.H, f.W, C, sp, [&](int z, int y, int row, int x, int c) {
         const int64_t coarse = ((int64_t)(z / 2) * (f.H / 2) + y / 2) * (f.W / 2), fine = (int64_t)row * f.W;
         const Channels<V> d = Channels<V>::load(dy, (coarse + x / 2) * cu + c);
         Channels<V> va, vg, o;
@@ -895,11 +912,11 @@ __global__ __launch_bounds__(256) void k_pool2_bwd(const __bf16* __restrict__ dy
 
 // Nearest 2x upsampling of `low` (Cl channels) and, beside it, the Cs channels of `skip`, into
 // channels [c0, c0 + Cl + Cs) of a fine tensor of Ct; C = Cl + Cs, all in units.
-template <int V>
+template <int V, Rows MODE>
 __global__ __launch_bounds__(256) void k_up2(const __bf16* __restrict__ low, int Cl, const __bf16* __restrict__ skip,
-                                             Grid3 f, FastDiv C, int Ct, int c0, __bf16* __restrict__ y) {
+                                             Grid3 f, FastDiv C, RowSplit sp, int Ct, int c0, __bf16* __restrict__ y) {
     const int Cs = (int)C.d - Cl;
-    each_row(f.D, f.H, f.W, C, [&](int z, int yy, int row, int x, int c) {
+    each_row<MODE>(f.D, f.H, f.W, C, sp, [&](int z, int yy, int row, int x, int c) {
         const int64_t coarse = ((int64_t)(z / 2) * (f.H / 2) + yy / 2) * (f.W / 2), fine = (int64_t)row * f.W;
         const bool up = c < Cl;
         const Channels<V> v = Channels<V>::load(up ? low : skip, up ? (coarse + x / 2) * Cl + c : (fine + x) * Cs + c - Cl);
@@ -909,11 +926,11 @@ __global__ __launch_bounds__(256) void k_up2(const __bf16* __restrict__ low, int
 
 // Adjoint of the upsampling: the sums over 2x2x2 voxels of channels [c0, c0 + C) of a fine tensor
 // of Ct, passed through the ReLU of the coarse layer (gate, null: none).  All counts in units.
-template <int V>
-__global__ __launch_bounds__(256) void k_up2_bwd(const __bf16* __restrict__ dy, Grid3 f, FastDiv C, int Ct, int c0,
+template <int V, Rows MODE>
+__global__ __launch_bounds__(256) void k_up2_bwd(const __bf16* __restrict__ dy, Grid3 f, FastDiv C, RowSplit sp, int Ct, int c0,
                                                  const __bf16* __restrict__ gate, __bf16* __restrict__ dx) {
     const int Wc = f.W / 2, cu = (int)C.d;
-    each_row(f.D / 2, f.H / 2, Wc, C, [&](int zc, int yc, int row, int xc, int c) {
+    each_row<MODE>(f.D / 2, f.H / 2, Wc, C, sp, [&](int zc, int yc, int row, int xc, int c) {
         const int64_t fine = ((int64_t)2 * zc * f.H + 2 * yc) * f.W;
         const int64_t at = ((int64_t)row * Wc + xc) * cu + c;
         Channels<V> in[8], vg, out;
@@ -1014,20 +1031,36 @@ inline bool aligned16(P... p) {
 }
 
 // Launch of a kernel that takes its D x H x W output in rows (each_row), C channels in units of 8
-// (wide) or 1: launch(channels per unit, workgroups, threads, units of a voxel).  A division of a
-// row's unit by the units of a voxel is exact below 2^32 (FastDiv), else left to the kernel.
+// (wide) or 1: launch(channels per unit, mode, workgroups, threads, units of a voxel, split).  A
+// workgroup to a row fills the chip where rows are many and long enough; else few long rows are cut
+// until 512 workgroups have a share (at least a unit to each thread), and many rows shorter than a
+// wave share workgroups (us a pass, a workgroup to a row and so: up of 24 channels on 2 x 6 x 1380 29.4
+// and 4.7, of 3 channels on 194 x 206 x 2 10.9 and 4.7, a launch each).  A division of a row's unit by the units
+// of a voxel is exact below 2^32 (FastDiv), else left to the kernel.
 constexpr int MAX_ROW_GROUPS = 1 << 24;  // a launch holds fewer than 2^32 threads
 template <class Fn>
 int rows_of(int64_t D, int64_t H, int64_t W, int C, bool wide, Fn&& launch) {
-    const int64_t rows = D * H, cu = wide ? C / 8 : C;
-    if (rows <= 0 || W * cu <= 0) return -2;
-    if (rows > INT32_MAX - MAX_ROW_GROUPS || W * cu > INT32_MAX - 256) return -1;
-    const int threads = (int)std::min<int64_t>(256, (W * cu + 63) / 64 * 64);
+    const int64_t rows = D * H, cu = wide ? C / 8 : C, n = W * cu;
+    if (rows <= 0 || n <= 0) return -2;
+    if (rows > INT32_MAX - MAX_ROW_GROUPS || n > INT32_MAX - 256) return -1;
     FastDiv c = fast_div((uint32_t)cu);
-    if (W * cu * cu >= (int64_t)1 << 32) c.mul = c.one = 0;
-    const int groups = (int)std::min<int64_t>(rows, MAX_ROW_GROUPS);
-    if (wide) launch(std::integral_constant<int, 8>{}, groups, threads, c);
-    else launch(std::integral_constant<int, 1>{}, groups, threads, c);
+    if (n * cu >= (int64_t)1 << 32) c.mul = c.one = 0;
+    RowSplit sp{1, 0};
+    auto with = [&](auto mode, int64_t groups, int threads) {
+        const int g = (int)std::min<int64_t>(groups, MAX_ROW_GROUPS);
+        if (wide) launch(std::integral_constant<int, 8>{}, mode, g, threads, c, sp);
+        else launch(std::integral_constant<int, 1>{}, mode, g, threads, c, sp);
+    };
+    if (n <= 64 && rows > 4096) {
+        while ((1 << sp.lanes) < n) ++sp.lanes;
+        const int64_t held = 256 >> sp.lanes;
+        with(std::integral_constant<Rows, Rows::SHARED>{}, (rows + held - 1) / held, 256);
+    } else if (rows < 512 && n > 256) {
+        sp.segs = (int)std::min<int64_t>((511 + rows) / rows, (n + 255) / 256);
+        with(std::integral_constant<Rows, Rows::CUT>{}, rows * sp.segs, 256);
+    } else {
+        with(std::integral_constant<Rows, Rows::WHOLE>{}, rows, (int)std::min<int64_t>(256, (n + 63) / 64 * 64));
+    }
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -1307,8 +1340,8 @@ int mfnn_pool2(const void* x, int32_t D, int32_t H, int32_t W, int32_t C, void* 
     if (D % 2 || H % 2 || W % 2) return -1;
     const Grid3 f{D, H, W};
     hipStream_t s = (hipStream_t)stream;
-    return rows_of(D / 2, H / 2, W / 2, C, C % 8 == 0 && aligned16(x, y), [&](auto V, int rows, int threads, FastDiv c) {
-        k_pool2<V><<<rows, threads, 0, s>>>((const __bf16*)x, f, c, (__bf16*)y);
+    return rows_of(D / 2, H / 2, W / 2, C, C % 8 == 0 && aligned16(x, y), [&](auto V, auto mode, int groups, int threads, FastDiv c, RowSplit sp) {
+        k_pool2<V, mode><<<groups, threads, 0, s>>>((const __bf16*)x, f, c, sp, (__bf16*)y);
     });
 }
 
@@ -1318,8 +1351,8 @@ int mfnn_pool2_merge(const void* dy, int32_t D, int32_t H, int32_t W, int32_t C,
     const Grid3 f{D, H, W};
     hipStream_t s = (hipStream_t)stream;
     const bool wide = C % 8 == 0 && ca % 8 == 0 && ca0 % 8 == 0 && aligned16(dy, a, gate, out);
-    return rows_of(D, H, W, C, wide, [&](auto V, int rows, int threads, FastDiv c) {
-        k_pool2_bwd<V><<<rows, threads, 0, s>>>((const __bf16*)dy, f, c, (const __bf16*)a, ca / V, ca0 / V,
+    return rows_of(D, H, W, C, wide, [&](auto V, auto mode, int groups, int threads, FastDiv c, RowSplit sp) {
+        k_pool2_bwd<V, mode><<<groups, threads, 0, s>>>((const __bf16*)dy, f, c, sp, (const __bf16*)a, ca / V, ca0 / V,
                                                 (const __bf16*)gate, (__bf16*)out);
     });
 }
@@ -1336,8 +1369,8 @@ int mfnn_up2_cat(const void* low, int32_t cl, const void* skip, int32_t cs, int3
     const Grid3 f{D, H, W};
     hipStream_t s = (hipStream_t)stream;
     const bool wide = cl % 8 == 0 && cs % 8 == 0 && ct % 8 == 0 && c0 % 8 == 0 && aligned16(low, skip, y);
-    return rows_of(D, H, W, cl + cs, wide, [&](auto V, int rows, int threads, FastDiv c) {
-        k_up2<V><<<rows, threads, 0, s>>>((const __bf16*)low, cl / V, (const __bf16*)skip, f, c, ct / V, c0 / V, (__bf16*)y);
+    return rows_of(D, H, W, cl + cs, wide, [&](auto V, auto mode, int groups, int threads, FastDiv c, RowSplit sp) {
+        k_up2<V, mode><<<groups, threads, 0, s>>>((const __bf16*)low, cl / V, (const __bf16*)skip, f, c, sp, ct / V, c0 / V, (__bf16*)y);
     });
 }
 
@@ -1347,8 +1380,8 @@ int mfnn_up2_split(const void* dy, int32_t D, int32_t H, int32_t W, int32_t C, i
     const Grid3 f{D, H, W};
     hipStream_t s = (hipStream_t)stream;
     const bool wide = C % 8 == 0 && ct % 8 == 0 && c0 % 8 == 0 && aligned16(dy, gate, dx);
-    return rows_of(D / 2, H / 2, W / 2, C, wide, [&](auto V, int rows, int threads, FastDiv c) {
-        k_up2_bwd<V><<<rows, threads, 0, s>>>((const __bf16*)dy, f, c, ct / V, c0 / V, (const __bf16*)gate, (__bf16*)dx);
+    return rows_of(D / 2, H / 2, W / 2, C, wide, [&](auto V, auto mode, int groups, int threads, FastDiv c, RowSplit sp) {
+        k_up2_bwd<V, mode><<<groups, threads, 0, s>>>((const __bf16*)dy, f, c, sp, ct / V, c0 / V, (const __bf16*)gate, (__bf16*)dx);
     });
 }
 

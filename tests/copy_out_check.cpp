@@ -1,8 +1,10 @@
 // Host harness of HostStaging (mf-lbm-cuda_amd/csrc/copy_out.h) for tests/test_copy_out_host.py:
 // the HIP calls that it makes are defined here, on host memory, so that a CPU runs it.  Built with
 // g++; argv[1] names the check, the exit status says whether it held.
+#include <atomic>
 #include <chrono>
 #include <csignal>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <set>
@@ -19,6 +21,7 @@ int made = 0;                       // hipHostMalloc calls
 int queued = 0, direct = 0;         // hipMemcpyAsync and hipMemcpy calls
 hipMemoryType kind = hipMemoryTypeUnregistered;  // of every destination
 hipError_t known = hipSuccess;
+int fail_at = 0;  // this queued copy fails
 void called() {
     std::lock_guard<std::mutex> lock(book);
     callers.insert(std::this_thread::get_id());
@@ -40,7 +43,7 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*) { call
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { called(); ++direct; std::memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
     called();
-    ++queued;
+    if (++queued == fail_at) return hipErrorUnknown;
     std::memcpy(d, s, n);
     return hipSuccess;
 }
@@ -50,9 +53,10 @@ namespace {
 using mflbm::HostStaging;
 
 std::vector<unsigned char> pattern(size_t n) {
+    std::vector<uint32_t> words(n / 4 + 1);
+    for (size_t i = 0; i < words.size(); ++i) words[i] = (uint32_t)(i + n) * 2654435761u;
     std::vector<unsigned char> v(n);
-    uint32_t x = 12345u + (uint32_t)n;
-    for (auto& b : v) b = (unsigned char)((x = x * 1664525u + 1013904223u) >> 24);
+    std::memcpy(v.data(), words.data(), n);
     return v;
 }
 
@@ -142,6 +146,39 @@ int worth() {
     many.release();
     return 0;
 }
+
+// a copy that fails at any chunk ends, says so, and leaves the slots fit for the next
+int errors() {
+    HostStaging h;
+    const size_t n = 20 * HostStaging::SLOT + 77;
+    if (!copies(h, n)) return 1;
+    const auto src = pattern(n);
+    std::vector<unsigned char> dst(n);
+    for (int k = 1; k <= 21; ++k) {
+        queued = 0;
+        fail_at = k;
+        if (h.copy(dst.data(), src.data(), n, nullptr) != hipErrorUnknown) return 1;
+        fail_at = 0;
+        if (!copies(h, n)) return 1;
+    }
+    h.release();
+    return 0;
+}
+
+// several threads, each on its own handle's slots or sharing one's
+int threads() {
+    HostStaging one, two;
+    std::atomic<int> good{0};
+    std::vector<std::thread> t;
+    for (int k = 0; k < 4; ++k)
+        t.emplace_back([&, k] {
+            for (int r = 0; r < 3; ++r) good += copies(k < 3 ? one : two, (13 + k) * HostStaging::SLOT + r);
+        });
+    for (auto& x : t) x.join();
+    one.release();
+    two.release();
+    return good == 12 ? 0 : 1;
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -152,6 +189,8 @@ int main(int argc, char** argv) {
     if (what == "contents") return contents();
     if (what == "order") return order();
     if (what == "calls") return calls();
+    if (what == "errors") return errors();
+    if (what == "threads") return threads();
     if (what == "worth") return worth();
     if (what == "destinations") return destinations();
     return 2;

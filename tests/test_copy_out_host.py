@@ -1,7 +1,7 @@
 """The staged copies to the host (HostStaging in mf-lbm-cuda_amd/csrc/copy_out.h) with the HIP calls
 replaced by host ones, on the CPU: contents at the sizes where chunks and slots change, the order
-of its locks, the thread that makes the HIP calls, the destinations that need no staging, and the
-copy that makes the slots."""
+of its locks, the thread that makes the HIP calls, the destinations that need no staging, the copy
+that makes the slots, errors, and copies from several threads."""
 import os
 import subprocess
 
@@ -19,7 +19,7 @@ def harness(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["contents", "order", "calls", "destinations", "worth"])
+@pytest.mark.parametrize("check", ["contents", "order", "calls", "destinations", "worth", "errors", "threads"])
 def test_staged_copy(harness, check):
     """exit status 1: it did not hold, 3: it did not end"""
     assert subprocess.run([harness, check], timeout=60).returncode == 0

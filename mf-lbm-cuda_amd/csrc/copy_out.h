@@ -22,10 +22,10 @@
 
 namespace mflbm {
 
-// Pinned slots of one handle: made once its large copies are worth them, given back with it.  One copy at a
-// time, of all handles: it holds the library's lock, which callers may hold already and which the
-// slots' allocation needs (a mutex of the slots' own, taken by a copy before that lock and by a
-// caller that held it after, could deadlock two threads).
+// Pinned slots of one handle: made once its large copies are worth them, given back with it.  One
+// large copy at a time, of all handles (large_copies).  A copy never waits for the library's lock,
+// which its caller may hold and another thread's handle may be created under: where the slots are to
+// be made and another thread holds it, the copy is hipMemcpy's.
 class HostStaging {
 public:
     static constexpr size_t WORKERS = 4, SLOTS = 6;
@@ -40,8 +40,9 @@ public:
 
     // dst[0, bytes) = src[0, bytes), after the work queued on `stream`; returns when it is there
     hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t stream) {
+        std::unique_lock<std::mutex> lock;
         if (bytes >= MIN_BYTES && pageable(dst)) {
-            std::lock_guard<std::recursive_mutex> lock(device_lock());
+            lock = std::unique_lock<std::mutex>(large_copies());
             copied_ = copied_ < WORTH_BYTES ? copied_ + bytes : copied_;
             if (copied_ >= WORTH_BYTES && make()) return staged(static_cast<char*>(dst), static_cast<const char*>(src), bytes, stream);
         }
@@ -68,8 +69,15 @@ private:
         return true;
     }
 
-    bool make() {  // under device_lock
+    static std::mutex& large_copies() {
+        static std::mutex m;
+        return m;
+    }
+
+    bool make() {  // under large_copies
         if (ring_) return true;
+        std::unique_lock<std::recursive_mutex> lock(device_lock(), std::try_to_lock);
+        if (!lock) return false;
         void* p = nullptr;
         bool ok = hipHostMalloc(&p, SLOTS * SLOT, hipHostMallocDefault) == hipSuccess;
         ring_ = ok ? static_cast<char*>(p) : nullptr;

@@ -165,6 +165,28 @@ int errors() {
     return 0;
 }
 
+// a copy does not wait for a thread that holds the library's lock (a handle that is being created)
+int waits() {
+    HostStaging h;
+    std::atomic<bool> done{false}, ok{false};
+    std::thread other;
+    bool early = false;
+    {
+        std::lock_guard<std::recursive_mutex> lock(mflbm::device_lock());
+        other = std::thread([&] {
+            ok = copies(h, 25 * HostStaging::SLOT);
+            done = true;
+        });
+        for (int t = 0; t < 100 && !early; ++t) {
+            std::this_thread::sleep_for(std::chrono::milliseconds(100));
+            early = done;
+        }
+    }
+    other.join();
+    h.release();
+    return early && ok ? 0 : 1;
+}
+
 // several threads, each on its own handle's slots or sharing one's
 int threads() {
     HostStaging one, two;
@@ -190,6 +212,7 @@ int main(int argc, char** argv) {
     if (what == "order") return order();
     if (what == "calls") return calls();
     if (what == "errors") return errors();
+    if (what == "waits") return waits();
     if (what == "threads") return threads();
     if (what == "worth") return worth();
     if (what == "destinations") return destinations();

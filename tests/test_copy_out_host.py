@@ -19,7 +19,7 @@ def harness(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["contents", "order", "calls", "destinations", "worth", "errors", "threads"])
+@pytest.mark.parametrize("check", ["contents", "order", "calls", "destinations", "worth", "errors", "threads", "waits"])
 def test_staged_copy(harness, check):
     """exit status 1: it did not hold, 3: it did not end"""
     assert subprocess.run([harness, check], timeout=60).returncode == 0

@@ -3,10 +3,14 @@
 //
 // Step sequence per time step (src/main_iteration_GPU.cu:1890-2055):
 //   collide (odd/even)  ->  periodic copies  ->  Zou-He in/outlet  ->  gradient chain
-// The gradient chain (phi extrapolation, normals + wetting, normal extrapolation,
-// curvature) runs as one fused tiled kernel that writes only the force records the next
+// By default that is three launches: the collision, which also writes the ghost phi of the
+// periodic and open boundaries, and the two kernels of the gradient chain on boxes (phi
+// extrapolation, normals + wetting; normal extrapolation, curvature), the second with the
+// boundary updates of the populations.  The chain writes only the force records the next
 // collision reads; the split kernels (one per reference kernel) fill the dense gradient
-// fields when they are downloaded, or run every step with MFLBM_FLAG_SPLIT_GRADIENT.
+// fields when they are downloaded, or run every step with MFLBM_FLAG_SPLIT_GRADIENT.  Periodic
+// axes of fewer than 8 nodes, the split kernels and the one-pass march (MFLBM_GRAD_SHAPE) have
+// the boundary updates in a launch of their own.
 // The reference synchronises the device after every launch; here all launches of a step
 // are stream-ordered and replayed from a captured graph.
 #include <hip/hip_runtime.h>

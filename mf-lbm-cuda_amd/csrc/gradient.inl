@@ -44,7 +44,7 @@ __device__ __forceinline__ float keep_if(bool f, float v) { return __int_as_floa
 
 // Four values of one node side by side, so that one vector access moves all four (16 B in
 // FP32, 32 B in FP64) and a row of nodes is one contiguous run: the two-pass chain's
-// (cn_x, cn_y, cn_z, c_norm) and its solid normals (snx, sny, snz, 0) of wetting nodes.
+// (cn_x, cn_y, cn_z, c_norm).
 template <typename T>
 struct alignas(4 * sizeof(T)) Vec4 {
     T x, y, z, w;
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(GRAD_THREADS) void k_gradient(GradArgs<T> A, StepCo
                 if (i < n) {
                     const int v = list[i], e = pos(v);
                     if (v & (1 << 14)) {
-                        // three scalar loads: the 4-vector copy measured no faster here (FP64)
+                        // three scalar loads: a copy as 4-vectors measured no faster here (FP64)
                         const int c = i4(d, ib + e % WX, jb + e / WX, q);
                         wn[m][0] = A.snx[c]; wn[m][1] = A.sny[c]; wn[m][2] = A.snz[c];
                     }
